@@ -31,6 +31,13 @@ extern "C" {
 #define ZBALHIP_LAYOUT_MAX_BLOCKS 50 /* scratch rows, reference dispatch_layout.h:33 (MAX_BLOCK) */
 
 /*
+ * OR-ed into quant_mode of zbalhip_dispatch_normal and zbalhip_dispatch_low_latency, mode of
+ * zbalhip_fused_permute_quant and base_is_inclusive of zbalhip_combine: the expert ids are an int64 array of which the
+ * low words count (what converting it to int32 would leave).
+ */
+#define ZBALHIP_IDS_ARE_I64 0x400
+
+/*
  * Router (no reference counterpart). logits [T,E] fp32 -> topk_idx [T,K]
  * int64 (idx_is_i64 != 0, the type the layout operator takes) or int32 (the
  * type the dispatch and fused operators take), topk_w [T,K] fp32.
@@ -51,19 +58,18 @@ ZBALHIP_API int32_t zbalhip_dispatch_layout(const void *topk_idx, int32_t idx_is
                                 int32_t *send_token_idx, int32_t *scratch, void *stream);
 
 /*
- * zbalhip_dispatch_layout for callers that cannot allocate device memory
- * (code under HIP graph capture, serving loops and harnesses that forbid
- * hipMalloc). No counterpart in the reference. Same arguments, outputs and
- * results as zbalhip_dispatch_layout, minus `scratch`: the per-block
- * histograms live in a file-scope device array of the library
- * (ZBALHIP_LAYOUT_MAX_BLOCKS * ZBALHIP_LAYOUT_STATIC_MAX_EXPERTS int32 =
- * 200 KiB on every GPU the library runs on, held until the process ends).
- * The call allocates and frees nothing. experts above
- * ZBALHIP_LAYOUT_STATIC_MAX_EXPERTS is refused with -2 and a last-error text.
- * All calls on one GPU share that array: calls that overlap on one GPU
- * (different streams, different threads) race; order them on one stream.
- * The first call on a GPU looks up the array's device address
- * (hipGetSymbolAddress): make it before a graph capture starts.
+ * zbalhip_dispatch_layout without `scratch` (which it takes for the reference's sake and does not touch), plus
+ * token_in_rank [T, ranks] i32: 1 where the token picks an expert of the rank, else 0 (may be null).
+ */
+ZBALHIP_API int32_t zbalhip_dispatch_layout_in_rank(const void *topk_idx, int32_t idx_is_i64, int64_t tokens, int64_t experts,
+                                        int64_t topk, int32_t ranks, int32_t *tokens_per_rank,
+                                        int32_t *tokens_per_expert, int32_t *send_token_idx, int32_t *token_in_rank,
+                                        void *stream);
+
+/*
+ * zbalhip_dispatch_layout for callers that cannot allocate device memory (code under HIP graph capture, serving loops
+ * and harnesses that forbid hipMalloc): no `scratch`, nothing allocated, no state between calls. No counterpart in the
+ * reference. experts above ZBALHIP_LAYOUT_STATIC_MAX_EXPERTS is refused with -2 and a last-error text.
  */
 #define ZBALHIP_LAYOUT_STATIC_MAX_EXPERTS 1024
 ZBALHIP_API int32_t zbalhip_dispatch_layout_static(const void *topk_idx, int32_t idx_is_i64, int64_t tokens, int64_t experts,
@@ -88,6 +94,18 @@ ZBALHIP_API int32_t zbalhip_dispatch_notify(const int32_t *const *tokens_per_exp
                                 int64_t experts, int64_t topk, int32_t *recv_data, int32_t *put_offset,
                                 int32_t *total_recv, int64_t *recv_tokens_per_expert, int32_t *balance_matrix,
                                 void *stream);
+
+/*
+ * zbalhip_dispatch_notify for a caller that needs the received counts on the host: returns when `host_counts`
+ * [experts / ranks] (host memory) holds them. `block` is from zbalhip_host_counts_alloc (a few KiB of pinned memory
+ * that the kernel writes directly); one call at a time per block. Refused while the stream is being captured.
+ */
+ZBALHIP_API int32_t zbalhip_dispatch_notify_counts(const int32_t *const *tokens_per_expert, int32_t ranks, int32_t my_rank,
+                                       int64_t experts, int64_t topk, int32_t *recv_data, int32_t *put_offset,
+                                       int32_t *total_recv, int64_t *recv_tokens_per_expert, int32_t *balance_matrix,
+                                       void *block, int64_t *host_counts, void *stream);
+ZBALHIP_API int32_t zbalhip_host_counts_alloc(void **block);
+ZBALHIP_API int32_t zbalhip_host_counts_free(void *block);
 
 /*
  * Replaces ZBALOpDispatchNormal (zbal_npu_operators.h:58-62; kernel

@@ -173,6 +173,29 @@ uint64_t zbal_fused_deep_moe_workspace_size(int64_t tokens, int64_t hidden, int6
                                             int64_t gmm1HLen, int64_t shareGmm1HLen, int64_t quantMode);
 
 /*
+ * extension: zbal_dispatch_normal_layout without its scratch operand, and with tokenInRank [T, ranks] int32: 1 where
+ * the token picks an expert of the rank, else 0.
+ */
+int32_t zbal_dispatch_normal_layout_in_rank(const zbal_tensor_info_t *topkIndex, int64_t tokens, int64_t expertNum,
+                                            int64_t topkNum, const zbal_tensor_info_t *tokensPerRank,
+                                            const zbal_tensor_info_t *tokensPerExpert,
+                                            const zbal_tensor_info_t *sendTokensIndex,
+                                            const zbal_tensor_info_t *tokenInRank, zbal_comm_t comm, aclrtStream stream,
+                                            int64_t flags);
+
+/*
+ * extension: zbal_dispatch_normal_notify for a caller that sizes its receive tensors from the counts: returns when
+ * hostCounts [E / ranks] (host memory) holds this rank's recvTokensPerExpert.
+ */
+int32_t zbal_dispatch_normal_notify_counts(const zbal_tensor_info_t *sendTokensPerExpert, int64_t sendCount,
+                                           int64_t topKNum, const zbal_tensor_info_t *recvBuff,
+                                           const zbal_tensor_info_t *totalRecvTokens,
+                                           const zbal_tensor_info_t *recvTokensPerExpert,
+                                           const zbal_tensor_info_t *pushTargetOffset,
+                                           const zbal_tensor_info_t *balanceMatrix, int64_t *hostCounts,
+                                           zbal_comm_t comm, aclrtStream stream, int64_t flags);
+
+/*
  * extension: softmax + top-k router. logits [T, E] fp32 -> topkIndex [T, K]
  * (int64, the type zbal_dispatch_normal_layout takes, or int32, the type
  * the dispatch and fused operators take: the descriptor's dataType says

@@ -118,6 +118,8 @@ SIGNATURES = {
     "zbal_recv": (_i32, [_vp, ctypes.c_size_t, _i32, _u32, _vp, _vp]),
     "zbal_dispatch_normal_notify": (_i32, [_TI, _i64, _i64, _TI, _TI, _TI, _TI, _TI, _vp, _vp, _i64]),
     "zbal_dispatch_normal_layout": (_i32, [_TI, _i64, _i64, _i64, _TI, _TI, _TI, _TI, _vp, _vp, _i64]),
+    "zbal_dispatch_normal_layout_in_rank": (_i32, [_TI, _i64, _i64, _i64, _TI, _TI, _TI, _TI, _vp, _vp, _i64]),
+    "zbal_dispatch_normal_notify_counts": (_i32, [_TI, _i64, _i64, _TI, _TI, _TI, _TI, _TI, _vp, _vp, _vp, _i64]),
     "zbal_dispatch_normal": (_i32, [_TI, _TI, _TI, _TI, _TI, _i64, _i32, _TI, _TI, _vp, _vp, _i64]),
     "zbal_combine_normal": (_i32, [_TI, _TI, _TI, _TI, _TI, _TI, _u16, _TI, _vp, _vp, _i64]),
     "zbal_dispatch_low_latency": (_i32, [_TI, _TI, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _TI, _TI, _TI, _TI, _TI,
@@ -131,6 +133,10 @@ SIGNATURES = {
     "zbalhip_topk_route": (_i32, [_vp, _i64, _i64, _i64, _vp, _i32, _vp, _vp]),
     "zbalhip_dispatch_layout": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp]),
     "zbalhip_dispatch_layout_static": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp]),
+    "zbalhip_dispatch_layout_in_rank": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp]),
+    "zbalhip_dispatch_notify_counts": (_i32, [_vp, _i32, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "zbalhip_host_counts_alloc": (_i32, [ctypes.POINTER(_vp)]),
+    "zbalhip_host_counts_free": (_i32, [_vp]),
     "zbalhip_dispatch_notify": (_i32, [_vp, _i32, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp]),
     "zbalhip_dispatch_normal": (_i32, [_vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _i32, _i32, _i64,
                                        _vp]),

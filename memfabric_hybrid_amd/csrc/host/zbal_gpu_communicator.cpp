@@ -17,6 +17,7 @@
 #include <cstring>
 #include <ctime>
 #include <fstream>
+#include <mutex>
 
 #include "zbal_hip_kernels.h"
 #include "zbal_host.h"
@@ -88,6 +89,48 @@ const char *ProfName(uint64_t frame)
         default: return nullptr;
     }
 }
+
+/*
+ * The pinned blocks that notify kernels write counts for the host into: one per call in progress. A few are kept for
+ * the next calls; they go with the communicator.
+ */
+class CountsBlocks {
+public:
+    ~CountsBlocks()
+    {
+        for (void *b : kept_) zbalhip_host_counts_free(b);
+    }
+    void *Take()
+    {
+        {
+            std::lock_guard<std::mutex> guard(mutex_);
+            if (!kept_.empty()) {
+                void *b = kept_.back();
+                kept_.pop_back();
+                return b;
+            }
+        }
+        void *b = nullptr;
+        return zbalhip_host_counts_alloc(&b) == 0 ? b : nullptr;
+    }
+    /* a block whose launch failed may still be written to: it is not used again */
+    void GiveBack(void *b, bool reusable)
+    {
+        {
+            std::lock_guard<std::mutex> guard(mutex_);
+            if (reusable && kept_.size() < kMost) {
+                kept_.push_back(b);
+                return;
+            }
+        }
+        zbalhip_host_counts_free(b);
+    }
+
+private:
+    static constexpr size_t kMost = 8;
+    std::mutex mutex_;
+    std::vector<void *> kept_;
+};
 
 class GpuCommunicator final : public Communicator {
 public:
@@ -176,6 +219,7 @@ public:
 private:
     uint64_t *traceHost_ = nullptr, *traceDev_ = nullptr;
     int64_t tracePoints_ = 0;
+    CountsBlocks countsBlocks_;
 
 public:
 
@@ -223,6 +267,9 @@ public:
         }
         return Translate(op, p, bytes, out);
     }
+
+    /* expert ids may be int32 or int64: the kernels read either where it lies */
+    static int32_t IdsFlag(const zbal_tensor_info_t *ids) { return ids->dataType == ZBAL_DATA_TYPE_INT64 ? ZBALHIP_IDS_ARE_I64 : 0; }
 
     static size_t ElemSize(zbal_datatype_t dt)
     {
@@ -279,7 +326,8 @@ public:
     int32_t DispatchNormalLayout(const zbal_tensor_info_t *topkIndex, int64_t tokens, int64_t expertNum,
                                  int64_t topkNum, const zbal_tensor_info_t *tokensPerRank,
                                  const zbal_tensor_info_t *tokensPerExpert, const zbal_tensor_info_t *sendTokensIndex,
-                                 const zbal_tensor_info_t *notifySendData, aclrtStream stream, int64_t) override
+                                 const zbal_tensor_info_t *notifySendData, aclrtStream stream, int64_t,
+                                 const zbal_tensor_info_t *tokenInRank) override
     {
         const char *op = "DispatchLayout";
         const int64_t R = info_.groupSize;
@@ -289,25 +337,30 @@ public:
                              Z_INVALID_PARAM);
         ZB_CHECK(op, "tokensPerRank", tokensPerRank, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, R);
         ZB_CHECK(op, "tokensPerExpert", tokensPerExpert, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, expertNum);
-        ZB_CHECK(op, "notifySendData", notifySendData, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32,
-                 (int64_t)ZBALHIP_LAYOUT_MAX_BLOCKS * expertNum);
+        /* the reference's scratch operand; callers of the extension, which takes tokenInRank, have none */
+        if (notifySendData)
+            ZB_CHECK(op, "notifySendData", notifySendData, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32,
+                     (int64_t)ZBALHIP_LAYOUT_MAX_BLOCKS * expertNum);
         if (tokens > 0) {
             ZB_CHECK(op, "topkIndex", topkIndex, ZBAL_DATA_TYPE_INT64, ZBAL_DATA_TYPE_INT32, tokens * topkNum);
             ZB_CHECK(op, "sendTokensIndex", sendTokensIndex, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32,
                      tokens * topkNum);
+            if (tokenInRank)
+                ZB_CHECK(op, "tokenInRank", tokenInRank, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, tokens * R);
         }
-        return Launched(op, zbalhip_dispatch_layout(topkIndex->data, topkIndex->dataType == ZBAL_DATA_TYPE_INT64,
-                                                    tokens, expertNum, topkNum, (int32_t)R,
-                                                    (int32_t *)tokensPerRank->data, (int32_t *)tokensPerExpert->data,
-                                                    (int32_t *)sendTokensIndex->data, (int32_t *)notifySendData->data,
-                                                    stream));
+        return Launched(op, zbalhip_dispatch_layout_in_rank(topkIndex->data, topkIndex->dataType == ZBAL_DATA_TYPE_INT64,
+                                                            tokens, expertNum, topkNum, (int32_t)R,
+                                                            (int32_t *)tokensPerRank->data,
+                                                            (int32_t *)tokensPerExpert->data,
+                                                            (int32_t *)sendTokensIndex->data,
+                                                            tokenInRank ? (int32_t *)tokenInRank->data : nullptr, stream));
     }
 
     int32_t DispatchNormalNotify(const zbal_tensor_info_t *sendTokensPerExpert, int64_t sendCount, int64_t topKNum,
                                  const zbal_tensor_info_t *recvBuff, const zbal_tensor_info_t *totalRecvTokens,
                                  const zbal_tensor_info_t *recvTokensPerExpert,
                                  const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,
-                                 aclrtStream stream, int64_t) override
+                                 aclrtStream stream, int64_t, int64_t *hostCounts) override
     {
         const char *op = "NotifyDispatch";
         const int64_t R = info_.groupSize, me = info_.myGroupRank;
@@ -324,6 +377,17 @@ public:
         /* the counts of the other ranks are read where they lie: at the same offset in each rank's window */
         const void *counts[ZBALHIP_MAX_REDUCE_PEERS];
         if (!PeerCopies(op, sendTokensPerExpert->data, (size_t)E * 4, counts)) return Z_INVALID_PARAM;
+        if (hostCounts) {
+            void *block = countsBlocks_.Take();
+            ZBAL_VALIDATE_RETURN(block != nullptr, op << " failed as no pinned memory is left", Z_ERROR);
+            const int32_t rc = zbalhip_dispatch_notify_counts((const int32_t *const *)counts, (int32_t)R, (int32_t)me, E, topKNum,
+                                                              (int32_t *)recvBuff->data, (int32_t *)pushTargetOffset->data,
+                                                              (int32_t *)totalRecvTokens->data,
+                                                              (int64_t *)recvTokensPerExpert->data,
+                                                              (int32_t *)balanceMatrix->data, block, hostCounts, stream);
+            countsBlocks_.GiveBack(block, rc == 0);
+            return Launched(op, rc);
+        }
         return Launched(op, zbalhip_dispatch_notify((const int32_t *const *)counts, (int32_t)R, (int32_t)me, E, topKNum,
                                                     (int32_t *)recvBuff->data, (int32_t *)pushTargetOffset->data,
                                                     (int32_t *)totalRecvTokens->data,
@@ -366,7 +430,7 @@ public:
                              Z_INVALID_PARAM);
         if (T == 0) return Z_OK;
         ZB_CHECK(op, "srcTokens", srcTokens, ZBAL_DATA_TYPE_BFP16, ZBAL_DATA_TYPE_FP16, T * H);
-        ZB_CHECK(op, "topkIndex", topkIndex, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
+        ZB_CHECK(op, "topkIndex", topkIndex, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT64, T * K);
         ZB_CHECK(op, "sendTokensIndex", sendTokensIndex, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
         ZB_CHECK(op, "pushTargetOffset", pushTargetOffset, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, expertNum * R);
         int64_t scalesPerRow = 0;
@@ -394,7 +458,7 @@ public:
         return Launched(op, zbalhip_dispatch_normal(srcTokens->data, srcTokens->dataType, (const int32_t *)topkIndex->data,
                                                     (const int32_t *)sendTokensIndex->data,
                                                     (const int32_t *)pushTargetOffset->data, T, H, K, expertNum,
-                                                    (int32_t)quantMode, (void *const *)dest,
+                                                    (int32_t)quantMode | IdsFlag(topkIndex), (void *const *)dest,
                                                     scalesPerRow > 0 ? (float *const *)scale : nullptr, (int32_t)R,
                                                     (int32_t)me, destRows, stream));
     }
@@ -423,14 +487,14 @@ public:
         ZB_CHECK(op, "destTokens", destTokens, srcTokens->dataType, srcTokens->dataType, T * H);
         ZB_CHECK(op, "srcTokensPerEp", srcTokensPerEp, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, expertNum * R);
         ZB_CHECK(op, "topKWeight", topKWeight, ZBAL_DATA_TYPE_FP32, ZBAL_DATA_TYPE_FP32, T * K);
-        ZB_CHECK(op, "topkIndex", topkIndex, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
+        ZB_CHECK(op, "topkIndex", topkIndex, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT64, T * K);
         ZB_CHECK(op, "sendTokensIndex", sendTokensIndex, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
         /* the expert outputs are read from the window of the rank that owns the expert; rows past what they hold are skipped */
         const int64_t srcRows = Numel(srcTokens) / H;
         const void *src[ZBALHIP_MAX_REDUCE_PEERS];
         if (!PeerCopies(op, srcTokens->data, (size_t)srcRows * H * 2, src)) return Z_INVALID_PARAM;
         return Launched(op, zbalhip_combine(src, (int32_t)R, (int32_t)me, srcRows, srcTokens->dataType,
-                                            (const int32_t *)srcTokensPerEp->data, 0, (const float *)topKWeight->data,
+                                            (const int32_t *)srcTokensPerEp->data, IdsFlag(topkIndex), (const float *)topKWeight->data,
                                             (const int32_t *)topkIndex->data, (const int32_t *)sendTokensIndex->data, T, H, K,
                                             expertNum, destTokens->data, stream));
     }
@@ -469,7 +533,7 @@ public:
         /* an empty batch has empty per-token tensors (torch hands out a null pointer for them): only the counts are written */
         if (T > 0) {
             ZB_CHECK(op, "x", x, ZBAL_DATA_TYPE_BFP16, ZBAL_DATA_TYPE_FP16, T * H);
-            ZB_CHECK(op, "expertIds", expertIds, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
+            ZB_CHECK(op, "expertIds", expertIds, ZBAL_DATA_TYPE_INT32, R == 1 ? ZBAL_DATA_TYPE_INT64 : ZBAL_DATA_TYPE_INT32, T * K);
             ZB_CHECK(op, "expandIdxOut", expandIdxOut, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
             /* every pick may be valid, so the packed output must hold tokens * topk rows */
             if (quantMode == 0) {
@@ -507,7 +571,7 @@ public:
         int64_t blocks = Numel(putOffset) / E;
         if (blocks > ZBALHIP_LAYOUT_MAX_BLOCKS) blocks = ZBALHIP_LAYOUT_MAX_BLOCKS;
         return Launched(op, zbalhip_dispatch_low_latency(x->data, x->dataType, (const int32_t *)expertIds->data, T, H, K, E,
-                                                         (int32_t)quantMode, (int32_t)expertTokenNumsType,
+                                                         (int32_t)quantMode | IdsFlag(expertIds), (int32_t)expertTokenNumsType,
                                                          expandXOut->data, (float *)dynamicScalesOut->data,
                                                          (int32_t *)expandIdxOut->data,
                                                          (int64_t *)expertTokenNumsOut->data,
@@ -537,7 +601,7 @@ public:
         ZBAL_VALIDATE_RETURN(expandX->dataType == xOut->dataType, op << " failed as source and destination types differ",
                              Z_INVALID_PARAM);
         ZB_CHECK(op, "xOut", xOut, expandX->dataType, expandX->dataType, T * H);
-        ZB_CHECK(op, "expertIds", expertIds, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
+        ZB_CHECK(op, "expertIds", expertIds, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT64, T * K);
         ZB_CHECK(op, "expertIdx", expertIdx, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
         ZB_CHECK(op, "epSendCounts", epSendCounts, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, moeExpertNum * R);
         ZB_CHECK(op, "expertScales", expertScales, ZBAL_DATA_TYPE_FP32, ZBAL_DATA_TYPE_FP32, T * K);
@@ -546,7 +610,7 @@ public:
         const void *src[ZBALHIP_MAX_REDUCE_PEERS];
         if (!PeerCopies(op, expandX->data, (size_t)srcRows * H * 2, src)) return Z_INVALID_PARAM;
         return Launched(op, zbalhip_combine(src, (int32_t)R, (int32_t)me, srcRows, expandX->dataType,
-                                            (const int32_t *)epSendCounts->data, 1, (const float *)expertScales->data,
+                                            (const int32_t *)epSendCounts->data, 1 | IdsFlag(expertIds), (const float *)expertScales->data,
                                             (const int32_t *)expertIds->data, (const int32_t *)expertIdx->data, T, H, K,
                                             moeExpertNum, xOut->data, stream));
     }
@@ -620,7 +684,7 @@ public:
         if (T > 0) { /* an empty batch has empty per-token tensors (null data): only expertTokenNums is written */
             ZB_CHECK(op, "x", x, ZBAL_DATA_TYPE_BFP16, ZBAL_DATA_TYPE_FP16, T * H);
             ZB_CHECK(op, "output", output, x->dataType, x->dataType, T * H);
-            ZB_CHECK(op, "expertIds", expertIds, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT32, T * K);
+            ZB_CHECK(op, "expertIds", expertIds, ZBAL_DATA_TYPE_INT32, ZBAL_DATA_TYPE_INT64, T * K);
             ZB_CHECK(op, "expertScales", expertScales, ZBAL_DATA_TYPE_FP32, ZBAL_DATA_TYPE_FP32, T * K);
         } else {
             ZBAL_VALIDATE_RETURN(x->dataType == ZBAL_DATA_TYPE_BFP16 || x->dataType == ZBAL_DATA_TYPE_FP16,
@@ -709,7 +773,7 @@ public:
             if (rc != 0) return Launched(op, rc);
         }
         rc = zbalhip_fused_permute_quant(x->data, x->dataType, (const int32_t *)expertIds->data, smooth, activeMask, T, H, K, E,
-                                         qmode, q1, xs, expandIdx, (int64_t *)expertTokenNums->data, rowOff,
+                                         qmode | IdsFlag(expertIds), q1, xs, expandIdx, (int64_t *)expertTokenNums->data, rowOff,
                                          sgl ? (uint32_t *)(sgl + rows * I) : nullptr, sgl ? rows : 0, layoutScratch,
                                          ZBALHIP_LAYOUT_MAX_BLOCKS, stream);
         if (rc != 0) return Launched(op, rc);
@@ -720,7 +784,7 @@ public:
                                   x->dataType, y, stream);
         if (rc != 0) return Launched(op, rc);
         const void *ySrc[1] = {y};
-        return Launched(op, zbalhip_combine(ySrc, 1, 0, rows, x->dataType, rowOff, 0, (const float *)expertScales->data,
+        return Launched(op, zbalhip_combine(ySrc, 1, 0, rows, x->dataType, rowOff, IdsFlag(expertIds), (const float *)expertScales->data,
                                             (const int32_t *)expertIds->data, expandIdx, T, H, K, E, output->data,
                                             stream));
     }

@@ -150,14 +150,14 @@ public:
                                          const zbal_tensor_info_t *tokensPerExpert,
                                          const zbal_tensor_info_t *sendTokensIndex,
                                          const zbal_tensor_info_t *notifySendData, aclrtStream stream,
-                                         int64_t flags) = 0;
+                                         int64_t flags, const zbal_tensor_info_t *tokenInRank = nullptr) = 0;
     virtual int32_t DispatchNormalNotify(const zbal_tensor_info_t *sendTokensPerExpert, int64_t sendCount,
                                          int64_t topKNum, const zbal_tensor_info_t *recvBuff,
                                          const zbal_tensor_info_t *totalRecvTokens,
                                          const zbal_tensor_info_t *recvTokensPerExpert,
                                          const zbal_tensor_info_t *pushTargetOffset,
                                          const zbal_tensor_info_t *balanceMatrix, aclrtStream stream,
-                                         int64_t flags) = 0;
+                                         int64_t flags, int64_t *hostCounts = nullptr) = 0;
     virtual int32_t DispatchNormal(const zbal_tensor_info_t *srcTokens, const zbal_tensor_info_t *topkIndex,
                                    const zbal_tensor_info_t *sendTokensIndex,
                                    const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,

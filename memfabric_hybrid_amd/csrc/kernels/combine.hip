@@ -32,7 +32,7 @@ struct PeerSource {
 template <int DT>
 __global__ void __launch_bounds__(kThreads)
 combine_kernel(PeerSource src, const int32_t *__restrict__ base, int base_inclusive,
-               const float *__restrict__ w, const int32_t *__restrict__ topk_idx,
+               const float *__restrict__ w, ExpertIds topk_idx,
                const int32_t *__restrict__ rank_in_expert, int hidden, int topk, int experts,
                uint16_t *__restrict__ out)
 {
@@ -131,6 +131,8 @@ extern "C" int32_t zbalhip_combine(const void *const *y, int32_t ranks, int32_t 
     if (dtype != ZDT_BF16 && dtype != ZDT_FP16) return ZBALHIP_INVALID;
     if (tokens < 0 || hidden <= 0 || hidden % 8 != 0 || topk <= 0 || topk > kMaxTopk || experts <= 0)
         return ZBALHIP_INVALID;
+    const ExpertIds ids = expert_ids(topk_idx, (base_is_inclusive & ZBALHIP_IDS_ARE_I64) != 0);
+    base_is_inclusive &= ~ZBALHIP_IDS_ARE_I64;
     if (ranks <= 0 || ranks > ZBALHIP_MAX_REDUCE_PEERS || my_rank < 0 || my_rank >= ranks || experts % ranks != 0 || y_rows < 0)
         return ZBALHIP_INVALID;
     PeerSource src = {};
@@ -152,10 +154,10 @@ extern "C" int32_t zbalhip_combine(const void *const *y, int32_t ranks, int32_t 
     const dim3 grid((unsigned)tokens, (unsigned)splits);
     hipStream_t st = (hipStream_t)stream;
     if (dtype == ZDT_BF16)
-        combine_kernel<ZDT_BF16><<<grid, threads, 0, st>>>(src, base, base_is_inclusive, w, topk_idx, send_token_idx,
+        combine_kernel<ZDT_BF16><<<grid, threads, 0, st>>>(src, base, base_is_inclusive, w, ids, send_token_idx,
                                                                      (int)hidden, (int)topk, (int)experts, (uint16_t *)out);
     else
-        combine_kernel<ZDT_FP16><<<grid, threads, 0, st>>>(src, base, base_is_inclusive, w, topk_idx, send_token_idx,
+        combine_kernel<ZDT_FP16><<<grid, threads, 0, st>>>(src, base, base_is_inclusive, w, ids, send_token_idx,
                                                                      (int)hidden, (int)topk, (int)experts, (uint16_t *)out);
     return zbalhip_check_launch();
 }

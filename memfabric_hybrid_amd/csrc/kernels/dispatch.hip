@@ -12,7 +12,7 @@
 #include "zbal_device.h"
 #include "zbal_hip_kernels.h"
 
-int32_t zbalhip_layout_ranges_internal(const int32_t *idx, int64_t tokens, int64_t experts, int64_t topk,
+int32_t zbalhip_layout_ranges_internal(const ExpertIds &idx, int64_t tokens, int64_t experts, int64_t topk,
                                        const uint8_t *active_mask, int32_t *send_token_idx, int32_t *hist, int nblk,
                                        int tokens_per_block, hipStream_t st);
 
@@ -20,7 +20,7 @@ int32_t zbalhip_ll_counts_internal(const int32_t *const *ids, int ranks, int me,
                                    int64_t experts, int32_t token_nums_type, int32_t *all_counts, int32_t *ep_recv_counts,
                                    int64_t *expert_token_nums, hipStream_t st);
 
-int32_t zbalhip_layout_fused_internal(const int32_t *idx, int64_t tokens, int64_t experts, int64_t topk,
+int32_t zbalhip_layout_fused_internal(const ExpertIds &idx, int64_t tokens, int64_t experts, int64_t topk,
                                       int32_t token_nums_type, const uint8_t *active_mask, int32_t *send_token_idx,
                                       int32_t *incl_i32, int32_t *row_off, int64_t *counts_i64, int64_t *nums_typed,
                                       hipStream_t st);
@@ -82,7 +82,7 @@ struct InlineLayout {
  * On return s_off[e] = rows before expert e, s_e[k] / s_rk[k] = expert and rank of pick k of token t. Negative ranks are
  * not routed: -1 an invalid expert id, -2 a token past the active ones (the combine leaves such a token's row alone).
  */
-__device__ __forceinline__ void inline_layout(const int32_t *__restrict__ idx, int t, int topk, int experts,
+__device__ __forceinline__ void inline_layout(const ExpertIds &idx, int t, int topk, int experts,
                                               const InlineLayout &il, int32_t *s_off, int32_t *s_e, int32_t *s_rk, int32_t *s_tmp)
 {
     const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = tid >> 6;
@@ -284,7 +284,7 @@ enum { LM_GIVEN = 0, LM_INLINE = 1, LM_TABLE = 2 };     /* where ranks and offse
 
 template <int XDT, int QM, int SLOTS, bool SMOOTH, int LM>
 __global__ void __launch_bounds__(kThreads)
-permute_quant_kernel(const uint16_t *__restrict__ x, const int32_t *__restrict__ topk_idx,
+permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                      const int32_t *__restrict__ rank_in_expert, const int32_t *__restrict__ base, int base_inclusive,
                      const float *__restrict__ smooth, int hidden, int topk, int experts, PeerRows pr, InlineLayout il,
                      RangeTable rt, uint32_t *__restrict__ clear_words, int64_t clear_count)
@@ -465,7 +465,7 @@ permute_quant_kernel(const uint16_t *__restrict__ x, const int32_t *__restrict__
 
 /* plain row copy (no quantisation): 16-byte chunks of 8 elements */
 __global__ void __launch_bounds__(kThreads)
-permute_copy_kernel(const uint16_t *__restrict__ x, const int32_t *__restrict__ topk_idx,
+permute_copy_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                     const int32_t *__restrict__ rank_in_expert, const int32_t *__restrict__ base, int base_inclusive,
                     int hidden, int topk, int experts, PeerRows pr)
 {
@@ -504,7 +504,7 @@ struct PermuteExtras {
 };
 
 template <int XDT, int QM, bool SMOOTH>
-int32_t launch_quant(const void *x, const int32_t *topk_idx, const int32_t *rank_in_expert, const int32_t *base,
+int32_t launch_quant(const void *x, const ExpertIds &topk_idx, const int32_t *rank_in_expert, const int32_t *base,
                      int base_inclusive, const float *smooth, int64_t tokens, int64_t hidden, int64_t topk,
                      int64_t experts, const PeerRows &pr, const PermuteExtras &ex, hipStream_t st)
 {
@@ -541,7 +541,7 @@ int32_t launch_quant(const void *x, const int32_t *topk_idx, const int32_t *rank
  * exclusive (or inclusive) per-expert row offset table on the device; `pr`
  * says where each rank's rows go.
  */
-static int32_t permute_launch(const void *x, int32_t x_dtype, const int32_t *topk_idx, const int32_t *rank_in_expert,
+static int32_t permute_launch(const void *x, int32_t x_dtype, const ExpertIds &topk_idx, const int32_t *rank_in_expert,
                               const int32_t *base, int base_inclusive, const float *smooth, int64_t tokens,
                               int64_t hidden, int64_t topk, int64_t experts, int quant, const PeerRows &pr, hipStream_t st,
                               const PermuteExtras &ex = PermuteExtras{})
@@ -599,6 +599,8 @@ extern "C" int32_t zbalhip_dispatch_normal(const void *x, int32_t x_dtype, const
                                            int64_t dest_rows, void *stream)
 {
     if (!x || !topk_idx || !send_token_idx || !put_offset || !dest) return ZBALHIP_INVALID;
+    const ExpertIds ids = expert_ids(topk_idx, (quant_mode & ZBALHIP_IDS_ARE_I64) != 0);
+    quant_mode &= ~ZBALHIP_IDS_ARE_I64;
     if (experts <= 0 || quant_mode < 0 || quant_mode > 2) return ZBALHIP_INVALID;
     if (ranks <= 0 || ranks > ZBALHIP_MAX_REDUCE_PEERS || my_rank < 0 || my_rank >= ranks || experts % ranks != 0 || dest_rows < 0)
         return ZBALHIP_INVALID;
@@ -614,7 +616,7 @@ extern "C" int32_t zbalhip_dispatch_normal(const void *x, int32_t x_dtype, const
     pr.e_loc = (int)(experts / ranks);
     pr.rows_cap = dest_rows;
     const int q = quant_mode == 0 ? QM_COPY : (quant_mode == 1 ? QM_INT8_EPS : QM_FP8);
-    return permute_launch(x, x_dtype, topk_idx, send_token_idx, put_offset, 0, nullptr, tokens, hidden, topk, experts, q, pr,
+    return permute_launch(x, x_dtype, ids, send_token_idx, put_offset, 0, nullptr, tokens, hidden, topk, experts, q, pr,
                           (hipStream_t)stream);
 }
 
@@ -628,6 +630,8 @@ extern "C" int32_t zbalhip_dispatch_low_latency(const void *x, int32_t x_dtype, 
     /* an empty batch has no per-token data: only the counts are written */
     if (!expert_token_nums || !ep_recv_counts || !scratch) return ZBALHIP_INVALID;
     if (tokens > 0 && (!x || !expert_ids || !expand_x || !expand_idx)) return ZBALHIP_INVALID;
+    const ExpertIds ids = ::expert_ids(expert_ids, (quant_mode & ZBALHIP_IDS_ARE_I64) != 0);
+    quant_mode &= ~ZBALHIP_IDS_ARE_I64;
     if (experts <= 0 || experts > 1024 || topk <= 0 || tokens < 0 || quant_mode < 0 || quant_mode > 2 ||
         scratch_blocks < 1)
         return ZBALHIP_INVALID;
@@ -642,13 +646,13 @@ extern "C" int32_t zbalhip_dispatch_low_latency(const void *x, int32_t x_dtype, 
         il.incl_i32 = ep_recv_counts;
         il.nums_typed = expert_token_nums;
         const PermuteExtras ex = {&il, nullptr, 0, nullptr};
-        return permute_launch(x, x_dtype, expert_ids, expand_idx, ep_recv_counts, 1, nullptr, tokens, hidden, topk, experts, q,
+        return permute_launch(x, x_dtype, ids, expand_idx, ep_recv_counts, 1, nullptr, tokens, hidden, topk, experts, q,
                               single_window(expand_x, dynamic_scales, experts, tokens * topk), st, ex);
     }
-    const int32_t rc = zbalhip_layout_fused_internal(expert_ids, tokens, experts, topk, token_nums_type, nullptr, expand_idx,
+    const int32_t rc = zbalhip_layout_fused_internal(ids, tokens, experts, topk, token_nums_type, nullptr, expand_idx,
                                                      ep_recv_counts, nullptr, nullptr, expert_token_nums, st);
     if (rc != ZBALHIP_OK) return rc;
-    return permute_launch(x, x_dtype, expert_ids, expand_idx, ep_recv_counts, 1, nullptr, tokens, hidden, topk, experts, q,
+    return permute_launch(x, x_dtype, ids, expand_idx, ep_recv_counts, 1, nullptr, tokens, hidden, topk, experts, q,
                           single_window(expand_x, dynamic_scales, experts, tokens * topk), st);
 }
 
@@ -681,11 +685,12 @@ extern "C" int32_t zbalhip_dispatch_low_latency_ranks(const void *x, int32_t x_d
                                             ep_recv_counts, expert_token_nums, st);
     if (rc != ZBALHIP_OK || tokens == 0) return rc;
     /* the rank of each of my picks among my own earlier picks of the same expert */
-    rc = zbalhip_layout_fused_internal(expert_ids[my_rank], tokens, experts, topk, 1, nullptr, expand_idx, nullptr, nullptr,
+    const ExpertIds ids = ::expert_ids(expert_ids[my_rank], false);
+    rc = zbalhip_layout_fused_internal(ids, tokens, experts, topk, 1, nullptr, expand_idx, nullptr, nullptr,
                                        nullptr, nullptr, st);
     if (rc != ZBALHIP_OK) return rc;
     const int q = quant_mode == 0 ? QM_COPY : (quant_mode == 1 ? QM_INT8_NOEPS : QM_FP8);
-    return permute_launch(x, x_dtype, expert_ids[my_rank], expand_idx, ep_recv_counts, 1, nullptr, tokens, hidden, topk,
+    return permute_launch(x, x_dtype, ids, expand_idx, ep_recv_counts, 1, nullptr, tokens, hidden, topk,
                           experts, q, pr, st);
 }
 
@@ -698,6 +703,8 @@ extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, c
 {
     if (!counts || !row_off || clear_count < 0 || (clear_count > 0 && !clear_words)) return ZBALHIP_INVALID;
     if (tokens > 0 && (!x || !expert_ids || !q1 || !xs || !expand_idx)) return ZBALHIP_INVALID;
+    const ExpertIds ids = ::expert_ids(expert_ids, (mode & ZBALHIP_IDS_ARE_I64) != 0);
+    mode &= ~ZBALHIP_IDS_ARE_I64;
     if (experts <= 0 || experts > 1024 || topk <= 0 || tokens < 0 || (mode != 1 && mode != 2)) return ZBALHIP_INVALID;
     if (mode == 2 && smooth) return ZBALHIP_INVALID;
     if (scratch_blocks < 0 || (scratch_blocks > 0 && !scratch)) return ZBALHIP_INVALID;
@@ -712,7 +719,7 @@ extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, c
         il.row_off = row_off;
         il.counts_i64 = counts;
         const PermuteExtras ex = {&il, clear_words, clear_count, nullptr};
-        return permute_launch(x, x_dtype, expert_ids, expand_idx, row_off, 0, smooth, tokens, hidden, topk, experts, q,
+        return permute_launch(x, x_dtype, ids, expand_idx, row_off, 0, smooth, tokens, hidden, topk, experts, q,
                               single_window(q1, xs, experts, tokens * topk), st, ex);
     }
     /* large batches with room for the ranges' histograms: a short layout launch, the rest of the layout inside the permute launch */
@@ -727,18 +734,18 @@ extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, c
         rt.expand_idx = expand_idx;
         rt.row_off = row_off;
         rt.counts_i64 = counts;
-        const int32_t rc = zbalhip_layout_ranges_internal(expert_ids, tokens, experts, topk, active_mask, expand_idx, scratch,
+        const int32_t rc = zbalhip_layout_ranges_internal(ids, tokens, experts, topk, active_mask, expand_idx, scratch,
                                                           rt.ranges, rt.tokens_per_range, st);
         if (rc != ZBALHIP_OK) return rc;
         const PermuteExtras ex = {nullptr, clear_words, clear_count, &rt};
-        return permute_launch(x, x_dtype, expert_ids, nullptr, nullptr, 0, smooth, tokens, hidden, topk, experts, q,
+        return permute_launch(x, x_dtype, ids, nullptr, nullptr, 0, smooth, tokens, hidden, topk, experts, q,
                               single_window(q1, xs, experts, tokens * topk), st, ex);
     }
-    const int32_t rc = zbalhip_layout_fused_internal(expert_ids, tokens, experts, topk, 1, active_mask, expand_idx, nullptr,
+    const int32_t rc = zbalhip_layout_fused_internal(ids, tokens, experts, topk, 1, active_mask, expand_idx, nullptr,
                                                      row_off, counts, nullptr, st);
     if (rc != ZBALHIP_OK) return rc;
     if (tokens == 0 && clear_count > 0) return zbalhip_fill_i32((int32_t *)clear_words, clear_count, 0, stream);
     const PermuteExtras ex = {nullptr, clear_words, clear_count, nullptr};
-    return permute_launch(x, x_dtype, expert_ids, expand_idx, row_off, 0, smooth, tokens, hidden, topk, experts, q,
+    return permute_launch(x, x_dtype, ids, expand_idx, row_off, 0, smooth, tokens, hidden, topk, experts, q,
                           single_window(q1, xs, experts, tokens * topk), st, ex);
 }

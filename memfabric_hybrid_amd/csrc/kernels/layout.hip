@@ -5,60 +5,21 @@
  *
  * The stable rank of a pick (its position among earlier picks of the same
  * expert, in flat (t,k) order) is computed without atomics on the result:
- * blocks own contiguous token ranges, a first pass leaves one histogram per
- * block in `scratch`, and the second pass starts each block from the sum of
- * the histograms of the blocks before it; inside a block, picks are ranked 64
- * at a time with wave ballots (lanes holding the same expert find each other
- * by intersecting one ballot per index bit) and the four waves of a block
- * commit their running counts in wave order.
+ * blocks own contiguous token ranges, each counts the picks before its own
+ * range, and inside a block picks are ranked 64 at a time with wave ballots
+ * (lanes holding the same expert find each other by intersecting one ballot
+ * per index bit).
  */
-#include <mutex>
+#include <time.h>
 
 #include "zbal_device.h"
 #include "zbal_hip_kernels.h"
 #include "zbal_layout_rank.h"
 
 #define ZB_MAX_EXPERTS 1024
-#define ZB_LAYOUT_THREADS 256
 #define ZB_FUSED_THREADS 1024
 
-/*
- * Per-block histograms of zbalhip_dispatch_layout_static: the rows its kernels otherwise find in the caller's
- * `scratch` argument, for the largest case the entry point takes. Every GPU the library runs on holds its own copy
- * for the life of the process (200 KiB). Host code never uses this name as an address: it asks the runtime for the
- * device address once per device (static_scratch_of) and hands that pointer to the kernels.
- */
-static __device__ __align__(256) int32_t scratch[ZBALHIP_LAYOUT_MAX_BLOCKS * ZB_MAX_EXPERTS];
-
 namespace {
-
-constexpr int ZB_MAX_DEVICES = 64;
-
-/*
- * This GPU's copy of `scratch`: its device address, looked up on the first call with that GPU current, and an event
- * that marks the end of the last launch sequence that used it. Calls are issued under `mu`, each waiting for that
- * event on its own stream first and recording it again after its last launch, so two callers on different streams
- * (or threads) take turns on the array instead of racing on it.
- */
-struct StaticScratch {
-    std::mutex mu;
-    int32_t *addr = nullptr;
-    hipEvent_t last_use = nullptr;
-};
-
-StaticScratch *static_scratch_of(int dev)
-{
-    static StaticScratch per_device[ZB_MAX_DEVICES];
-    StaticScratch &s = per_device[dev];
-    std::lock_guard<std::mutex> guard(s.mu);
-    if (s.addr == nullptr) {
-        void *p = nullptr;
-        if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || p == nullptr) return nullptr;
-        if (hipEventCreateWithFlags(&s.last_use, hipEventDisableTiming) != hipSuccess) return nullptr;
-        s.addr = static_cast<int32_t *>(p);
-    }
-    return &s;
-}
 
 struct LayoutPlan {
     int nblk;
@@ -79,85 +40,44 @@ inline LayoutPlan plan_layout(int64_t tokens, int64_t topk, int max_blocks)
     return p;
 }
 
-template <typename IdxT>
-__global__ void __launch_bounds__(ZB_LAYOUT_THREADS)
-layout_hist_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int experts, int ranks, int tpb,
-                   int32_t *__restrict__ scratch, int32_t *__restrict__ tokens_per_rank)
+/*
+ * What a layout launch writes; every pointer may be null. send_token_idx [T, K]; incl_i32 [E] running sums; row_off
+ * [E + 1] exclusive offsets; counts_i32 / counts_i64 [E]; nums_typed [E] counts (type 1) or running sums (type 0);
+ * tokens_per_rank [ranks]: tokens with a pick of one of the rank's experts; token_in_rank [T, ranks]: 1 where the token
+ * has such a pick, else 0.
+ */
+struct LayoutOutputs {
+    int32_t *send_token_idx, *incl_i32, *row_off, *counts_i32;
+    int64_t *counts_i64, *nums_typed;
+    int32_t *tokens_per_rank, *token_in_rank;
+    int ranks, token_nums_type;
+};
+
+/* bit r of the returned mask: the token's picks [i0, i0 + topk) include an expert of rank first_rank + r (r < 32) */
+__device__ __forceinline__ uint32_t token_ranks(const ExpertIds &idx, int64_t i0, int topk, int experts, int e_loc, int first_rank)
 {
-    __shared__ int32_t hist[ZB_MAX_EXPERTS];
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) hist[e] = 0;
-    if (blockIdx.x == 0 && tokens_per_rank)
-        for (int r = threadIdx.x; r < ranks; r += blockDim.x) tokens_per_rank[r] = 0;
-    __syncthreads();
-    const int64_t p0 = (int64_t)blockIdx.x * tpb * topk;
-    int64_t p1 = p0 + (int64_t)tpb * topk;
-    const int64_t pend = (int64_t)tokens * topk;
-    if (p1 > pend) p1 = pend;
-    for (int64_t i = p0 + threadIdx.x; i < p1; i += blockDim.x) {
-        int64_t e = (int64_t)idx[i];
-        if (e >= 0 && e < experts) atomicAdd(&hist[e], 1);
+    uint32_t mask = 0;
+    for (int k = 0; k < topk; ++k) {
+        const int e = idx[i0 + k];
+        if (e < 0 || e >= experts) continue;
+        const int r = (e_loc == experts ? 0 : e / e_loc) - first_rank;
+        if (r >= 0 && r < 32) mask |= 1u << r;
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) scratch[(int64_t)blockIdx.x * experts + e] = hist[e];
-}
-
-template <typename IdxT>
-__global__ void __launch_bounds__(ZB_LAYOUT_THREADS)
-layout_rank_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int experts, int ranks, int tpb, int nbits,
-                   const int32_t *__restrict__ scratch, int32_t *__restrict__ send_token_idx,
-                   int32_t *__restrict__ tokens_per_rank)
-{
-    __shared__ int32_t run[ZB_MAX_EXPERTS];
-    __shared__ int32_t rcnt[ZB_MAX_EXPERTS];
-    __shared__ __align__(16) uint8_t cnt[ZB_LAYOUT_THREADS / 64 * ZB_MAX_EXPERTS];
-    const int b = blockIdx.x;
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) {
-        int32_t s = 0;
-        for (int bb = 0; bb < b; ++bb) s += scratch[(int64_t)bb * experts + e];
-        run[e] = s;
-    }
-    for (int r = threadIdx.x; r < ranks; r += blockDim.x) rcnt[r] = 0;
-    __syncthreads();
-
-    const int tok0 = b * tpb;
-    int tok1 = tok0 + tpb;
-    if (tok1 > tokens) tok1 = tokens;
-    rank_picks(idx, (int64_t)tok0 * topk, (int64_t)tok1 * topk, experts, nbits, run, cnt, send_token_idx);
-
-    /* tokens per rank: one count per (token, rank) no matter how many of the token's picks land there */
-    if (tokens_per_rank) {
-        const int e_loc = experts / ranks;
-        for (int t = tok0 + threadIdx.x; t < tok1; t += blockDim.x) {
-            for (int k = 0; k < topk; ++k) {
-                int64_t e = (int64_t)idx[(int64_t)t * topk + k];
-                if (e < 0 || e >= experts) continue;
-                const int r = (int)(e / e_loc);
-                bool first = true;
-                for (int k2 = 0; k2 < k; ++k2) {
-                    int64_t e2 = (int64_t)idx[(int64_t)t * topk + k2];
-                    if (e2 >= 0 && e2 < experts && (int)(e2 / e_loc) == r) first = false;
-                }
-                if (first) atomicAdd(&rcnt[r], 1);
-            }
-        }
-        __syncthreads();
-        for (int r = threadIdx.x; r < ranks; r += blockDim.x)
-            if (rcnt[r]) atomicAdd(&tokens_per_rank[r], rcnt[r]);
-    }
+    return mask;
 }
 
 /*
- * The whole layout in one launch, for the callers that need ranks and offsets but no per-rank counts: every
- * block first counts the picks that precede its own range (the index array is a few hundred KiB and sits in L2,
- * so reading it again per block is cheaper than a launch), ranks its own picks, and the last block, whose running
- * counts are then the totals, scans them into the offsets. Every output pointer except send_token_idx may be null.
+ * The whole layout in one launch: every block first counts the picks that precede its own range (the index array is a
+ * few hundred KiB and sits in L2, so reading it again per block is cheaper than a launch), ranks its own picks, and the
+ * last block, whose running counts are then the totals, scans them into the offsets and counts the tokens per rank.
+ * With per-rank counts on 4096 tokens of 8 int64 picks over 32 experts this replaces a histogram, a ranking and a scan
+ * launch (4.7 + 20.3 + 6.1 us; the ranking blocks summed up to 49 histograms one after the other) and five elementwise
+ * launches that worked token_in_rank out.
  */
-template <typename IdxT>
+template <bool RANKS>
 __global__ void __launch_bounds__(ZB_FUSED_THREADS)
-layout_fused_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int experts, int tpb, int nbits,
-                    int token_nums_type, const uint8_t *__restrict__ active_mask, int32_t *__restrict__ send_token_idx,
-                    int32_t *__restrict__ incl_i32, int32_t *__restrict__ row_off /* [E+1] */,
-                    int64_t *__restrict__ counts_i64, int64_t *__restrict__ nums_typed)
+layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, int nbits,
+                    const uint8_t *__restrict__ active_mask, LayoutOutputs o)
 {
     __shared__ int32_t run[ZB_MAX_EXPERTS];
     __shared__ int32_t wsum[ZB_FUSED_THREADS / 64];
@@ -186,37 +106,42 @@ layout_fused_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int expe
     int tok0 = blockIdx.x * tpb;
     int tok1 = tok0 + tpb;
     if (tok1 > tokens) tok1 = tokens;
+    const int e_loc = RANKS ? experts / o.ranks : experts;
+    if (RANKS && o.token_in_rank)
+        for (int i = tok0 * o.ranks + threadIdx.x; i < tok1 * o.ranks; i += blockDim.x) {
+            const int t = i / o.ranks;
+            o.token_in_rank[i] = (int)(token_ranks(idx, (int64_t)t * topk, topk, experts, e_loc, i - t * o.ranks) & 1u);
+        }
     for (int64_t i = (int64_t)(tok0 > active ? tok0 : active) * topk + threadIdx.x; i < (int64_t)tok1 * topk; i += blockDim.x)
-        send_token_idx[i] = -2;
+        o.send_token_idx[i] = -2;
     if (tok0 > active) tok0 = active;
     if (tok1 > active) tok1 = active;
     const int64_t p0 = (int64_t)tok0 * topk, p1 = (int64_t)tok1 * topk;
-    constexpr int PER = 16 / (int)sizeof(IdxT);      /* indices per 16-byte load */
-    const int64_t nvec = ((uintptr_t)idx & 15) == 0 ? p0 / PER : 0;
+    const int per = 4 / idx.stride();                /* ids per 16-byte load */
+    const int64_t nvec = ((uintptr_t)idx.p & 15) == 0 ? p0 / per : 0;
     /* four 16-byte loads per lane are requested before the first is counted: a chain of round trips to L2 otherwise */
     for (int64_t v0 = threadIdx.x; v0 < nvec; v0 += 4 * (int64_t)blockDim.x) {
         u32x4 raw[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int64_t v = v0 + u * (int64_t)blockDim.x;
-            raw[u] = v < nvec ? *reinterpret_cast<const u32x4 *>(idx + v * PER) : u32x4{~0u, ~0u, ~0u, ~0u};
+            raw[u] = v < nvec ? *reinterpret_cast<const u32x4 *>(idx.p + v * 4) : u32x4{~0u, ~0u, ~0u, ~0u};
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                int64_t e;
-                if (sizeof(IdxT) == 4) e = (int32_t)raw[u][j];
-                else e = (int64_t)(((uint64_t)raw[u][2 * j + 1] << 32) | raw[u][2 * j]);
-                if (e >= 0 && e < experts) atomicAdd(&run[(int)e], 1);
+            for (int j = 0; j < 4; ++j) {
+                if (idx.kind != IDS_I32 && (j & 1)) continue;
+                const int e = idx.kind == IDS_I32 ? (int)raw[u][j] : idx.of_words(raw[u][j], raw[u][j | 1]);
+                if (e >= 0 && e < experts) atomicAdd(&run[e], 1);
             }
     }
-    for (int64_t i = nvec * PER + threadIdx.x; i < p0; i += blockDim.x) {
-        const int64_t e = (int64_t)idx[i];
-        if (e >= 0 && e < experts) atomicAdd(&run[(int)e], 1);
+    for (int64_t i = nvec * per + threadIdx.x; i < p0; i += blockDim.x) {
+        const int e = idx[i];
+        if (e >= 0 && e < experts) atomicAdd(&run[e], 1);
     }
     __syncthreads();
-    rank_picks(idx, p0, p1, experts, nbits, run, cnt, send_token_idx);
+    rank_picks(idx, p0, p1, experts, nbits, run, cnt, o.send_token_idx);
     if (blockIdx.x != gridDim.x - 1) return;
 
     /* rank_picks ends on a barrier: run[] now holds the totals */
@@ -228,8 +153,8 @@ layout_fused_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int expe
         int32_t s = c;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
-            const int32_t o = __shfl_up(s, off, 64);
-            if (lane >= off) s += o;
+            const int32_t other = __shfl_up(s, off, 64);
+            if (lane >= off) s += other;
         }
         if (lane == 63) wsum[wave] = s;
         __syncthreads();
@@ -241,11 +166,37 @@ layout_fused_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int expe
         carry += chunk_total;
         __syncthreads();
         if (e < experts) {
-            if (incl_i32) incl_i32[e] = s;
-            if (row_off) { row_off[e] = s - c; if (e == experts - 1) row_off[experts] = s; }
-            if (counts_i64) counts_i64[e] = c;
-            if (nums_typed) nums_typed[e] = token_nums_type == 0 ? (int64_t)s : (int64_t)c;
+            if (o.incl_i32) o.incl_i32[e] = s;
+            if (o.row_off) { o.row_off[e] = s - c; if (e == experts - 1) o.row_off[experts] = s; }
+            if (o.counts_i32) o.counts_i32[e] = c;
+            if (o.counts_i64) o.counts_i64[e] = c;
+            if (o.nums_typed) o.nums_typed[e] = o.token_nums_type == 0 ? (int64_t)s : (int64_t)c;
         }
+    }
+    /* tokens per rank: one count per (token, rank) no matter how many of the token's picks land there, 32 ranks per pass */
+    if (RANKS && o.tokens_per_rank) {
+        int32_t *rcnt = run;                        /* the totals have been written out */
+        for (int r = threadIdx.x; r < o.ranks; r += blockDim.x) rcnt[r] = 0;
+        __syncthreads();
+        for (int first = 0; first < o.ranks; first += 32) {
+            const int nr = o.ranks - first < 32 ? o.ranks - first : 32;
+            int32_t mine = 0;                       /* ranks == 1: counted in a register */
+            for (int t = threadIdx.x; t < tokens; t += blockDim.x) {
+                uint32_t mask = token_ranks(idx, (int64_t)t * topk, topk, experts, e_loc, first);
+                if (o.ranks == 1) { mine += (int32_t)(mask & 1u); continue; }
+                for (; mask; mask &= mask - 1) {
+                    const int r = __ffs((int)mask) - 1;
+                    if (r < nr) atomicAdd(&rcnt[first + r], 1);
+                }
+            }
+            if (o.ranks == 1) {
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off, 64);
+                if (lane == 0 && mine) atomicAdd(&rcnt[0], mine);
+            }
+        }
+        __syncthreads();
+        for (int r = threadIdx.x; r < o.ranks; r += blockDim.x) o.tokens_per_rank[r] = rcnt[r];
     }
 }
 
@@ -258,9 +209,9 @@ layout_fused_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int expe
  * its own itself (LDS atomics: a fraction of what ranking them costs), so no block waits for another, and the block of
  * the last slice ends up with the whole range's histogram and writes it.
  */
-template <typename IdxT, bool SLICED>
+template <bool SLICED>
 __global__ void __launch_bounds__(ZB_FUSED_THREADS)
-layout_ranges_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int experts, int tpb, int subs_arg, int nbits,
+layout_ranges_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, int subs_arg, int nbits,
                      const uint8_t *__restrict__ active_mask, int32_t *__restrict__ send_token_idx,
                      int32_t *__restrict__ hist)
 {
@@ -300,8 +251,8 @@ layout_ranges_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int exp
     if (sl1 > active) sl1 = active;
     if (SLICED) {       /* the picks of this range in front of the slice: counted only */
         for (int64_t i = (int64_t)tok0 * topk + threadIdx.x; i < (int64_t)sl0 * topk; i += blockDim.x) {
-            const int64_t e = (int64_t)idx[i];
-            if (e >= 0 && e < experts) atomicAdd(&run[(int)e], 1);
+            const int e = idx[i];
+            if (e >= 0 && e < experts) atomicAdd(&run[e], 1);
         }
         __syncthreads();
     }
@@ -311,24 +262,26 @@ layout_ranges_kernel(const IdxT *__restrict__ idx, int tokens, int topk, int exp
         for (int e = threadIdx.x; e < experts; e += blockDim.x) hist[(int64_t)range * experts + e] = run[e];
 }
 
+/* where a notify launch leaves the counts for a host that waits for them: pinned memory that the GPU writes directly */
+struct HostCounts {
+    int64_t counts[ZB_MAX_EXPERTS];
+    uint64_t ready;                /* the number of the launch that wrote the counts, stored after them */
+};
+
 /*
- * One block: totals per expert from the per-block histograms (or from a
- * ready histogram when nblk == 0), then an inclusive scan over experts.
- * Every output pointer may be null.
+ * Notify for a group of one rank, one block: the offsets are the exclusive running sum of the counts. With `host` the
+ * counts also go to pinned host memory, followed by a flag, so that a caller who has to know them spins on that word
+ * instead of queueing a copy behind the kernel and waiting for the stream.
  */
 __global__ void __launch_bounds__(ZB_MAX_EXPERTS)
-layout_scan_kernel(const int32_t *__restrict__ hist, int nblk, int experts, int topk, int token_nums_type,
-                   int32_t *__restrict__ counts_i32, int32_t *__restrict__ excl_i32, int32_t *__restrict__ incl_i32,
-                   int32_t *__restrict__ row_off /* [E+1] */, int64_t *__restrict__ counts_i64,
-                   int64_t *__restrict__ nums_typed, int32_t *__restrict__ total, int32_t *__restrict__ balance)
+notify_one_kernel(const int32_t *__restrict__ tokens_per_expert, int experts, int topk, int32_t *__restrict__ recv_data,
+                  int32_t *__restrict__ put_offset, int64_t *__restrict__ recv_tokens_per_expert,
+                  int32_t *__restrict__ total, int32_t *__restrict__ balance, HostCounts *host, uint64_t launch)
 {
     __shared__ int32_t wsum[ZB_MAX_EXPERTS / 64];
     const int e = threadIdx.x;
-    int32_t c = 0;
-    if (e < experts) {
-        if (nblk == 0) c = hist[e];
-        else for (int b = 0; b < nblk; ++b) c += hist[(int64_t)b * experts + e];
-    }
+    const int32_t c = e < experts ? tokens_per_expert[e] : 0;
+    if (host && e < experts) host->counts[e] = c;
     int32_t s = c;
     const int lane = e & 63, wave = e >> 6;
 #pragma unroll
@@ -337,24 +290,21 @@ layout_scan_kernel(const int32_t *__restrict__ hist, int nblk, int experts, int 
         if (lane >= off) s += o;
     }
     if (lane == 63) wsum[wave] = s;
+    if (host) __threadfence_system();
     __syncthreads();
+    if (host && e == 0) __hip_atomic_store(&host->ready, launch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     int32_t add = 0;
     for (int w = 0; w < wave; ++w) add += wsum[w];
     s += add;
     if (e < experts) {
-        if (counts_i32) counts_i32[e] = c;
-        if (excl_i32) excl_i32[e] = s - c;
-        if (incl_i32) incl_i32[e] = s;
-        if (row_off) { row_off[e] = s - c; if (e == experts - 1) row_off[experts] = s; }
-        if (counts_i64) counts_i64[e] = c;
-        if (nums_typed) nums_typed[e] = token_nums_type == 0 ? (int64_t)s : (int64_t)c;
+        recv_data[e] = c;
+        put_offset[e] = s - c;
+        recv_tokens_per_expert[e] = c;
         if (e == experts - 1) {
-            if (total) *total = s;
-            if (balance) {
-                const int32_t bs = s / topk;
-                balance[0] = bs > 0 ? 0 : -1;
-                balance[1] = bs > 0 ? bs - 1 : -1;
-            }
+            *total = s;
+            const int32_t bs = s / topk;
+            balance[0] = bs > 0 ? 0 : -1;
+            balance[1] = bs > 0 ? bs - 1 : -1;
         }
     }
 }
@@ -596,48 +546,37 @@ inline int ceil_log2(int64_t v)
 
 } // namespace
 
-/* Used by the other translation units of the library (fused path, low-latency dispatch). */
-int32_t zbalhip_layout_internal(const void *idx, int32_t idx_is_i64, int64_t tokens, int64_t experts, int64_t topk,
-                                int32_t ranks, int32_t *tokens_per_rank, int32_t *send_token_idx, int32_t *scratch,
-                                int max_blocks, int *nblk_out, hipStream_t st)
+static int32_t launch_fused_layout(const ExpertIds &idx, int64_t tokens, int64_t experts, int64_t topk,
+                                   const uint8_t *active_mask, const LayoutOutputs &o, hipStream_t st)
 {
-    const LayoutPlan p = plan_layout(tokens, topk, max_blocks);
-    const int nbits = ceil_log2(experts);
-    if (idx_is_i64) {
-        layout_hist_kernel<int64_t><<<p.nblk, ZB_LAYOUT_THREADS, 0, st>>>(
-            (const int64_t *)idx, (int)tokens, (int)topk, (int)experts, ranks, p.tokens_per_block, scratch,
-            tokens_per_rank);
-        layout_rank_kernel<int64_t><<<p.nblk, ZB_LAYOUT_THREADS, 0, st>>>(
-            (const int64_t *)idx, (int)tokens, (int)topk, (int)experts, ranks, p.tokens_per_block, nbits, scratch,
-            send_token_idx, tokens_per_rank);
-    } else {
-        layout_hist_kernel<int32_t><<<p.nblk, ZB_LAYOUT_THREADS, 0, st>>>(
-            (const int32_t *)idx, (int)tokens, (int)topk, (int)experts, ranks, p.tokens_per_block, scratch,
-            tokens_per_rank);
-        layout_rank_kernel<int32_t><<<p.nblk, ZB_LAYOUT_THREADS, 0, st>>>(
-            (const int32_t *)idx, (int)tokens, (int)topk, (int)experts, ranks, p.tokens_per_block, nbits, scratch,
-            send_token_idx, tokens_per_rank);
-    }
-    *nblk_out = p.nblk;
+    const LayoutPlan p = plan_layout(tokens, topk, 64);
+    if (o.tokens_per_rank || o.token_in_rank)
+        layout_fused_kernel<true><<<p.nblk, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,
+                                                                     p.tokens_per_block, ceil_log2(experts), active_mask, o);
+    else
+        layout_fused_kernel<false><<<p.nblk, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,
+                                                                      p.tokens_per_block, ceil_log2(experts), active_mask, o);
     return zbalhip_check_launch();
 }
 
-/* ranks + offsets in one launch (no per-rank counts, no scratch) */
-int32_t zbalhip_layout_fused_internal(const int32_t *idx, int64_t tokens, int64_t experts, int64_t topk,
+/* Used by the other translation units of the library (fused path, low-latency dispatch): ranks + offsets in one launch */
+int32_t zbalhip_layout_fused_internal(const ExpertIds &idx, int64_t tokens, int64_t experts, int64_t topk,
                                       int32_t token_nums_type, const uint8_t *active_mask, int32_t *send_token_idx,
                                       int32_t *incl_i32, int32_t *row_off, int64_t *counts_i64, int64_t *nums_typed,
                                       hipStream_t st)
 {
-    const LayoutPlan p = plan_layout(tokens, topk, 64);
-    layout_fused_kernel<int32_t><<<p.nblk, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,
-                                                                    p.tokens_per_block, ceil_log2(experts), token_nums_type,
-                                                                    active_mask, send_token_idx, incl_i32, row_off,
-                                                                    counts_i64, nums_typed);
-    return zbalhip_check_launch();
+    LayoutOutputs o = {};
+    o.send_token_idx = send_token_idx;
+    o.incl_i32 = incl_i32;
+    o.row_off = row_off;
+    o.counts_i64 = counts_i64;
+    o.nums_typed = nums_typed;
+    o.token_nums_type = token_nums_type;
+    return launch_fused_layout(idx, tokens, experts, topk, active_mask, o, st);
 }
 
 /* ranks within token ranges + one histogram per range, for the permute kernel's table mode; returns the ranges' size */
-int32_t zbalhip_layout_ranges_internal(const int32_t *idx, int64_t tokens, int64_t experts, int64_t topk,
+int32_t zbalhip_layout_ranges_internal(const ExpertIds &idx, int64_t tokens, int64_t experts, int64_t topk,
                                        const uint8_t *active_mask, int32_t *send_token_idx, int32_t *hist, int nblk,
                                        int tokens_per_block, hipStream_t st)
 {
@@ -651,10 +590,10 @@ int32_t zbalhip_layout_ranges_internal(const int32_t *idx, int64_t tokens, int64
     subs = subs < 1 ? 1 : (subs > 8 ? 8 : subs);
     if (subs > tokens_per_block) subs = tokens_per_block;
     if (subs == 1)
-        layout_ranges_kernel<int32_t, false><<<(unsigned)nblk, ZB_FUSED_THREADS, 0, st>>>(
+        layout_ranges_kernel<false><<<(unsigned)nblk, ZB_FUSED_THREADS, 0, st>>>(
             idx, (int)tokens, (int)topk, (int)experts, tokens_per_block, 1, ceil_log2(experts), active_mask, send_token_idx, hist);
     else
-        layout_ranges_kernel<int32_t, true><<<(unsigned)(nblk * subs), ZB_FUSED_THREADS, 0, st>>>(
+        layout_ranges_kernel<true><<<(unsigned)(nblk * subs), ZB_FUSED_THREADS, 0, st>>>(
             idx, (int)tokens, (int)topk, (int)experts, tokens_per_block, (int)subs, ceil_log2(experts), active_mask,
             send_token_idx, hist);
     return zbalhip_check_launch();
@@ -669,17 +608,6 @@ int32_t zbalhip_ll_counts_internal(const int32_t *const *ids, int ranks, int me,
     const int threads = (int)((experts + 63) / 64 * 64);
     ll_counts_kernel<<<1, threads, 0, st>>>(all, ranks, me, (int)tokens, (int)topk, (int)experts, token_nums_type, all_counts,
                                             ep_recv_counts, expert_token_nums);
-    return zbalhip_check_launch();
-}
-
-int32_t zbalhip_scan_internal(const int32_t *hist, int nblk, int64_t experts, int64_t topk, int32_t token_nums_type,
-                              int32_t *counts_i32, int32_t *excl_i32, int32_t *incl_i32, int32_t *row_off,
-                              int64_t *counts_i64, int64_t *nums_typed, int32_t *total, int32_t *balance,
-                              hipStream_t st)
-{
-    int threads = (int)((experts + 63) / 64 * 64);
-    layout_scan_kernel<<<1, threads, 0, st>>>(hist, nblk, (int)experts, (int)topk, token_nums_type, counts_i32,
-                                              excl_i32, incl_i32, row_off, counts_i64, nums_typed, total, balance);
     return zbalhip_check_launch();
 }
 
@@ -722,16 +650,27 @@ extern "C" int32_t zbalhip_dispatch_layout(const void *topk_idx, int32_t idx_is_
                                            int32_t *tokens_per_expert, int32_t *send_token_idx, int32_t *scratch,
                                            void *stream)
 {
-    if (!topk_idx || !tokens_per_rank || !tokens_per_expert || !send_token_idx || !scratch) return ZBALHIP_INVALID;
+    if (!scratch) return ZBALHIP_INVALID;
+    return zbalhip_dispatch_layout_in_rank(topk_idx, idx_is_i64, tokens, experts, topk, ranks, tokens_per_rank,
+                                           tokens_per_expert, send_token_idx, nullptr, stream);
+}
+
+extern "C" int32_t zbalhip_dispatch_layout_in_rank(const void *topk_idx, int32_t idx_is_i64, int64_t tokens,
+                                                   int64_t experts, int64_t topk, int32_t ranks,
+                                                   int32_t *tokens_per_rank, int32_t *tokens_per_expert,
+                                                   int32_t *send_token_idx, int32_t *token_in_rank, void *stream)
+{
+    if (!topk_idx || !tokens_per_rank || !tokens_per_expert || !send_token_idx) return ZBALHIP_INVALID;
     if (!layout_args_ok(tokens, experts, topk) || ranks <= 0 || ranks > experts || experts % ranks != 0)
         return ZBALHIP_INVALID;
-    int nblk = 0;
-    int32_t rc = zbalhip_layout_internal(topk_idx, idx_is_i64, tokens, experts, topk, ranks, tokens_per_rank,
-                                         send_token_idx, scratch, ZBALHIP_LAYOUT_MAX_BLOCKS, &nblk,
-                                         (hipStream_t)stream);
-    if (rc != ZBALHIP_OK) return rc;
-    return zbalhip_scan_internal(scratch, nblk, experts, topk, 1, tokens_per_expert, nullptr, nullptr, nullptr, nullptr,
-                                 nullptr, nullptr, nullptr, (hipStream_t)stream);
+    if (token_in_rank && tokens > 0x7fffffff / ranks) return ZBALHIP_INVALID;
+    LayoutOutputs o = {};
+    o.send_token_idx = send_token_idx;
+    o.counts_i32 = tokens_per_expert;
+    o.tokens_per_rank = tokens_per_rank;
+    o.token_in_rank = token_in_rank;
+    o.ranks = ranks;
+    return launch_fused_layout(expert_ids(topk_idx, idx_is_i64 != 0, true), tokens, experts, topk, nullptr, o, (hipStream_t)stream);
 }
 
 extern "C" int32_t zbalhip_dispatch_layout_static(const void *topk_idx, int32_t idx_is_i64, int64_t tokens, int64_t experts,
@@ -743,36 +682,14 @@ extern "C" int32_t zbalhip_dispatch_layout_static(const void *topk_idx, int32_t 
         zbalhip_set_last_error("zbalhip_dispatch_layout_static: more experts than the static scratch holds (1024)");
         return ZBALHIP_INVALID;
     }
-    if (!layout_args_ok(tokens, experts, topk) || ranks <= 0 || ranks > experts || experts % ranks != 0)
-        return ZBALHIP_INVALID;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= ZB_MAX_DEVICES) return ZBALHIP_RT_ERROR;
-    StaticScratch *ss = static_scratch_of(dev);
-    if (ss == nullptr) return ZBALHIP_RT_ERROR;
-    hipStream_t st = (hipStream_t)stream;
-    /*
-     * Under stream capture the order of the array's users is the captured graph's own business (an event recorded
-     * outside of the capture cannot be waited for inside it); everywhere else this call queues behind the last one.
-     */
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool capturing = st != nullptr && hipStreamIsCapturing(st, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
-    std::lock_guard<std::mutex> guard(ss->mu);
-    if (!capturing && hipStreamWaitEvent(st, ss->last_use, 0) != hipSuccess) return ZBALHIP_RT_ERROR;
-    /* the histogram kernel writes every row that the rank and scan kernels read: nothing has to start at zero */
-    int nblk = 0;
-    int32_t rc = zbalhip_layout_internal(topk_idx, idx_is_i64, tokens, experts, topk, ranks, tokens_per_rank,
-                                         send_token_idx, ss->addr, ZBALHIP_LAYOUT_MAX_BLOCKS, &nblk, st);
-    if (rc == ZBALHIP_OK)
-        rc = zbalhip_scan_internal(ss->addr, nblk, experts, topk, 1, tokens_per_expert, nullptr, nullptr, nullptr, nullptr,
-                                   nullptr, nullptr, nullptr, st);
-    if (!capturing && hipEventRecord(ss->last_use, st) != hipSuccess && rc == ZBALHIP_OK) rc = ZBALHIP_RT_ERROR;
-    return rc;
+    return zbalhip_dispatch_layout_in_rank(topk_idx, idx_is_i64, tokens, experts, topk, ranks, tokens_per_rank,
+                                           tokens_per_expert, send_token_idx, nullptr, stream);
 }
 
-extern "C" int32_t zbalhip_dispatch_notify(const int32_t *const *tokens_per_expert, int32_t ranks, int32_t my_rank,
-                                           int64_t experts, int64_t topk, int32_t *recv_data, int32_t *put_offset,
-                                           int32_t *total_recv, int64_t *recv_tokens_per_expert, int32_t *balance_matrix,
-                                           void *stream)
+static int32_t launch_notify(const int32_t *const *tokens_per_expert, int32_t ranks, int32_t my_rank, int64_t experts,
+                             int64_t topk, int32_t *recv_data, int32_t *put_offset, int32_t *total_recv,
+                             int64_t *recv_tokens_per_expert, int32_t *balance_matrix, HostCounts *host, uint64_t launch,
+                             hipStream_t st)
 {
     if (!tokens_per_expert || !recv_data || !put_offset || !total_recv || !recv_tokens_per_expert || !balance_matrix)
         return ZBALHIP_INVALID;
@@ -781,14 +698,83 @@ extern "C" int32_t zbalhip_dispatch_notify(const int32_t *const *tokens_per_expe
         return ZBALHIP_INVALID;
     for (int r = 0; r < ranks; ++r)
         if (!tokens_per_expert[r]) return ZBALHIP_INVALID;
-    if (ranks == 1)
-        return zbalhip_scan_internal(tokens_per_expert[0], 0, experts, topk, 1, recv_data, put_offset, nullptr, nullptr,
-                                     recv_tokens_per_expert, nullptr, total_recv, balance_matrix, (hipStream_t)stream);
+    const int threads = (int)((experts + 63) / 64 * 64);
+    if (ranks == 1) {
+        notify_one_kernel<<<1, threads, 0, st>>>(tokens_per_expert[0], (int)experts, (int)topk, recv_data, put_offset,
+                                                 recv_tokens_per_expert, total_recv, balance_matrix, host, launch);
+        return zbalhip_check_launch();
+    }
     CountsOfRanks counts = {};
     for (int r = 0; r < ranks; ++r) counts.p[r] = tokens_per_expert[r];
-    const int threads = (int)((experts + 63) / 64 * 64);
-    notify_ranks_kernel<<<1, threads, 0, (hipStream_t)stream>>>(counts, ranks, my_rank, (int)experts, (int)topk, recv_data,
-                                                                put_offset, total_recv, recv_tokens_per_expert,
-                                                                balance_matrix);
+    notify_ranks_kernel<<<1, threads, 0, st>>>(counts, ranks, my_rank, (int)experts, (int)topk, recv_data, put_offset,
+                                               total_recv, recv_tokens_per_expert, balance_matrix);
     return zbalhip_check_launch();
+}
+
+extern "C" int32_t zbalhip_dispatch_notify(const int32_t *const *tokens_per_expert, int32_t ranks, int32_t my_rank,
+                                           int64_t experts, int64_t topk, int32_t *recv_data, int32_t *put_offset,
+                                           int32_t *total_recv, int64_t *recv_tokens_per_expert, int32_t *balance_matrix,
+                                           void *stream)
+{
+    return launch_notify(tokens_per_expert, ranks, my_rank, experts, topk, recv_data, put_offset, total_recv,
+                         recv_tokens_per_expert, balance_matrix, nullptr, 0, (hipStream_t)stream);
+}
+
+extern "C" int32_t zbalhip_host_counts_alloc(void **block)
+{
+    if (!block) return ZBALHIP_INVALID;
+    if (hipHostMalloc(block, sizeof(HostCounts), hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess)
+        return ZBALHIP_RT_ERROR;
+    static_cast<HostCounts *>(*block)->ready = 0;
+    return ZBALHIP_OK;
+}
+
+extern "C" int32_t zbalhip_host_counts_free(void *block)
+{
+    return block == nullptr || hipHostFree(block) == hipSuccess ? ZBALHIP_OK : ZBALHIP_RT_ERROR;
+}
+
+extern "C" int32_t zbalhip_dispatch_notify_counts(const int32_t *const *tokens_per_expert, int32_t ranks, int32_t my_rank,
+                                                  int64_t experts, int64_t topk, int32_t *recv_data, int32_t *put_offset,
+                                                  int32_t *total_recv, int64_t *recv_tokens_per_expert,
+                                                  int32_t *balance_matrix, void *block, int64_t *host_counts, void *stream)
+{
+    if (!block || !host_counts) return ZBALHIP_INVALID;
+    hipStream_t st = (hipStream_t)stream;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (st != nullptr && hipStreamIsCapturing(st, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone) {
+        zbalhip_set_last_error("NotifyDispatch failed as the counts cannot be read back while the stream is being captured");
+        return ZBALHIP_RT_ERROR;
+    }
+    HostCounts *host = static_cast<HostCounts *>(block);
+    const uint64_t launch = host->ready + 1;
+    const int32_t rc = launch_notify(tokens_per_expert, ranks, my_rank, experts, topk, recv_data, put_offset, total_recv,
+                                     recv_tokens_per_expert, balance_matrix, host, launch, st);
+    if (rc != ZBALHIP_OK) return rc;
+    if (ranks > 1) {
+        const size_t bytes = (size_t)(experts / ranks) * sizeof(int64_t);
+        if (hipMemcpyAsync(host->counts, recv_tokens_per_expert, bytes, hipMemcpyDeviceToHost, st) != hipSuccess) return ZBALHIP_RT_ERROR;
+        if (hipStreamSynchronize(st) != hipSuccess) return ZBALHIP_RT_ERROR;
+    } else {
+        /*
+         * The flag arrives a few microseconds after the kernels in front of this one have run. A stream with long work
+         * queued is not spun on for more than a millisecond; the runtime's wait takes over, and reports a stream that
+         * will never get there.
+         */
+        timespec t0, t1;
+        clock_gettime(CLOCK_MONOTONIC, &t0);
+        bool arrived = false;
+        for (int spin = 0; !arrived; ++spin) {
+            arrived = __atomic_load_n(&host->ready, __ATOMIC_ACQUIRE) == launch;
+            if (arrived) break;
+            __builtin_ia32_pause();
+            if ((spin & 63) != 63) continue;
+            clock_gettime(CLOCK_MONOTONIC, &t1);
+            if ((t1.tv_sec - t0.tv_sec) * 1000000000ll + (t1.tv_nsec - t0.tv_nsec) > 1000000) break;
+        }
+        if (!arrived && hipStreamSynchronize(st) != hipSuccess) return ZBALHIP_RT_ERROR;
+        if (!arrived && __atomic_load_n(&host->ready, __ATOMIC_ACQUIRE) != launch) return ZBALHIP_RT_ERROR;
+    }
+    for (int64_t e = 0; e < experts / ranks; ++e) host_counts[e] = host->counts[e];
+    return ZBALHIP_OK;
 }

@@ -141,6 +141,29 @@ __device__ __forceinline__ float zb_expf(float x)
     return (p * s1) * s2;
 }
 
+/*
+ * Expert ids, read where the caller has them: an int32 array (stride 1) or an int64 one (stride 2), so that int64 ids
+ * need no converting launch in front of the kernel. IDS_FULL: an int64 id outside of int32 is no expert (-1);
+ * otherwise its low word counts, which is what converting the array first would have left.
+ */
+enum { IDS_I32 = 0, IDS_LOW = 1, IDS_FULL = 2 };
+struct ExpertIds {
+    const int32_t *p;
+    int kind;
+    __device__ __forceinline__ int stride() const { return kind == IDS_I32 ? 1 : 2; }
+    __device__ __forceinline__ int32_t of_words(uint32_t lo, uint32_t hi) const { return kind == IDS_FULL && hi != 0u ? -1 : (int32_t)lo; }
+    __device__ __forceinline__ int32_t operator[](int64_t i) const
+    {
+        if (kind == IDS_I32) return p[i];
+        const u32x2 w = reinterpret_cast<const u32x2 *>(p)[i];
+        return of_words(w[0], w[1]);
+    }
+};
+inline ExpertIds expert_ids(const void *p, bool is_i64, bool full = false)
+{
+    return {(const int32_t *)p, !is_i64 ? IDS_I32 : (full ? IDS_FULL : IDS_LOW)};
+}
+
 /* ---- wave64 reductions ------------------------------------------------------ */
 
 __device__ __forceinline__ float zb_wave_max(float v)

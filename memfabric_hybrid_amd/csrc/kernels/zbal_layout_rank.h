@@ -14,8 +14,7 @@
  * groups in `cnt` (one byte per wave and expert, a group has at most 64 members) and a pick's rank is the running
  * count plus the groups of the waves before its own. Ends on a barrier.
  */
-template <typename IdxT>
-__device__ __forceinline__ void rank_picks(const IdxT *__restrict__ idx, int64_t p0, int64_t p1, int experts, int nbits,
+__device__ __forceinline__ void rank_picks(const ExpertIds &idx, int64_t p0, int64_t p1, int experts, int nbits,
                                            int32_t *run, uint8_t *cnt /* [waves][experts rounded up to 4] */,
                                            int32_t *__restrict__ send_token_idx)
 {
@@ -28,10 +27,9 @@ __device__ __forceinline__ void rank_picks(const IdxT *__restrict__ idx, int64_t
 
     for (int it = 0; it < iters; ++it) {
         const int64_t i = p0 + (int64_t)it * threads + threadIdx.x;
-        int64_t e64 = (i < p1) ? (int64_t)idx[i] : -1;
+        const int e = (i < p1) ? idx[i] : -1;
         for (int j = threadIdx.x; j < nwaves * pad / 4; j += threads) reinterpret_cast<uint32_t *>(cnt)[j] = 0u;
-        const bool valid = (e64 >= 0 && e64 < experts);
-        const int e = valid ? (int)e64 : 0;
+        const bool valid = (e >= 0 && e < experts);
         uint64_t peers = __ballot(valid);
         for (int bit = 0; bit < nbits; ++bit) {
             const bool one = (e >> bit) & 1;
