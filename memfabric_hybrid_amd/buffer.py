@@ -200,25 +200,11 @@ class Buffer:
         if token_nums_type not in (0, 1):
             raise ValueError("expert_token_nums_type is invalid")
         self._wait(previous_event)
-        K = topk_idx.size(1)
-        note = self.runtime.notify(num_tokens_per_expert, K)
-        counts = None
-        if num_worst_tokens > 0:
-            rows = num_worst_tokens
-        else:
-            counts = note["recv_per_expert"].cpu()          # the one host synchronisation (zbal_deepep.cpp:359, 379)
-            total = int(counts.sum().item())
-            rows = 1 if total == 0 else total               # zbal_deepep.cpp:360
-        qm = capi.QUANT_INT8 if use_quant else capi.NO_QUANT
-        recv_x, recv_x_scales, _, h = self.runtime.dispatch(x, topk_idx, topk_weights, num_tokens_per_expert, qm,
-                                                            recv_rows=rows, notified=note)
-        num_recv_tokens_per_expert_list: List[int] = []
-        if counts is not None:
-            run = 0
-            for c in counts.tolist():
-                run = run + int(c) if token_nums_type == 0 else int(c)
-                num_recv_tokens_per_expert_list.append(run)
-        handle = (is_token_in_rank, topk_idx, topk_weights, h["put_offset"], h["balance_matrix"])
+        # without num_worst_tokens: the one host synchronisation (zbal_deepep.cpp:359, 379), at least one row (:360)
+        recv_x, recv_x_scales, num_recv_tokens_per_expert_list, put_offset, balance_matrix = self.runtime.dispatch_counts(
+            x, topk_idx, num_tokens_per_expert, capi.QUANT_INT8 if use_quant else capi.NO_QUANT, num_worst_tokens,
+            token_nums_type == 0)
+        handle = (is_token_in_rank, topk_idx, topk_weights, put_offset, balance_matrix)
         return ((recv_x, recv_x_scales) if use_quant else recv_x, None, None, num_recv_tokens_per_expert_list, handle,
                 self._event(async_finish))
 
@@ -238,7 +224,7 @@ class Buffer:
                 topk_weights_ori.dtype != torch.float32:
             raise ValueError("topk_weights check failed")
         self._wait(previous_event)
-        h = dict(put_offset=put_offset, balance_matrix=balance_matrix, expert_ids=topk_idx.to(torch.int32),
+        h = dict(put_offset=put_offset, balance_matrix=balance_matrix, expert_ids=topk_idx,
                  send_token_idx=self.runtime.send_token_idx, num_experts=put_offset.size(1))
         out = self.runtime.combine(x, h, topk_weights_ori)
         return out, None, self._event(async_finish)
@@ -295,7 +281,7 @@ class Buffer:
             blocks += [torch.zeros((1, topk_weights.size(1)), dtype=topk_weights.dtype, device=topk_weights.device)
                        for _ in range(pad["count"])]
             new_idx, new_scales = pad["topk_idx"], torch.cat(blocks, 0)
-        h = dict(expert_ids=new_idx.to(torch.int32), expand_idx=src_info, ep_recv_count=layout_range,
+        h = dict(expert_ids=new_idx, expand_idx=src_info, ep_recv_count=layout_range,
                  num_experts=num_experts)
         combined = self.runtime.low_latency_combine(x, new_scales, h)
         if pad is not None:
@@ -349,7 +335,7 @@ class Buffer:
         """A list of per-expert weights -> the list of their pre-packed forms. The whole list is one cache entry and
         one pre-pack launch (the experts stacked); the per-expert results are views of that one tensor."""
         ws = list(ws)
-        if all(getattr(t, "zbal_prepacked", False) for t in ws):
+        if capi.native().all_prepacked(ws):
             return ws
         key = ("list",) + tuple(self._weight_key(t) for t in ws)
         packed = self._cache_get(key, ws)
@@ -400,7 +386,7 @@ class Buffer:
         sw1 = self._packed_weight(share_gmm1_weight, int4) if has_share else None
         sw2 = self._packed_weight(share_gmm2_weight, int4) if has_share else None
         out, share_out, nums = self.runtime.fused_deep_moe(
-            x, topk_idx.int(), w1, gmm1_permuted_weight_scale, w2, gmm2_weight_scale, topk_weights, num_experts,
+            x, topk_idx, w1, gmm1_permuted_weight_scale, w2, gmm2_weight_scale, topk_weights, num_experts,
             quant_mode=quant_mode, expert_smooth_scales=expert_smooth_scales, share_gmm1_weight=sw1,
             share_gmm1_scale=share_gmm1_scale if has_share else None, share_gmm2_weight=sw2,
             share_gmm2_scale=share_gmm2_scale if has_share else None, share_smooth_scales=share_smooth_scales,

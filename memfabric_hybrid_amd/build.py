@@ -1,4 +1,5 @@
-"""Builds libzbal.so (HIP kernels for gfx950 + the C++ host layer) in-tree.
+"""Builds libzbal.so (HIP kernels for gfx950 + the C++ host layer) and _zbal_torch.so (the operator layer's native
+calls, against torch's headers) in-tree.
 
     python -m memfabric_hybrid_amd.build            # incremental
     python -m memfabric_hybrid_amd.build --force    # recompile everything
@@ -8,9 +9,11 @@ with -ffp-contract=off (products and sums round separately unless written as
 fmaf) and with packed fp32 instructions disabled.
 """
 import concurrent.futures
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -18,6 +21,7 @@ CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(CSRC, "_obj")
 LIB_DIR = os.path.join(PKG, "lib")
 LIB = os.path.join(LIB_DIR, "libzbal.so")
+TORCH_LIB = os.path.join(LIB_DIR, "_zbal_torch.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 KERNELS = ["layout", "dispatch", "combine", "reduce", "prepack", "gemm"]
@@ -54,6 +58,22 @@ def _run(cmd):
     return r.stdout
 
 
+def build_torch_adaptor(force=False):
+    """The native calls under operators.py. Links against the torch that will import it; libzbal.so is looked up at run time."""
+    src = os.path.join(CSRC, "torch", "zbal_torch.cpp")
+    if not force and _newer(TORCH_LIB, [src] + _headers()):
+        return TORCH_LIB
+    os.makedirs(LIB_DIR, exist_ok=True)
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    inc = os.path.join(torch_dir, "include")
+    _run(["g++"] + [f for f in HOST_FLAGS if f != "-Wextra"] +
+         ["-shared", "-DUSE_ROCM", "-I" + os.path.join(ROOT, "include"), "-isystem", inc, "-isystem",
+          os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", os.path.join(ROCM, "include"),
+          "-I" + sysconfig.get_paths()["include"], src, "-o", TORCH_LIB, "-L" + os.path.join(torch_dir, "lib"),
+          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-ldl"])
+    return TORCH_LIB
+
+
 def build_library(force=False, verbose=False):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -72,10 +92,12 @@ def build_library(force=False, verbose=False):
         objs.append(obj)
         if force or not _newer(obj, [src] + hdrs):
             jobs.append(["g++"] + HOST_FLAGS + INCLUDES + ["-c", src, "-o", obj])
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(jobs) + 1)) as ex:
+        adaptor = ex.submit(build_torch_adaptor, force)
         for out in ex.map(_run, jobs):
             if verbose and out.strip():
                 print(out)
+        adaptor.result()
     if jobs or force or not os.path.exists(LIB):
         _run([os.path.join(ROCM, "bin", "hipcc"), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs +
              ["-L" + os.path.join(ROCM, "lib"), "-lamdhip64", "-Wl,-rpath," + os.path.join(ROCM, "lib")])

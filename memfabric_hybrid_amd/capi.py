@@ -12,6 +12,7 @@ import os
 _PKG = os.path.dirname(os.path.abspath(__file__))
 # ZBAL_LIB: another build of the library (the host layer under sanitizers, `python -m memfabric_hybrid_amd.build --asan`)
 LIB_PATH = os.environ.get("ZBAL_LIB") or os.path.join(_PKG, "lib", "libzbal.so")
+NATIVE_PATH = os.path.join(_PKG, "lib", "_zbal_torch.so")
 
 ZBAL_MAX_TENSOR_DIM = 12
 ZBAL_COMM_NAME_MAX = 128
@@ -181,6 +182,27 @@ def load():
     return lib
 
 
+_native = None
+
+
+def native():
+    """The operator layer's native calls (csrc/torch/zbal_torch.cpp), bound to the library that load() returns."""
+    global _native
+    if _native is None:
+        import importlib.util
+        import torch                     # the module links against torch's libraries
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError("_zbal_torch.so is missing (%s): build it with `python -m memfabric_hybrid_amd.build`; "
+                               "there is no fallback implementation" % NATIVE_PATH)
+        spec = importlib.util.spec_from_file_location("_zbal_torch", NATIVE_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.bind(os.path.abspath(LIB_PATH), check, torch.OutOfMemoryError)
+        _native = module
+    return _native
+
+
 _GI = ctypes.POINTER(CommGroupInfo)
 _f32, _bool = ctypes.c_float, ctypes.c_bool
 # the C++-linkage launchers of include/zbal_amd_operators.h: name -> argument types (all return int32_t; references
@@ -295,6 +317,4 @@ def tensor_info(t, dtype=None, weight_format=0, shape=None):
 
 def stream_ptr(stream=None):
     """hipStream_t of a torch stream (default: the current one) as an integer."""
-    import torch
-    s = torch.cuda.current_stream() if stream is None else stream
-    return ctypes.c_void_p(s.cuda_stream)
+    return ctypes.c_void_p(native().current_stream() if stream is None else stream.cuda_stream)

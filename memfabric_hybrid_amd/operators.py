@@ -4,7 +4,8 @@
 app/zbal/src/csrc/adaptor/deepep/zbal_deepep.cpp), the C++ object the
 reference's Python `Buffer` keeps as `self.runtime`: it allocates the
 operators' tensors with the reference's shapes and dtypes and makes one or
-more calls through the zbal C ABI per method. Nothing here synchronises with
+more calls through the zbal C ABI per method, in native code
+(csrc/torch/zbal_torch.cpp). Nothing here synchronises with
 the host; the DeepEP-compatible signatures, handle tuples and Python lists
 live in buffer.py. Differences from the reference's adaptor, all deliberate:
   * no host synchronisation between notify and dispatch (the reference reads
@@ -86,7 +87,9 @@ class OperatorBuffer:
             raise RuntimeError("memfabric_hybrid_amd needs a GPU; there is no CPU path")
         self.device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
         self.lib = capi.load()
+        self.native = capi.native()
         self.comm = _acquire(self.device.index or 0)
+        self._comm, self._dev = self.comm.value, self.device.index or 0      # as the native calls take them
         self.send_token_idx = None       # kept between layout, dispatch and combine (zbal_deepep.cpp:254,305,423)
         self._tables = {}                # device address tables of tensor-list operands
         self._closed = False
@@ -110,68 +113,26 @@ class OperatorBuffer:
     def _ti(t, **kw):
         return ctypes.byref(capi.tensor_info(t, **kw))
 
-    def _list_ti(self, seq, num_experts, live, **kw):
-        """Descriptor of a tensor list: shape and type of the stacked tensor, `data` = a device table of the
-        per-expert addresses (kept in a small cache, so repeated calls with the same tensors copy nothing). The
-        descriptor holds the table's raw address only, so the table itself is appended to `live`, which the caller
-        keeps until its operator call has been issued: the cache may drop its own reference at any insertion."""
-        if len(seq) != num_experts:
-            raise ValueError("a tensor list needs one tensor per expert")
-        first = seq[0]
-        per = tuple(first.shape[1:]) if first.shape[0] == 1 and first.dim() == 3 else tuple(first.shape)
-        for t in seq:
-            if not t.is_contiguous() or t.dtype != first.dtype or t.numel() != first.numel():
-                raise ValueError("tensor-list entries must be contiguous and alike")
-        key = tuple(t.data_ptr() for t in seq)
-        table = self._tables.pop(key, None)
-        if table is None:
-            table = torch.tensor(key, dtype=torch.int64).to(self.device)
-        self._tables[key] = table        # most recently used last
-        while len(self._tables) > 64:
-            del self._tables[next(iter(self._tables))]
-        live.append(table)
-        ti = capi.tensor_info(first, shape=(num_experts,) + per, **kw)
-        ti.data = table.data_ptr()
-        return ctypes.byref(ti)
-
     # -- router (extension) ------------------------------------------------------------------
     def topk_route(self, logits, num_topk, idx_dtype=torch.int64):
         """idx_dtype: torch.int64 (what get_dispatch_layout takes) or torch.int32 (what dispatch / fused_deep_moe take)"""
-        T = logits.shape[0]
-        idx = self._empty((T, num_topk), idx_dtype)
-        w = self._empty((T, num_topk), torch.float32)
-        capi.check("zbal_moe_topk_route", self.lib.zbal_moe_topk_route(
-            self._ti(logits), num_topk, self._ti(idx), self._ti(w), self.comm, capi.stream_ptr(), 0))
-        return idx, w
+        return self.native.topk_route(self._comm, self._dev, logits, num_topk, idx_dtype == torch.int64)
 
     # -- normal mode -------------------------------------------------------------------------
     def get_dispatch_layout(self, topk_idx, num_experts):
         """zbal_deepep.cpp:209-257. Returns (num_tokens_per_rank, None, num_tokens_per_expert, is_token_in_rank, None)."""
         assert topk_idx.dim() == 2 and topk_idx.is_contiguous() and topk_idx.dtype == torch.int64
-        T, K = topk_idx.shape
-        per_expert = self._empty((num_experts,), torch.int32)
-        per_rank = self._empty((self.num_ranks,), torch.int32)
-        send_idx = self._empty((T, K), torch.int32)
-        scratch = self._empty((num_experts * 50,), torch.int32)
-        capi.check("zbal_dispatch_normal_layout", self.lib.zbal_dispatch_normal_layout(
-            self._ti(topk_idx), T, num_experts, K, self._ti(per_rank), self._ti(per_expert), self._ti(send_idx),
-            self._ti(scratch), self.comm, capi.stream_ptr(), 0))
-        self.send_token_idx = send_idx
-        valid = (topk_idx >= 0) & (topk_idx < num_experts)
-        is_token_in_rank = valid.any(dim=1, keepdim=True).to(torch.int32)   # the reference leaves this unwritten
+        # (the reference leaves is_token_in_rank unwritten)
+        per_rank, per_expert, self.send_token_idx, is_token_in_rank = self.native.layout(self._comm, self._dev, topk_idx,
+                                                                                         num_experts)
         return per_rank, None, per_expert, is_token_in_rank, None
 
     def notify(self, num_tokens_per_expert, num_topk):
         """zbal_deepep.cpp:318-357: received counts, exclusive put offsets and the balance matrix, left on the device."""
-        E = num_tokens_per_expert.shape[0]
-        note = dict(recv_data=self._empty((1, E), torch.int32), recv_per_expert=self._empty((E,), torch.int64),
-                    put_offset=self._empty((1, E), torch.int32), balance_matrix=self._empty((1, 2), torch.int32),
-                    total_recv=self._empty((1,), torch.int32))
-        capi.check("zbal_dispatch_normal_notify", self.lib.zbal_dispatch_normal_notify(
-            self._ti(num_tokens_per_expert), E, num_topk, self._ti(note["recv_data"]), self._ti(note["total_recv"]),
-            self._ti(note["recv_per_expert"]), self._ti(note["put_offset"]), self._ti(note["balance_matrix"]),
-            self.comm, capi.stream_ptr(), 0))
-        return note
+        recv_data, recv_per_expert, put_offset, balance, total = self.native.notify(self._comm, self._dev,
+                                                                                    num_tokens_per_expert, num_topk)
+        return dict(recv_data=recv_data, recv_per_expert=recv_per_expert, put_offset=put_offset, balance_matrix=balance,
+                    total_recv=total)
 
     def dispatch(self, x, topk_idx, topk_weights, num_tokens_per_expert, quant_mode=capi.NO_QUANT, recv_rows=None,
                  notified=None):
@@ -186,75 +147,39 @@ class OperatorBuffer:
         note = self.notify(num_tokens_per_expert, K) if notified is None else notified
         put_offset, balance = note["put_offset"], note["balance_matrix"]
         rows = max(T * K, 1) if recv_rows is None else max(int(recv_rows), 1)
-        if quant_mode == capi.NO_QUANT:
-            recv_x = self._empty((rows, H), x.dtype)
-            scales = self._empty((1,), torch.float32)
-        elif quant_mode == capi.QUANT_INT8:
-            recv_x = self._empty((rows, H), torch.int8)
-            scales = self._empty((rows,), torch.float32)
-        else:
-            recv_x = self._empty((rows, H), torch.float8_e4m3fn)
-            scales = self._empty((rows, H // 128), torch.float32)
-        capi.check("zbal_dispatch_normal", self.lib.zbal_dispatch_normal(
-            self._ti(x), self._ti(expert_ids), self._ti(self.send_token_idx), self._ti(put_offset), self._ti(balance),
-            E, quant_mode, self._ti(recv_x), self._ti(scales), self.comm, capi.stream_ptr(), 0))
+        recv_x, scales = self.native.dispatch(self._comm, self._dev, x, expert_ids, self.send_token_idx, put_offset, balance,
+                                              E, quant_mode, rows)
         handle = dict(put_offset=put_offset, balance_matrix=balance, expert_ids=expert_ids,
                       send_token_idx=self.send_token_idx, total_recv=note["total_recv"], num_experts=E)
         return recv_x, scales, note["recv_per_expert"], handle
 
+    def dispatch_counts(self, x, topk_idx, num_tokens_per_expert, quant_mode, num_worst_tokens, running_sums):
+        """notify() and dispatch() as one native call, the counts read back unless num_worst_tokens says how many rows
+        to allow for. Returns (recv_x, recv_x_scales, list of received counts, put_offset, balance_matrix)."""
+        assert self.send_token_idx is not None, "call get_dispatch_layout first"
+        return self.native.dispatch_counts(self._comm, self._dev, x, topk_idx, self.send_token_idx, num_tokens_per_expert,
+                                           quant_mode, num_worst_tokens, running_sums)
+
     def combine(self, x, handle, topk_weights):
         """zbal_deepep.cpp:395-452."""
-        T, K = handle["expert_ids"].shape
-        H = x.shape[1]
-        out = self._empty((T, H), x.dtype)
-        capi.check("zbal_combine_normal", self.lib.zbal_combine_normal(
-            self._ti(x), self._ti(handle["put_offset"]), self._ti(topk_weights), self._ti(handle["expert_ids"]),
-            self._ti(handle["send_token_idx"]), self._ti(handle["balance_matrix"]), handle["num_experts"],
-            self._ti(out), self.comm, capi.stream_ptr(), 0))
-        return out
+        return self.native.combine(self._comm, self._dev, x, handle["put_offset"], topk_weights, handle["expert_ids"],
+                                   handle["send_token_idx"], handle["balance_matrix"], handle["num_experts"])
 
     # -- low-latency mode ----------------------------------------------------------------------
     def low_latency_dispatch(self, x, topk_idx, num_max_dispatch_tokens_per_rank, num_experts, use_fp8=True,
                              fp8_block_scale=False):
         """zbal_deepep.cpp:454-565. Returns (packed_recv_x, packed_recv_x_scales, packed_recv_count, handle)."""
-        T, H = x.shape
-        K = topk_idx.shape[1]
-        expert_ids = topk_idx.to(torch.int32)
-        rows = max(T * K, 1)
         token_nums_type = int(os.environ.get("MOE_EXPERT_TOKEN_NUMS_TYPE", "1"))
-        if not use_fp8:
-            qm, recv = capi.NO_QUANT, self._empty((rows, H), x.dtype)
-            scales = self._empty((rows,), torch.float32)
-        elif fp8_block_scale:
-            qm, recv = capi.QUANT_FP8_B128, self._empty((rows, H), torch.float8_e4m3fn)
-            scales = self._empty((rows, H // 128), torch.float32)
-        else:
-            qm, recv = capi.QUANT_INT8, self._empty((rows, H), torch.int8)
-            scales = self._empty((rows,), torch.float32)
-        expand_idx = self._empty((rows,), torch.int32)
-        ep_recv_count = self._empty((num_experts,), torch.int32)
-        packed_recv_count = self._empty((num_experts,), torch.int64)
-        put_offset = self._empty((num_experts,), torch.int32)
-        put_offset_status = self._empty((num_experts,), torch.float32)
-        capi.check("zbal_dispatch_low_latency", self.lib.zbal_dispatch_low_latency(
-            self._ti(x), self._ti(expert_ids), num_experts, 1, 0, qm, max(T, num_max_dispatch_tokens_per_rank), 0,
-            token_nums_type, self._ti(recv), self._ti(scales), self._ti(expand_idx), self._ti(packed_recv_count),
-            self._ti(ep_recv_count), self._ti(put_offset), self._ti(put_offset_status), self.comm, capi.stream_ptr(),
-            0))
-        handle = dict(expert_ids=expert_ids, expand_idx=expand_idx, ep_recv_count=ep_recv_count,
-                      num_experts=num_experts)
+        qm = capi.NO_QUANT if not use_fp8 else capi.QUANT_FP8_B128 if fp8_block_scale else capi.QUANT_INT8
+        recv, scales, packed_recv_count, expand_idx, ep_recv_count = self.native.ll_dispatch(
+            self._comm, self._dev, x, topk_idx, num_max_dispatch_tokens_per_rank, num_experts, qm, token_nums_type)
+        handle = dict(expert_ids=topk_idx, expand_idx=expand_idx, ep_recv_count=ep_recv_count, num_experts=num_experts)
         return recv, scales, packed_recv_count, handle
 
     def low_latency_combine(self, x, topk_weights, handle):
         """zbal_deepep.cpp:567-656."""
-        T, K = handle["expert_ids"].shape
-        H = x.shape[1]
-        out = self._empty((T, H), x.dtype)
-        capi.check("zbal_combine_low_latency", self.lib.zbal_combine_low_latency(
-            self._ti(x), self._ti(handle["expert_ids"]), self._ti(handle["expand_idx"], shape=(T, K)),
-            self._ti(handle["ep_recv_count"]), self._ti(topk_weights), self._ti(out), handle["num_experts"],
-            self.comm, capi.stream_ptr(), 0))
-        return out
+        return self.native.ll_combine(self._comm, self._dev, x, handle["expert_ids"], handle["expand_idx"],
+                                      handle["ep_recv_count"], topk_weights, handle["num_experts"])
 
     # -- fused MoE ------------------------------------------------------------------------------
     def prepack_weight(self, w, int4=False):
@@ -287,41 +212,8 @@ class OperatorBuffer:
         expert. x_active_mask [T] bool: only the first sum(mask) tokens are routed; the other rows of `out` keep
         their contents. is_tensor_list: the four routed-expert operands are sequences of per-expert tensors (each
         pre-packed on its own, [1,N,K] or [N,K]); the library receives one device table of addresses per operand."""
-        T, H = x.shape
-        K = topk_idx.shape[1]
-        n1 = gmm1_permuted_weight[0].shape[-2] if is_tensor_list else gmm1_permuted_weight.shape[1]
-        shared = share_gmm1_weight is not None
-        sn1 = share_gmm1_weight.shape[-2] if shared else 0
-        expert_ids = topk_idx if topk_idx.dtype == torch.int32 else topk_idx.to(torch.int32)
-        if workspace is None:
-            workspace = self._empty((self.fused_workspace_bytes(T, H, K, num_experts, n1, quant_mode, sn1),), torch.uint8)
-        if out is None:
-            out = self._empty((T, H), x.dtype)
-        if shared and share_out is None:
-            share_out = self._empty((T, H), x.dtype)
-        if not shared:
-            share_out = None
-        token_nums = self._empty((num_experts,), torch.int64)
-        wdt = {0: None, 1: None, 2: capi.DT_FP8_E4M3, 3: capi.DT_INT4X2}[quant_mode]
-        null = ctypes.byref(capi.TensorInfo())
-        live = []                        # this call's address tables, referenced until the call has been issued
-        if is_tensor_list:
-            def wti(t, **kw):
-                return self._list_ti(t, num_experts, live, **kw)
-        else:
-            wti = self._ti
-        capi.check("zbal_fused_deep_moe", self.lib.zbal_fused_deep_moe(
-            self._ti(x), self._ti(expert_ids),
-            wti(gmm1_permuted_weight, dtype=wdt, weight_format=capi.WEIGHT_FORMAT_PREPACKED),
-            wti(gmm1_permuted_weight_scale),
-            wti(gmm2_weight, dtype=wdt, weight_format=capi.WEIGHT_FORMAT_PREPACKED), wti(gmm2_weight_scale),
-            self._ti(topk_weights), self._ti(expert_smooth_scales) if expert_smooth_scales is not None else null,
-            self._ti(share_gmm1_weight, dtype=wdt, weight_format=capi.WEIGHT_FORMAT_PREPACKED) if shared else null,
-            self._ti(share_gmm1_scale) if shared else null,
-            self._ti(share_gmm2_weight, dtype=wdt, weight_format=capi.WEIGHT_FORMAT_PREPACKED) if shared else null,
-            self._ti(share_gmm2_scale) if shared else null,
-            self._ti(share_smooth_scales) if share_smooth_scales is not None else null,
-            self._ti(x_active_mask.view(torch.uint8)) if x_active_mask is not None else null,
-            self._ti(out), self._ti(share_out) if shared else null, self._ti(token_nums), self._ti(workspace),
-            num_experts, quant_mode, 0, n1, sn1, int(is_tensor_list), self.comm, capi.stream_ptr(), 0))
-        return out, share_out, token_nums
+        return self.native.fused(
+            self._comm, self._dev, x, topk_idx, gmm1_permuted_weight, gmm1_permuted_weight_scale, gmm2_weight,
+            gmm2_weight_scale, topk_weights, num_experts, quant_mode, expert_smooth_scales, share_gmm1_weight,
+            share_gmm1_scale, share_gmm2_weight, share_gmm2_scale, share_smooth_scales, x_active_mask, workspace, out,
+            share_out, is_tensor_list, self._tables)
