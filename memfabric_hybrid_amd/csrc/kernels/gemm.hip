@@ -14,9 +14,9 @@
  * scales 16-byte vectors, gate/up pairs of the SwiGLU sit in the same lane,
  * and results leave as 8-element vectors.
  *
- * Workgroup tile: 256 (or 128) token rows x 256 output channels x 128 K-bytes
- * per step, eight (four) waves, each wave 64 rows x 128 channels = 4x8 MFMA
- * tiles (128 accumulator registers). For GMM1 the 256 channels are 128 gate
+ * Workgroup tile: 64 to 320 token rows x 256 output channels x 128 K-bytes per
+ * step, eight waves; in the 256-row shape each wave has 64 rows x 128 channels
+ * = 4x8 MFMA tiles (128 accumulator registers). For GMM1 the 256 channels are 128 gate
  * columns j and the matching 128 up columns I+j, so the SwiGLU product and,
  * in the fp8 mode, the complete 1x128 requantisation happen in registers.
  * K slabs go from HBM to LDS by DMA, in a swizzled order that the weights are
@@ -99,11 +99,12 @@ __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float 
  * rows, for token row (RG*mt + wm)*16 + lane%16 of the tile (RG = row groups of waves; a wave's 16-row sub-tiles
  * are dealt round-robin over the row groups, so a tile that is not full leaves every SIMD the same share). The pre-pack put channels 32*(nt/2) + 8*(lane/16) + 4*(nt%2) + i in
  * those rows (zb_block_row_channel), so the sub-tiles nt = 2s and 2s+1 together are eight consecutive channels.
- * `lds_rowmax` is [2][tile_rows] floats of scratch for the row maxima of the two channel halves (GMM1 only).
+ * A wave's NT channel sub-tiles are 16 * NT consecutive channels (GMM1: 8 * NT gate and the matching 8 * NT up columns).
+ * `lds_rowmax` is [16 / NT][tile_rows] floats of scratch for the row maxima of the waves' channel ranges (GMM1 only).
  */
-template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM>
-__device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &tc, f32x4 (&accf)[MTM][8],
-                                         i32x4 (&acci)[MTM][8], int row_begin, int row_end, int wm, int wn, int lane,
+template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT>
+__device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &tc, f32x4 (&accf)[MTM][NT],
+                                         i32x4 (&acci)[MTM][NT], int row_begin, int row_end, int wm, int wn, int lane,
                                          float *lds_rowmax, int tile_rows, const float *es)
 {
     /*
@@ -128,8 +129,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             if (MODE == MODE_W8A8) xs = es_row[(RG * mt + wm) * 16 + frag_row];
             else if (MODE == MODE_W4A8) xs = p.a_scale[row];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {         /* sub-tiles 2s and 2s+1: eight consecutive channels from n */
-                const int nl = wn * 128 + s * 32 + q8;       /* within the tile */
+            for (int s = 0; s < NT / 2; ++s) {    /* sub-tiles 2s and 2s+1: eight consecutive channels from n */
+                const int nl = wn * (16 * NT) + s * 32 + q8;       /* within the tile */
                 const int n = tc.n_tile * BN + nl;
                 float ws[8];
                 if constexpr (MODE == MODE_W8A8) {
@@ -164,8 +165,9 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             }
         }
     } else {
-        /* SwiGLU on gate sub-tile nt and up sub-tile nt+4: columns j = n_tile*128 + wn*64 + 32*(nt/2) + q8 + 4*(nt%2) + i */
-        float sg[MTM][4][4];
+        /* SwiGLU on gate sub-tile nt and up sub-tile nt + NT/2: columns j = n_tile*128 + 32*(t/2) + q8 + 4*(t%2) + i with t = wn*NT/2 + nt */
+        constexpr int UP = NT / 2, COL_GROUPS = 16 / NT;
+        float sg[MTM][UP][4];
         float rmax[MTM];
 #pragma unroll
         for (int mt = 0; mt < MTM; ++mt) {
@@ -181,8 +183,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             else if (MODE == MODE_W4A8) xs = p.a_scale[row < p.max_rows ? row : p.max_rows - 1];
             rmax[mt] = 0.0f;
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) {
-                const int jl = wn * 64 + (nt >> 1) * 32 + q8 + (nt & 1) * 4;       /* within the tile's 128 SwiGLU columns */
+            for (int nt = 0; nt < UP; ++nt) {
+                const int t = wn * UP + nt, jl = (t >> 1) * 32 + q8 + (t & 1) * 4;       /* within the tile's 128 SwiGLU columns */
                 float g[4], u[4];
                 if constexpr (MODE == MODE_W8A8) {
                     const f32x4 wg = *reinterpret_cast<const f32x4 *>(es + jl);             /* gate scales, then up scales */
@@ -190,14 +192,14 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         g[i] = ((float)acci[mt][nt][i] * wg[i]) * xs;
-                        u[i] = ((float)acci[mt][nt + 4][i] * wu[i]) * xs;
+                        u[i] = ((float)acci[mt][nt + UP][i] * wu[i]) * xs;
                     }
                 } else if constexpr (MODE == MODE_FP8) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) { g[i] = accf[mt][nt][i]; u[i] = accf[mt][nt + 4][i]; }
+                    for (int i = 0; i < 4; ++i) { g[i] = accf[mt][nt][i]; u[i] = accf[mt][nt + UP][i]; }
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) { g[i] = accf[mt][nt][i] * xs; u[i] = accf[mt][nt + 4][i] * xs; }
+                    for (int i = 0; i < 4; ++i) { g[i] = accf[mt][nt][i] * xs; u[i] = accf[mt][nt + UP][i] * xs; }
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -223,27 +225,31 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
         for (int mt = 0; mt < MTM; ++mt) {
             const int lr = (RG * mt + wm) * 16 + frag_row;
             const int row = row_begin + lr;
-            const float amax_tile = fmaxf(lds_rowmax[lr], lds_rowmax[tile_rows + lr]);
+            float amax_tile = lds_rowmax[lr];
+#pragma unroll
+            for (int g = 1; g < COL_GROUPS; ++g) amax_tile = fmaxf(amax_tile, lds_rowmax[g * tile_rows + lr]);
             if (row >= row_end) continue;
             if constexpr (MODE == MODE_FP8) {
                 const float amax = fmaxf(amax_tile, 1e-4f);
                 const float mult = 448.0f / amax;
                 uint8_t *q2 = (uint8_t *)p.out;
+                uint32_t q[UP];
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {         /* sub-tiles 2s and 2s+1: eight consecutive columns */
-                    const int j = tc.n_tile * 128 + wn * 64 + s * 32 + q8;
-                    u32x2 v;
+                for (int nt = 0; nt < UP; ++nt)
+                    q[nt] = pack4_e4m3(sg[mt][nt][0] * mult, sg[mt][nt][1] * mult, sg[mt][nt][2] * mult, sg[mt][nt][3] * mult);
+                uint8_t *q2row = q2 + (int64_t)row * I + tc.n_tile * 128;
+                if constexpr (UP == 1) {
+                    *reinterpret_cast<uint32_t *>(q2row + (wn >> 1) * 32 + q8 + (wn & 1) * 4) = q[0];
+                } else {
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        v[h] = pack4_e4m3(sg[mt][2 * s + h][0] * mult, sg[mt][2 * s + h][1] * mult, sg[mt][2 * s + h][2] * mult,
-                                          sg[mt][2 * s + h][3] * mult);
-                    *reinterpret_cast<u32x2 *>(q2 + (int64_t)row * I + j) = v;
+                    for (int s = 0; s < UP / 2; ++s)      /* sub-tiles 2s and 2s+1: eight consecutive columns */
+                        *reinterpret_cast<u32x2 *>(q2row + wn * (8 * NT) + s * 32 + q8) = u32x2{q[2 * s], q[2 * s + 1]};
                 }
                 if (wn == 0 && lane < 16) p.out_scale[(int64_t)row * (I / 128) + tc.n_tile] = amax * (1.0f / 448.0f);
             } else {
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt) {
-                    const int j = tc.n_tile * 128 + wn * 64 + (nt >> 1) * 32 + q8 + (nt & 1) * 4;
+                for (int nt = 0; nt < UP; ++nt) {
+                    const int t = wn * UP + nt, j = tc.n_tile * 128 + (t >> 1) * 32 + q8 + (t & 1) * 4;
                     const f32x4 v = f32x4{sg[mt][nt][0], sg[mt][nt][1], sg[mt][nt][2], sg[mt][nt][3]};
                     *reinterpret_cast<f32x4 *>(p.sgl_ws + (int64_t)row * I + j) = v;
                 }
@@ -255,8 +261,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
 
 /* ------------------------------------------------------------------------------------------------------
  * The grouped GEMM kernel (W8A8, fp8, W4A8): TM token rows x 256 channels x 128 K elements per workgroup,
- * eight waves (four row groups x two 128-channel halves; a wave's rows are the 16-row sub-tiles s with
- * s % 4 = its row group), one workgroup per CU.
+ * eight waves (RG row groups x 8 / RG channel ranges; a wave's rows are the 16-row sub-tiles s with
+ * s % RG = its row group), one workgroup per CU.
  *
  * K slabs go from HBM to LDS without passing through registers: every wave issues
  * global_load_lds_dwordx4, which deposits the 64 lanes' 16-byte chunks in 1 KiB of consecutive LDS
@@ -267,11 +273,12 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
  * pairs, so the read is free of bank conflicts whether the LDS serves 8 or 16 lanes per pass; plain
  * row-major storage would put all 16 rows on the same slot.
  *
- * Three shapes are built. TM = 256 and TM = 320 with two stages of 64 / 72 KiB (the slab for step k+1 is in
- * flight while step k is multiplied) have the arithmetic intensity that many-row experts need; the 320-row
- * shape gives every wave a fifth sub-tile. TM = 128 with three stages of 48 KiB is for
- * few-row experts, where the job is to stream every weight byte once at HBM speed: it keeps two weight slabs
- * (64 KiB) in flight per CU, two sub-tiles per wave, and skips the MFMAs of sub-tiles past the expert's end.
+ * TM = 256 and TM = 320 with two stages of 64 / 72 KiB (the slab for step k+1 is in flight while step k is
+ * multiplied) have the arithmetic intensity that many-row experts need; the 320-row shape gives every wave a fifth
+ * sub-tile. TM = 128 and TM = 64 with three or four stages are for few-row experts, where the job is to stream every
+ * weight byte once at HBM speed: two weight slabs or more stay in flight per CU, and the MFMAs of sub-tiles past the
+ * expert's end are skipped; W4A8, bound by its vector instructions, also has a 192-row shape. The few-row shapes and
+ * that one split a tile over one or two row groups of waves instead of four (FewRows, launch_w4a8).
  * Either way there is one barrier per step.
  *
  * W4A8: the weight slab stays packed in LDS (64 bytes per channel; block layout and nibble order as written by
@@ -282,12 +289,14 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
 constexpr int D_MAX_KB = 256;                 /* K up to 32768 */
 constexpr int D_MAX_EXPERTS = 1024;
 
-/* WRB = bytes of one weight row per slab: 128 (8-bit) or 64 (packed int4) */
-template <int TM, int NSTAGE, int WRB>
+/* WRB = bytes of one weight row per slab: 128 (8-bit) or 64 (packed int4); RG = row groups of waves */
+template <int TM, int NSTAGE, int WRB, int RG>
 struct DmaShape {
-    static constexpr int ROW_GROUPS = 4;                   /* row groups of two waves each: eight waves, two per SIMD */
+    static constexpr int NW = 8;                           /* eight waves, two per SIMD */
+    static constexpr int ROW_GROUPS = RG;
+    static constexpr int COL_GROUPS = NW / RG;             /* the waves of a row group split the tile's 256 channels */
+    static constexpr int NT = 16 / COL_GROUPS;             /* 16-channel sub-tiles per wave: 8 or 4 */
     static constexpr int MTM = (TM / 16 + ROW_GROUPS - 1) / ROW_GROUPS;   /* 16-row sub-tiles per wave, at most: 2, 4, or 5 in the 320-row shape */
-    static constexpr int NW = ROW_GROUPS * 2;
     static constexpr int THREADS = NW * 64;
     static constexpr int A_BYTES = TM * BKB;
     static constexpr int W_BYTES = BN * WRB;
@@ -299,13 +308,14 @@ struct DmaShape {
     static constexpr int PARTS = W_PARTS > A_PARTS ? W_PARTS : A_PARTS;
     static constexpr bool TWO_PHASE = TM == 256;            /* the tiles of short experts run after all the others (see the kernel) */
     /* two buffers of per-tile scales, floats each: fp8 2 x D_MAX_KB weight block scales; W8A8 256 channel + TM token scales */
-    static constexpr int SW_STRIDE = TM > 256 ? 576 : 2 * D_MAX_KB;
+    static constexpr int SW_STRIDE = WRB == 64 ? 0 : (TM > 256 ? 576 : 2 * D_MAX_KB);      /* W4A8 has its own (lds_gs) */
     static constexpr int SW_BYTES = 2 * SW_STRIDE * 4;
-    static_assert(SW_STRIDE >= 2 * D_MAX_KB && SW_STRIDE >= 256 + TM, "scale buffer too small");
-    static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES + NSTAGE * TM * 4 + 2 * TM * 4 + SW_BYTES +
+    static_assert(WRB == 64 || (SW_STRIDE >= 2 * D_MAX_KB && SW_STRIDE >= 256 + TM), "scale buffer too small");
+    static constexpr int SA_FLOATS = WRB == 64 ? 0 : NSTAGE * TM;      /* the fp8 mode's activation block scales */
+    static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES + SA_FLOATS * 4 + COL_GROUPS * TM * 4 + SW_BYTES +
                                      2 * (MAX_EXPERTS + 1) * 4 + (WRB == 64 ? NSTAGE * BN * 2 : 0) +
                                      (TWO_PHASE ? MAX_EXPERTS * 2 + (MAX_EXPERTS + 1) * 4 : 0);
-    static_assert(PARTS >= 2 && (PARTS % 4 == 0 || PARTS == 2 || (NSTAGE == 2 && PARTS == 5)),
+    static_assert(PARTS >= 2 && (TM % (8 * NW) == 0 || NSTAGE == 2),
                   "the issue schedule hands out parts q * PARTS / 4 .. (q + 1) * PARTS / 4 - 1 of a slab with quarter q of a step");
     static_assert(NW <= HALF_BLOCKS && HALF_BLOCKS % NW == 0, "a wave's W blocks must not straddle a weight half");
     static_assert(LDS_BYTES <= 160 * 1024, "tile does not fit the LDS");
@@ -375,6 +385,25 @@ __device__ __forceinline__ void wait_vmcnt()
     __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+/*
+ * Wait for the oldest slab in flight with `later` (MOST at most) younger slabs left alone; OPS operations per slab, one
+ * more where `extra` (wave-uniform).
+ */
+template <int MOST, int OPS>
+__device__ __forceinline__ void wait_slab(int later, bool extra)
+{
+    if constexpr (MOST > 0) {
+        if (later >= MOST) {
+            if (extra) wait_vmcnt<MOST * (OPS + 1)>();
+            else wait_vmcnt<MOST * OPS>();
+        } else {
+            wait_slab<MOST - 1, OPS>(later, extra);
+        }
+    } else {
+        wait_vmcnt<0>();
+    }
+}
+
 /* what a workgroup needs to know about one tile; every member is wave-uniform and lives in scalar registers */
 struct DmaTile {
     bool valid;
@@ -385,7 +414,7 @@ struct DmaTile {
     const uint16_t *gs_mine;          /* W4A8: fp16 group scales, slab 0, of the weight half this wave brings in (wave % 2) */
 };
 
-template <int MODE, bool GMM1, int OUT_DT, int TM, int NSTAGE, bool WSTREAM>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int NSTAGE, int RG, bool WSTREAM>
 /*
  * Eight waves, two per SIMD (256 registers each), in every shape. The 128-row shape used to run four waves with the
  * wave tile of the 256-row shape (64 x 128), one per SIMD with nobody to cover its waits; as eight waves of 32 x 128
@@ -396,18 +425,17 @@ __global__ void __launch_bounds__(512, 2)
 grouped_gemm_dma_kernel(GemmParams p)
 {
     static_assert(MODE == MODE_W8A8 || MODE == MODE_FP8 || MODE == MODE_W4A8, "unknown mode");
-    static_assert(NSTAGE == 2 || NSTAGE == 3, "two or three stages");
     constexpr int WRB = MODE == MODE_W4A8 ? 64 : 128;
-    using S = DmaShape<TM, NSTAGE, WRB>;
+    using S = DmaShape<TM, NSTAGE, WRB, RG>;
+    constexpr int COL_GROUPS = S::COL_GROUPS, NT = S::NT;
     constexpr int NW = S::NW, STAGE_BYTES = S::STAGE_BYTES, A_BYTES = S::A_BYTES, W_PARTS = S::W_PARTS, PARTS = S::PARTS;
     constexpr int HALF_BLOCKS = S::HALF_BLOCKS, W_BLOCK_BYTES = 128 * WRB;     /* one 128-channel block of one slab */
-    constexpr int RG = S::ROW_GROUPS;                /* row groups of waves; 16-row sub-tile s of a tile belongs to group s % RG */
     using Tile = DmaTile;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     float *lds_sa = reinterpret_cast<float *>(smem + NSTAGE * STAGE_BYTES);   /* [NSTAGE][TM] */
-    float *lds_rowmax = lds_sa + NSTAGE * TM;                                 /* [2][TM] */
+    float *lds_rowmax = lds_sa + S::SA_FLOATS;                                 /* [COL_GROUPS][TM] */
     constexpr int SW_STRIDE = S::SW_STRIDE;
-    float *lds_sw = lds_rowmax + 2 * TM;                                      /* [2 tiles][SW_STRIDE]: fp8 [2][D_MAX_KB] weight block scales */
+    float *lds_sw = lds_rowmax + COL_GROUPS * TM;                                      /* [2 tiles][SW_STRIDE]: fp8 [2][D_MAX_KB] weight block scales */
     int *lds_mtp = reinterpret_cast<int *>(lds_sw + 2 * SW_STRIDE);            /* [experts + 1] tiles of TM rows before expert e */
     int *lds_roff = lds_mtp + (S::MAX_EXPERTS + 1);                            /* [experts + 1] copy of row_off */
     uint16_t *lds_gs = reinterpret_cast<uint16_t *>(lds_roff + (S::MAX_EXPERTS + 1));   /* [NSTAGE][BN] W4A8 group scales (fp16) */
@@ -417,7 +445,8 @@ grouped_gemm_dma_kernel(GemmParams p)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const int wm = wave_u >> 1, wn = wave_u & 1;      /* wave-uniform, so everything derived from them lives in scalar registers */
+    /* row group (16-row sub-tile s of a tile belongs to group s % RG) and channel range; wave-uniform, so everything derived from them lives in scalar registers */
+    const int wm = wave_u / COL_GROUPS, wn = wave_u % COL_GROUPS;
     const int n_tiles = GMM1 ? (p.N / 2) / 128 : p.N / BN;
     const int K = p.K;
     const int KB = K / 128;
@@ -620,14 +649,15 @@ grouped_gemm_dma_kernel(GemmParams p)
     const bool gs_wave = MODE == MODE_W4A8 && wave < 2;            /* wave h brings the group scales of weight half h */
     const uint32_t lds_gs0 = __builtin_amdgcn_readfirstlane(lds_addr(lds_gs) + (wave & 1) * 256);
     /*
-     * The 320-row shape has no register to spare for the transfers' lane offsets across a K step: there they are worked
+     * The tallest shapes have no register to spare for the transfers' lane offsets across a K step: there they are worked
      * out afresh for every transfer from a copy of the lane number that the K loop makes opaque once per step (kept
      * across the loop they were spilled, and a reload waits for the slabs in flight).
      */
+    constexpr bool FRESH_OFFSETS = TM > 256 || (MODE == MODE_W4A8 && TM >= 192);
     int lane_dma = lane;
     /* part j of a slab: the wave's j-th block of the W tile (j < W_PARTS), of the A tile (j < A_PARTS) and, with part 0, the scales */
     auto issue_part = [&](const Tile &t, int kb, int stage, int j) __attribute__((always_inline)) {
-        const int lane_x = TM > 256 ? lane_dma : lane;
+        const int lane_x = FRESH_OFFSETS ? lane_dma : lane;
         const int r0 = 8 * wave_u + (lane_x >> 3);
         const uint32_t a_chunk = ((lane_x & 7) ^ ((r0 & 7) ^ ((r0 >> 3) & 1))) * 16;
         const uint32_t w_off = wave_u * 1024 + lane_x * 16;
@@ -715,12 +745,12 @@ grouped_gemm_dma_kernel(GemmParams p)
     const int off_lo = frag_row * BKB + ((g2 ^ key) * 16), off_hi = frag_row * BKB + (((g2 + 1) ^ key) * 16);
     /* int4: one 16-byte chunk per lane, chunk lane/16 of channel lane%16 of the 16-channel block, at its swizzled slot */
     const int w4_off = frag_row * 64 + (((lane >> 4) ^ ((frag_row >> 2) & 3)) * 16);
-    int w_sub[8], w_ch[8];
+    int w_sub[NT], w_ch[NT];
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
         int r;
-        if (GMM1) r = (nt < 4) ? wn * 64 + nt * 16 : 128 + wn * 64 + (nt - 4) * 16;
-        else r = wn * 128 + nt * 16;
+        if (GMM1) r = (nt < NT / 2) ? wn * (8 * NT) + nt * 16 : 128 + wn * (8 * NT) + (nt - NT / 2) * 16;
+        else r = wn * (16 * NT) + nt * 16;
         w_sub[nt] = A_BYTES + r * WRB;
         w_ch[nt] = zb_block_row_channel(r);       /* tile-local channel held by the sub-tile's first block row */
     }
@@ -740,12 +770,12 @@ grouped_gemm_dma_kernel(GemmParams p)
         load_tile(lid, nxt);
 
         constexpr int MTM = S::MTM;
-        f32x4 accf[MTM][8];
-        i32x4 acci[MTM][8];
+        f32x4 accf[MTM][NT];
+        i32x4 acci[MTM][NT];
 #pragma unroll
         for (int mt = 0; mt < MTM; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < 8; ++nt) {
+            for (int nt = 0; nt < NT; ++nt) {
                 accf[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 acci[mt][nt] = i32x4{0, 0, 0, 0};
             }
@@ -762,16 +792,14 @@ grouped_gemm_dma_kernel(GemmParams p)
         auto k_loop = [&](auto mt_tag) __attribute__((always_inline)) {
         constexpr int MT = decltype(mt_tag)::value;
         for (int kb = 0; kb < KB; ++kb) {
-            /* the slab after this one exists if the tile or the sequence goes on; its loads may stay in flight */
-            const bool later = kb + 1 < KB || nxt.valid;
-            if (NSTAGE == 3 && later) {
-                if (extra_op_wave) wait_vmcnt<OPS + 1>();
-                else wait_vmcnt<OPS>();
-            } else {
-                wait_vmcnt<0>();
-            }
+            /*
+             * The slabs after this one that have been asked for, NSTAGE - 2 at most, may stay in flight: there are that
+             * many while the sequence goes on (the host guarantees KB >= NSTAGE - 1), fewer at its very end.
+             */
+            const int later = nxt.valid ? NSTAGE - 2 : KB - 1 - kb;
+            wait_slab<NSTAGE - 2, OPS>(later, extra_op_wave);
             __syncthreads();                /* slab kb has landed for everybody; the stage read in the step before is free */
-            if constexpr (TM > 256) asm volatile("" : "+v"(lane_dma));
+            if constexpr (FRESH_OFFSETS) asm volatile("" : "+v"(lane_dma));
             /*
              * The next tile's weight block scales go into the buffer the tile before this one used. Every wave is
              * past this tile's first barrier now, so none of them still reads that buffer; the transfers are older
@@ -801,6 +829,12 @@ grouped_gemm_dma_kernel(GemmParams p)
             auto issue_quarter = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
                 for (int j = q * PARTS / 4; j < (q + 1) * PARTS / 4; ++j) issue_part(ft, fill_kb, fill_stage, j);
+            };
+            /* the quarters that go out with channel sub-tile nt: one each with the first four, two each where a wave has only two */
+            auto issue_at = [&](int nt) __attribute__((always_inline)) {
+                constexpr int EACH = NT < 4 ? 4 / NT : 1;
+#pragma unroll
+                for (int q = nt * EACH; q < nt * EACH + EACH && q < 4; ++q) issue_quarter(q);
             };
             auto load_w = [&](int nt) -> i32x8 {
                 const u32x4 lo = *reinterpret_cast<const u32x4 *>(sb + w_sub[nt] + off_lo);
@@ -859,13 +893,13 @@ grouped_gemm_dma_kernel(GemmParams p)
                                  * GPU, 4096 tokens over 32 experts: 0.563 against 0.590 ms; the first GEMM the other way
                                  * round, 1.16 against 1.00 ms).
                                  */
-                                const float swx = wn == 1 ? sw1 : sw0;
+                                const float swx = wn >= COL_GROUPS / 2 ? sw1 : sw0;
                                 float sc[MN];
 #pragma unroll
                                 for (int m = 0; m < MN; ++m)
                                     sc[m] = lds_sa[cur_stage * TM + (RG * (M0 + m) + wm) * 16 + frag_row] * swx;
 #pragma unroll
-                                for (int nt = 0; nt < 8; ++nt) {
+                                for (int nt = 0; nt < NT; ++nt) {
                                     const i32x8 wfj = (M0 == 0 && nt == 0) ? wf_first : load_w(nt);
                                     if (M0 == 0 && more && (nt == 0 || nt == 2)) { issue_quarter(nt); issue_quarter(nt + 1); }
                                     f32x4 part = mfma_fp8_16x16x128(wfj, af[A0]);
@@ -901,16 +935,16 @@ grouped_gemm_dma_kernel(GemmParams p)
                             }
                             f32x4 part = mfma_fp8_16x16x128(wf, af[0]);
 #pragma unroll
-                            for (int nt = 0; nt < 8; ++nt) {
+                            for (int nt = 0; nt < NT; ++nt) {
                                 i32x8 wf_n = wf;
-                                if (nt + 1 < 8) wf_n = load_w(nt + 1);
+                                if (nt + 1 < NT) wf_n = load_w(nt + 1);
                                 if (M0 == 0 && more && (nt == 0 || nt == 2)) { issue_quarter(nt); issue_quarter(nt + 1); }
-                                const bool second = GMM1 ? (nt >= 4) : (wn == 1);
+                                const bool second = GMM1 ? (nt >= NT / 2) : (wn >= COL_GROUPS / 2);
 #pragma unroll
                                 for (int m = 0; m < MN; ++m) {
                                     f32x4 nxt_part = part;
                                     if (m + 1 < MN) nxt_part = mfma_fp8_16x16x128(wf, af[m + 1]);
-                                    else if (nt + 1 < 8) nxt_part = mfma_fp8_16x16x128(wf_n, af[0]);
+                                    else if (nt + 1 < NT) nxt_part = mfma_fp8_16x16x128(wf_n, af[0]);
                                     const float sc = second ? s1[m] : s0[m];
 #pragma unroll
                                     for (int i = 0; i < 4; ++i) accf[M0 + m][nt][i] = __builtin_fmaf(part[i], sc, accf[M0 + m][nt][i]);
@@ -933,21 +967,21 @@ grouped_gemm_dma_kernel(GemmParams p)
                         i32x8 wf = wf_first;
                         f32x4 part = mfma_fp8_16x16x128(wf, af[0]);
     #pragma unroll
-                        for (int nt = 0; nt < 8; ++nt) {
+                        for (int nt = 0; nt < NT; ++nt) {
                             i32x8 wf_n = wf;
-                            if (nt + 1 < 8) wf_n = load_w(nt + 1);
+                            if (nt + 1 < NT) wf_n = load_w(nt + 1);
                             /* the 256-row fp8 loop hands the slab out in two halves (0.6 % faster, measured against quarters on one GPU; the other loops are slower that way) */
                             if (TM == 256) {
                                 if (more && (nt == 0 || nt == 2)) { issue_quarter(nt); issue_quarter(nt + 1); }
-                            } else if (nt < 4 && more) {
-                                issue_quarter(nt);
+                            } else if (more) {
+                                issue_at(nt);
                             }
-                            const bool second = GMM1 ? (nt >= 4) : (wn == 1);
+                            const bool second = GMM1 ? (nt >= NT / 2) : (wn >= COL_GROUPS / 2);
     #pragma unroll
                             for (int mt = 0; mt < MT; ++mt) {
                                 f32x4 nxt_part = part;
                                 if (mt + 1 < MT) nxt_part = mfma_fp8_16x16x128(wf, af[mt + 1]);
-                                else if (nt + 1 < 8) nxt_part = mfma_fp8_16x16x128(wf_n, af[0]);
+                                else if (nt + 1 < NT) nxt_part = mfma_fp8_16x16x128(wf_n, af[0]);
                                 const float sc = second ? s1[mt] : s0[mt];
     #pragma unroll
                                 for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(part[i], sc, accf[mt][nt][i]);
@@ -966,40 +1000,53 @@ grouped_gemm_dma_kernel(GemmParams p)
                     const uint16_t *gsb = lds_gs + cur_stage * BN;
                     auto load_pk = [&](int nt) -> u32x4 { return *reinterpret_cast<const u32x4 *>(sb + w_sub[nt] + w4_off); };
                     auto load_gs = [&](int nt) -> u32x2 { return *reinterpret_cast<const u32x2 *>(gsb + lane_ch + w_ch[nt]); };
+                    /*
+                     * The sums start at the bits of 1.5 * 2^23: |pair sum| <= 128 * 128 * 128 = 2^21, so the result read as a
+                     * float is 1.5 * 2^23 + sum, exactly, and one subtraction makes it the float a conversion would. On
+                     * this GPU v_cvt_f32_i32 and v_fma_mix_f32 issue at half the rate of v_sub_f32 and v_fma_f32 (2.1
+                     * and 2.0 ns against 1.2 and 1.3 per instruction and SIMD, two waves), and next to nothing of
+                     * either hides under an MFMA, so the scales are also widened once per channel sub-tile.
+                     */
+                    constexpr float MAGIC = 12582912.0f;
+                    i32x4 magic = {0x4b400000, 0x4b400000, 0x4b400000, 0x4b400000};
+                    asm volatile("" : "+v"(magic));
                     auto lo4 = [](uint32_t v) -> int { return (int)((v << 4) & 0xf0f0f0f0u); };
                     auto hi4 = [](uint32_t v) -> int { return (int)(v & 0xf0f0f0f0u); };
                     auto mfma_pair = [&](const u32x4 &pk, const i32x8 &a) -> i32x4 {
                         const i32x4 w0 = i32x4{lo4(pk[0]), hi4(pk[0]), lo4(pk[1]), hi4(pk[1])};
                         const i32x4 w1 = i32x4{lo4(pk[2]), hi4(pk[2]), lo4(pk[3]), hi4(pk[3])};
-                        i32x4 part = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, i32x4{a[0], a[1], a[2], a[3]}, i32x4{0, 0, 0, 0}, 0, 0, 0);
+                        i32x4 part = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, i32x4{a[0], a[1], a[2], a[3]}, magic, 0, 0, 0);
                         return __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, i32x4{a[4], a[5], a[6], a[7]}, part, 0, 0, 0);
                     };
+                    constexpr bool LATE_SCALES = TM == 192;      /* no two registers to spare for fetching the scales ahead */
                     /* the packed chunk and the raw fp16 scales of the next channel sub-tile are fetched one sub-tile ahead */
                     u32x4 pk = load_pk(0);
                     u32x2 gsr = load_gs(0);
                     i32x4 part = mfma_pair(pk, af[0]);
 #pragma unroll
-                    for (int nt = 0; nt < 8; ++nt) {
+                    for (int nt = 0; nt < NT; ++nt) {
                         u32x4 pkn = pk;
                         u32x2 gsn = gsr;
-                        if (nt + 1 < 8) {
+                        if (nt + 1 < NT) {
                             pkn = load_pk(nt + 1);
-                            gsn = load_gs(nt + 1);
+                            if (!LATE_SCALES) gsn = load_gs(nt + 1);
                         }
-                        if (nt < 4 && more) issue_quarter(nt);
-                        const float gs[4] = {zb_fp16_to_f32(gsr[0] & 0xffffu), zb_fp16_to_f32(gsr[0] >> 16),
-                                             zb_fp16_to_f32(gsr[1] & 0xffffu), zb_fp16_to_f32(gsr[1] >> 16)};
+                        if (more) issue_at(nt);
+                        float gs[4] = {zb_fp16_to_f32(gsr[0] & 0xffffu), zb_fp16_to_f32(gsr[0] >> 16),
+                                       zb_fp16_to_f32(gsr[1] & 0xffffu), zb_fp16_to_f32(gsr[1] >> 16)};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) if (TM <= 128) asm("" : "+v"(gs[i]));      /* or the compiler folds the widening into v_fma_mix_f32 */
 #pragma unroll
                         for (int mt = 0; mt < MT; ++mt) {
                             i32x4 nxt_part = part;
                             if (mt + 1 < MT) nxt_part = mfma_pair(pk, af[mt + 1]);
-                            else if (nt + 1 < 8) nxt_part = mfma_pair(pkn, af[0]);
+                            else if (nt + 1 < NT) nxt_part = mfma_pair(pkn, af[0]);
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf((float)part[i], gs[i], accf[mt][nt][i]);
+                            for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(__int_as_float(part[i]) - MAGIC, gs[i], accf[mt][nt][i]);
                             part = nxt_part;
                         }
                         pk = pkn;
-                        gsr = gsn;
+                        gsr = LATE_SCALES && nt + 1 < NT ? load_gs(nt + 1) : gsn;
                     }
                 } else {
                     /*
@@ -1008,9 +1055,9 @@ grouped_gemm_dma_kernel(GemmParams p)
                      * SIMD's other wave covers the read.)
                      */
 #pragma unroll
-                    for (int nt = 0; nt < 8; ++nt) {
+                    for (int nt = 0; nt < NT; ++nt) {
                         const i32x8 wf = nt == 0 ? wf_first : load_w(nt);
-                        if (nt < 4 && more) issue_quarter(nt);
+                        if (more) issue_at(nt);
                         const i32x4 wf0 = i32x4{wf[0], wf[1], wf[2], wf[3]}, wf1 = i32x4{wf[4], wf[5], wf[6], wf[7]};
 #pragma unroll
                         for (int mt = 0; mt < MT; ++mt)
@@ -1025,7 +1072,11 @@ grouped_gemm_dma_kernel(GemmParams p)
             }
         }
         };
-        if (MTM >= 5 && mt_act == 5) k_loop(std::integral_constant<int, MTM >= 5 ? 5 : MTM>{});
+        static_assert(MTM <= 8, "sub-tiles per wave");
+        if (MTM >= 8 && mt_act == 8) k_loop(std::integral_constant<int, MTM >= 8 ? 8 : MTM>{});
+        else if (MTM >= 7 && mt_act == 7) k_loop(std::integral_constant<int, MTM >= 7 ? 7 : MTM>{});
+        else if (MTM >= 6 && mt_act == 6) k_loop(std::integral_constant<int, MTM >= 6 ? 6 : MTM>{});
+        else if (MTM >= 5 && mt_act == 5) k_loop(std::integral_constant<int, MTM >= 5 ? 5 : MTM>{});
         else if (MTM >= 4 && mt_act == 4) k_loop(std::integral_constant<int, MTM >= 4 ? 4 : MTM>{});
         else if (MTM >= 3 && mt_act == 3) k_loop(std::integral_constant<int, MTM >= 3 ? 3 : MTM>{});
         else if (MTM >= 2 && mt_act == 2) k_loop(std::integral_constant<int, MTM >= 2 ? 2 : MTM>{});
@@ -1035,7 +1086,7 @@ grouped_gemm_dma_kernel(GemmParams p)
 #pragma unroll
             for (int mt = 0; mt < MTM; ++mt)
 #pragma unroll
-                for (int nt = 0; nt < 8; ++nt)
+                for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) accf[mt][nt][i] *= 0.0625f;
         }
@@ -1050,7 +1101,7 @@ grouped_gemm_dma_kernel(GemmParams p)
          */
         int lane_e = lane;
         asm volatile("" : "+v"(lane_e));
-        epilogue<MODE, GMM1, OUT_DT, RG, S::MTM>(p, tc, accf, acci, cur.row_begin, cur.row_end, wm, wn, lane_e, lds_rowmax, TM,
+        epilogue<MODE, GMM1, OUT_DT, RG, S::MTM, NT>(p, tc, accf, acci, cur.row_begin, cur.row_end, wm, wn, lane_e, lds_rowmax, TM,
                                          lds_sw + sw_buf * SW_STRIDE);
         if (!nxt.valid) break;
         cur = nxt;
@@ -1119,13 +1170,13 @@ inline unsigned grid_for(int64_t max_rows, int64_t experts, int n_tiles, int til
  * finds its kernel unprepared does it itself, and fails with a clear error if the stream is capturing.
  * Returns the device's CU count through n_cus.
  */
-template <int MODE, bool GMM1, int OUT_DT, int TM, int NSTAGE, bool WSTREAM>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int NSTAGE, int RG, bool WSTREAM>
 int32_t prepare_shape(hipStream_t st, int *n_cus)
 {
-    using S = DmaShape<TM, NSTAGE, MODE == MODE_W4A8 ? 64 : 128>;
+    using S = DmaShape<TM, NSTAGE, MODE == MODE_W4A8 ? 64 : 128, RG>;
     static std::mutex mu;          /* one per kernel instantiation: guards its per-device set-up below */
     static int cus[64] = {};
-    const void *kern = reinterpret_cast<const void *>(&grouped_gemm_dma_kernel<MODE, GMM1, OUT_DT, TM, NSTAGE, WSTREAM>);
+    const void *kern = reinterpret_cast<const void *>(&grouped_gemm_dma_kernel<MODE, GMM1, OUT_DT, TM, NSTAGE, RG, WSTREAM>);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return ZBALHIP_RT_ERROR;
     std::lock_guard<std::mutex> guard(mu);
@@ -1146,31 +1197,48 @@ int32_t prepare_shape(hipStream_t st, int *n_cus)
 }
 
 /* launched with one persistent workgroup per CU, or fewer when there are not that many tiles */
-template <int MODE, bool GMM1, int OUT_DT, int TM, int NSTAGE, bool WSTREAM = false>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int NSTAGE, int RG, bool WSTREAM = false>
 int32_t launch_dma_shape(const GemmParams &p, int n_tiles, hipStream_t st)
 {
-    using S = DmaShape<TM, NSTAGE, MODE == MODE_W4A8 ? 64 : 128>;
+    using S = DmaShape<TM, NSTAGE, MODE == MODE_W4A8 ? 64 : 128, RG>;
     int n_cus = 0;
-    const int32_t rc = prepare_shape<MODE, GMM1, OUT_DT, TM, NSTAGE, WSTREAM>(st, &n_cus);
+    const int32_t rc = prepare_shape<MODE, GMM1, OUT_DT, TM, NSTAGE, RG, WSTREAM>(st, &n_cus);
     if (rc != ZBALHIP_OK) return rc;
     unsigned grid = grid_for(p.max_rows, p.experts, n_tiles, TM);
     const unsigned resident = (unsigned)(n_cus + 7) / 8 * 8;
     if (grid > resident) grid = resident;
-    grouped_gemm_dma_kernel<MODE, GMM1, OUT_DT, TM, NSTAGE, WSTREAM><<<grid, S::THREADS, S::LDS_BYTES, st>>>(p);
+    grouped_gemm_dma_kernel<MODE, GMM1, OUT_DT, TM, NSTAGE, RG, WSTREAM><<<grid, S::THREADS, S::LDS_BYTES, st>>>(p);
     return zbalhip_check_launch();
 }
+
+/*
+ * The shapes with few rows: rows, stages, row groups of waves. The few-row kernels are weight streams, and what a step
+ * costs beside the transfer of its slab is the waves' own work after the barrier, so the waves split the channels
+ * rather than the rows: with two row groups (W4A8's first GEMM: one) a weight fragment is read from LDS, and unpacked,
+ * by two waves instead of four, and a tile of 16 or 32 rows keeps all eight waves busy instead of two or four.
+ */
+template <int MODE, bool GMM1> struct FewRows {
+    static constexpr int RG_W4 = GMM1 ? 1 : 2;
+    static constexpr int RG = MODE == MODE_W4A8 ? RG_W4 : 2;
+    static constexpr int STAGES_64 = MODE == MODE_W4A8 ? 4 : 3;
+};
 
 /* every shape a launch of (MODE, GMM1, OUT_DT) can take */
 template <int MODE, bool GMM1, int OUT_DT>
 int32_t prepare_mode()
 {
+    using F = FewRows<MODE, GMM1>;
     int n = 0;
-    int32_t rc = prepare_shape<MODE, GMM1, OUT_DT, 256, 2, false>(nullptr, &n);
-    if constexpr (MODE != MODE_W4A8)
-        if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 320, 2, false>(nullptr, &n);
-    if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, false>(nullptr, &n);
-    if constexpr (MODE != MODE_W4A8)
-        if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, true>(nullptr, &n);
+    int32_t rc = prepare_shape<MODE, GMM1, OUT_DT, 256, 2, 4, false>(nullptr, &n);
+    if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG, false>(nullptr, &n);
+    if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 64, F::STAGES_64, F::RG, true>(nullptr, &n);
+    if constexpr (MODE == MODE_W4A8) {
+        if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, 2, false>(nullptr, &n);
+        if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 192, 3, 2, false>(nullptr, &n);
+    } else {
+        if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 320, 2, 4, false>(nullptr, &n);
+        if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG, true>(nullptr, &n);
+    }
     return rc;
 }
 
@@ -1186,13 +1254,11 @@ int32_t prepare_mode()
  *     192 rows 2.314 / 1.204 against 2.108 / 1.148;
  *   - W8A8, 32 experts: 128 rows 0.243 / 0.129 against 0.254 / 0.138; 192 rows 0.289 / 0.146 against 0.275 / 0.150;
  *     256 rows 0.342 / 0.174 against 0.303 / 0.163. 256 experts: 128 rows 1.788 / 0.892 against 1.799 / 0.931;
- *     192 rows 2.197 / 1.093 against 2.016 / 1.106;
- *   - W4A8: 96 rows 0.358 / 0.171 against 0.366 / 0.178; 128 rows 0.503 / 0.237 against 0.457 / 0.216.
+ *     192 rows 2.197 / 1.093 against 2.016 / 1.106.
  */
 template <int MODE, bool GMM1>
 inline int64_t few_rows_limit(const GemmParams &p, int n_tiles)
 {
-    if (MODE == MODE_W4A8) return 96;
     if (GMM1) return 128;
     const bool few_tiles = (int64_t)p.experts * n_tiles <= 1024;
     return (MODE == MODE_FP8 && !few_tiles) ? 128 : 192;
@@ -1217,30 +1283,66 @@ inline int64_t few_rows_limit(const GemmParams &p, int n_tiles)
  */
 constexpr int64_t kTallRowsLimitFp8 = 1536;
 
+/*
+ * W4A8: the smaller the slab (16 KiB of weights), the more a step's own work shows, and the compute-bound sizes are
+ * bound by vector instructions, a quarter of which unpack weights once per row group of waves. Shapes by rows per
+ * expert on average, first / second GEMM in us on 4096 x 3072 / 1536 x 4096, 128 experts, random routing, one GPU,
+ * old (four row groups, 128 or 256 rows) against now:
+ *   - up to 48: 64 rows, 4 stages, streaming hint: 1 row 152 / 82 -> 104 / 58, 4 rows 222 / 108 -> 155 / 78, 32 rows
+ *     263 / 127 -> 197 / 102, 44 rows 278 / 135 -> 213 / 109 (53 rows: 244 / 124, the next shape 242 / 118);
+ *   - up to 100: 128 rows, 3 stages: 64 rows 308 / 145 -> 255 / 124, 96 rows 362 / 166 -> 316 / 150;
+ *   - up to 640: 192 rows, 3 stages, two row groups: 112 rows 436 / 186 -> 368 / 169, 128 rows 440 / 197 -> 380 / 174,
+ *     256 rows 757 / 329 -> 697 / 329, 512 rows 1289 / 585 -> 1237 / 571; except where most experts just miss one tile
+ *     of it and make two of half the height, which the 128-row shape does cheaper (187 rows, 64 experts of 2048 x 2048
+ *     / 1024 x 2048: 145 / 60 against 128 / 54);
+ *   - beyond: 256 rows (1024 rows: 2456 / 1098 against 2507 / 1185).
+ */
+template <bool GMM1, int OUT_DT>
+int32_t launch_w4a8(const GemmParams &p, int n_tiles, hipStream_t st)
+{
+    using F = FewRows<MODE_W4A8, GMM1>;
+    const int64_t rows = p.max_rows, e = p.experts;
+    if (rows <= 48 * e && p.K >= 128 * (F::STAGES_64 - 1))
+        return launch_dma_shape<MODE_W4A8, GMM1, OUT_DT, 64, F::STAGES_64, F::RG, true>(p, n_tiles, st);
+    if (p.K >= 256) {
+        if (rows <= 100 * e) return launch_dma_shape<MODE_W4A8, GMM1, OUT_DT, 128, 3, F::RG>(p, n_tiles, st);
+        if (rows > 160 * e && rows <= 224 * e) return launch_dma_shape<MODE_W4A8, GMM1, OUT_DT, 128, 3, 2>(p, n_tiles, st);
+        if (rows <= 640 * e) return launch_dma_shape<MODE_W4A8, GMM1, OUT_DT, 192, 3, 2>(p, n_tiles, st);
+    }
+    return launch_dma_shape<MODE_W4A8, GMM1, OUT_DT, 256, 2, 4>(p, n_tiles, st);
+}
+
 template <int MODE, bool GMM1, int OUT_DT>
 int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
 {
-    if ((int64_t)p.max_rows <= few_rows_limit<MODE, GMM1>(p, n_tiles) * (int64_t)p.experts && p.K >= 256) {
-        /*
-         * With few rows per expert nearly every expert has a single row tile and its weight slabs are read once: they
-         * are requested with the streaming hint. Measured on 32 experts of 7168 x 4096 / 2048 x 7168, first / second
-         * GEMM: at 32 rows per expert on average fp8 11 % / 2 % and W8A8 7 % / 6 % faster (decode layer, Zipf routing:
-         * 0.304 -> 0.288 ms); at 64 rows W8A8 4.5 % / 2 % faster, fp8 equal; at 96 rows W8A8 3 % / 0 % faster, fp8
-         * 4 % / 1 % slower; at 128 rows, where row tiles share slabs through the L2, both 5-9 % slower. W4A8's few-row
-         * kernel is bound by its unpack and promote instructions: 1-2 % with the hint at 32-96 rows, left as it is.
-         */
-        if constexpr (MODE != MODE_W4A8) {
-            const int64_t stream_limit = MODE == MODE_W8A8 ? 96 : 32;
-            if ((int64_t)p.max_rows <= stream_limit * (int64_t)p.experts) return launch_dma_shape<MODE, GMM1, OUT_DT, 128, 3, true>(p, n_tiles, st);
+    if constexpr (MODE == MODE_W4A8) {
+        return launch_w4a8<GMM1, OUT_DT>(p, n_tiles, st);
+    } else {
+        using F = FewRows<MODE, GMM1>;
+        const int64_t rows = p.max_rows, e = p.experts;
+        if (rows <= few_rows_limit<MODE, GMM1>(p, n_tiles) * e && p.K >= 256) {
+            /*
+             * Where nearly every expert has a single row tile its weight slabs are read once: they are requested with the
+             * streaming hint. Measured on 32 experts of 7168 x 4096 / 2048 x 7168, without / with, rows per expert:
+             * fp8 25 rows 165 / 91 -> 147 / 85 us, 64 rows 177 / 100 -> 153 / 99, 100 rows 194 / 109 -> 180 / 112, 128 rows
+             * 284 / 132 -> 288 / 146; W8A8 64 rows 195 / 100 -> 175 / 97, on 128 experts of 4096 x 3072 / 1536 x 4096
+             * 81 rows 367 / 180 -> 348 / 170, 128 rows 453 / 216 -> 523 / 238 (row tiles that share slabs through the L2).
+             */
+            const int64_t stream_limit = GMM1 ? 100 : (MODE == MODE_W8A8 ? 96 : 84);
+            /*
+             * A handful of rows: half the tile height, so the transfers of absent rows shrink as well (one row: 55.9 / 22.8
+             * -> 54.8 / 21.2 us on the experts above, 22.9 / 11.1 -> 21.6 / 9.8 on 64 of 2048 x 2048 / 1024 x 2048; equal from
+             * 4 to 32 rows). The limit leaves room for popular experts, whose rows would make several tiles of 64.
+             */
+            if (rows <= 8 * e) return launch_dma_shape<MODE, GMM1, OUT_DT, 64, F::STAGES_64, F::RG, true>(p, n_tiles, st);
+            if (rows <= stream_limit * e) return launch_dma_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG, true>(p, n_tiles, st);
+            return launch_dma_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG>(p, n_tiles, st);
         }
-        return launch_dma_shape<MODE, GMM1, OUT_DT, 128, 3>(p, n_tiles, st);
+        using Tall = DmaShape<320, 2, 128, 4>;
+        const bool tall_pays = MODE == MODE_W8A8 || rows <= kTallRowsLimitFp8 * e;
+        if (tall_pays && e <= Tall::MAX_EXPERTS) return launch_dma_shape<MODE, GMM1, OUT_DT, 320, 2, 4>(p, n_tiles, st);
+        return launch_dma_shape<MODE, GMM1, OUT_DT, 256, 2, 4>(p, n_tiles, st);
     }
-    if constexpr (MODE != MODE_W4A8) {
-        using Tall = DmaShape<320, 2, 128>;
-        const bool tall_pays = MODE == MODE_W8A8 || (int64_t)p.max_rows <= kTallRowsLimitFp8 * (int64_t)p.experts;
-        if (tall_pays && p.experts <= Tall::MAX_EXPERTS) return launch_dma_shape<MODE, GMM1, OUT_DT, 320, 2>(p, n_tiles, st);
-    }
-    return launch_dma_shape<MODE, GMM1, OUT_DT, 256, 2>(p, n_tiles, st);
 }
 
 } // namespace

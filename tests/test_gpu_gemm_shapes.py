@@ -1,0 +1,75 @@
+"""Every shape the grouped GEMMs choose by rows per expert, with row counts at the edges of its tiles (sub-tiles of 16
+rows, one or two row groups of waves, one tile more), against the oracle. The K loops run at their shortest (as many
+slabs as the pipeline has stages ahead) and longer."""
+import numpy as np
+import pytest
+import torch
+
+from memfabric_hybrid_amd import capi
+from memfabric_hybrid_amd.operators import OperatorBuffer
+from oracle import oracle as zo
+from test_gpu_gemm import assert_requant_close, fp8_operands, gmm1, gmm2
+from zbal_testlib import FP8_GEMM_ELEM_TOL, assert_fp8_close, dev, host, rng
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def buf():
+    b = OperatorBuffer()
+    yield b
+    torch.cuda.synchronize()
+    b.close()
+
+
+# rows per expert on average: the classes of W4A8 end at 48, 100, 160, 224 and 640, those of the 8-bit modes at 8, 84-100
+EDGES = {"few": [0, 1, 15, 16, 17, 2, 8, 5, 0, 3], "64": [1, 0, 16, 31, 33, 63, 64, 65, 80, 127],
+         "100": [0, 96, 97, 127, 128, 129, 112, 64, 1, 200], "160": [191, 192, 193, 176, 177, 0, 30, 160, 161, 256],
+         "224": [128, 129, 256, 257, 192, 255, 0, 144, 300, 250], "640": [384, 385, 192, 577, 1, 0, 600, 383, 500, 191]}
+
+
+@pytest.mark.parametrize("edges", sorted(EDGES))
+@pytest.mark.parametrize("K,N", [(256, 512), (384, 256), (640, 1280)])
+def test_w4a8_shapes_bit_exact(buf, edges, K, N):
+    counts = np.array(EDGES[edges], dtype=np.int64)
+    E, rows = len(counts), int(counts.sum())
+    a = rng(1).integers(-128, 128, (rows, K)).astype(np.int8)
+    a[:3] = -128                                    # with -8 below: the largest sums a scale group can have
+    xs = rng(2).uniform(0.005, 0.05, rows).astype(np.float32)
+    w = rng(3).integers(-8, 8, (E, K, N)).astype(np.int8)
+    w[:, :, :40] = -8
+    gs = rng(4).uniform(0.001, 0.01, (E, K // 128, N)).astype(np.float16).view(np.uint16)
+    packed = buf.prepack_weight(dev(w), int4=True)
+    assert np.array_equal(host(gmm2(buf, dev(a), dev(xs), packed, dev(gs), capi.DT_FP16, counts, K, N, 3)),
+                          zo.gmm2_w4a8(a, xs, w, gs, counts))
+    q2, s2, _ = gmm1(buf, dev(a), dev(xs), packed, dev(gs), counts, K, N, 3)
+    r_q2, r_s2, _ = zo.gmm1_swiglu_quant_w4a8(a, xs, w, gs, counts)
+    assert np.array_equal(host(s2).view(np.uint32), r_s2.view(np.uint32)) and np.array_equal(host(q2), r_q2)
+
+
+@pytest.mark.parametrize("edges", ["few", "64", "100"])
+@pytest.mark.parametrize("K,N", [(256, 512), (640, 1280)])
+def test_8_bit_shapes(buf, edges, K, N):
+    counts = np.array(EDGES[edges], dtype=np.int64)
+    E, rows = len(counts), int(counts.sum())
+    a = rng(1).integers(-127, 128, (rows, K)).astype(np.int8)
+    xs = rng(2).uniform(0.005, 0.05, rows).astype(np.float32)
+    w = rng(3).integers(-128, 128, (E, K, N)).astype(np.int8)
+    ws = rng(4).uniform(0.0015, 0.0045, (E, N)).astype(np.float32)
+    packed = buf.prepack_weight(dev(w))
+    assert np.array_equal(host(gmm2(buf, dev(a), dev(xs), packed, dev(ws), capi.DT_FP32, counts, K, N, 1)),
+                          zo.grouped_gemm_w8a8_dequant(a, xs, w, ws, counts))
+    q2, s2, _ = gmm1(buf, dev(a), dev(xs), packed, dev(ws), counts, K, N, 1)
+    r_q2, r_s2 = zo.gmm1_swiglu_quant_w8a8(a, xs, w, ws, counts)[:2]
+    assert np.array_equal(host(s2).view(np.uint32), r_s2.view(np.uint32)) and np.array_equal(host(q2), r_q2)
+
+    a, sa, w, sw = fp8_operands(E, K, N, rows, 20)
+    packed = buf.prepack_weight(dev(w))
+    y = gmm2(buf, dev(a), dev(sa), packed, dev(sw), capi.DT_FP32, counts, K, N, 2)
+    assert_fp8_close(zo.bf16_to_f32(host(y)), zo.bf16_to_f32(zo.gmm2_fp8(a, sa, w, sw, counts)), "fp8 GEMM", FP8_GEMM_ELEM_TOL)
+    q2, s2, _ = gmm1(buf, dev(a), dev(sa), packed, dev(sw), counts, K, N, 2)
+    r_q2, r_s2, _ = zo.gmm1_swiglu_quant_fp8(a, sa, w, sw, counts)
+    blocks = (rows, N // 256, 128)
+    assert np.allclose(host(s2), r_s2, rtol=1e-4)
+    assert_requant_close(zo.e4m3_to_f32(host(q2)).reshape(blocks) * host(s2)[:, :, None],
+                         zo.e4m3_to_f32(r_q2).reshape(blocks) * r_s2[:, :, None], host(q2), r_q2)
