@@ -58,11 +58,13 @@ __device__ __forceinline__ int64_t pick_row(const int32_t *__restrict__ base, in
 }
 
 /*
- * Small batches: the permute kernel works the layout out itself. With at most kInlineMaxPicks picks in all, every
- * workgroup counts the whole index array (a few KiB that sit in L2) into an LDS histogram, scans it into the
- * exclusive row offsets and counts the same-expert picks that precede each of its own token's picks: no layout
- * launch in front of the permute, and no dependency between workgroups. Workgroup 0 also writes the layout's
- * outputs (any of them may be null); every workgroup writes its token's expand_idx entries.
+ * Small batches: the permute kernel works the layout out itself, with no layout launch in front of it and no dependency
+ * between workgroups. A pick's destination row is the number of picks that sort before it (lower expert, or the same
+ * expert and an earlier pick), so with at most kInlineMaxPicks picks in all every workgroup reads the whole index array
+ * (a few KiB that sit in L2) and each thread compares its share of the picks with those of the workgroup's token, in
+ * registers; the counts meet in LDS behind the one barrier that the row's absmax needs anyway. (A histogram in LDS, its
+ * scan and the ranks, with a barrier after each, took 10.4 us where this takes 6: 128 tokens of 8 picks, 32 experts.)
+ * One workgroup more works the layout's outputs out and does nothing else.
  */
 constexpr int kInlineMaxPicks = 4096;
 constexpr int kInlineMaxTopk = 32;
@@ -78,63 +80,43 @@ struct InlineLayout {
     int64_t *nums_typed;          /* [E] counts (type 1) or running sums (type 0) */
 };
 
-/*
- * On return s_off[e] = rows before expert e, s_e[k] / s_rk[k] = expert and rank of pick k of token t. Negative ranks are
- * not routed: -1 an invalid expert id, -2 a token past the active ones (the combine leaves such a token's row alone).
- */
-__device__ __forceinline__ void inline_layout(const ExpertIds &idx, int t, int topk, int experts,
-                                              const InlineLayout &il, int32_t *s_off, int32_t *s_e, int32_t *s_rk, int32_t *s_tmp)
+/* how many tokens the mask routes (all of them without one); `s` is one word of LDS; holds barriers if there is a mask */
+__device__ __forceinline__ int active_tokens(const uint8_t *mask, int tokens, int32_t *s)
+{
+    if (mask == nullptr) return tokens;
+    if (threadIdx.x == 0) *s = 0;
+    __syncthreads();
+    int part = 0;
+    for (int t = threadIdx.x; t < tokens; t += blockDim.x) part += mask[t] != 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
+    if ((threadIdx.x & 63) == 0 && part) atomicAdd(s, part);
+    __syncthreads();
+    return *s;
+}
+
+/* the layout's outputs, by one workgroup; any of them may be null */
+__device__ __forceinline__ void write_inline_layout(const ExpertIds &idx, int topk, int experts, const InlineLayout &il,
+                                                    int32_t *s_hist, int32_t *s_tmp)
 {
     const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = tid >> 6;
-    for (int e = tid; e < experts; e += nthr) s_off[e] = 0;
-    /* the first four indices of this lane are requested together with the token's own picks (no mask: every token counts) */
-    int first[4] = {-1, -1, -1, -1};
-    if (il.active_mask == nullptr) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (tid + u * nthr < il.tokens * topk) first[u] = idx[tid + u * nthr];
-    }
-    if (tid < topk) {
-        s_e[tid] = idx[(int64_t)t * topk + tid];
-        s_rk[tid] = 0;
-    }
-    if (tid == 0) s_tmp[0] = 0;
+    for (int e = tid; e < experts; e += nthr) s_hist[e] = 0;
+    const int n = active_tokens(il.active_mask, il.tokens, s_tmp) * topk;
     __syncthreads();
-    int active = il.tokens;
-    if (il.active_mask) {
-        int part = 0;
-        for (int tt = tid; tt < il.tokens; tt += nthr) part += il.active_mask[tt] != 0;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
-        if (lane == 0 && part) atomicAdd(&s_tmp[0], part);
-        __syncthreads();
-        active = s_tmp[0];
-    }
-    const int n = active * topk, mine0 = t * topk;
-    /* four indices per lane are requested before the first is used: the loop is a chain of round trips to L2 otherwise */
     for (int i0 = tid; i0 < n; i0 += 4 * nthr) {
         int ev[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (i0 == tid && il.active_mask == nullptr) ev[u] = first[u];
-            else ev[u] = i0 + u * nthr < n ? idx[i0 + u * nthr] : -1;
-        }
+        for (int u = 0; u < 4; ++u) ev[u] = i0 + u * nthr < n ? idx[i0 + u * nthr] : -1;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = ev[u], i = i0 + u * nthr;
-            if (e < 0 || e >= experts) continue;
-            atomicAdd(&s_off[e], 1);
-            if (i < mine0 + topk)
-                for (int k = 0; k < topk; ++k)
-                    if (e == s_e[k] && i < mine0 + k) atomicAdd(&s_rk[k], 1);
-        }
+        for (int u = 0; u < 4; ++u)
+            if (ev[u] >= 0 && ev[u] < experts) atomicAdd(&s_hist[ev[u]], 1);
     }
     __syncthreads();
-    /* exclusive scan of the counts, in place: a thread owns `chunk` consecutive experts */
+    /* a thread owns `chunk` consecutive experts */
     const int chunk = (experts + nthr - 1) / nthr, b0 = tid * chunk;
     int32_t sum = 0;
     for (int j = 0; j < chunk; ++j)
-        if (b0 + j < experts) sum += s_off[b0 + j];
+        if (b0 + j < experts) sum += s_hist[b0 + j];
     int32_t incl = sum;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -145,28 +127,65 @@ __device__ __forceinline__ void inline_layout(const ExpertIds &idx, int t, int t
     __syncthreads();
     for (int w = 0; w < wave; ++w) incl += s_tmp[1 + w];
     int32_t run = incl - sum;
-    const bool writer = blockIdx.x == 0;
-    for (int j = 0; j < chunk; ++j) {
+    for (int j = 0; j < chunk && b0 + j < experts; ++j) {
         const int e = b0 + j;
-        if (e >= experts) break;
-        const int32_t c = s_off[e];
-        s_off[e] = run;
-        if (writer) {
-            if (il.row_off) il.row_off[e] = run;
-            if (il.incl_i32) il.incl_i32[e] = run + c;
-            if (il.counts_i64) il.counts_i64[e] = c;
-            if (il.nums_typed) il.nums_typed[e] = il.token_nums_type == 0 ? (int64_t)(run + c) : (int64_t)c;
-        }
+        const int32_t c = s_hist[e];
+        if (il.row_off) il.row_off[e] = run;
+        if (il.incl_i32) il.incl_i32[e] = run + c;
+        if (il.counts_i64) il.counts_i64[e] = c;
+        if (il.nums_typed) il.nums_typed[e] = il.token_nums_type == 0 ? (int64_t)(run + c) : (int64_t)c;
         run += c;
-        if (writer && e == experts - 1 && il.row_off) il.row_off[experts] = run;
+        if (e == experts - 1 && il.row_off) il.row_off[experts] = run;
     }
-    if (tid < topk) {
-        const int e = s_e[tid];
-        const int32_t rk = t >= active ? -2 : ((e >= 0 && e < experts) ? s_rk[tid] : -1);
-        s_rk[tid] = rk;
-        il.expand_idx[(int64_t)t * topk + tid] = rk;
+}
+
+/* a token's picks, one per lane (lane k holds pick k, every wave a copy): expert and destination row, -1 where not routed */
+struct LanePicks {
+    int e;
+    int32_t row;
+};
+
+/*
+ * This wave's part of the counts: lane k returns, for pick k of token t, (picks of lower experts) << 16 | (picks that
+ * sort before it), over the wave's share of the picks [0, n). my_e: lane k's pick.
+ */
+__device__ __forceinline__ int32_t count_before(const ExpertIds &idx, int t, int topk, int experts, int n, int my_e)
+{
+    const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63;
+    constexpr int KG = 8;                              /* picks per pass over the array */
+    int32_t result = 0;
+    for (int k0 = 0; k0 < topk; k0 += KG) {
+        int32_t first[KG], self[KG], below[KG], before[KG];
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            const int e = __builtin_amdgcn_readlane(my_e, (k0 + k) & 63);
+            first[k] = e << 13;                        /* keys: expert << 13 | pick, kInlineMaxPicks < 2^13 */
+            self[k] = first[k] | (t * topk + k0 + k);
+            below[k] = before[k] = 0;
+        }
+        for (int i0 = tid; i0 < n; i0 += 4 * nthr) {
+            int key[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = i0 + u * nthr;
+                const int e = i < n ? idx[i] : -1;
+                key[u] = e >= 0 && e < experts ? (e << 13 | i) : 0x7fffffff;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int k = 0; k < KG; ++k) {
+                    below[k] += key[u] < first[k] ? 1 : 0;
+                    before[k] += key[u] < self[k] ? 1 : 0;
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            const int32_t sum = zb_wave_sum_dpp(below[k] << 16 | before[k]);
+            if (lane == k0 + k) result = sum;
+        }
     }
-    __syncthreads();
+    return result;
 }
 
 /*
@@ -282,6 +301,62 @@ __device__ __forceinline__ u32x4 pack16_e4m3(const float (&v)[16], float mult)
  */
 enum { LM_GIVEN = 0, LM_INLINE = 1, LM_TABLE = 2 };     /* where ranks and offsets come from */
 
+/*
+ * Picks k0 + lane of token t where ranks and offsets come from a layout launch. The index and rank loads go out before
+ * the row's, the offset's (which depends on them) after: resolve_given takes them up.
+ */
+struct GivenPicks {
+    int e;
+    int32_t rank;
+};
+__device__ __forceinline__ GivenPicks request_given(const ExpertIds &idx, const int32_t *__restrict__ rank_in_expert, int t, int topk, int k)
+{
+    GivenPicks g = {-1, -1};
+    if (k < topk) {
+        g.e = idx[(int64_t)t * topk + k];
+        g.rank = rank_in_expert[(int64_t)t * topk + k];
+    }
+    return g;
+}
+__device__ __forceinline__ LanePicks resolve_given(const GivenPicks &g, const int32_t *__restrict__ base, int base_inclusive,
+                                                   int experts, const PeerRows &pr)
+{
+    LanePicks p = {g.e, -1};
+    /* rank < 0: the layout masked this token out */
+    if (g.e >= 0 && g.e < experts && g.rank >= 0) p.row = (int32_t)pick_row(base, base_inclusive, pr, g.e, g.rank);
+    return p;
+}
+
+/* window of the rank that owns expert e */
+__device__ __forceinline__ int window_of(const PeerRows &pr, int e) { return pr.ranks == 1 ? 0 : e / pr.e_loc; }
+
+/*
+ * The workgroup's token in inline mode, in two halves with one barrier of the caller's between them: the wave's counts
+ * go to LDS, their sums come back as destination rows. Writes the token's expand_idx.
+ */
+__device__ __forceinline__ void inline_counts(const ExpertIds &idx, int t, int topk, int experts, int active, int my_e,
+                                              int32_t (*s_cnt)[kInlineMaxTopk])
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int32_t c = count_before(idx, t, topk, experts, active * topk, my_e);
+    if (lane < topk) s_cnt[wave][lane] = c;
+}
+__device__ __forceinline__ LanePicks inline_rows(int t, int topk, int experts, int active, int my_e, const InlineLayout &il,
+                                                 const PeerRows &pr, int32_t (*s_cnt)[kInlineMaxTopk])
+{
+    const int lane = threadIdx.x & 63, nwaves = (blockDim.x + 63) >> 6;
+    LanePicks p = {my_e, -1};
+    if (lane < topk) {
+        int32_t c = 0;
+        for (int w = 0; w < nwaves; ++w) c += s_cnt[w][lane];
+        const bool valid = my_e >= 0 && my_e < experts, routed = valid && t < active;
+        const int32_t row = c & 0xffff, rank = t >= active ? -2 : (valid ? row - (c >> 16) : -1);
+        if (routed && row < pr.rows_cap) p.row = row;
+        if (threadIdx.x < 64) il.expand_idx[(int64_t)t * topk + lane] = rank;
+    }
+    return p;
+}
+
 template <int XDT, int QM, int SLOTS, bool SMOOTH, int LM>
 __global__ void __launch_bounds__(kThreads)
 permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
@@ -293,25 +368,25 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
     __shared__ float red[kThreads / 64];
     __shared__ int32_t s_off[INLINE ? kInlineMaxExperts : (TABLE ? kTableMaxExperts : 1)];
     __shared__ int32_t s_before[TABLE ? kTableMaxExperts : 1], s_tab[TABLE ? kTableMaxEntries : 1];
-    __shared__ int32_t s_e[kInlineMaxTopk], s_rk[INLINE ? kInlineMaxTopk : 1], s_tmp[8];
-    __shared__ int64_t s_row[kInlineMaxTopk];
-    const int t = blockIdx.x;
+    __shared__ int32_t s_cnt[kThreads / 64][kInlineMaxTopk], s_tmp[8];
+    const int lane = threadIdx.x & 63;
     const int nseg = hidden / kElemsPerLane;
     /* words the next stage wants at zero (the row maxima the int modes' first GEMM accumulates into) */
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < clear_count; i += (int64_t)gridDim.x * blockDim.x)
         clear_words[i] = 0u;
-    /*
-     * Where the token's picks go is worked out by one lane per pick while the row is on its way (the picks' index,
-     * rank and offset loads depend on each other: done pick after pick inside the store loop they cost topk round
-     * trips to L2 per workgroup): index and rank are requested before the row, the offset after it.
-     * s_row[k] < 0: pick k is not routed.
-     */
-    const bool picker = !INLINE && threadIdx.x < topk && threadIdx.x < kInlineMaxTopk;
-    int pick_e = -1, pick_rk = -1;
-    if (picker) {
-        pick_e = topk_idx[(int64_t)t * topk + threadIdx.x];
-        pick_rk = TABLE ? rt.expand_idx[(int64_t)t * topk + threadIdx.x] : rank_in_expert[(int64_t)t * topk + threadIdx.x];
+    if (INLINE && blockIdx.x == 0) {
+        write_inline_layout(topk_idx, topk, experts, il, s_off, s_tmp);
+        return;
     }
+    const int t = INLINE ? blockIdx.x - 1 : blockIdx.x;
+    /*
+     * Where the token's picks go is worked out by one lane per pick, in every wave, while the row is on its way (the
+     * picks' index, rank and offset loads depend on each other: done pick after pick inside the store loop they cost
+     * topk round trips to L2 per workgroup).
+     */
+    GivenPicks given = {-1, -1};
+    if (INLINE) given.e = lane < topk ? topk_idx[(int64_t)t * topk + lane] : -1;
+    else given = request_given(topk_idx, TABLE ? rt.expand_idx : rank_in_expert, t, topk, lane);
     int32_t tabv[TABLE ? kTablePerThread : 1];
     if constexpr (TABLE) table_request(rt, experts, tabv);
     /* the row is requested here (streamed: it is read once) and first used after the picks are resolved: the two latencies overlap */
@@ -325,47 +400,50 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
             raw[s][1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + (int64_t)t * hidden + (int64_t)seg * 16 + 8));
         }
     }
+    LanePicks picks = {-1, -1};
+    int active = 0;
     if constexpr (INLINE) {
-        inline_layout(topk_idx, t, topk, experts, il, s_off, s_e, s_rk, s_tmp);
-        if (threadIdx.x < topk) {
-            const int32_t rk = s_rk[threadIdx.x];
-            const int64_t row = rk < 0 ? -1 : (int64_t)s_off[s_e[threadIdx.x]] + rk;
-            s_row[threadIdx.x] = row < pr.rows_cap ? row : -1;
-        }
+        active = active_tokens(il.active_mask, il.tokens, s_tmp);
+        inline_counts(topk_idx, t, topk, experts, active, given.e, s_cnt);
     } else if constexpr (TABLE) {
         table_layout(rt, tabv, t / rt.tokens_per_range, experts, t == 0, s_tab, s_off, s_before, s_tmp);
-        if (picker) {
-            int64_t row = -1;
-            if (pick_e >= 0 && pick_e < experts && pick_rk >= 0) {       /* rank < 0: the layout masked this token out */
-                const int32_t rk = s_before[pick_e] + pick_rk;
-                rt.expand_idx[(int64_t)t * topk + threadIdx.x] = rk;       /* the rank within the expert: what the combine reads */
-                row = (int64_t)s_off[pick_e] + rk;
-                if (row >= pr.rows_cap) row = -1;
-            }
-            s_e[threadIdx.x] = pick_e;
-            s_row[threadIdx.x] = row;
+        picks.e = given.e;
+        if (given.e >= 0 && given.e < experts && given.rank >= 0) {       /* rank < 0: the layout masked this token out */
+            const int32_t rk = s_before[given.e] + given.rank, row = s_off[given.e] + rk;
+            if (threadIdx.x < 64) rt.expand_idx[(int64_t)t * topk + lane] = rk;   /* the rank within the expert: what the combine reads */
+            if (row < pr.rows_cap) picks.row = row;
         }
-    } else if (picker) {
-        const bool routed = pick_e >= 0 && pick_e < experts && pick_rk >= 0;      /* rank < 0: the layout masked this token out */
-        s_e[threadIdx.x] = pick_e;
-        s_row[threadIdx.x] = routed ? pick_row(base, base_inclusive, pr, pick_e, pick_rk) : -1;
+    } else {
+        picks = resolve_given(given, base, base_inclusive, experts, pr);
     }
-    __syncthreads();
     float v[SLOTS][16];
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) cvt16<XDT>(raw[s][0], raw[s][1], v[s]);
-    /* destination of pick k of this token: false if the pick is not routed (uniform across the workgroup) */
-    auto resolve = [&](int k, int &e, int64_t &row) __attribute__((always_inline)) -> bool {
-        if (INLINE || k < kInlineMaxTopk) {
-            e = s_e[k];
-            row = s_row[k];
-            return row >= 0;
+    constexpr bool ROW_MAX = QM != QM_FP8 && !SMOOTH;
+    if constexpr (ROW_MAX) {
+        float amax = 0.0f;
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[s][i]));
+        amax = zb_wave_reduce_dpp<true>(amax);
+        if (lane == 0) red[threadIdx.x >> 6] = amax;
+    }
+    if constexpr (ROW_MAX || INLINE) __syncthreads();
+    if constexpr (INLINE) picks = inline_rows(t, topk, experts, active, given.e, il, pr, s_cnt);
+    /* f(pick's expert, window, row) for every routed pick of the token; wave-uniform */
+    auto for_each_pick = [&](auto f) __attribute__((always_inline)) {
+        for (int k0 = 0; k0 < topk; k0 += 64) {
+            if (!INLINE && !TABLE && k0 > 0)
+                picks = resolve_given(request_given(topk_idx, rank_in_expert, t, topk, k0 + lane), base, base_inclusive, experts, pr);
+            const int n = topk - k0 < 64 ? topk - k0 : 64;
+            for (int k = 0; k < n; ++k) {
+                const int32_t row = __builtin_amdgcn_readlane(picks.row, k);
+                if (row < 0) continue;
+                const int e = __builtin_amdgcn_readlane(picks.e, k);
+                f(e, window_of(pr, e), (int64_t)row);
+            }
         }
-        e = topk_idx[(int64_t)t * topk + k];          /* more picks per token than the table holds: one by one */
-        const int rk = rank_in_expert[(int64_t)t * topk + k];
-        if (e < 0 || e >= experts || rk < 0) return false;
-        row = pick_row(base, base_inclusive, pr, e, rk);
-        return row >= 0;
     };
 
     if constexpr (QM == QM_FP8) {
@@ -384,12 +462,9 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
             sc[s] = amax * (1.0f / 448.0f);
         }
         const int nblk128 = hidden / 128;
-        for (int k = 0; k < topk; ++k) {
-            int e;
-            int64_t row;
-            if (!resolve(k, e, row)) continue;
-            uint8_t *dest = pr.dest[e / pr.e_loc];
-            float *dest_scale = pr.scale[e / pr.e_loc];
+        for_each_pick([&](int, int win, int64_t row) __attribute__((always_inline)) {
+            uint8_t *dest = pr.dest[win];
+            float *dest_scale = pr.scale[win];
 #pragma unroll
             for (int s = 0; s < SLOTS; ++s) {
                 const int seg = s * blockDim.x + threadIdx.x;
@@ -398,14 +473,10 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                     if ((seg & 7) == 0) dest_scale[row * nblk128 + (seg >> 3)] = sc[s];
                 }
             }
-        }
+        });
     } else if constexpr (!SMOOTH) {
-        float amax = 0.0f;
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[s][i]));
-        amax = zb_block_max(amax, red);
+        float amax = red[0];
+        for (int w = 1; w < (int)((blockDim.x + 63) >> 6); ++w) amax = fmaxf(amax, red[w]);
         float sq, stored;
         if (QM == QM_INT8_NOEPS && amax == 0.0f) { sq = 0.0f; stored = 0.0f; }
         else {
@@ -415,25 +486,19 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
         u32x4 q[SLOTS];
 #pragma unroll
         for (int s = 0; s < SLOTS; ++s) q[s] = pack16_i8(v[s], sq);
-        for (int k = 0; k < topk; ++k) {
-            int e;
-            int64_t row;
-            if (!resolve(k, e, row)) continue;
-            uint8_t *dest = pr.dest[e / pr.e_loc];
+        for_each_pick([&](int, int win, int64_t row) __attribute__((always_inline)) {
+            uint8_t *dest = pr.dest[win];
 #pragma unroll
             for (int s = 0; s < SLOTS; ++s) {
                 const int seg = s * blockDim.x + threadIdx.x;
                 if (seg < nseg)
                     *reinterpret_cast<u32x4 *>(dest + row * hidden + (int64_t)seg * 16) = q[s];
             }
-            if (threadIdx.x == 0) pr.scale[e / pr.e_loc][row] = stored;
-        }
+            if (threadIdx.x == 0) pr.scale[win][row] = stored;
+        });
     } else {
-        for (int k = 0; k < topk; ++k) {
-            int e;
-            int64_t row;
-            if (!resolve(k, e, row)) continue; /* uniform across the block */
-            uint8_t *dest = pr.dest[e / pr.e_loc];
+        for_each_pick([&](int e, int win, int64_t row) __attribute__((always_inline)) {
+            uint8_t *dest = pr.dest[win];
             float sv[SLOTS][16];
             float amax = 0.0f;
 #pragma unroll
@@ -458,38 +523,64 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                     *reinterpret_cast<u32x4 *>(dest + row * hidden + (int64_t)seg * 16) = q;
                 }
             }
-            if (threadIdx.x == 0) pr.scale[e / pr.e_loc][row] = stored;
-        }
+            if (threadIdx.x == 0) pr.scale[win][row] = stored;
+        });
     }
 }
 
-/* plain row copy (no quantisation): 16-byte chunks of 8 elements */
+/* plain row copy (no quantisation): 16-byte chunks of 8 elements, UNROLL of them per lane and pass */
+template <int LM, int UNROLL>
 __global__ void __launch_bounds__(kThreads)
 permute_copy_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                     const int32_t *__restrict__ rank_in_expert, const int32_t *__restrict__ base, int base_inclusive,
-                    int hidden, int topk, int experts, PeerRows pr)
+                    int hidden, int topk, int experts, PeerRows pr, InlineLayout il)
 {
-    const int t = blockIdx.x;
+    constexpr bool INLINE = LM == LM_INLINE;
+    __shared__ int32_t s_off[INLINE ? kInlineMaxExperts : 1], s_cnt[kThreads / 64][kInlineMaxTopk], s_tmp[8];
+    if (INLINE && blockIdx.x == 0) {
+        write_inline_layout(topk_idx, topk, experts, il, s_off, s_tmp);
+        return;
+    }
+    const int t = INLINE ? blockIdx.x - 1 : blockIdx.x, lane = threadIdx.x & 63;
     const int nchunk = hidden / 8;
-    for (int c0 = 0; c0 < nchunk; c0 += blockDim.x * 4) {
-        u32x4 v[4];
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(x + (int64_t)t * hidden);
+    GivenPicks given = {-1, -1};
+    if (INLINE) given.e = lane < topk ? topk_idx[(int64_t)t * topk + lane] : -1;
+    else given = request_given(topk_idx, rank_in_expert, t, topk, lane);
+    u32x4 v[UNROLL];
+    auto load = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < UNROLL; ++u) {
             const int c = c0 + u * blockDim.x + threadIdx.x;
-            if (c < nchunk) v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + (int64_t)t * hidden + (int64_t)c * 8));
+            if (c < nchunk) v[u] = __builtin_nontemporal_load(src + c);
         }
-        for (int k = 0; k < topk; ++k) {
-            const int e = topk_idx[(int64_t)t * topk + k];
-            const int rk = rank_in_expert[(int64_t)t * topk + k];
-            if (e < 0 || e >= experts || rk < 0) continue;      /* rk < 0: the layout masked this token out */
-            const int64_t row = pick_row(base, base_inclusive, pr, e, rk);
-            if (row < 0) continue;
-            uint16_t *dest = reinterpret_cast<uint16_t *>(pr.dest[e / pr.e_loc]);
+    };
+    load(0);
+    LanePicks first;
+    if constexpr (INLINE) {
+        const int active = active_tokens(il.active_mask, il.tokens, s_tmp);
+        inline_counts(topk_idx, t, topk, experts, active, given.e, s_cnt);
+        __syncthreads();
+        first = inline_rows(t, topk, experts, active, given.e, il, pr, s_cnt);
+    } else {
+        first = resolve_given(given, base, base_inclusive, experts, pr);
+    }
+    for (int c0 = 0; c0 < nchunk; c0 += blockDim.x * UNROLL) {
+        if (c0 > 0) load(c0);
+        LanePicks picks = first;
+        for (int k0 = 0; k0 < topk; k0 += 64) {
+            if (!INLINE && k0 > 0)
+                picks = resolve_given(request_given(topk_idx, rank_in_expert, t, topk, k0 + lane), base, base_inclusive, experts, pr);
+            const int n = topk - k0 < 64 ? topk - k0 : 64;
+            for (int k = 0; k < n; ++k) {
+                const int32_t row = __builtin_amdgcn_readlane(picks.row, k);
+                if (row < 0) continue;
+                u32x4 *dest = reinterpret_cast<u32x4 *>(pr.dest[window_of(pr, __builtin_amdgcn_readlane(picks.e, k))] + (int64_t)row * hidden * 2);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int c = c0 + u * blockDim.x + threadIdx.x;
-                if (c < nchunk)
-                    *reinterpret_cast<u32x4 *>(dest + row * hidden + (int64_t)c * 8) = v[u];
+                for (int u = 0; u < UNROLL; ++u) {
+                    const int c = c0 + u * blockDim.x + threadIdx.x;
+                    if (c < nchunk) dest[c] = v[u];       /* (non-temporal stores: 4096 x 7168 3-5 % slower) */
+                }
             }
         }
     }
@@ -516,7 +607,7 @@ int32_t launch_quant(const void *x, const ExpertIds &topk_idx, const int32_t *ra
     const InlineLayout il = ex.inline_layout ? *ex.inline_layout : InlineLayout{};
     const RangeTable rt = ex.range_table ? *ex.range_table : RangeTable{};
 #define ZB_LAUNCH_I(S, LMV)                                                                                       \
-    permute_quant_kernel<XDT, QM, S, SMOOTH, LMV><<<(unsigned)tokens, threads, 0, st>>>(                           \
+    permute_quant_kernel<XDT, QM, S, SMOOTH, LMV><<<(unsigned)(tokens + (LMV == LM_INLINE ? 1 : 0)), threads, 0, st>>>( \
         (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, smooth, (int)hidden, (int)topk,       \
         (int)experts, pr, il, rt, ex.clear_words, ex.clear_count)
 #define ZB_LAUNCH(S)                                                                                              \
@@ -550,9 +641,18 @@ static int32_t permute_launch(const void *x, int32_t x_dtype, const ExpertIds &t
     if (hidden <= 0 || hidden > 16 * kThreads * 4 || topk <= 0 || tokens < 0) return ZBALHIP_INVALID;
     if (tokens == 0) return ZBALHIP_OK;
     if (quant == QM_COPY) {
-        if (hidden % 8 != 0 || ex.inline_layout || ex.clear_count) return ZBALHIP_INVALID;
-        permute_copy_kernel<<<(unsigned)tokens, kThreads, 0, st>>>((const uint16_t *)x, topk_idx, rank_in_expert, base,
-                                                                 base_inclusive, (int)hidden, (int)topk, (int)experts, pr);
+        if (hidden % 8 != 0 || ex.range_table || ex.clear_count) return ZBALHIP_INVALID;
+        const int nchunk = (int)(hidden / 8);
+        int threads = (nchunk + 63) / 64 * 64;
+        if (threads > kThreads) threads = kThreads;
+        if (ex.inline_layout)
+            permute_copy_kernel<LM_INLINE, 4><<<(unsigned)tokens + 1, threads, 0, st>>>(
+                (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, (int)hidden, (int)topk, (int)experts, pr,
+                *ex.inline_layout);
+        else
+            permute_copy_kernel<LM_GIVEN, 4><<<(unsigned)tokens, threads, 0, st>>>(
+                (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, (int)hidden, (int)topk, (int)experts, pr,
+                InlineLayout{});
         return zbalhip_check_launch();
     }
     if (hidden % 16 != 0 || (quant == QM_FP8 && hidden % 128 != 0)) return ZBALHIP_INVALID;
@@ -572,10 +672,10 @@ static int32_t permute_launch(const void *x, int32_t x_dtype, const ExpertIds &t
     return ZBALHIP_INVALID;
 }
 
-/* the permute kernel can work the layout out itself when the batch is this small (inline_layout above) */
-static bool layout_fits_inline(int64_t tokens, int64_t topk, int64_t experts, int quant)
+/* the permute kernel can work the layout out itself when the batch is this small (InlineLayout above) */
+static bool layout_fits_inline(int64_t tokens, int64_t topk, int64_t experts)
 {
-    return quant != QM_COPY && tokens > 0 && tokens * topk <= kInlineMaxPicks && topk <= kInlineMaxTopk &&
+    return tokens > 0 && tokens * topk <= kInlineMaxPicks && topk <= kInlineMaxTopk &&
            experts <= kInlineMaxExperts;
 }
 
@@ -638,7 +738,7 @@ extern "C" int32_t zbalhip_dispatch_low_latency(const void *x, int32_t x_dtype, 
     hipStream_t st = (hipStream_t)stream;
     const int q = quant_mode == 0 ? QM_COPY : (quant_mode == 1 ? QM_INT8_NOEPS : QM_FP8);
     if (tokens > 0 && q != QM_COPY && !dynamic_scales) return ZBALHIP_INVALID;
-    if (layout_fits_inline(tokens, topk, experts, q)) {      /* one launch: the permute kernel derives ranks and counts itself */
+    if (layout_fits_inline(tokens, topk, experts)) {      /* one launch: the permute kernel derives ranks and counts itself */
         InlineLayout il = {};
         il.tokens = (int)tokens;
         il.token_nums_type = token_nums_type;
@@ -710,7 +810,7 @@ extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, c
     if (scratch_blocks < 0 || (scratch_blocks > 0 && !scratch)) return ZBALHIP_INVALID;
     hipStream_t st = (hipStream_t)stream;
     const int q = mode == 2 ? QM_FP8 : QM_INT8_NOEPS;
-    if (layout_fits_inline(tokens, topk, experts, q)) {      /* one launch: the permute kernel derives ranks and offsets itself */
+    if (layout_fits_inline(tokens, topk, experts)) {      /* one launch: the permute kernel derives ranks and offsets itself */
         InlineLayout il = {};
         il.active_mask = active_mask;
         il.tokens = (int)tokens;

@@ -1114,19 +1114,19 @@ grouped_gemm_dma_kernel(GemmParams p)
  * one wave takes one row at a time and every lane asks for its (up to eight) 16-byte pieces of the row before it
  * converts the first. Measured on 131 072 rows of 1536 values (read 805 MB, write 201 MB): 256 threads with one piece
  * in flight per lane 200 us (5.0 TB/s), two waves with four pieces 182 us, one wave with eight 166 us (6.1 TB/s).
+ * A small batch waits for round trips: the row and its maximum are asked for together with the number of rows that
+ * there are (rows past it hold nothing of use, but are inside the scratch, which has max_rows).
  */
 constexpr int kRequantThreads = 64, kRequantPieces = 8;
 
 __global__ void __launch_bounds__(kRequantThreads)
 requant_rows_kernel(const float *__restrict__ sgl, const uint32_t *__restrict__ rowmax, const int32_t *__restrict__ row_off,
-                    int experts, int I, int8_t *__restrict__ q2, float *__restrict__ scale2)
+                    int experts, int max_rows, int I, int8_t *__restrict__ q2, float *__restrict__ scale2)
 {
     const int total = row_off[experts];
     const int vecs = I / 4;
-    for (int row = blockIdx.x; row < total; row += gridDim.x) {
-        const float mx = __uint_as_float(rowmax[row]);
-        const float inv = mx == 0.0f ? 0.0f : 1.0f / mx;
-        if (threadIdx.x == 0) scale2[row] = mx * (1.0f / 127.0f);
+    for (int row = blockIdx.x; row < max_rows; row += gridDim.x) {
+        const uint32_t mx_bits = rowmax[row];
         const f32x4 *src = reinterpret_cast<const f32x4 *>(sgl + (int64_t)row * I);
         uint32_t *dst = reinterpret_cast<uint32_t *>(q2 + (int64_t)row * I);
         for (int c0 = 0; c0 < vecs; c0 += kRequantThreads * kRequantPieces) {
@@ -1136,6 +1136,9 @@ requant_rows_kernel(const float *__restrict__ sgl, const uint32_t *__restrict__ 
                 const int c = c0 + u * kRequantThreads + (int)threadIdx.x;
                 v[u] = c < vecs ? __builtin_nontemporal_load(src + c) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             }
+            if (row >= total) return;
+            const float mx = __uint_as_float(mx_bits), inv = mx == 0.0f ? 0.0f : 1.0f / mx;
+            if (c0 == 0 && threadIdx.x == 0) scale2[row] = mx * (1.0f / 127.0f);
 #pragma unroll
             for (int u = 0; u < kRequantPieces; ++u) {
                 const int c = c0 + u * kRequantThreads + (int)threadIdx.x;
@@ -1380,7 +1383,7 @@ extern "C" int32_t zbalhip_gmm1_swiglu_quant(const void *a, const float *a_scale
         if (rc != ZBALHIP_OK) return rc;
     }
     int64_t rb = max_rows < 16384 ? max_rows : 16384;
-    requant_rows_kernel<<<(unsigned)rb, kRequantThreads, 0, st>>>(sgl_ws, p.rowmax, row_off, (int)experts, (int)(n1 / 2),
+    requant_rows_kernel<<<(unsigned)rb, kRequantThreads, 0, st>>>(sgl_ws, p.rowmax, row_off, (int)experts, (int)max_rows, (int)(n1 / 2),
                                                     (int8_t *)q2, scale2);
     return zbalhip_check_launch();
 }

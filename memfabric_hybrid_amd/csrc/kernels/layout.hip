@@ -57,19 +57,48 @@ struct LayoutOutputs {
 __device__ __forceinline__ uint32_t token_ranks(const ExpertIds &idx, int64_t i0, int topk, int experts, int e_loc, int first_rank)
 {
     uint32_t mask = 0;
-    for (int k = 0; k < topk; ++k) {
-        const int e = idx[i0 + k];
-        if (e < 0 || e >= experts) continue;
-        const int r = (e_loc == experts ? 0 : e / e_loc) - first_rank;
-        if (r >= 0 && r < 32) mask |= 1u << r;
+    for (int k0 = 0; k0 < topk; k0 += 8) {
+        int e[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) e[k] = k0 + k < topk ? idx[i0 + k0 + k] : -1;      /* requested together */
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (e[k] < 0 || e[k] >= experts) continue;
+            const int r = (e_loc == experts ? 0 : e[k] / e_loc) - first_rank;
+            if (r >= 0 && r < 32) mask |= 1u << r;
+        }
     }
     return mask;
+}
+
+/* one count per (token, rank) no matter how many of the token's picks land there, 32 ranks per pass; by one block */
+__device__ __forceinline__ void count_tokens_per_rank(const ExpertIds &idx, int tokens, int topk, int experts, int e_loc,
+                                                      const LayoutOutputs &o, int32_t *rcnt)
+{
+    for (int r = threadIdx.x; r < o.ranks; r += blockDim.x) rcnt[r] = 0;
+    __syncthreads();
+    for (int first = 0; first < o.ranks; first += 32) {
+        int32_t mine = 0;                       /* ranks == 1: counted in a register */
+        for (int t = threadIdx.x; t < tokens; t += blockDim.x) {
+            uint32_t mask = token_ranks(idx, (int64_t)t * topk, topk, experts, e_loc, first);
+            if (o.ranks == 1) mine += (int32_t)(mask & 1u);
+            else
+                for (; mask; mask &= mask - 1) atomicAdd(&rcnt[first + __ffs((int)mask) - 1], 1);
+        }
+        if (o.ranks == 1) {
+            mine = zb_wave_sum_dpp(mine);
+            if ((threadIdx.x & 63) == 0 && mine) atomicAdd(&rcnt[0], mine);
+        }
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r < o.ranks; r += blockDim.x) o.tokens_per_rank[r] = rcnt[r];
 }
 
 /*
  * The whole layout in one launch: every block first counts the picks that precede its own range (the index array is a
  * few hundred KiB and sits in L2, so reading it again per block is cheaper than a launch), ranks its own picks, and the
- * last block, whose running counts are then the totals, scans them into the offsets and counts the tokens per rank.
+ * last block, whose running counts are then the totals, scans them into the offsets. One block more counts the tokens
+ * per rank (RANKS).
  * With per-rank counts on 4096 tokens of 8 int64 picks over 32 experts this replaces a histogram, a ranking and a scan
  * launch (4.7 + 20.3 + 6.1 us; the ranking blocks summed up to 49 histograms one after the other) and five elementwise
  * launches that worked token_in_rank out.
@@ -83,6 +112,12 @@ layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, i
     __shared__ int32_t wsum[ZB_FUSED_THREADS / 64];
     __shared__ int32_t s_active;
     __shared__ __align__(16) uint8_t cnt[ZB_FUSED_THREADS / 64 * ZB_MAX_EXPERTS];
+    const int e_loc = RANKS ? experts / o.ranks : experts;
+    const int last = (int)gridDim.x - (RANKS ? 2 : 1);
+    if (RANKS && (int)blockIdx.x > last) {
+        if (o.tokens_per_rank) count_tokens_per_rank(idx, tokens, topk, experts, e_loc, o, run);
+        return;
+    }
     for (int e = threadIdx.x; e < experts; e += blockDim.x) run[e] = 0;
     if (threadIdx.x == 0) s_active = 0;
     __syncthreads();
@@ -106,7 +141,6 @@ layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, i
     int tok0 = blockIdx.x * tpb;
     int tok1 = tok0 + tpb;
     if (tok1 > tokens) tok1 = tokens;
-    const int e_loc = RANKS ? experts / o.ranks : experts;
     if (RANKS && o.token_in_rank)
         for (int i = tok0 * o.ranks + threadIdx.x; i < tok1 * o.ranks; i += blockDim.x) {
             const int t = i / o.ranks;
@@ -142,7 +176,7 @@ layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, i
     }
     __syncthreads();
     rank_picks(idx, p0, p1, experts, nbits, run, cnt, o.send_token_idx);
-    if (blockIdx.x != gridDim.x - 1) return;
+    if ((int)blockIdx.x != last) return;
 
     /* rank_picks ends on a barrier: run[] now holds the totals */
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -172,31 +206,6 @@ layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, i
             if (o.counts_i64) o.counts_i64[e] = c;
             if (o.nums_typed) o.nums_typed[e] = o.token_nums_type == 0 ? (int64_t)s : (int64_t)c;
         }
-    }
-    /* tokens per rank: one count per (token, rank) no matter how many of the token's picks land there, 32 ranks per pass */
-    if (RANKS && o.tokens_per_rank) {
-        int32_t *rcnt = run;                        /* the totals have been written out */
-        for (int r = threadIdx.x; r < o.ranks; r += blockDim.x) rcnt[r] = 0;
-        __syncthreads();
-        for (int first = 0; first < o.ranks; first += 32) {
-            const int nr = o.ranks - first < 32 ? o.ranks - first : 32;
-            int32_t mine = 0;                       /* ranks == 1: counted in a register */
-            for (int t = threadIdx.x; t < tokens; t += blockDim.x) {
-                uint32_t mask = token_ranks(idx, (int64_t)t * topk, topk, experts, e_loc, first);
-                if (o.ranks == 1) { mine += (int32_t)(mask & 1u); continue; }
-                for (; mask; mask &= mask - 1) {
-                    const int r = __ffs((int)mask) - 1;
-                    if (r < nr) atomicAdd(&rcnt[first + r], 1);
-                }
-            }
-            if (o.ranks == 1) {
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off, 64);
-                if (lane == 0 && mine) atomicAdd(&rcnt[0], mine);
-            }
-        }
-        __syncthreads();
-        for (int r = threadIdx.x; r < o.ranks; r += blockDim.x) o.tokens_per_rank[r] = rcnt[r];
     }
 }
 
@@ -551,7 +560,7 @@ static int32_t launch_fused_layout(const ExpertIds &idx, int64_t tokens, int64_t
 {
     const LayoutPlan p = plan_layout(tokens, topk, 64);
     if (o.tokens_per_rank || o.token_in_rank)
-        layout_fused_kernel<true><<<p.nblk, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,
+        layout_fused_kernel<true><<<p.nblk + 1, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,
                                                                      p.tokens_per_block, ceil_log2(experts), active_mask, o);
     else
         layout_fused_kernel<false><<<p.nblk, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,

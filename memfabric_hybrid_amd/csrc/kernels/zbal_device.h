@@ -195,6 +195,18 @@ template <bool IS_MAX> __device__ __forceinline__ float zb_wave_reduce_dpp(float
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
 }
 
+/* sum over the wave, in every lane */
+__device__ __forceinline__ int32_t zb_wave_sum_dpp(int32_t x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false);     /* the steps of zb_wave_reduce_dpp */
+    x += __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x140, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
 /* max over groups of 2^LOG2 consecutive lanes */
 template <int LOG2> __device__ __forceinline__ float zb_group_max(float v)
 {
