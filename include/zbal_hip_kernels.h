@@ -96,14 +96,16 @@ ZBALHIP_API int32_t zbalhip_dispatch_notify(const int32_t *const *tokens_per_exp
                                 void *stream);
 
 /*
- * zbalhip_dispatch_notify for a caller that needs the received counts on the host: returns when `host_counts`
- * [experts / ranks] (host memory) holds them. `block` is from zbalhip_host_counts_alloc (a few KiB of pinned memory
- * that the kernel writes directly); one call at a time per block. Refused while the stream is being captured.
+ * zbalhip_dispatch_notify for a caller that needs the received counts on the host as well: the kernel also writes them
+ * to `block` (from zbalhip_host_counts_alloc: a few KiB of pinned memory), and zbalhip_host_counts_wait with the ticket
+ * returns when they have arrived, with the first n = experts / ranks of them in `host_counts`. Work queued behind the
+ * notify in between is not waited for. One notify at a time per block. Refused while the stream is being captured.
  */
 ZBALHIP_API int32_t zbalhip_dispatch_notify_counts(const int32_t *const *tokens_per_expert, int32_t ranks, int32_t my_rank,
                                        int64_t experts, int64_t topk, int32_t *recv_data, int32_t *put_offset,
                                        int32_t *total_recv, int64_t *recv_tokens_per_expert, int32_t *balance_matrix,
-                                       void *block, int64_t *host_counts, void *stream);
+                                       void *block, uint64_t *ticket, void *stream);
+ZBALHIP_API int32_t zbalhip_host_counts_wait(void *block, uint64_t ticket, int64_t n, int64_t *host_counts, void *stream);
 ZBALHIP_API int32_t zbalhip_host_counts_alloc(void **block);
 ZBALHIP_API int32_t zbalhip_host_counts_free(void *block);
 

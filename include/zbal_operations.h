@@ -184,16 +184,24 @@ int32_t zbal_dispatch_normal_layout_in_rank(const zbal_tensor_info_t *topkIndex,
                                             int64_t flags);
 
 /*
- * extension: zbal_dispatch_normal_notify for a caller that sizes its receive tensors from the counts: returns when
- * hostCounts [E / ranks] (host memory) holds this rank's recvTokensPerExpert.
+ * extension: zbal_dispatch_normal_notify for a caller that also needs this rank's recvTokensPerExpert on the host.
+ * zbal_dispatch_normal_notify_end, on the same stream, returns when hostCounts [E / ranks] (host memory) holds them; it
+ * does not wait for work queued in between (the dispatch). Every notify_begin that succeeded is followed by one
+ * notify_end with its `pending`.
  */
-int32_t zbal_dispatch_normal_notify_counts(const zbal_tensor_info_t *sendTokensPerExpert, int64_t sendCount,
-                                           int64_t topKNum, const zbal_tensor_info_t *recvBuff,
-                                           const zbal_tensor_info_t *totalRecvTokens,
-                                           const zbal_tensor_info_t *recvTokensPerExpert,
-                                           const zbal_tensor_info_t *pushTargetOffset,
-                                           const zbal_tensor_info_t *balanceMatrix, int64_t *hostCounts,
-                                           zbal_comm_t comm, aclrtStream stream, int64_t flags);
+typedef struct {
+    void *block;
+    uint64_t ticket;
+} zbal_pending_counts_t;
+int32_t zbal_dispatch_normal_notify_begin(const zbal_tensor_info_t *sendTokensPerExpert, int64_t sendCount,
+                                          int64_t topKNum, const zbal_tensor_info_t *recvBuff,
+                                          const zbal_tensor_info_t *totalRecvTokens,
+                                          const zbal_tensor_info_t *recvTokensPerExpert,
+                                          const zbal_tensor_info_t *pushTargetOffset,
+                                          const zbal_tensor_info_t *balanceMatrix, zbal_pending_counts_t *pending,
+                                          zbal_comm_t comm, aclrtStream stream, int64_t flags);
+int32_t zbal_dispatch_normal_notify_end(zbal_pending_counts_t *pending, int64_t sendCount, int64_t *hostCounts,
+                                        zbal_comm_t comm, aclrtStream stream, int64_t flags);
 
 /*
  * extension: softmax + top-k router. logits [T, E] fp32 -> topkIndex [T, K]

@@ -76,6 +76,10 @@ def get_low_latency_rdma_size_hint(num_max_dispatch_tokens_per_rank: int, hidden
     return num_max_dispatch_tokens_per_rank
 
 
+def _no_hook() -> None:
+    """The receive hook of the low-latency calls: there is nothing to wait for."""
+
+
 PADDING_SIZE = 1      # an empty batch is padded to this many tokens (zbal_deepep.cpp:85, 470-490)
 
 
@@ -257,14 +261,14 @@ class Buffer:
                 ts.append(torch.arange(0, K, dtype=topk_idx.dtype, device=topk_idx.device).reshape(1, K))
             new_x, new_idx = torch.cat(xs, 0), torch.cat(ts, 0)
             self._pad = dict(count=pad, ori_x=x.clone(), topk_idx=new_idx)
-        recv, scales, packed_recv_count, h = self.runtime.low_latency_dispatch(
-            new_x, new_idx, num_max_dispatch_tokens_per_rank, num_experts, use_fp8=use_fp8)
-        handle = (h["expand_idx"], h["ep_recv_count"], num_max_dispatch_tokens_per_rank, x.size(1), num_experts,
-                  packed_recv_count)
-        kept = (x, topk_idx, recv, scales, packed_recv_count, h["expand_idx"], h["ep_recv_count"],
-                cumulative_local_expert_recv_stats)
-        return ((recv, scales) if use_fp8 else recv, packed_recv_count, handle,
-                self._event(async_finish, kept if async_finish else None), (lambda: None))
+        rt = self.runtime               # one native call; rt.low_latency_dispatch wraps the same
+        recv, scales, packed_recv_count, expand_idx, ep_recv_count = rt.native.ll_dispatch(
+            rt._comm, rt._dev, new_x, new_idx, num_max_dispatch_tokens_per_rank, num_experts,
+            capi.QUANT_INT8 if use_fp8 else capi.NO_QUANT)
+        handle = (expand_idx, ep_recv_count, num_max_dispatch_tokens_per_rank, x.size(1), num_experts, packed_recv_count)
+        kept = (x, topk_idx, recv, scales, packed_recv_count, expand_idx, ep_recv_count,
+                cumulative_local_expert_recv_stats) if async_finish else None
+        return ((recv, scales) if use_fp8 else recv, packed_recv_count, handle, self._event(async_finish, kept), _no_hook)
 
     def low_latency_combine(self, x: torch.Tensor, topk_idx: torch.Tensor, topk_weights: torch.Tensor, handle: tuple,
                             zero_copy: bool = False, async_finish: bool = False, return_recv_hook: bool = False,
@@ -281,17 +285,16 @@ class Buffer:
             blocks += [torch.zeros((1, topk_weights.size(1)), dtype=topk_weights.dtype, device=topk_weights.device)
                        for _ in range(pad["count"])]
             new_idx, new_scales = pad["topk_idx"], torch.cat(blocks, 0)
-        h = dict(expert_ids=new_idx, expand_idx=src_info, ep_recv_count=layout_range,
-                 num_experts=num_experts)
-        combined = self.runtime.low_latency_combine(x, new_scales, h)
+        rt = self.runtime
+        combined = rt.native.ll_combine(rt._comm, rt._dev, x, new_idx, src_info, layout_range, new_scales, num_experts)
         if pad is not None:
             combined = pad["ori_x"] if pad["count"] == PADDING_SIZE else combined[:PADDING_SIZE - pad["count"]]
             self._pad = None
         if out is not None:
             out.copy_(combined)
             combined = out
-        kept = (x, topk_idx, topk_weights, src_info, layout_range, combined)
-        return combined, self._event(async_finish, kept if async_finish else None), (lambda: None)
+        kept = (x, topk_idx, topk_weights, src_info, layout_range, combined) if async_finish else None
+        return combined, self._event(async_finish, kept), _no_hook
 
     # ---- fused MoE --------------------------------------------------------------------------------------
     def prepack_weight(self, w: torch.Tensor, int4: bool = False) -> torch.Tensor:

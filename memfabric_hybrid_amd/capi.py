@@ -40,6 +40,11 @@ class TensorInfo(ctypes.Structure):
                 ("shape", ctypes.c_uint32 * ZBAL_MAX_TENSOR_DIM), ("reserved", ctypes.c_uint16 * 1)]
 
 
+class PendingCounts(ctypes.Structure):
+    """zbal_pending_counts_t"""
+    _fields_ = [("block", ctypes.c_void_p), ("ticket", ctypes.c_uint64)]
+
+
 class BootstrapOptions(ctypes.Structure):
     _fields_ = [("flags", ctypes.c_uint32), ("btType", ctypes.c_int32), ("ipPort", ctypes.c_char * 64),
                 ("worldSize", ctypes.c_uint16), ("rankId", ctypes.c_uint16), ("deviceId", ctypes.c_uint16),
@@ -120,7 +125,9 @@ SIGNATURES = {
     "zbal_dispatch_normal_notify": (_i32, [_TI, _i64, _i64, _TI, _TI, _TI, _TI, _TI, _vp, _vp, _i64]),
     "zbal_dispatch_normal_layout": (_i32, [_TI, _i64, _i64, _i64, _TI, _TI, _TI, _TI, _vp, _vp, _i64]),
     "zbal_dispatch_normal_layout_in_rank": (_i32, [_TI, _i64, _i64, _i64, _TI, _TI, _TI, _TI, _vp, _vp, _i64]),
-    "zbal_dispatch_normal_notify_counts": (_i32, [_TI, _i64, _i64, _TI, _TI, _TI, _TI, _TI, _vp, _vp, _vp, _i64]),
+    "zbal_dispatch_normal_notify_begin": (_i32, [_TI, _i64, _i64, _TI, _TI, _TI, _TI, _TI, ctypes.POINTER(PendingCounts), _vp,
+                                                 _vp, _i64]),
+    "zbal_dispatch_normal_notify_end": (_i32, [ctypes.POINTER(PendingCounts), _i64, _vp, _vp, _vp, _i64]),
     "zbal_dispatch_normal": (_i32, [_TI, _TI, _TI, _TI, _TI, _i64, _i32, _TI, _TI, _vp, _vp, _i64]),
     "zbal_combine_normal": (_i32, [_TI, _TI, _TI, _TI, _TI, _TI, _u16, _TI, _vp, _vp, _i64]),
     "zbal_dispatch_low_latency": (_i32, [_TI, _TI, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _TI, _TI, _TI, _TI, _TI,
@@ -136,6 +143,7 @@ SIGNATURES = {
     "zbalhip_dispatch_layout_static": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp]),
     "zbalhip_dispatch_layout_in_rank": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp]),
     "zbalhip_dispatch_notify_counts": (_i32, [_vp, _i32, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "zbalhip_host_counts_wait": (_i32, [_vp, _u64, _i64, _vp, _vp]),
     "zbalhip_host_counts_alloc": (_i32, [ctypes.POINTER(_vp)]),
     "zbalhip_host_counts_free": (_i32, [_vp]),
     "zbalhip_dispatch_notify": (_i32, [_vp, _i32, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp]),

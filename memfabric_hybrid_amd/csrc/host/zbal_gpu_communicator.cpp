@@ -360,7 +360,7 @@ public:
                                  const zbal_tensor_info_t *recvBuff, const zbal_tensor_info_t *totalRecvTokens,
                                  const zbal_tensor_info_t *recvTokensPerExpert,
                                  const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,
-                                 aclrtStream stream, int64_t, int64_t *hostCounts) override
+                                 aclrtStream stream, int64_t, zbal_pending_counts_t *pending) override
     {
         const char *op = "NotifyDispatch";
         const int64_t R = info_.groupSize, me = info_.myGroupRank;
@@ -377,15 +377,16 @@ public:
         /* the counts of the other ranks are read where they lie: at the same offset in each rank's window */
         const void *counts[ZBALHIP_MAX_REDUCE_PEERS];
         if (!PeerCopies(op, sendTokensPerExpert->data, (size_t)E * 4, counts)) return Z_INVALID_PARAM;
-        if (hostCounts) {
-            void *block = countsBlocks_.Take();
-            ZBAL_VALIDATE_RETURN(block != nullptr, op << " failed as no pinned memory is left", Z_ERROR);
+        if (pending) {
+            pending->block = countsBlocks_.Take();
+            ZBAL_VALIDATE_RETURN(pending->block != nullptr, op << " failed as no pinned memory is left", Z_ERROR);
             const int32_t rc = zbalhip_dispatch_notify_counts((const int32_t *const *)counts, (int32_t)R, (int32_t)me, E, topKNum,
                                                               (int32_t *)recvBuff->data, (int32_t *)pushTargetOffset->data,
                                                               (int32_t *)totalRecvTokens->data,
                                                               (int64_t *)recvTokensPerExpert->data,
-                                                              (int32_t *)balanceMatrix->data, block, hostCounts, stream);
-            countsBlocks_.GiveBack(block, rc == 0);
+                                                              (int32_t *)balanceMatrix->data, pending->block, &pending->ticket,
+                                                              stream);
+            if (rc != 0) countsBlocks_.GiveBack(pending->block, false);
             return Launched(op, rc);
         }
         return Launched(op, zbalhip_dispatch_notify((const int32_t *const *)counts, (int32_t)R, (int32_t)me, E, topKNum,
@@ -393,6 +394,15 @@ public:
                                                     (int32_t *)totalRecvTokens->data,
                                                     (int64_t *)recvTokensPerExpert->data,
                                                     (int32_t *)balanceMatrix->data, stream));
+    }
+
+    int32_t DispatchNormalNotifyEnd(zbal_pending_counts_t *pending, int64_t sendCount, int64_t *hostCounts,
+                                    aclrtStream stream) override
+    {
+        const int32_t rc = zbalhip_host_counts_wait(pending->block, pending->ticket, sendCount / info_.groupSize, hostCounts, stream);
+        countsBlocks_.GiveBack(pending->block, rc == 0);
+        pending->block = nullptr;
+        return Launched("NotifyDispatch", rc);
     }
 
     static bool TokensShape(const char *op, const zbal_tensor_info_t *x, int64_t *tokens, int64_t *hidden)

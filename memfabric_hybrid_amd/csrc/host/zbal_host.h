@@ -157,7 +157,9 @@ public:
                                          const zbal_tensor_info_t *recvTokensPerExpert,
                                          const zbal_tensor_info_t *pushTargetOffset,
                                          const zbal_tensor_info_t *balanceMatrix, aclrtStream stream,
-                                         int64_t flags, int64_t *hostCounts = nullptr) = 0;
+                                         int64_t flags, zbal_pending_counts_t *pending = nullptr) = 0;
+    virtual int32_t DispatchNormalNotifyEnd(zbal_pending_counts_t *pending, int64_t sendCount, int64_t *hostCounts,
+                                            aclrtStream stream) = 0;
     virtual int32_t DispatchNormal(const zbal_tensor_info_t *srcTokens, const zbal_tensor_info_t *topkIndex,
                                    const zbal_tensor_info_t *sendTokensIndex,
                                    const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,

@@ -746,9 +746,9 @@ extern "C" int32_t zbalhip_host_counts_free(void *block)
 extern "C" int32_t zbalhip_dispatch_notify_counts(const int32_t *const *tokens_per_expert, int32_t ranks, int32_t my_rank,
                                                   int64_t experts, int64_t topk, int32_t *recv_data, int32_t *put_offset,
                                                   int32_t *total_recv, int64_t *recv_tokens_per_expert,
-                                                  int32_t *balance_matrix, void *block, int64_t *host_counts, void *stream)
+                                                  int32_t *balance_matrix, void *block, uint64_t *ticket, void *stream)
 {
-    if (!block || !host_counts) return ZBALHIP_INVALID;
+    if (!block || !ticket) return ZBALHIP_INVALID;
     hipStream_t st = (hipStream_t)stream;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (st != nullptr && hipStreamIsCapturing(st, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone) {
@@ -756,34 +756,40 @@ extern "C" int32_t zbalhip_dispatch_notify_counts(const int32_t *const *tokens_p
         return ZBALHIP_RT_ERROR;
     }
     HostCounts *host = static_cast<HostCounts *>(block);
-    const uint64_t launch = host->ready + 1;
+    *ticket = ranks == 1 ? host->ready + 1 : 0;
     const int32_t rc = launch_notify(tokens_per_expert, ranks, my_rank, experts, topk, recv_data, put_offset, total_recv,
-                                     recv_tokens_per_expert, balance_matrix, host, launch, st);
-    if (rc != ZBALHIP_OK) return rc;
-    if (ranks > 1) {
-        const size_t bytes = (size_t)(experts / ranks) * sizeof(int64_t);
-        if (hipMemcpyAsync(host->counts, recv_tokens_per_expert, bytes, hipMemcpyDeviceToHost, st) != hipSuccess) return ZBALHIP_RT_ERROR;
-        if (hipStreamSynchronize(st) != hipSuccess) return ZBALHIP_RT_ERROR;
-    } else {
+                                     recv_tokens_per_expert, balance_matrix, host, *ticket, st);
+    if (rc != ZBALHIP_OK || ranks == 1) return rc;
+    const size_t bytes = (size_t)(experts / ranks) * sizeof(int64_t);
+    return hipMemcpyAsync(host->counts, recv_tokens_per_expert, bytes, hipMemcpyDeviceToHost, st) == hipSuccess ? ZBALHIP_OK : ZBALHIP_RT_ERROR;
+}
+
+extern "C" int32_t zbalhip_host_counts_wait(void *block, uint64_t ticket, int64_t n, int64_t *host_counts, void *stream)
+{
+    if (!block || !host_counts || n < 0 || n > ZB_MAX_EXPERTS) return ZBALHIP_INVALID;
+    HostCounts *host = static_cast<HostCounts *>(block);
+    bool arrived = false;
+    if (ticket != 0) {
         /*
-         * The flag arrives a few microseconds after the kernels in front of this one have run. A stream with long work
+         * The flag arrives a few microseconds after the kernels in front of the notify have run. A stream with long work
          * queued is not spun on for more than a millisecond; the runtime's wait takes over, and reports a stream that
          * will never get there.
          */
         timespec t0, t1;
         clock_gettime(CLOCK_MONOTONIC, &t0);
-        bool arrived = false;
-        for (int spin = 0; !arrived; ++spin) {
-            arrived = __atomic_load_n(&host->ready, __ATOMIC_ACQUIRE) == launch;
+        for (int spin = 0;; ++spin) {
+            arrived = __atomic_load_n(&host->ready, __ATOMIC_ACQUIRE) == ticket;
             if (arrived) break;
             __builtin_ia32_pause();
             if ((spin & 63) != 63) continue;
             clock_gettime(CLOCK_MONOTONIC, &t1);
             if ((t1.tv_sec - t0.tv_sec) * 1000000000ll + (t1.tv_nsec - t0.tv_nsec) > 1000000) break;
         }
-        if (!arrived && hipStreamSynchronize(st) != hipSuccess) return ZBALHIP_RT_ERROR;
-        if (!arrived && __atomic_load_n(&host->ready, __ATOMIC_ACQUIRE) != launch) return ZBALHIP_RT_ERROR;
     }
-    for (int64_t e = 0; e < experts / ranks; ++e) host_counts[e] = host->counts[e];
+    if (!arrived) {
+        if (hipStreamSynchronize((hipStream_t)stream) != hipSuccess) return ZBALHIP_RT_ERROR;
+        if (ticket != 0 && __atomic_load_n(&host->ready, __ATOMIC_ACQUIRE) != ticket) return ZBALHIP_RT_ERROR;
+    }
+    for (int64_t e = 0; e < n; ++e) host_counts[e] = host->counts[e];
     return ZBALHIP_OK;
 }

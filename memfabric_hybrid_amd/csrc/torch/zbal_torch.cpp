@@ -18,7 +18,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
-#include <string>
+#include <cstdlib>
+#include <cstring>
 #include <vector>
 
 #include "zbal.h"
@@ -31,7 +32,8 @@ struct Library {
     decltype(&zbal_moe_topk_route) topk_route;
     decltype(&zbal_dispatch_normal_layout_in_rank) layout;
     decltype(&zbal_dispatch_normal_notify) notify;
-    decltype(&zbal_dispatch_normal_notify_counts) notify_counts;
+    decltype(&zbal_dispatch_normal_notify_begin) notify_begin;
+    decltype(&zbal_dispatch_normal_notify_end) notify_end;
     decltype(&zbal_dispatch_normal) dispatch;
     decltype(&zbal_combine_normal) combine;
     decltype(&zbal_dispatch_low_latency) ll_dispatch;
@@ -150,8 +152,11 @@ at::Tensor expert_ids(const at::Tensor &t)
 
 /*
  * The outputs of one call. Large ones have an allocation each; the small ones (indices, counts, offsets) share one:
- * several tensors over one storage, each at a 256-byte boundary.
+ * several tensors over one storage, each at a 256-byte boundary. (An allocation is 0.8 us of host time; a tensor kept
+ * for long pins only what it shares the storage with, hence the limit.)
  */
+constexpr int64_t kShareBytes = 1 << 20;
+
 class Outputs {
 public:
     explicit Outputs(c10::Device dev) : dev_(dev) {}
@@ -287,8 +292,8 @@ struct Note {
     at::Tensor recv_data, recv_per_expert, put_offset, balance, total;
 };
 
-/* host_counts: also wait for the counts and leave them there */
-Note notify_call(const Frame &f, const at::Tensor &per_expert, int64_t topk, std::vector<int64_t> *host_counts)
+/* pending: the counts are wanted on the host as well */
+Note notify_call(const Frame &f, const at::Tensor &per_expert, int64_t topk, zbal_pending_counts_t *pending)
 {
     const int64_t E = per_expert.size(0);
     Outputs out(f.dev);
@@ -297,10 +302,9 @@ Note notify_call(const Frame &f, const at::Tensor &per_expert, int64_t topk, std
     Note n{out.make(o0, {1, E}, at::kInt), out.make(o1, {E}, at::kLong), out.make(o2, {1, E}, at::kInt),
            out.make(o3, {1, 2}, at::kInt), out.make(o4, {1}, at::kInt)};
     const Info i0(per_expert), i1(n.recv_data), i2(n.total), i3(n.recv_per_expert), i4(n.put_offset), i5(n.balance);
-    if (host_counts) host_counts->resize((size_t)E);
     check("zbal_dispatch_normal_notify", unlocked([&] {
-              return host_counts ? L.notify_counts(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, host_counts->data(), f.comm, f.stream, 0)
-                                 : L.notify(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, f.comm, f.stream, 0);
+              return pending ? L.notify_begin(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, pending, f.comm, f.stream, 0)
+                             : L.notify(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, f.comm, f.stream, 0);
           }));
     return n;
 }
@@ -313,13 +317,13 @@ PyObject *notify(PyObject *const *args, Py_ssize_t nargs)
     return tuple_of(wrap(n.recv_data), wrap(n.recv_per_expert), wrap(n.put_offset), wrap(n.balance), wrap(n.total));
 }
 
-/* the receive tensors of `rows` rows for one quantisation mode: rows, scales */
-void receive(Outputs &out, int64_t qm, const at::Tensor &x, int64_t rows, int64_t none_scales, at::Tensor *recv, at::Tensor *scales)
+/* the receive tensors of `rows` rows for one quantisation mode: rows, scales (one unused scale without quantisation) */
+void receive(Outputs &out, int64_t qm, const at::Tensor &x, int64_t rows, at::Tensor *recv, at::Tensor *scales)
 {
     const int64_t H = x.size(1);
     if (qm == NO_QUANT) {
         *recv = out.big({rows, H}, x.scalar_type());
-        *scales = out.big({none_scales}, at::kFloat);
+        *scales = out.big({1}, at::kFloat);
     } else if (qm == QUANT_BF16_2_INT8) {
         *recv = out.big({rows, H}, at::kChar);
         *scales = out.big({rows}, at::kFloat);
@@ -333,7 +337,7 @@ void dispatch_call(const Frame &f, const at::Tensor &x, const at::Tensor &ids, c
                    const at::Tensor &balance, int64_t E, int64_t qm, int64_t rows, at::Tensor *recv, at::Tensor *scales)
 {
     Outputs out(f.dev);
-    receive(out, qm, x, rows, 1, recv, scales);
+    receive(out, qm, x, rows, recv, scales);
     const Info i0(x), i1(ids), i2(send), i3(put_offset), i4(balance), i5(*recv), i6(*scales);
     check("zbal_dispatch_normal", unlocked([&] {
               return L.dispatch(*i0, *i1, *i2, *i3, *i4, E, (zbal_quant_mode_t)qm, *i5, *i6, f.comm, f.stream, 0);
@@ -352,35 +356,46 @@ PyObject *dispatch(PyObject *const *args, Py_ssize_t nargs)
 /*
  * Notify and dispatch in one call. (comm, dev, x, ids, send_idx, per_expert, quant_mode, worst_rows, running) ->
  * (recv, scales, list of received counts, put_offset, balance_matrix). worst_rows > 0: that many rows, an empty list
- * and no wait for the GPU; else the counts are read back (one wait), recv has their sum of rows (one at least), and
- * the list holds them, or their running sums.
+ * and no wait for the GPU; else the counts are read back, recv has their sum of rows (one at least), and the list holds
+ * them, or their running sums. The read-back does not hold the GPU up: the dispatch goes into tensors with a row for
+ * every pick and is queued before the counts are waited for; what is returned are the rows that there are.
  */
 PyObject *dispatch_counts(PyObject *const *args, Py_ssize_t nargs)
 {
     const Frame f(args, nargs, 9);
-    const at::Tensor &x = f.t(2);
-    const at::Tensor ids = expert_ids(f.t(3)), &per_expert = f.t(5);
-    const int64_t worst = f.n(7);
-    std::vector<int64_t> counts;
-    const Note n = notify_call(f, per_expert, f.t(3).size(1), worst > 0 ? nullptr : &counts);
-    int64_t rows = worst, run = 0;
-    PyObject *list = PyList_New((Py_ssize_t)counts.size());
-    if (worst <= 0) {
-        int64_t total = 0;
-        const bool running = f.n(8) != 0;
-        for (size_t e = 0; e < counts.size(); ++e) {
-            total += counts[e];
-            run = running ? run + counts[e] : counts[e];
-            PyList_SET_ITEM(list, (Py_ssize_t)e, PyLong_FromLongLong(run));
-        }
-        rows = total == 0 ? 1 : total;
-    }
+    const at::Tensor &x = f.t(2), &per_expert = f.t(5);
+    const at::Tensor ids = expert_ids(f.t(3));
+    const int64_t worst = f.n(7), E = per_expert.size(0), qm = f.n(6), most = ids.numel() > 0 ? ids.numel() : 1;
+    zbal_pending_counts_t pending = {};
+    const Note n = notify_call(f, per_expert, ids.size(1), worst > 0 ? nullptr : &pending);
     at::Tensor recv, scales;
-    try {
-        dispatch_call(f, x, ids, f.t(4), n.put_offset, n.balance, per_expert.size(0), f.n(6), rows, &recv, &scales);
-    } catch (...) {
-        Py_DECREF(list);
-        throw;
+    std::vector<int64_t> counts;
+    if (worst > 0) {
+        dispatch_call(f, x, ids, f.t(4), n.put_offset, n.balance, E, qm, worst, &recv, &scales);
+    } else {
+        counts.resize((size_t)E);
+        auto wait = [&] { return L.notify_end(&pending, E, counts.data(), f.comm, f.stream, 0); };
+        try {
+            dispatch_call(f, x, ids, f.t(4), n.put_offset, n.balance, E, qm, most, &recv, &scales);
+        } catch (...) {
+            (void)wait();
+            throw;
+        }
+        check("zbal_dispatch_normal_notify", unlocked(wait));
+    }
+    int64_t total = 0;
+    for (const int64_t c : counts) total += c;
+    const int64_t rows = total == 0 ? 1 : total;
+    if (worst <= 0 && rows < most) {
+        recv = recv.narrow(0, 0, rows);
+        if (qm != NO_QUANT) scales = scales.narrow(0, 0, rows);
+    }
+    PyObject *list = PyList_New((Py_ssize_t)counts.size());
+    const bool running = f.n(8) != 0;
+    int64_t run = 0;
+    for (size_t e = 0; e < counts.size(); ++e) {
+        run = running ? run + counts[e] : counts[e];
+        PyList_SET_ITEM(list, (Py_ssize_t)e, PyLong_FromLongLong(run));
     }
     return tuple_of(wrap(recv), wrap(scales), list, wrap(n.put_offset), wrap(n.balance));
 }
@@ -401,21 +416,36 @@ PyObject *combine(PyObject *const *args, Py_ssize_t nargs)
     return wrap(out);
 }
 
-/* (comm, dev, x, ids, max_tokens, experts, quant_mode, token_nums_type) -> (recv, scales, recv_count, expand_idx, ep_recv_count) */
+/* MOE_EXPERT_TOKEN_NUMS_TYPE (zbal_deepep.cpp:497), 1 where it is not set */
+int64_t token_nums_type()
+{
+    const char *v = getenv("MOE_EXPERT_TOKEN_NUMS_TYPE");
+    if (v == nullptr) return 1;
+    char *end = nullptr;
+    const long n = strtol(v, &end, 10);
+    if (end == v || *end != 0) fail(PyExc_ValueError, "MOE_EXPERT_TOKEN_NUMS_TYPE is not a number");
+    return n;
+}
+
+/* (comm, dev, x, ids, max_tokens, experts, quant_mode) -> (recv, scales, recv_count, expand_idx, ep_recv_count) */
 PyObject *ll_dispatch(PyObject *const *args, Py_ssize_t nargs)
 {
-    const Frame f(args, nargs, 8);
+    const Frame f(args, nargs, 7);
     const at::Tensor &x = f.t(2);
     const at::Tensor ids = expert_ids(f.t(3));
-    const int64_t T = x.size(0), K = ids.size(1), rows = T * K > 0 ? T * K : 1, E = f.n(5), qm = f.n(6), most = f.n(4), type = f.n(7);
+    const int64_t T = x.size(0), K = ids.size(1), H = x.size(1), rows = T * K > 0 ? T * K : 1, E = f.n(5), qm = f.n(6), most = f.n(4),
+                  type = token_nums_type(), blocks = qm == QUANT_BF16_2_FP8E4M3_B128 ? H / 128 : 1;
+    const at::ScalarType rt = qm == NO_QUANT ? x.scalar_type() : qm == QUANT_BF16_2_INT8 ? at::kChar : at::kFloat8_e4m3fn;
     Outputs out(f.dev);
+    const bool share = rows * H * (int64_t)c10::elementSize(rt) <= kShareBytes;
+    const size_t orecv = share ? out.plan(rows * H, rt) : 0, oscale = out.plan(rows * blocks, at::kFloat);
     const size_t o0 = out.plan(rows, at::kInt), o1 = out.plan(E, at::kInt), o2 = out.plan(E, at::kLong), o3 = out.plan(E, at::kInt),
                  o4 = out.plan(E, at::kFloat);
     const at::Tensor expand_idx = out.make(o0, {rows}, at::kInt), ep_recv = out.make(o1, {E}, at::kInt),
                      nums = out.make(o2, {E}, at::kLong), put_offset = out.make(o3, {E}, at::kInt),
                      status = out.make(o4, {E}, at::kFloat);
-    at::Tensor recv, scales;
-    receive(out, qm, x, rows, rows, &recv, &scales);
+    const at::Tensor recv = share ? out.make(orecv, {rows, H}, rt) : out.big({rows, H}, rt),
+                     scales = qm == QUANT_BF16_2_FP8E4M3_B128 ? out.make(oscale, {rows, blocks}, at::kFloat) : out.make(oscale, {rows}, at::kFloat);
     const Info i0(x), i1(ids), i2(recv), i3(scales), i4(expand_idx), i5(nums), i6(ep_recv), i7(put_offset), i8(status);
     check("zbal_dispatch_low_latency", unlocked([&] {
               return L.ll_dispatch(*i0, *i1, E, 1, 0, qm, T > most ? T : most, 0, type, *i2, *i3, *i4, *i5, *i6, *i7, *i8, f.comm,
@@ -598,7 +628,8 @@ PyObject *bind(PyObject *const *args, Py_ssize_t nargs)
     void *h = dlopen(path, RTLD_NOW | RTLD_LOCAL);
     if (h == nullptr) fail(PyExc_RuntimeError, dlerror());
     if (!find(h, "zbal_moe_topk_route", &L.topk_route) || !find(h, "zbal_dispatch_normal_layout_in_rank", &L.layout) ||
-        !find(h, "zbal_dispatch_normal_notify", &L.notify) || !find(h, "zbal_dispatch_normal_notify_counts", &L.notify_counts) ||
+        !find(h, "zbal_dispatch_normal_notify", &L.notify) || !find(h, "zbal_dispatch_normal_notify_begin", &L.notify_begin) ||
+        !find(h, "zbal_dispatch_normal_notify_end", &L.notify_end) ||
         !find(h, "zbal_dispatch_normal", &L.dispatch) || !find(h, "zbal_combine_normal", &L.combine) ||
         !find(h, "zbal_dispatch_low_latency", &L.ll_dispatch) || !find(h, "zbal_combine_low_latency", &L.ll_combine) ||
         !find(h, "zbal_fused_deep_moe", &L.fused) || !find(h, "zbal_fused_deep_moe_workspace_size", &L.fused_workspace))

@@ -18,7 +18,6 @@ live in buffer.py. Differences from the reference's adaptor, all deliberate:
 torch is used for device memory and streams only.
 """
 import ctypes
-import os
 import threading
 
 import torch
@@ -169,10 +168,9 @@ class OperatorBuffer:
     def low_latency_dispatch(self, x, topk_idx, num_max_dispatch_tokens_per_rank, num_experts, use_fp8=True,
                              fp8_block_scale=False):
         """zbal_deepep.cpp:454-565. Returns (packed_recv_x, packed_recv_x_scales, packed_recv_count, handle)."""
-        token_nums_type = int(os.environ.get("MOE_EXPERT_TOKEN_NUMS_TYPE", "1"))
         qm = capi.NO_QUANT if not use_fp8 else capi.QUANT_FP8_B128 if fp8_block_scale else capi.QUANT_INT8
         recv, scales, packed_recv_count, expand_idx, ep_recv_count = self.native.ll_dispatch(
-            self._comm, self._dev, x, topk_idx, num_max_dispatch_tokens_per_rank, num_experts, qm, token_nums_type)
+            self._comm, self._dev, x, topk_idx, num_max_dispatch_tokens_per_rank, num_experts, qm)
         handle = dict(expert_ids=topk_idx, expand_idx=expand_idx, ep_recv_count=ep_recv_count, num_experts=num_experts)
         return recv, scales, packed_recv_count, handle
 

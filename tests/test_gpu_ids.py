@@ -58,7 +58,7 @@ def test_layout_in_one_launch(buf, T, K, E, R, npdt):
 
 @pytest.mark.parametrize("E", [1, 63, 64, 65, 1024])
 def test_counts_read_back_by_the_notify_kernel(buf, E):
-    """Several calls in a row, with work queued in front, give the counts of that call."""
+    """Several calls in a row, with work queued in front and behind, give the counts of that call."""
     out = {k: torch.empty(n, dtype=t, device="cuda") for k, n, t in
            (("recv", E, torch.int32), ("put", E, torch.int32), ("total", 1, torch.int32), ("per", E, torch.int64),
             ("bal", 2, torch.int32))}
@@ -69,9 +69,13 @@ def test_counts_read_back_by_the_notify_kernel(buf, E):
         busy = torch.randn((2048, 2048), device="cuda")
         for _ in range(10 * rep):
             busy = busy @ busy * 1e-3
-        capi.check("notify", buf.lib.zbal_dispatch_normal_notify_counts(
+        pending = capi.PendingCounts()
+        capi.check("begin", buf.lib.zbal_dispatch_normal_notify_begin(
             ref(ti(counts)), E, 4, ref(ti(out["recv"])), ref(ti(out["total"])), ref(ti(out["per"])), ref(ti(out["put"])),
-            ref(ti(out["bal"])), got.ctypes.data, buf.comm, capi.stream_ptr(), 0))
+            ref(ti(out["bal"])), ref(pending), buf.comm, capi.stream_ptr(), 0))
+        busy = busy @ busy                                   # work behind the notify
+        capi.check("end", buf.lib.zbal_dispatch_normal_notify_end(ref(pending), E, got.ctypes.data, buf.comm,
+                                                                  capi.stream_ptr(), 0))
         assert np.array_equal(got, c)
         assert np.array_equal(host(out["put"]), np.cumsum(c) - c) and host(out["total"])[0] == c.sum()
         assert np.array_equal(host(out["per"]), c)
