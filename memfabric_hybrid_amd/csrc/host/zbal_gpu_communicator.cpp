@@ -240,7 +240,8 @@ public:
                 out[r] = static_cast<const uint8_t *>(p) + ((int64_t)info_.worldRank[r] - me) * (int64_t)info_.peerStride;
             return true;
         }
-        const std::vector<PeerWindow> peers = Peers();
+        std::lock_guard<std::mutex> guard(peersMutex_);
+        const std::vector<PeerWindow> &peers = info_.peers;
         const PeerWindow &mine = peers[info_.myGroupRank];
         const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(mine.base);
         if (mine.base == nullptr || a < b || a + bytes > b + mine.size) {
@@ -261,7 +262,7 @@ public:
     /* the copies of `p` in every rank's window; a group of one needs no window: its only copy is `p` itself */
     bool PeerCopies(const char *op, const void *p, size_t bytes, const void **out) const
     {
-        if (info_.groupSize == 1 && info_.peerStride == 0 && Peers()[0].base == nullptr) {
+        if (info_.groupSize == 1 && info_.peerStride == 0 && NoWindow()) {
             out[0] = p;
             return true;
         }
@@ -299,7 +300,7 @@ public:
         }
         const size_t es = ElemSize(dt);
         const void *peer[ZBALHIP_MAX_REDUCE_PEERS];
-        if (info_.groupSize == 1 && info_.peerStride == 0 && Peers()[0].base == nullptr) {
+        if (info_.groupSize == 1 && info_.peerStride == 0 && NoWindow()) {
             peer[0] = send; /* a group of one needs no window */
         } else if (!Translate(opName, send, (sliceOffsetElems + count) * es, peer)) {
             return Z_INVALID_PARAM;

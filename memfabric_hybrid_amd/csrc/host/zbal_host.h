@@ -135,10 +135,11 @@ public:
         std::lock_guard<std::mutex> guard(peersMutex_);
         info_.peers[rank] = w;
     }
-    std::vector<PeerWindow> Peers() const
+    /* no window registered for this rank */
+    bool NoWindow() const
     {
         std::lock_guard<std::mutex> guard(peersMutex_);
-        return info_.peers;
+        return info_.peers[info_.myGroupRank].base == nullptr;
     }
 
     virtual int32_t AllReduce(const void *send, void *recv, void *buffer, size_t count, zbal_datatype_t dt,

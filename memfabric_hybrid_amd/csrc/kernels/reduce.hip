@@ -138,20 +138,66 @@ __device__ __forceinline__ typename Elem<DT>::acc_t fold_elem(typename Elem<DT>:
     }
 }
 
-template <int DT, int OP, int N>
-__global__ void __launch_bounds__(256)
-reduce_kernel(ReducePtrs in, int n_in, int64_t nvec, u32x4 *__restrict__ out)
+/* one element of a buffer, as the fold wants it, and back */
+template <int DT> __device__ __forceinline__ typename Elem<DT>::acc_t load_elem(const void *p, int64_t j)
 {
     typedef typename Elem<DT>::acc_t A;
-    constexpr int PER = Elem<DT>::per;
+    if constexpr (DT == ZDT_FP32) return ((const float *)p)[j];
+    else if constexpr (DT == ZDT_INT32) return (A)((const uint32_t *)p)[j];
+    else if constexpr (DT == ZDT_INT64) return ((const int64_t *)p)[j];
+    else if constexpr (DT == ZDT_INT8) return (A)((const int8_t *)p)[j];
+    else if constexpr (DT == ZDT_INT16) return (A)((const int16_t *)p)[j];
+    else return zb_half_to_f32<DT>(((const uint16_t *)p)[j]);
+}
+template <int DT> __device__ __forceinline__ void store_elem(void *out, int64_t j, typename Elem<DT>::acc_t v)
+{
+    if constexpr (DT == ZDT_FP32) ((float *)out)[j] = v;
+    else if constexpr (DT == ZDT_INT32) ((uint32_t *)out)[j] = (uint32_t)v;
+    else if constexpr (DT == ZDT_INT64) ((int64_t *)out)[j] = v;
+    else if constexpr (DT == ZDT_INT8) ((int8_t *)out)[j] = (int8_t)v;
+    else if constexpr (DT == ZDT_INT16) ((int16_t *)out)[j] = (int16_t)v;
+    else ((uint16_t *)out)[j] = (uint16_t)zb_f32_to_half<DT>(v);
+}
+
+/* [0, head) element by element, then nvec 16-byte vectors of the output, then the rest up to count element by element */
+struct ReduceSpan {
+    int64_t count, nvec;
+    int head;
+    int chunk;                      /* consecutive blocks per XCD and turn, 0: blocks in order */
+};
+
+constexpr int kMaxReduceThreads = 1024;
+typedef u32x4 __attribute__((aligned(1))) u32x4_any_offset;      /* global loads may sit at any byte */
+
+/*
+ * The output's vectors are aligned; ANY_OFFSET: the inputs' need not be, and are read with vector loads that are only
+ * aligned to their elements (reduce-scatter slices of odd length: 2 x 10^8 halves 287 us element by element, as this was
+ * done before, 148 so; loads from the dword below, shifted into place, are slower again, 1 ms, for the registers they
+ * take over 16 inputs). The few elements around the vectors belong to the last block, so there is one launch whatever
+ * the offsets and the length.
+ */
+template <int DT, int OP, int N, bool ANY_OFFSET>
+__global__ void __launch_bounds__(kMaxReduceThreads)
+reduce_kernel(ReducePtrs in, int n_in, ReduceSpan sp, void *__restrict__ out_base)
+{
+    typedef typename Elem<DT>::acc_t A;
+    constexpr int PER = Elem<DT>::per, ESZ = 16 / PER;
+    const int64_t skip = (int64_t)sp.head * ESZ;
+    typedef std::conditional_t<ANY_OFFSET, u32x4_any_offset, u32x4> vec_in;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    u32x4 *out = reinterpret_cast<u32x4 *>((char *)out_base + skip);
+    int64_t b = blockIdx.x;
+    if (sp.chunk) {                 /* gridDim.x is a multiple of 8 * chunk then */
+        const int64_t turn = b / (8 * sp.chunk), r = b - turn * (8 * sp.chunk);
+        b = turn * (8 * sp.chunk) + (r & 7) * sp.chunk + (r >> 3);
+    }
     trace_record(in, false);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nvec; i += stride) {
+    for (int64_t i = b * blockDim.x + threadIdx.x; i < sp.nvec; i += stride) {
         u32x4 v[N];
 #pragma unroll
         for (int p = 0; p < N; ++p)
             if (N != ZBALHIP_MAX_REDUCE_PEERS || p < n_in)
-                v[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(in.p[p]) + i);
+                v[p] = __builtin_nontemporal_load(reinterpret_cast<const vec_in *>((const char *)in.p[p] + skip) + i);
         A acc[PER], cur[PER];
         unpack<DT>(v[0], acc);
 #pragma unroll
@@ -164,86 +210,53 @@ reduce_kernel(ReducePtrs in, int n_in, int64_t nvec, u32x4 *__restrict__ out)
         }
         out[i] = pack<DT>(acc);      /* inputs are streamed (non-temporal loads); the plain store measured 5% faster than a non-temporal one */
     }
+    if (blockIdx.x == gridDim.x - 1) {
+        const int64_t rest = sp.head + sp.nvec * PER, n = sp.head + (sp.count - rest);
+        for (int64_t k = threadIdx.x; k < n; k += blockDim.x) {
+            const int64_t j = k < sp.head ? k : rest + (k - sp.head);
+            A acc = load_elem<DT>(in.p[0], j);
+            for (int p = 1; p < n_in; ++p) acc = fold_elem<DT, OP>(acc, load_elem<DT>(in.p[p], j));
+            store_elem<DT>(out_base, j, acc);
+        }
+    }
     trace_record(in, true);
 }
 
-/* elements past the last whole 16-byte vector */
 template <int DT, int OP>
-__global__ void reduce_tail_kernel(ReducePtrs in, int n_in, int64_t first, int64_t count, void *out)
+int32_t launch_reduce(const ReducePtrs &ptrs, int n_in, int64_t count, void *out, bool same_offset, hipStream_t st)
 {
-    typedef typename Elem<DT>::acc_t A;
-    constexpr int ESZ = 16 / Elem<DT>::per;
-    const int64_t j = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= count) return;
-    auto load = [&](const void *p) -> A {
-        if constexpr (ESZ == 4 && DT == ZDT_FP32) return ((const float *)p)[j];
-        else if constexpr (ESZ == 4) return (A)((const uint32_t *)p)[j];
-        else if constexpr (ESZ == 8) return ((const int64_t *)p)[j];
-        else if constexpr (DT == ZDT_INT8) return (A)((const int8_t *)p)[j];
-        else if constexpr (DT == ZDT_INT16) return (A)((const int16_t *)p)[j];
-        else return zb_half_to_f32<DT>(((const uint16_t *)p)[j]);
-    };
-    A acc = load(in.p[0]);
-    for (int p = 1; p < n_in; ++p) acc = fold_elem<DT, OP>(acc, load(in.p[p]));
-    if constexpr (ESZ == 4 && DT == ZDT_FP32) ((float *)out)[j] = acc;
-    else if constexpr (ESZ == 4) ((uint32_t *)out)[j] = (uint32_t)acc;
-    else if constexpr (ESZ == 8) ((int64_t *)out)[j] = acc;
-    else if constexpr (DT == ZDT_INT8) ((int8_t *)out)[j] = (int8_t)acc;
-    else if constexpr (DT == ZDT_INT16) ((int16_t *)out)[j] = (int16_t)acc;
-    else ((uint16_t *)out)[j] = (uint16_t)zb_f32_to_half<DT>(acc);
-}
-
-/* element by element over [first, count): the tail of the vector path, and the whole job when the bases disagree about their alignment */
-template <int DT, int OP>
-void launch_scalar(const ReducePtrs &ptrs, int n_in, int64_t first, int64_t count, void *out, hipStream_t st)
-{
-    const int64_t n = count - first;
-    if (n <= 0) return;
-    if (n <= 64) reduce_tail_kernel<DT, OP><<<1, 64, 0, st>>>(ptrs, n_in, first, count, out);
-    else reduce_tail_kernel<DT, OP><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(ptrs, n_in, first, count, out);
-}
-
-/*
- * `head` = elements in front of the first 16-byte boundary, the same for every base (0 when they are aligned), or
- * -1 when the bases sit at different offsets from a boundary: then no vector of one lines up with a vector of the
- * others, and the job runs element by element (correct, several times slower; reduce-scatter slices of odd length are
- * the case it is for).
- */
-template <int DT, int OP>
-int32_t launch_reduce(ReducePtrs ptrs, int n_in, int64_t count, void *out, int head, hipStream_t st)
-{
-    constexpr int PER = Elem<DT>::per;
-    constexpr int ESZ = 16 / PER;
-    if (head < 0) {
-        launch_scalar<DT, OP>(ptrs, n_in, 0, count, out, st);
-        return zbalhip_check_launch();
+    constexpr int PER = Elem<DT>::per, ESZ = 16 / PER;
+    ReduceSpan sp = {};
+    const unsigned mis = (unsigned)((uintptr_t)out & 15u);
+    const int64_t head = mis ? (16 - mis) / ESZ : 0;
+    sp.count = count;
+    sp.head = (int)(head < count ? head : count);
+    sp.nvec = (count - sp.head) / PER;
+    /*
+     * One 16-byte vector per thread: short-lived workgroups stream faster (6.2 TB/s for 8 x 256 MiB) than a capped grid
+     * with a grid-stride loop (5.3 TB/s); the loop only serves huge counts. From 8 Mi vectors on (128 MiB of output):
+     * workgroups of 1024, and each XCD takes 512 KiB in a row of every buffer, so that it needs fewer pages at a time
+     * (three sets of 8 x 256 MiB in turn, more than the address caches hold: 423 -> 408 us; 256 threads in order 423,
+     * 1024 in order 416, 256 KiB and 2 MiB in a row 430).
+     */
+    const bool big = sp.nvec >= (8ll << 20);
+    const int threads = big ? kMaxReduceThreads : 256;
+    int64_t blocks = (sp.nvec + threads - 1) / threads;
+    const int64_t cap = 1 << 22;
+    if (blocks > cap) blocks = cap;
+    if (blocks < 1) blocks = 1;
+    if (big) {
+        sp.chunk = 32;
+        blocks = (blocks + 255) / 256 * 256;
     }
-    if (head > 0) {
-        if (head > count) head = (int)count;
-        launch_scalar<DT, OP>(ptrs, n_in, 0, head, out, st);
-        for (int p = 0; p < n_in; ++p) ptrs.p[p] = (const char *)ptrs.p[p] + (size_t)head * ESZ;
-        out = (char *)out + (size_t)head * ESZ;
-        count -= head;
-        if (count == 0) return zbalhip_check_launch();
-    }
-    const int64_t nvec = count / PER;
-    if (nvec > 0) {
-        /* one 16-byte vector per thread: measured on MI355X, short-lived workgroups stream faster (6.2 TB/s for
-           8 x 256 MiB) than a capped grid with a grid-stride loop (5.3 TB/s); the loop only serves huge counts */
-        int64_t blocks = (nvec + 255) / 256;
-        const int64_t cap = 1 << 22;
-        if (blocks > cap) blocks = cap;
-        u32x4 *o = (u32x4 *)out;
-        switch (n_in) {
-            case 1: reduce_kernel<DT, OP, 1><<<(unsigned)blocks, 256, 0, st>>>(ptrs, n_in, nvec, o); break;
-            case 2: reduce_kernel<DT, OP, 2><<<(unsigned)blocks, 256, 0, st>>>(ptrs, n_in, nvec, o); break;
-            case 4: reduce_kernel<DT, OP, 4><<<(unsigned)blocks, 256, 0, st>>>(ptrs, n_in, nvec, o); break;
-            case 8: reduce_kernel<DT, OP, 8><<<(unsigned)blocks, 256, 0, st>>>(ptrs, n_in, nvec, o); break;
-            default:
-                reduce_kernel<DT, OP, ZBALHIP_MAX_REDUCE_PEERS><<<(unsigned)blocks, 256, 0, st>>>(ptrs, n_in, nvec, o);
-        }
-    }
-    launch_scalar<DT, OP>(ptrs, n_in, nvec * PER, count, out, st);
+#define ZB_REDUCE(N, ANY) reduce_kernel<DT, OP, N, ANY><<<(unsigned)blocks, threads, 0, st>>>(ptrs, n_in, sp, out)
+    if (!same_offset) ZB_REDUCE(ZBALHIP_MAX_REDUCE_PEERS, true);
+    else if (n_in == 1) ZB_REDUCE(1, false);
+    else if (n_in == 2) ZB_REDUCE(2, false);
+    else if (n_in == 4) ZB_REDUCE(4, false);
+    else if (n_in == 8) ZB_REDUCE(8, false);
+    else ZB_REDUCE(ZBALHIP_MAX_REDUCE_PEERS, false);
+#undef ZB_REDUCE
     return zbalhip_check_launch();
 }
 
@@ -259,12 +272,11 @@ template <int DT> int32_t dispatch_op(const ReducePtrs &ptrs, int n_in, int64_t 
         if (m % ESZ) return ZBALHIP_INVALID;
         same = same && m == mis;
     }
-    const int head = !same ? -1 : (mis ? (int)((16 - mis) / ESZ) : 0);
     switch (op) {
-        case OP_PROD: return launch_reduce<DT, OP_PROD>(ptrs, n_in, count, out, head, st);
-        case OP_SUM: return launch_reduce<DT, OP_SUM>(ptrs, n_in, count, out, head, st);
-        case OP_MAX: return launch_reduce<DT, OP_MAX>(ptrs, n_in, count, out, head, st);
-        case OP_MIN: return launch_reduce<DT, OP_MIN>(ptrs, n_in, count, out, head, st);
+        case OP_PROD: return launch_reduce<DT, OP_PROD>(ptrs, n_in, count, out, same, st);
+        case OP_SUM: return launch_reduce<DT, OP_SUM>(ptrs, n_in, count, out, same, st);
+        case OP_MAX: return launch_reduce<DT, OP_MAX>(ptrs, n_in, count, out, same, st);
+        case OP_MIN: return launch_reduce<DT, OP_MIN>(ptrs, n_in, count, out, same, st);
         default: return ZBALHIP_INVALID;
     }
 }
