@@ -1,0 +1,406 @@
+/*
+ * The grouped GEMM as a weight stream: the kernel for experts with few rows each, and for int4 weights with any number.
+ *
+ * A weight byte is wanted by one wave only, so the weights do not go through LDS: a wave keeps the fragments of the next
+ * four slabs (128 K each) of its own 32 channels in flight in registers, in exactly the order the pre-pack stores them
+ * (a 16-channel sub-tile of a slab is 2 KiB of consecutive bytes, int4 1 KiB), and nothing in the stream waits for
+ * another wave. The activations, which all eight waves read, come in chunks of four slabs through two LDS buffers filled
+ * by DMA: one barrier per four slabs. Workgroup tile: TM rows x 256 channels; a wave has all rows of its 32 channels
+ * (first GEMM: 16 gate and the matching 16 up columns), so a weight is unpacked once, and the epilogue is that of the
+ * kernel that stages the slabs (gemm.hip).
+ *
+ * With 128 registers per lane and at most 80 KiB of LDS two workgroups are resident per CU: four waves per SIMD to cover
+ * each other's waits, 256 KiB of 8-bit weights in flight, one workgroup's start and epilogue behind the other's stream.
+ * Workgroups are not persistent: the dispatcher evens out what a fixed sequence of tiles per CU cannot (528 tiles on 256
+ * CUs, popular experts).
+ *
+ * What bounds it: 8-bit weights the HBM stream (6.1-6.6 TB/s), int4 the vector instructions that unpack and scale
+ * (active in 43 % of the cycles, MFMA in 16 %, at 32 rows per expert). Layers against the staging kernel on one GPU, other
+ * weights on every pass: W8A8, 128 experts of 4096 x 3072 / 1536 x 4096, top-8, 509 tokens 487 -> 461 us, Zipf(1.2)
+ * routing 508 -> 457; 64 of 2048 x 2048 / 1024 x 2048, top-6, 200 tokens 111 -> 97. W4A8, 128 experts: 20 tokens 188 -> 166,
+ * 509 tokens 320 -> 271, Zipf 397 -> 294, 2048 Zipf 842 -> 562, 16384 (96 rows) 3913 -> 3749.
+ */
+#ifndef ZBAL_GEMM_STREAM_H_
+#define ZBAL_GEMM_STREAM_H_
+
+#include "zbal_gemm_tile.h"
+
+namespace {
+
+template <int MODE, int TM> struct StreamShape {
+    /* at many rows per expert (TM = 96) the L2 serves the weights: two slabs of look-ahead do, and leave room for six row sub-tiles */
+    static constexpr int PF = TM > 64 ? 2 : 4;                  /* slabs in flight, and slabs per activation chunk */
+    static constexpr int MT_STEP = 4 / PF;                      /* row sub-tiles come in ones, or in twos: then two slabs of them are one transfer of every wave */
+    static constexpr int NW = 8, NT = 2, THREADS = NW * 64;
+    static constexpr int MTM = TM / 16;
+    static constexpr int LOADS = MODE == MODE_W4A8 ? 1 : 2;     /* 16-byte loads per lane, sub-tile and slab */
+    static constexpr int WRB = MODE == MODE_W4A8 ? 64 : 128;    /* bytes of a weight row per slab */
+    static constexpr int A_BYTES = PF * TM * BKB;               /* one chunk: [slab][row][128 bytes, swizzled] */
+    static constexpr int SA_FLOATS = MODE == MODE_FP8 ? PF * 64 : 0;      /* one chunk's block scales, [slab][64 rows] */
+    static constexpr int GS_BYTES = MODE == MODE_W4A8 ? PF * BN * 2 : 0;  /* one chunk's fp16 group scales, [slab][channel] */
+    static constexpr int ES_FLOATS = MODE == MODE_W8A8 ? 256 + (TM + 63) / 64 * 64 : (MODE == MODE_FP8 ? 2 * 256 : 0);
+    static constexpr int LDS_BYTES = 2 * (A_BYTES + SA_FLOATS * 4 + GS_BYTES) + ES_FLOATS * 4 + NW * TM * 4;
+    static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
+};
+
+/*
+ * A weight load whose wait is counted by hand. The compiler counts its own loads exactly, but not the LDS-DMA transfers
+ * issued from inline asm, so its waits reach that many loads too far: half of what an int4 wave has in flight. The value
+ * may only be touched after a wait_w() that names it (tests/test_kernel_asm_checks.py reads the generated code for that);
+ * `s_nop 4`: a scalar base fresh from a vector instruction (see dma16_sv).
+ */
+template <bool STREAM>
+__device__ __forceinline__ void load16_sv(u32x4 &v, uint32_t lane_off, const uint8_t *uniform_base)
+{
+    if constexpr (STREAM) asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %1, %2 nt" : "=v"(v) : "v"(lane_off), "s"(uniform_base));
+    else asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %1, %2" : "=v"(v) : "v"(lane_off), "s"(uniform_base));
+}
+template <int N> __device__ __forceinline__ void wait_w(u32x4 (&w)[2][1])
+{
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(w[0][0]), "+v"(w[1][0]) : "n"(N));
+}
+template <int N> __device__ __forceinline__ void wait_w(u32x4 (&w)[2][2])
+{
+    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]) : "n"(N));
+}
+
+template <int MODE, bool GMM1, int OUT_DT, int TM>
+__global__ void __launch_bounds__(512, 4)
+grouped_gemm_stream_kernel(GemmParams p)
+{
+    using S = StreamShape<MODE, TM>;
+    constexpr int PF = S::PF, NT = S::NT, MTM = S::MTM, LOADS = S::LOADS, NW = S::NW, WRB = S::WRB;
+    constexpr int W_BLOCK_BYTES = 128 * WRB;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    float *lds_sa = reinterpret_cast<float *>(smem + 2 * S::A_BYTES);
+    uint16_t *lds_gs = reinterpret_cast<uint16_t *>(lds_sa + 2 * S::SA_FLOATS);
+    float *lds_es = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(lds_gs) + 2 * S::GS_BYTES);
+    float *lds_rowmax = lds_es + S::ES_FLOATS;
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_tiles = GMM1 ? (p.N / 2) / 128 : p.N / BN;
+    const int K = p.K, KB = K / 128, I = p.N / 2, E = p.experts;
+
+    /*
+     * This workgroup's tile. A column is one expert with rows and 256 of its channels: the weights one row tile streams. The
+     * columns are dealt to the XCDs in turn, so every XCD streams the same bytes whatever the routing (a contiguous run of
+     * tiles each left the XCDs of the popular experts, whose row tiles share weights in the L2, idle early); the row tiles
+     * of a column follow each other on its XCD. Every wave works the tile out for itself, without a barrier.
+     */
+    auto rows_of = [&](int base, int &lo, int &hi) {
+        lo = hi = 0;
+        if (base + lane < E) { lo = p.row_off[base + lane]; hi = p.row_off[base + lane + 1]; }
+    };
+    int lo[2], hi[2];                                              /* experts 0 .. 127, one per lane each: one round trip for all of them */
+    rows_of(0, lo[0], hi[0]);
+    rows_of(64, lo[1], hi[1]);
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    auto columns_before = [&](int y) { return (y - xcd + 7) >> 3; };      /* of this XCD, among columns 0 .. y - 1 */
+    int expert = -1, n_tile = 0, m_tile = 0, mt_e = 1, first_row = 0, end_row = 0;
+    for (int base = 0, tiles = 0, used = 0; base < E; base += 64) {
+        int l = lo[0], h = hi[0];
+        if (base == 64) { l = lo[1]; h = hi[1]; }
+        else if (base > 64) rows_of(base, l, h);
+        const int m = (h - l + TM - 1) / TM;
+        const uint64_t busy = __ballot(m > 0);
+        const int c0 = (used + __builtin_amdgcn_mbcnt_hi((uint32_t)(busy >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)busy, 0))) * n_tiles;
+        const int mine = (columns_before(c0 + n_tiles) - columns_before(c0)) * m;
+        int incl = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += o;
+        }
+        const uint64_t past = __ballot(tiles + incl > slot);
+        if (past) {
+            const int src = __ffsll((long long)past) - 1;
+            expert = base + src;
+            mt_e = __builtin_amdgcn_readlane(m, src);
+            first_row = __builtin_amdgcn_readlane(l, src);
+            end_row = __builtin_amdgcn_readlane(h, src);
+            const int at = slot - tiles - __builtin_amdgcn_readlane(incl - mine, src), col = at / mt_e;
+            m_tile = at - col * mt_e;
+            const int first_col = __builtin_amdgcn_readlane(c0, src);
+            n_tile = (columns_before(first_col) + col) * 8 + xcd - first_col;
+            break;
+        }
+        tiles += __builtin_amdgcn_readlane(incl, 63);
+        used += __popcll(busy);
+    }
+    if (expert < 0) return;
+    const int height = ((end_row - first_row + mt_e - 1) / mt_e + 15) & ~15;      /* even tiles, as in the other kernel */
+    const int row_begin = first_row + m_tile * height;
+    const int row_end = row_begin + height < end_row ? row_begin + height : end_row;
+    const int last_rel = row_end - 1 - row_begin;
+
+    /* the wave's two 16-channel sub-tiles: block rows r0, r0 + 16 .. of one 128-channel block, or the same rows of a gate and an up block */
+    const uint8_t *wb = expert_base<uint8_t>(p.w, p.w_is_list, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
+    const int col0 = GMM1 ? n_tile : n_tile * 2, col1 = GMM1 ? I / 128 + n_tile : n_tile * 2 + 1;
+    const uint8_t *w_src[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int r = GMM1 ? wave * 16 : (wave & 3) * 32 + nt * 16;
+        const int col = GMM1 ? (nt == 0 ? col0 : col1) : (wave < 4 ? col0 : col1);
+        w_src[nt] = uniform_ptr(wb + (int64_t)col * KB * W_BLOCK_BYTES + r * WRB);
+    }
+    const int frag_row = lane & 15;
+    const int key = (lane & 7) ^ ((lane >> 3) & 1), g2 = (lane >> 4) * 2;
+    const int off_lo = frag_row * BKB + ((g2 ^ key) * 16), off_hi = frag_row * BKB + (((g2 + 1) ^ key) * 16);
+    /*
+     * 8-bit weights: a load takes eight whole rows (1 KiB of consecutive bytes), lane (g, i) chunk 2g + i/8 of row i%8, and
+     * half_rows() trades between the two loads of a sub-tile what the MFMA wants elsewhere. Half of each of 16 rows per
+     * load, as the MFMA has them, asks for every line twice (W8A8, 32 experts of 7168 x 4096, one token: GMM1 80 -> 104 us).
+     */
+    const int w8_row = lane & 7, w8_chunk = g2 + ((lane >> 3) & 1);
+    const int w8_off[2] = {w8_row * BKB + ((w8_chunk ^ w8_row) * 16), (8 + w8_row) * BKB + ((w8_chunk ^ w8_row ^ 1) * 16)};
+    const int w4_off = frag_row * 64 + (((lane >> 4) ^ ((frag_row >> 2) & 3)) * 16);
+
+    typedef u32x4 Slabs[PF][NT][LOADS];
+    auto load_w = [&](auto stream_tag, Slabs &wr, int s, int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int h = 0; h < LOADS; ++h) {
+                load16_sv<decltype(stream_tag)::value>(wr[s][nt][h], LOADS == 1 ? w4_off : w8_off[h], w_src[nt] + (int64_t)kb * W_BLOCK_BYTES);
+            }
+    };
+
+    /*
+     * The activations (and what scales them) of slabs kb0 .. kb0 + 3, to buffer b: MT + (scales ? 1 : 0) operations of every
+     * wave. Rows past the tile's end repeat its last one.
+     */
+    const uint32_t lds_a0 = lds_addr(smem);
+    auto issue_chunk = [&](auto mt_tag, int kb0, int b) __attribute__((always_inline)) {
+        constexpr int MT = decltype(mt_tag)::value;
+        int lane_x = lane;
+        asm volatile("" : "+v"(lane_x));           /* the lane offsets are worked out afresh: there is no register to keep them in */
+        const int r = lane_x >> 3;
+        const int s = wave & (PF - 1);
+#pragma unroll
+        for (int j = 0; j < MT / S::MT_STEP; ++j) {                /* slab s of row block wave / PF + j * (8 / PF) */
+            const int rb = wave / PF + j * (NW / PF);
+            int rel = rb * 8 + r;
+            const uint32_t chunk16 = ((lane_x & 7) ^ (r ^ (rb & 1))) * 16;
+            if (rel > last_rel) rel = last_rel;
+            dma16_sv(p.a + (int64_t)row_begin * K + (int64_t)(kb0 + s) * BKB, (uint32_t)rel * (uint32_t)K + chunk16,
+                     lds_a0 + b * S::A_BYTES + s * (TM * BKB) + rb * 1024);
+        }
+        static_assert(MODE != MODE_FP8 || TM <= 64, "one lane per row");
+        if (MODE == MODE_FP8) {                                    /* waves s and s + 4 bring the same */
+            const int rel = lane_x > last_rel ? last_rel : lane_x;
+            dma4_sv(p.a_scale + (int64_t)row_begin * KB + kb0 + s, (uint32_t)rel * (uint32_t)KB * 4u,
+                    lds_addr(lds_sa) + (b * S::SA_FLOATS + s * 64) * 4);
+        }
+        if (MODE == MODE_W4A8) {
+            const uint16_t *gs = expert_base<uint16_t>(p.wscale, p.w_is_list, expert, (int64_t)KB * p.N);
+            const int sg = (wave >> 1) & (PF - 1);
+            gs += (int64_t)(kb0 + sg) * p.N + ((wave & 1) ? col1 : col0) * 128;
+            dma4_sv(reinterpret_cast<const float *>(gs), lane_x * 4u, lds_addr(lds_gs) + b * S::GS_BYTES + sg * (BN * 2) + (wave & 1) * 256);
+        }
+    };
+
+    /* what the epilogue (W8A8) or the K loop (fp8) needs of the tile's scales; older than everything else, so there first */
+    if constexpr (MODE == MODE_W8A8) {
+        const uint32_t dst0 = lds_addr(lds_es);
+        if (wave < (TM + 63) / 64) {
+            const int rel = wave * 64 + lane > last_rel ? last_rel : wave * 64 + lane;
+            dma4_sv(p.a_scale + row_begin, (uint32_t)rel * 4u, dst0 + 1024 + wave * 256);
+        }
+        if (wave >= 4) {
+            const int w4 = wave - 4;
+            if (GMM1 || !p.wscale_is_bf16) {
+                const float *wsb = expert_base<float>(p.wscale, p.w_is_list, expert, p.N);
+                const float *src = !GMM1 ? wsb + n_tile * BN + w4 * 64 : (w4 < 2 ? wsb + n_tile * 128 + w4 * 64 : wsb + I + n_tile * 128 + (w4 - 2) * 64);
+                dma4_sv(src, lane * 4u, dst0 + w4 * 256);
+            } else if (w4 < 2) {
+                const uint16_t *wsb = expert_base<uint16_t>(p.wscale, p.w_is_list, expert, p.N);
+                dma4_sv(reinterpret_cast<const float *>(wsb + n_tile * BN + w4 * 128), lane * 4u, dst0 + w4 * 256);
+            }
+        }
+    } else if constexpr (MODE == MODE_FP8) {
+        const int sw_stride = p.N / 128;
+        const float *base = expert_base<float>(p.wscale, p.w_is_list, expert, (int64_t)KB * sw_stride);
+        for (int b = (wave & 3) * 64; b < KB; b += 256) {
+            if (b + lane < KB)
+                dma4_sv(base + (wave < 4 ? col0 : col1), (uint32_t)(b + lane) * (uint32_t)sw_stride * 4u,
+                        lds_addr(lds_es) + ((wave < 4 ? 0 : 256) + b) * 4);
+        }
+    }
+
+    f32x4 accf[MTM][NT];
+    i32x4 acci[MTM][NT];
+#pragma unroll
+    for (int mt = 0; mt < MTM; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            accf[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            acci[mt][nt] = i32x4{0, 0, 0, 0};
+        }
+
+    i32x4 magic = {0x4b400000, 0x4b400000, 0x4b400000, 0x4b400000};      /* W4A8: see multiply() */
+    if constexpr (MODE == MODE_W4A8) asm volatile("" : "+v"(magic));
+    /* one slab over the first MT row sub-tiles: fragments of slot s, activations of slab s of buffer b */
+    auto multiply = [&](auto mt_tag, const Slabs &wr, int s, int b, int kb) __attribute__((always_inline)) {
+        constexpr int MT = decltype(mt_tag)::value;
+        const uint8_t *ab = smem + b * S::A_BYTES + s * (TM * BKB);
+        auto load_a = [&](int mt) -> i32x8 {
+            const u32x4 lo = *reinterpret_cast<const u32x4 *>(ab + mt * (16 * BKB) + off_lo);
+            const u32x4 hi = *reinterpret_cast<const u32x4 *>(ab + mt * (16 * BKB) + off_hi);
+            return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+        };
+        /* fragment of channel sub-tile nt: rows 0-7 of the first load beside rows 8-15 of the second, chunk 2g before chunk 2g + 1 */
+        auto half_rows = [&](int nt) -> i32x8 {
+            const u32x4 r0 = wr[s][nt][0], r8 = wr[s][nt][LOADS - 1];
+            i32x8 w;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {      /* row_ror:8, into lanes 8-15 and 0-7 of each 16 */
+                w[i] = __builtin_amdgcn_update_dpp((int)r0[i], (int)r8[i], 0x128, 0xf, 0xc, false);
+                w[4 + i] = __builtin_amdgcn_update_dpp((int)r8[i], (int)r0[i], 0x128, 0xf, 0x3, false);
+            }
+            return w;
+        };
+        if constexpr (MODE == MODE_W8A8) {
+            i32x8 w[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) w[nt] = half_rows(nt);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const i32x8 a = load_a(mt);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    acci[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{w[nt][0], w[nt][1], w[nt][2], w[nt][3]},
+                                                                         i32x4{a[0], a[1], a[2], a[3]}, acci[mt][nt], 0, 0, 0);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    acci[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{w[nt][4], w[nt][5], w[nt][6], w[nt][7]},
+                                                                         i32x4{a[4], a[5], a[6], a[7]}, acci[mt][nt], 0, 0, 0);
+            }
+        } else if constexpr (MODE == MODE_FP8) {
+            const float sw0 = lds_es[kb], sw1 = lds_es[256 + kb];
+            i32x8 w[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                w[nt] = half_rows(nt);
+                asm volatile("" : "+v"(w[nt]));
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const i32x8 a = load_a(mt);
+                const float sa = lds_sa[b * S::SA_FLOATS + s * 64 + mt * 16 + frag_row];
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    const f32x4 part = mfma_fp8_16x16x128(w[nt], a);
+                    const float sc = sa * ((GMM1 ? nt == 1 : wave >= 4) ? sw1 : sw0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(part[i], sc, accf[mt][nt][i]);
+                }
+                asm volatile("" ::: "memory");
+            }
+        } else {
+            /* the arithmetic of the other kernel's W4A8 loop (see there): sums from the bits of 1.5 * 2^23, weights times 16 */
+            constexpr float MAGIC = 12582912.0f;
+            auto lo4 = [](uint32_t v) -> int { return (int)((v << 4) & 0xf0f0f0f0u); };
+            auto hi4 = [](uint32_t v) -> int { return (int)(v & 0xf0f0f0f0u); };
+            i32x4 w0[NT], w1[NT];
+            float gs[NT][4];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const u32x4 pk = wr[s][nt][0];
+                w0[nt] = i32x4{lo4(pk[0]), hi4(pk[0]), lo4(pk[1]), hi4(pk[1])};
+                w1[nt] = i32x4{lo4(pk[2]), hi4(pk[2]), lo4(pk[3]), hi4(pk[3])};
+                const int r = GMM1 ? nt * 128 + wave * 16 : wave * 32 + nt * 16;
+                const u32x2 g = *reinterpret_cast<const u32x2 *>(lds_gs + (b * PF + s) * BN + (lane >> 4) * 8 + zb_block_row_channel(r));
+                gs[nt][0] = zb_fp16_to_f32(g[0] & 0xffffu);
+                gs[nt][1] = zb_fp16_to_f32(g[0] >> 16);
+                gs[nt][2] = zb_fp16_to_f32(g[1] & 0xffffu);
+                gs[nt][3] = zb_fp16_to_f32(g[1] >> 16);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) asm("" : "+v"(gs[nt][i]));
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const i32x8 a = load_a(mt);
+                i32x4 part[NT];
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    part[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0[nt], i32x4{a[0], a[1], a[2], a[3]}, magic, 0, 0, 0);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    part[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1[nt], i32x4{a[4], a[5], a[6], a[7]}, part[nt], 0, 0, 0);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(__int_as_float(part[nt][i]) - MAGIC, gs[nt][i], accf[mt][nt][i]);
+            }
+        }
+    };
+
+    const int mt_act = (row_end - row_begin + 15) >> 4;
+    auto k_loop = [&](auto mt_tag, auto stream_tag) __attribute__((always_inline)) {
+        constexpr int MT = decltype(mt_tag)::value;
+        constexpr int L = NT * LOADS;                                   /* loads per slab */
+        constexpr int D = MT / S::MT_STEP + (MODE == MODE_W8A8 ? 0 : 1);      /* transfers per chunk */
+        Slabs wr;
+        issue_chunk(mt_tag, 0, 0);
+#pragma unroll
+        for (int s = 0; s < PF; ++s) load_w(stream_tag, wr, s, s);
+        /* issued since chunk c's transfers: the fragments of its slabs, L each; since slab s's fragments: three more slabs, and D */
+        auto begin_chunk = [&]() __attribute__((always_inline)) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(PF * L) : "memory");
+        };
+        int b = 0, kb0 = 0;
+        for (; kb0 + PF < KB; kb0 += PF) {
+            begin_chunk();               /* chunk kb0's activations have landed for everybody, and nobody reads the other buffer any more */
+            issue_chunk(mt_tag, kb0 + PF, b ^ 1);
+#pragma unroll
+            for (int s = 0; s < PF; ++s) {
+                wait_w<(PF - 1) * L + D>(wr[s]);
+                multiply(mt_tag, wr, s, b, kb0 + s);
+                __builtin_amdgcn_sched_barrier(0);
+                load_w(stream_tag, wr, s, kb0 + PF + s);
+            }
+            b ^= 1;
+        }
+        begin_chunk();
+        if constexpr (PF == 4) {
+            wait_w<3 * L>(wr[0]);
+            multiply(mt_tag, wr, 0, b, kb0);
+            wait_w<2 * L>(wr[1]);
+            multiply(mt_tag, wr, 1, b, kb0 + 1);
+        }
+        wait_w<L>(wr[PF - 2]);
+        multiply(mt_tag, wr, PF - 2, b, kb0 + PF - 2);
+        wait_w<0>(wr[PF - 1]);
+        multiply(mt_tag, wr, PF - 1, b, kb0 + PF - 1);
+    };
+    auto k_loop_mt = [&](auto stream_tag) __attribute__((always_inline)) {
+        constexpr int ST = S::MT_STEP;
+        if (MTM >= 4 * ST && mt_act > 3 * ST) k_loop(std::integral_constant<int, MTM >= 4 * ST ? 4 * ST : MTM>{}, stream_tag);
+        else if (MTM >= 3 * ST && mt_act > 2 * ST) k_loop(std::integral_constant<int, MTM >= 3 * ST ? 3 * ST : MTM>{}, stream_tag);
+        else if (MTM >= 2 * ST && mt_act > ST) k_loop(std::integral_constant<int, MTM >= 2 * ST ? 2 * ST : MTM>{}, stream_tag);
+        else k_loop(std::integral_constant<int, ST>{}, stream_tag);
+    };
+    /* weights that the other row tiles of the column want too stay in the L2 for them; the others leave no trace in it */
+    if (mt_e == 1) k_loop_mt(std::true_type{});
+    else k_loop_mt(std::false_type{});
+    if constexpr (MODE == MODE_W4A8) {
+#pragma unroll
+        for (int mt = 0; mt < MTM; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) accf[mt][nt][i] *= 0.0625f;
+    }
+    TileCoord tc;
+    tc.expert = expert;
+    tc.m_tile = 0;
+    tc.n_tile = n_tile;
+    int lane_e = lane;
+    asm volatile("" : "+v"(lane_e));               /* as in the other kernel: nothing of the epilogue's stays live across the K loop */
+    epilogue<MODE, GMM1, OUT_DT, 1, MTM, NT>(p, tc, accf, acci, row_begin, row_end, 0, wave, lane_e, lds_rowmax, TM, lds_es);
+}
+
+} // namespace
+
+#endif /* ZBAL_GEMM_STREAM_H_ */

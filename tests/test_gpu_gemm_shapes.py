@@ -25,11 +25,17 @@ def buf():
 # rows per expert on average: the classes of W4A8 end at 48, 100, 160, 224 and 640, those of the 8-bit modes at 8, 84-100
 EDGES = {"few": [0, 1, 15, 16, 17, 2, 8, 5, 0, 3], "64": [1, 0, 16, 31, 33, 63, 64, 65, 80, 127],
          "100": [0, 96, 97, 127, 128, 129, 112, 64, 1, 200], "160": [191, 192, 193, 176, 177, 0, 30, 160, 161, 256],
+         "47": [47, 48, 49, 33, 32, 31, 0, 17, 64, 1], "53": [63, 64, 65, 49, 48, 128, 50, 0, 20, 33],
+         "sparse": [0] * 63 + [5, 70] + [0] * 66 + [16, 1] + [0] * 60 + [33, 2], "1000": [1000, 769, 96, 97, 1151, 1153, 767, 800, 0, 700],
          "224": [128, 129, 256, 257, 192, 255, 0, 144, 300, 250], "640": [384, 385, 192, 577, 1, 0, 600, 383, 500, 191]}
 
 
+# whole chunks of the streaming kernel's slabs, channel tiles in eighths and not
+STREAM_SHAPES = [(512, 512), (1024, 2304), (1536, 768)]
+
+
 @pytest.mark.parametrize("edges", sorted(EDGES))
-@pytest.mark.parametrize("K,N", [(256, 512), (384, 256), (640, 1280)])
+@pytest.mark.parametrize("K,N", [(256, 512), (384, 256), (640, 1280)] + STREAM_SHAPES)
 def test_w4a8_shapes_bit_exact(buf, edges, K, N):
     counts = np.array(EDGES[edges], dtype=np.int64)
     E, rows = len(counts), int(counts.sum())
@@ -47,8 +53,8 @@ def test_w4a8_shapes_bit_exact(buf, edges, K, N):
     assert np.array_equal(host(s2).view(np.uint32), r_s2.view(np.uint32)) and np.array_equal(host(q2), r_q2)
 
 
-@pytest.mark.parametrize("edges", ["few", "64", "100"])
-@pytest.mark.parametrize("K,N", [(256, 512), (640, 1280)])
+@pytest.mark.parametrize("edges", ["few", "47", "53", "64", "100", "sparse"])
+@pytest.mark.parametrize("K,N", [(256, 512), (640, 1280)] + STREAM_SHAPES)
 def test_8_bit_shapes(buf, edges, K, N):
     counts = np.array(EDGES[edges], dtype=np.int64)
     E, rows = len(counts), int(counts.sum())

@@ -85,3 +85,56 @@ def test_gemm_kernels_spill_no_vector_registers(gemm_asm):
     counts = [int(m.group(1)) for m in (re.search(r"\.vgpr_spill_count:\s+(\d+)", l) for l in gemm_asm) if m]
     assert len(counts) >= 20, counts
     assert all(c == 0 for c in counts), counts
+
+
+def _vector_registers(token):
+    m = re.match(r"v\[(\d+):(\d+)\]$", token)
+    if m:
+        return set(range(int(m.group(1)), int(m.group(2)) + 1))
+    m = re.match(r"v(\d+)$", token)
+    return {int(m.group(1))} if m else set()
+
+
+def _touched_in_flight(lines):
+    """(line number, instruction) of everything in a streaming kernel that names a register whose load has not been waited
+    for, and the number of such loads. The text is followed straight on; what was in flight is forgotten where it stops."""
+    found, loads, inside, flight = [], 0, False, []
+    for i, line in enumerate(lines):
+        t = line.split(";")[0].strip()
+        m = re.match(r"(_Z\w+):$", t)
+        if m:
+            inside, flight = "grouped_gemm_stream_kernel" in m.group(1), []
+        if not inside or not _is_instruction(t):
+            continue
+        op = t.split()[0]
+        if op == "s_waitcnt":
+            m = re.search(r"vmcnt\((\d+)\)", t)
+            if m:
+                flight = flight[-int(m.group(1)):] if int(m.group(1)) else []
+            continue
+        if op in ("s_branch", "s_endpgm"):
+            flight = []
+            continue
+        tokens = [x.split()[0] for x in t[len(op):].split(",") if x.split()]
+        used = set().union(*[_vector_registers(x) for x in tokens]) if tokens else set()
+        if any(f & used for f in flight):
+            found.append((i + 1, t))
+        if re.match(r"(global|scratch|flat|buffer)_", op):
+            is_load = op.startswith("global_load") and "lds" not in op
+            flight.append(_vector_registers(tokens[0]) if is_load else set())
+            loads += is_load
+    return found, loads
+
+
+def test_scanner_sees_a_register_in_flight():
+    lines = ["_ZN1_26grouped_gemm_stream_kernelE:", "global_load_dwordx4 v[4:7], v1, s[8:9] nt", "global_load_lds_dwordx4 v25, s[8:9]",
+             "s_waitcnt vmcnt(1)", "v_mov_b32_e32 v2, v5", "global_load_dwordx4 v[8:11], v1, s[8:9]", "s_waitcnt vmcnt(1)",
+             "v_mfma_i32_16x16x64_i8 v[0:3], v[8:11], v[4:7], v[0:3]"]
+    found, loads = _touched_in_flight(lines)
+    assert loads == 2 and [n for n, _ in found] == [8]
+
+
+def test_streamed_fragments_are_waited_for(gemm_asm):
+    found, loads = _touched_in_flight(gemm_asm)
+    assert loads > 300, "the scan did not find the streaming kernels' loads (%d)" % loads
+    assert not found, "%d instructions touch a register in flight, e.g. %r" % (len(found), found[:3])
