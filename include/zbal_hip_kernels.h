@@ -332,6 +332,34 @@ ZBALHIP_API int32_t zbalhip_gmm2_dequant(const void *a, const float *a_scale, co
                              int64_t k, int64_t n, int32_t mode, int32_t out_dtype, void *y, void *stream);
 
 /*
+ * The stages of the fused operator with a shared expert riding along (same K and N as the routed experts, same scale
+ * types): its tokens are one expert's rows more, so its weights stream in the same launches. Its rows lie behind the
+ * max_rows = tokens * topk rows that the routed experts can have, `rows` = tokens of them in token order; q1, xs, q2,
+ * scale2 and sgl_ws hold max_rows + rows rows, and row_off one entry more: row_off[experts + 1] = end of its rows, which
+ * the permute stage writes (x_active_mask cuts them short, as it does the routed rows). Second GEMM: row i of the shared
+ * expert goes to row i of `out`. smooth of the permute stage: [H] (int8 only, and only if the routed experts have one).
+ */
+typedef struct {
+    const void *weight, *scale;
+    int64_t rows;
+    void *out;
+} zbalhip_shared_expert_t;
+ZBALHIP_API int32_t zbalhip_fused_permute_quant_shared(const void *x, int32_t x_dtype, const int32_t *expert_ids, const float *smooth,
+                                    const uint8_t *active_mask,
+                                    int64_t tokens, int64_t hidden, int64_t topk, int64_t experts, int32_t mode,
+                                    void *q1, float *xs, int32_t *expand_idx, int64_t *counts, int32_t *row_off,
+                                    uint32_t *clear_words, int64_t clear_count, int32_t *scratch, int32_t scratch_blocks,
+                                    const float *shared_smooth, void *stream);
+ZBALHIP_API int32_t zbalhip_gmm1_swiglu_quant_shared(const void *a, const float *a_scale, const void *w1, const void *w1scale,
+                                  const int32_t *row_off, int64_t experts, int64_t max_rows, int64_t k, int64_t n1,
+                                  int32_t mode, void *q2, float *scale2, float *sgl_ws,
+                                  const zbalhip_shared_expert_t *shared, void *stream);
+ZBALHIP_API int32_t zbalhip_gmm2_dequant_shared(const void *a, const float *a_scale, const void *w2, const void *wscale,
+                             int32_t wscale_dtype, const int32_t *row_off, int64_t experts, int64_t max_rows,
+                             int64_t k, int64_t n, int32_t mode, int32_t out_dtype, void *y,
+                             const zbalhip_shared_expert_t *shared, void *stream);
+
+/*
  * One-time set-up of every grouped-GEMM kernel on the current GPU (each raises its dynamic-LDS limit before its
  * first launch, which cannot be recorded into a graph). No counterpart in the reference. Optional: a launch whose
  * kernel is still unprepared does it itself, and refuses with an error if its stream is being captured. The host

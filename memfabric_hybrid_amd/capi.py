@@ -162,6 +162,10 @@ SIGNATURES = {
                                            _vp, _i64, _vp, _i32, _vp]),
     "zbalhip_dispatch_low_latency_ranks": (_i32, [_vp, _i32, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _vp, _vp, _i32, _i32, _i64,
                                                   _vp, _vp, _vp, _vp, _vp]),
+    "zbalhip_fused_permute_quant_shared": (_i32, [_vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp,
+                                                  _vp, _i64, _vp, _i32, _vp, _vp]),
+    "zbalhip_gmm1_swiglu_quant_shared": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp]),
+    "zbalhip_gmm2_dequant_shared": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _vp, _vp, _vp]),
     "zbalhip_gmm1_swiglu_quant": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp]),
     "zbalhip_gmm2_dequant": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _vp, _vp]),
     "zbalhip_gemm_prepare": (_i32, []),

@@ -728,7 +728,7 @@ public:
             activeMask = (const uint8_t *)xActiveMask->data;
         }
         FusedWorkspace ws;
-        ZBAL_VALIDATE_RETURN(PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, &ws), op << " failed as the shapes are invalid",
+        ZBAL_VALIDATE_RETURN(PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, false, &ws), op << " failed as the shapes are invalid",
                              Z_INVALID_PARAM);
         ZBAL_VALIDATE_RETURN(workspace->data != nullptr && (reinterpret_cast<uintptr_t>(workspace->data) & 255u) == 0,
                              op << " failed as the workspace is null or not 256-byte aligned", Z_INVALID_PARAM);
@@ -737,8 +737,20 @@ public:
             ZBAL_LOG_AND_SET_LAST_ERROR(op << " failed as the workspace holds " << wsBytes << " bytes, needs " << ws.total);
             return Z_ERROR;
         }
+        /*
+         * A shared expert of the routed experts' width and scale types runs in their launches, as one expert more: alone it
+         * has a tile per 256 channels, 16 or 28 of them on 256 CUs (7168 x 4096 / 2048 x 7168, 32 experts: 1 token W8A8 141 ->
+         * 85 us, 37 tokens fp8 307 -> 279, 300 tokens 494 -> 380, 2000 tokens equal). With many rows it fills the GPU by itself, and
+         * its rows next to experts of a quarter as many are no gain (4096 tokens fp8 1945 -> 2054): then, and where the workspace
+         * holds no rows for it, it takes turns with them.
+         */
+        FusedWorkspace along;
+        const bool ride = shared && T > 0 && SN1 == N1 && shareWscale2Dt == wscale2Dt && (smooth != nullptr) == (shareSmooth != nullptr) &&
+                          E < 1024 && T * K <= 640 * E && T * (K + 1) <= 0x7fffffff &&
+                          PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, true, &along) && wsBytes >= along.total;
+        if (ride) ws = along;
         uint8_t *base = (uint8_t *)workspace->data;
-        const int64_t rows = T * K;
+        const int64_t rows = T * K, allRows = rows + (ride ? T : 0);
         void *q1 = base + ws.q1;
         float *xs = (float *)(base + ws.xs);
         int32_t *expandIdx = (int32_t *)(base + ws.expand_idx);
@@ -760,7 +772,10 @@ public:
                                                             stream));
         }
         int32_t rc = 0;
-        if (shared) {
+        const zbalhip_shared_expert_t along1 = {ride ? shareGmm1Weight->data : nullptr, ride ? shareGmm1Scale->data : nullptr, T, nullptr};
+        const zbalhip_shared_expert_t along2 = {ride ? shareGmm2Weight->data : nullptr, ride ? shareGmm2Scale->data : nullptr, T,
+                                                ride ? shareOutput->data : nullptr};
+        if (shared && !ride) {
             /*
              * The shared expert is the same pipeline with one expert that every token picks once: the rows stay in
              * token order, so the second GEMM writes shareOutput directly. It runs first and borrows the routed
@@ -783,16 +798,22 @@ public:
                                       SI, H, mode, x->dataType, shareOutput->data, stream);
             if (rc != 0) return Launched(op, rc);
         }
-        rc = zbalhip_fused_permute_quant(x->data, x->dataType, (const int32_t *)expertIds->data, smooth, activeMask, T, H, K, E,
-                                         qmode | IdsFlag(expertIds), q1, xs, expandIdx, (int64_t *)expertTokenNums->data, rowOff,
-                                         sgl ? (uint32_t *)(sgl + rows * I) : nullptr, sgl ? rows : 0, layoutScratch,
-                                         ZBALHIP_LAYOUT_MAX_BLOCKS, stream);
+        uint32_t *rowMax = sgl ? (uint32_t *)(sgl + allRows * I) : nullptr;
+        const int32_t *ids = (const int32_t *)expertIds->data;
+        const int32_t permuteMode = qmode | IdsFlag(expertIds);
+        int64_t *counts = (int64_t *)expertTokenNums->data;
+        rc = ride ? zbalhip_fused_permute_quant_shared(x->data, x->dataType, ids, smooth, activeMask, T, H, K, E, permuteMode, q1, xs,
+                                                       expandIdx, counts, rowOff, rowMax, sgl ? allRows : 0, layoutScratch,
+                                                       ZBALHIP_LAYOUT_MAX_BLOCKS, shareSmooth, stream)
+                  : zbalhip_fused_permute_quant(x->data, x->dataType, ids, smooth, activeMask, T, H, K, E, permuteMode, q1, xs,
+                                                expandIdx, counts, rowOff, rowMax, sgl ? allRows : 0, layoutScratch,
+                                                ZBALHIP_LAYOUT_MAX_BLOCKS, stream);
         if (rc != 0) return Launched(op, rc);
-        rc = zbalhip_gmm1_swiglu_quant(q1, xs, gmm1Weight->data, gmm1Scale->data, rowOff, E, rows, H, N1,
-                                       gemmMode | clearedFlag, q2, scale2, sgl, stream);
+        rc = zbalhip_gmm1_swiglu_quant_shared(q1, xs, gmm1Weight->data, gmm1Scale->data, rowOff, E, rows, H, N1,
+                                              gemmMode | clearedFlag, q2, scale2, sgl, ride ? &along1 : nullptr, stream);
         if (rc != 0) return Launched(op, rc);
-        rc = zbalhip_gmm2_dequant(q2, scale2, gmm2Weight->data, gmm2Scale->data, wscale2Dt, rowOff, E, rows, I, H, gemmMode,
-                                  x->dataType, y, stream);
+        rc = zbalhip_gmm2_dequant_shared(q2, scale2, gmm2Weight->data, gmm2Scale->data, wscale2Dt, rowOff, E, rows, I, H, gemmMode,
+                                         x->dataType, y, ride ? &along2 : nullptr, stream);
         if (rc != 0) return Launched(op, rc);
         const void *ySrc[1] = {y};
         return Launched(op, zbalhip_combine(ySrc, 1, 0, rows, x->dataType, rowOff, IdsFlag(expertIds), (const float *)expertScales->data,
@@ -840,7 +861,7 @@ CommunicatorPtr MakeGpuCommunicator(const GroupInfo &info) { return std::make_sh
 
 
 bool PlanFusedWorkspace(int64_t tokens, int64_t hidden, int64_t topk, int64_t experts, int64_t n1, int64_t shareN1,
-                        int64_t quantMode, FusedWorkspace *ws)
+                        int64_t quantMode, bool ridesAlong, FusedWorkspace *ws)
 {
     if (tokens < 0 || hidden <= 0 || topk <= 0 || experts <= 0 || n1 <= 0 || shareN1 < 0 || quantMode < 0 || quantMode > 3)
         return false;
@@ -849,19 +870,20 @@ bool PlanFusedWorkspace(int64_t tokens, int64_t hidden, int64_t topk, int64_t ex
     const uint64_t T = (uint64_t)(tokens > 0 ? tokens : 1);
     const uint64_t H = hidden, I = n1 / 2, SI = shareN1 / 2, E = experts;
     const bool fp8 = quantMode == 2;
-    /* the shared expert's pass (T rows, width SI) reuses the regions of the routed pass (rows rows, width I) */
+    const uint64_t all = rows + (ridesAlong ? T : 0);      /* rows of what the GEMMs read and hand on */
+    /* a shared expert's pass of its own (T rows, width SI) reuses the regions of the routed pass (rows rows, width I) */
     auto both = [&](uint64_t routed, uint64_t shared) { return SI > 0 && shared > routed ? shared : routed; };
     uint64_t off = 0;
     auto take = [&](uint64_t bytes) { uint64_t o = off; off = Align256(off + bytes); return o; };
-    ws->q1 = take(rows * H);
-    ws->xs = take(rows * (fp8 ? H / 128 : 1) * 4);
+    ws->q1 = take(all * H);
+    ws->xs = take(all * (fp8 ? H / 128 : 1) * 4);
     ws->expand_idx = take(rows * 4);
     ws->counts = take(E * 8);
-    ws->row_off = take((E + 1) * 4);
+    ws->row_off = take((E + 2) * 4);
     ws->layout_scratch = take((uint64_t)ZBALHIP_LAYOUT_MAX_BLOCKS * E * 4);
-    ws->q2 = take(both(rows * I, T * SI));
-    ws->scale2 = take(both(rows * (fp8 ? (I + 127) / 128 : 1), T * (fp8 ? (SI + 127) / 128 : 1)) * 4);
-    ws->sgl = fp8 ? off : take(both(rows * (I + 1), T * (SI + 1)) * 4);
+    ws->q2 = take(both(all * I, T * SI));
+    ws->scale2 = take(both(all * (fp8 ? (I + 127) / 128 : 1), T * (fp8 ? (SI + 127) / 128 : 1)) * 4);
+    ws->sgl = fp8 ? off : take(both(all * (I + 1), T * (SI + 1)) * 4);
     ws->y = take(both(rows * H * 2, Align256(T * 4) + 256));
     ws->total = off;
     return true;

@@ -240,8 +240,12 @@ struct FusedWorkspace {
     uint64_t q1, xs, expand_idx, counts, row_off, layout_scratch, q2, scale2, sgl, y, total;
 };
 /* shareN1 = output width of the shared expert's first GEMM, 0 without a shared expert */
+/*
+ * ridesAlong: with room for a shared expert's rows behind the routed ones (shareN1 == n1), so that it runs in the routed
+ * experts' launches. Without: it takes turns with them in the same regions.
+ */
 bool PlanFusedWorkspace(int64_t tokens, int64_t hidden, int64_t topk, int64_t experts, int64_t n1, int64_t shareN1,
-                        int64_t quantMode, FusedWorkspace *ws);
+                        int64_t quantMode, bool ridesAlong, FusedWorkspace *ws);
 
 } // namespace zbal
 

@@ -95,13 +95,21 @@ __device__ __forceinline__ int active_tokens(const uint8_t *mask, int tokens, in
     return *s;
 }
 
+/* a shared expert: every active token's row once more, row t at first_row + t (end null: none) */
+struct SharedRows {
+    int64_t first_row;
+    int32_t *end;                 /* first_row + active tokens goes here */
+    const float *smooth;          /* [H], where the routed experts have smooth scales */
+};
+
 /* the layout's outputs, by one workgroup; any of them may be null */
 __device__ __forceinline__ void write_inline_layout(const ExpertIds &idx, int topk, int experts, const InlineLayout &il,
-                                                    int32_t *s_hist, int32_t *s_tmp)
+                                                    const SharedRows &sh, int32_t *s_hist, int32_t *s_tmp)
 {
     const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = tid >> 6;
     for (int e = tid; e < experts; e += nthr) s_hist[e] = 0;
-    const int n = active_tokens(il.active_mask, il.tokens, s_tmp) * topk;
+    const int active = active_tokens(il.active_mask, il.tokens, s_tmp), n = active * topk;
+    if (sh.end && tid == 0) *sh.end = (int32_t)(sh.first_row + active);
     __syncthreads();
     for (int i0 = tid; i0 < n; i0 += 4 * nthr) {
         int ev[4];
@@ -362,7 +370,7 @@ __global__ void __launch_bounds__(kThreads)
 permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                      const int32_t *__restrict__ rank_in_expert, const int32_t *__restrict__ base, int base_inclusive,
                      const float *__restrict__ smooth, int hidden, int topk, int experts, PeerRows pr, InlineLayout il,
-                     RangeTable rt, uint32_t *__restrict__ clear_words, int64_t clear_count)
+                     RangeTable rt, SharedRows sh, uint32_t *__restrict__ clear_words, int64_t clear_count)
 {
     constexpr bool INLINE = LM == LM_INLINE, TABLE = LM == LM_TABLE;
     __shared__ float red[kThreads / 64];
@@ -375,10 +383,14 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < clear_count; i += (int64_t)gridDim.x * blockDim.x)
         clear_words[i] = 0u;
     if (INLINE && blockIdx.x == 0) {
-        write_inline_layout(topk_idx, topk, experts, il, s_off, s_tmp);
+        write_inline_layout(topk_idx, topk, experts, il, sh, s_off, s_tmp);
         return;
     }
     const int t = INLINE ? blockIdx.x - 1 : blockIdx.x;
+    if (!INLINE && sh.end && t == 0) {
+        const int n = active_tokens(il.active_mask, il.tokens, s_tmp);
+        if (threadIdx.x == 0) *sh.end = (int32_t)(sh.first_row + n);
+    }
     /*
      * Where the token's picks go is worked out by one lane per pick, in every wave, while the row is on its way (the
      * picks' index, rank and offset loads depend on each other: done pick after pick inside the store loop they cost
@@ -431,7 +443,9 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
     }
     if constexpr (ROW_MAX || INLINE) __syncthreads();
     if constexpr (INLINE) picks = inline_rows(t, topk, experts, active, given.e, il, pr, s_cnt);
-    /* f(pick's expert, window, row) for every routed pick of the token; wave-uniform */
+    /* rank -2: the layout masked the token out */
+    const bool shares = sh.end && (INLINE ? t < active : __builtin_amdgcn_readlane(given.rank, 0) != -2);
+    /* f(pick's expert, window, row) for every routed pick of the token, and for the shared expert (-1); wave-uniform */
     auto for_each_pick = [&](auto f) __attribute__((always_inline)) {
         for (int k0 = 0; k0 < topk; k0 += 64) {
             if (!INLINE && !TABLE && k0 > 0)
@@ -444,6 +458,7 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                 f(e, window_of(pr, e), (int64_t)row);
             }
         }
+        if (shares) f(-1, 0, sh.first_row + t);
     };
 
     if constexpr (QM == QM_FP8) {
@@ -499,6 +514,7 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
     } else {
         for_each_pick([&](int e, int win, int64_t row) __attribute__((always_inline)) {
             uint8_t *dest = pr.dest[win];
+            const float *sm = e < 0 ? sh.smooth : smooth + (int64_t)e * hidden;
             float sv[SLOTS][16];
             float amax = 0.0f;
 #pragma unroll
@@ -506,7 +522,7 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                 const int seg = s * blockDim.x + threadIdx.x;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const float m = (seg < nseg) ? smooth[(int64_t)e * hidden + seg * 16 + i] : 0.0f;
+                    const float m = (seg < nseg) ? sm[seg * 16 + i] : 0.0f;
                     sv[s][i] = v[s][i] * m;
                     amax = fmaxf(amax, fabsf(sv[s][i]));
                 }
@@ -538,7 +554,7 @@ permute_copy_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
     constexpr bool INLINE = LM == LM_INLINE;
     __shared__ int32_t s_off[INLINE ? kInlineMaxExperts : 1], s_cnt[kThreads / 64][kInlineMaxTopk], s_tmp[8];
     if (INLINE && blockIdx.x == 0) {
-        write_inline_layout(topk_idx, topk, experts, il, s_off, s_tmp);
+        write_inline_layout(topk_idx, topk, experts, il, SharedRows{}, s_off, s_tmp);
         return;
     }
     const int t = INLINE ? blockIdx.x - 1 : blockIdx.x, lane = threadIdx.x & 63;
@@ -592,6 +608,8 @@ struct PermuteExtras {
     uint32_t *clear_words;
     int64_t clear_count;
     const RangeTable *range_table;         /* non-null: ranks within token ranges + the ranges' histograms (large batches) */
+    SharedRows shared;
+    const uint8_t *active_mask;            /* with a shared expert, whatever the layout comes from */
 };
 
 template <int XDT, int QM, bool SMOOTH>
@@ -604,12 +622,16 @@ int32_t launch_quant(const void *x, const ExpertIds &topk_idx, const int32_t *ra
     if (threads > kThreads) threads = kThreads;
     if (ex.range_table) threads = kThreads;       /* the table's scan gives every expert a thread */
     const int slots = (nseg + threads - 1) / threads;
-    const InlineLayout il = ex.inline_layout ? *ex.inline_layout : InlineLayout{};
+    InlineLayout il = ex.inline_layout ? *ex.inline_layout : InlineLayout{};
+    if (!ex.inline_layout) {
+        il.active_mask = ex.active_mask;
+        il.tokens = (int)tokens;
+    }
     const RangeTable rt = ex.range_table ? *ex.range_table : RangeTable{};
 #define ZB_LAUNCH_I(S, LMV)                                                                                       \
     permute_quant_kernel<XDT, QM, S, SMOOTH, LMV><<<(unsigned)(tokens + (LMV == LM_INLINE ? 1 : 0)), threads, 0, st>>>( \
         (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, smooth, (int)hidden, (int)topk,       \
-        (int)experts, pr, il, rt, ex.clear_words, ex.clear_count)
+        (int)experts, pr, il, rt, ex.shared, ex.clear_words, ex.clear_count)
 #define ZB_LAUNCH(S)                                                                                              \
     do {                                                                                                          \
         if (ex.inline_layout) ZB_LAUNCH_I(S, LM_INLINE);                                                          \
@@ -745,7 +767,7 @@ extern "C" int32_t zbalhip_dispatch_low_latency(const void *x, int32_t x_dtype, 
         il.expand_idx = expand_idx;
         il.incl_i32 = ep_recv_counts;
         il.nums_typed = expert_token_nums;
-        const PermuteExtras ex = {&il, nullptr, 0, nullptr};
+        const PermuteExtras ex = {&il, nullptr, 0, nullptr, {}, nullptr};
         return permute_launch(x, x_dtype, ids, expand_idx, ep_recv_counts, 1, nullptr, tokens, hidden, topk, experts, q,
                               single_window(expand_x, dynamic_scales, experts, tokens * topk), st, ex);
     }
@@ -794,12 +816,11 @@ extern "C" int32_t zbalhip_dispatch_low_latency_ranks(const void *x, int32_t x_d
                           experts, q, pr, st);
 }
 
-extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, const int32_t *expert_ids,
-                                               const float *smooth, const uint8_t *active_mask, int64_t tokens,
-                                               int64_t hidden, int64_t topk,
-                                               int64_t experts, int32_t mode, void *q1, float *xs, int32_t *expand_idx,
-                                               int64_t *counts, int32_t *row_off, uint32_t *clear_words,
-                                               int64_t clear_count, int32_t *scratch, int32_t scratch_blocks, void *stream)
+static int32_t fused_permute_quant(const void *x, int32_t x_dtype, const int32_t *expert_ids, const float *smooth,
+                                   const uint8_t *active_mask, int64_t tokens, int64_t hidden, int64_t topk, int64_t experts,
+                                   int32_t mode, void *q1, float *xs, int32_t *expand_idx, int64_t *counts, int32_t *row_off,
+                                   uint32_t *clear_words, int64_t clear_count, int32_t *scratch, int32_t scratch_blocks,
+                                   const SharedRows &sh, void *stream)
 {
     if (!counts || !row_off || clear_count < 0 || (clear_count > 0 && !clear_words)) return ZBALHIP_INVALID;
     if (tokens > 0 && (!x || !expert_ids || !q1 || !xs || !expand_idx)) return ZBALHIP_INVALID;
@@ -818,7 +839,7 @@ extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, c
         il.expand_idx = expand_idx;
         il.row_off = row_off;
         il.counts_i64 = counts;
-        const PermuteExtras ex = {&il, clear_words, clear_count, nullptr};
+        const PermuteExtras ex = {&il, clear_words, clear_count, nullptr, sh, nullptr};
         return permute_launch(x, x_dtype, ids, expand_idx, row_off, 0, smooth, tokens, hidden, topk, experts, q,
                               single_window(q1, xs, experts, tokens * topk), st, ex);
     }
@@ -837,7 +858,7 @@ extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, c
         const int32_t rc = zbalhip_layout_ranges_internal(ids, tokens, experts, topk, active_mask, expand_idx, scratch,
                                                           rt.ranges, rt.tokens_per_range, st);
         if (rc != ZBALHIP_OK) return rc;
-        const PermuteExtras ex = {nullptr, clear_words, clear_count, &rt};
+        const PermuteExtras ex = {nullptr, clear_words, clear_count, &rt, sh, active_mask};
         return permute_launch(x, x_dtype, ids, nullptr, nullptr, 0, smooth, tokens, hidden, topk, experts, q,
                               single_window(q1, xs, experts, tokens * topk), st, ex);
     }
@@ -845,7 +866,31 @@ extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, c
                                                      row_off, counts, nullptr, st);
     if (rc != ZBALHIP_OK) return rc;
     if (tokens == 0 && clear_count > 0) return zbalhip_fill_i32((int32_t *)clear_words, clear_count, 0, stream);
-    const PermuteExtras ex = {nullptr, clear_words, clear_count, nullptr};
+    const PermuteExtras ex = {nullptr, clear_words, clear_count, nullptr, sh, active_mask};
     return permute_launch(x, x_dtype, ids, expand_idx, row_off, 0, smooth, tokens, hidden, topk, experts, q,
                           single_window(q1, xs, experts, tokens * topk), st, ex);
+}
+
+extern "C" int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, const int32_t *expert_ids,
+                                               const float *smooth, const uint8_t *active_mask, int64_t tokens,
+                                               int64_t hidden, int64_t topk,
+                                               int64_t experts, int32_t mode, void *q1, float *xs, int32_t *expand_idx,
+                                               int64_t *counts, int32_t *row_off, uint32_t *clear_words,
+                                               int64_t clear_count, int32_t *scratch, int32_t scratch_blocks, void *stream)
+{
+    return fused_permute_quant(x, x_dtype, expert_ids, smooth, active_mask, tokens, hidden, topk, experts, mode, q1, xs, expand_idx,
+                               counts, row_off, clear_words, clear_count, scratch, scratch_blocks, SharedRows{}, stream);
+}
+
+extern "C" int32_t zbalhip_fused_permute_quant_shared(const void *x, int32_t x_dtype, const int32_t *expert_ids,
+                                                      const float *smooth, const uint8_t *active_mask, int64_t tokens,
+                                                      int64_t hidden, int64_t topk, int64_t experts, int32_t mode, void *q1,
+                                                      float *xs, int32_t *expand_idx, int64_t *counts, int32_t *row_off,
+                                                      uint32_t *clear_words, int64_t clear_count, int32_t *scratch,
+                                                      int32_t scratch_blocks, const float *shared_smooth, void *stream)
+{
+    if (!row_off || tokens <= 0 || experts <= 0 || (smooth != nullptr) != (shared_smooth != nullptr)) return ZBALHIP_INVALID;
+    const SharedRows sh = {tokens * topk, row_off + experts + 1, shared_smooth};
+    return fused_permute_quant(x, x_dtype, expert_ids, smooth, active_mask, tokens, hidden, topk, experts, mode, q1, xs, expand_idx,
+                               counts, row_off, clear_words, clear_count, scratch, scratch_blocks, sh, stream);
 }

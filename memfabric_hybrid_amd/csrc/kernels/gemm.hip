@@ -194,7 +194,7 @@ grouped_gemm_dma_kernel(GemmParams p)
             int mt = 0, rows_e = 0;
             if (e < E) {
                 const int lo = p.row_off[e];
-                rows_e = p.row_off[e + 1] - lo;
+                rows_e = p.row_off[e + 1] - first_row_of(p, e);
                 mt = (rows_e + TM - 1) / TM;
                 if (TWO_PHASE && rows_e <= TM / 2) mt = 0;      /* a short expert's only tile is not a main tile */
                 lds_roff[e] = lo;
@@ -225,7 +225,7 @@ grouped_gemm_dma_kernel(GemmParams p)
                     const int e = base + lane;
                     bool mine = false;
                     if (e < E) {
-                        const int rows = p.row_off[e + 1] - p.row_off[e];
+                        const int rows = p.row_off[e + 1] - first_row_of(p, e);
                         mine = rows > 0 && rows <= TM / 2 && (rows > TM / 4) == (cls == 2);
                     }
                     const uint64_t bal = __ballot(mine);
@@ -295,7 +295,7 @@ grouped_gemm_dma_kernel(GemmParams p)
          * sub-tiles cost (the K loop leaves out the absent ones), so this is no more work, and no tile is so short
          * that it runs ahead of the tiles it shares slabs with.
          */
-        const int first_row = __builtin_amdgcn_readfirstlane(lds_roff[expert]);
+        const int first_row = expert == p.shared_index ? p.shared_row : __builtin_amdgcn_readfirstlane(lds_roff[expert]);
         const int end_row = __builtin_amdgcn_readfirstlane(lds_roff[expert + 1]);
         const int n_row_tiles = (end_row - first_row + TM - 1) / TM;
         const int height = (((end_row - first_row + n_row_tiles - 1) / n_row_tiles) + 15) & ~15;
@@ -306,11 +306,11 @@ grouped_gemm_dma_kernel(GemmParams p)
         t.sa_base = p.a_scale + (int64_t)t.row_begin * KB;
         /* weights come pre-packed as 16 KiB blocks of 128 channels x 128 K-bytes in LDS order ([E][N/128][K/128]) */
         const int col0 = GMM1 ? t.n_tile : t.n_tile * 2, col1 = GMM1 ? I / 128 + t.n_tile : t.n_tile * 2 + 1;
-        const uint8_t *wb = expert_base<uint8_t>(p.w, p.w_is_list, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
+        const uint8_t *wb = weights_of<uint8_t>(p, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
         t.w_half[0] = wb + ((int64_t)col0 * KB) * W_BLOCK_BYTES;
         t.w_half[1] = wb + ((int64_t)col1 * KB) * W_BLOCK_BYTES;
         if (MODE == MODE_W4A8) {      /* fp16 group scales [E][K/128][N]: the slab's 128 scales of each half are 256 bytes */
-            const uint16_t *gs = expert_base<uint16_t>(p.wscale, p.w_is_list, expert, (int64_t)KB * p.N);
+            const uint16_t *gs = scales_of<uint16_t>(p, expert, (int64_t)KB * p.N);
             t.gs_mine = gs + ((wave_u & 1) ? col1 : col0) * 128;
         }
     };
@@ -414,7 +414,7 @@ grouped_gemm_dma_kernel(GemmParams p)
     auto issue_sw = [&](const Tile &t, int buf) __attribute__((always_inline)) {
         if (MODE != MODE_FP8) return;
         const int sw_stride = p.N / 128;
-        const float *base = expert_base<float>(p.wscale, p.w_is_list, t.expert, (int64_t)KB * sw_stride);
+        const float *base = scales_of<float>(p, t.expert, (int64_t)KB * sw_stride);
         const int c0 = GMM1 ? t.n_tile : t.n_tile * 2, c1 = GMM1 ? I / 128 + t.n_tile : t.n_tile * 2 + 1;
         for (int b = wave_u * 64; b < KB; b += NW * 64) {
             if (b + lane < KB) {
@@ -440,14 +440,14 @@ grouped_gemm_dma_kernel(GemmParams p)
         }
         if (wave_u < 4) {
             if (GMM1) {
-                const float *wsb = expert_base<float>(p.wscale, p.w_is_list, t.expert, p.N);
+                const float *wsb = scales_of<float>(p, t.expert, p.N);
                 const float *src = wave_u < 2 ? wsb + t.n_tile * 128 + wave_u * 64 : wsb + I + t.n_tile * 128 + (wave_u - 2) * 64;
                 dma4_sv(src, lane * 4u, __builtin_amdgcn_readfirstlane(dst0 + wave_u * 256));
             } else if (!p.wscale_is_bf16) {
-                const float *wsb = expert_base<float>(p.wscale, p.w_is_list, t.expert, p.N);
+                const float *wsb = scales_of<float>(p, t.expert, p.N);
                 dma4_sv(wsb + t.n_tile * BN + wave_u * 64, lane * 4u, __builtin_amdgcn_readfirstlane(dst0 + wave_u * 256));
             } else if (wave_u < 2) {
-                const uint16_t *wsb = expert_base<uint16_t>(p.wscale, p.w_is_list, t.expert, p.N);
+                const uint16_t *wsb = scales_of<uint16_t>(p, t.expert, p.N);
                 dma4_sv(reinterpret_cast<const float *>(wsb + t.n_tile * BN + wave_u * 128), lane * 4u,
                         __builtin_amdgcn_readfirstlane(dst0 + wave_u * 256));
             }
@@ -839,9 +839,10 @@ constexpr int kRequantThreads = 64, kRequantPieces = 8;
 
 __global__ void __launch_bounds__(kRequantThreads)
 requant_rows_kernel(const float *__restrict__ sgl, const uint32_t *__restrict__ rowmax, const int32_t *__restrict__ row_off,
-                    int experts, int max_rows, int I, int8_t *__restrict__ q2, float *__restrict__ scale2)
+                    int experts, int shared_row, int max_rows, int I, int8_t *__restrict__ q2, float *__restrict__ scale2)
 {
-    const int total = row_off[experts];
+    /* rows [0, total) and, of a shared expert (the last of `experts`), [shared_row, end); shared_row = max_rows without one */
+    const int total = row_off[shared_row < max_rows ? experts - 1 : experts], end = row_off[experts];
     const int vecs = I / 4;
     for (int row = blockIdx.x; row < max_rows; row += gridDim.x) {
         const uint32_t mx_bits = rowmax[row];
@@ -854,7 +855,7 @@ requant_rows_kernel(const float *__restrict__ sgl, const uint32_t *__restrict__ 
                 const int c = c0 + u * kRequantThreads + (int)threadIdx.x;
                 v[u] = c < vecs ? __builtin_nontemporal_load(src + c) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             }
-            if (row >= total) return;
+            if (row >= total && (row < shared_row || row >= end)) break;
             const float mx = __uint_as_float(mx_bits), inv = mx == 0.0f ? 0.0f : 1.0f / mx;
             if (c0 == 0 && threadIdx.x == 0) scale2[row] = mx * (1.0f / 127.0f);
 #pragma unroll
@@ -1125,10 +1126,31 @@ int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
 
 } // namespace
 
-extern "C" int32_t zbalhip_gmm1_swiglu_quant(const void *a, const float *a_scale, const void *w1, const void *w1scale,
-                                             const int32_t *row_off, int64_t experts, int64_t max_rows, int64_t k,
-                                             int64_t n1, int32_t mode, void *q2, float *scale2, float *sgl_ws,
-                                             void *stream)
+/* the shared expert that rides along: one expert more, its rows from max_rows on (`shared` null: none) */
+static void with_shared(GemmParams &p, const zbalhip_shared_expert_t *shared, int64_t out_row_bytes)
+{
+    p.shared_index = -1;
+    if (!shared) return;
+    p.shared_index = p.experts;
+    p.shared_row = p.max_rows;
+    p.experts += 1;
+    p.max_rows += (int)shared->rows;
+    p.shared_w = (const uint8_t *)shared->weight;
+    p.shared_wscale = shared->scale;
+    p.shared_out = (void *)((uintptr_t)shared->out - (uintptr_t)p.shared_row * (uintptr_t)out_row_bytes);
+}
+
+static bool shared_is_valid(const zbalhip_shared_expert_t *shared, int64_t experts, bool needs_out)
+{
+    if (!shared) return true;
+    return experts < 1024 && shared->rows > 0 && shared->weight && shared->scale && !misaligned16(shared->weight) &&
+           !misaligned16(shared->scale) && (!needs_out || (shared->out && !misaligned16(shared->out)));
+}
+
+extern "C" int32_t zbalhip_gmm1_swiglu_quant_shared(const void *a, const float *a_scale, const void *w1, const void *w1scale,
+                                                    const int32_t *row_off, int64_t experts, int64_t max_rows, int64_t k,
+                                                    int64_t n1, int32_t mode, void *q2, float *scale2, float *sgl_ws,
+                                                    const zbalhip_shared_expert_t *shared, void *stream)
 {
     const int w_is_list = (mode & ZBALHIP_WEIGHTS_AS_LISTS) != 0;
     const bool rowmax_cleared = (mode & ZBALHIP_ROWMAX_CLEARED) != 0;
@@ -1138,35 +1160,42 @@ extern "C" int32_t zbalhip_gmm1_swiglu_quant(const void *a, const float *a_scale
     if (misaligned16(a) || misaligned16(w1) || misaligned16(w1scale) || misaligned16(q2) || misaligned16(sgl_ws)) return ZBALHIP_INVALID;
     if (experts <= 0 || experts > 1024 || max_rows < 0 || k <= 0 || k % 128 != 0 || k > 128 * 256 || n1 <= 0 || n1 % 256 != 0)
         return ZBALHIP_INVALID;
+    if (!shared_is_valid(shared, experts, false)) return ZBALHIP_INVALID;
     if (max_rows == 0) return ZBALHIP_OK;
     hipStream_t st = (hipStream_t)stream;
     GemmParams p = {};
     p.a = (const uint8_t *)a; p.a_scale = a_scale; p.w = (const uint8_t *)w1; p.wscale = w1scale; p.row_off = row_off;
     p.experts = (int)experts; p.max_rows = (int)max_rows; p.K = (int)k; p.N = (int)n1;
     p.out = q2; p.out_scale = scale2; p.sgl_ws = sgl_ws; p.w_is_list = w_is_list;
+    with_shared(p, shared, 0);
     const int n_tiles = (int)(n1 / 2 / 128);
     if (mode == MODE_FP8) return launch_dma<MODE_FP8, true, ZDT_BF16>(p, n_tiles, st);
     if (!sgl_ws) return ZBALHIP_INVALID;
     /* the row maxima live behind the SwiGLU values in the same scratch allocation */
-    p.rowmax = (uint32_t *)(sgl_ws + max_rows * (n1 / 2));
-    if (!rowmax_cleared) fill_u32_kernel<<<(unsigned)((max_rows + 255) / 256), 256, 0, st>>>(p.rowmax, max_rows, 0u);
-    if (mode == MODE_W8A8) {
-        const int32_t rc = launch_dma<MODE_W8A8, true, ZDT_BF16>(p, n_tiles, st);
-        if (rc != ZBALHIP_OK) return rc;
-    } else {
-        const int32_t rc = launch_dma<MODE_W4A8, true, ZDT_BF16>(p, n_tiles, st);
-        if (rc != ZBALHIP_OK) return rc;
-    }
-    int64_t rb = max_rows < 16384 ? max_rows : 16384;
-    requant_rows_kernel<<<(unsigned)rb, kRequantThreads, 0, st>>>(sgl_ws, p.rowmax, row_off, (int)experts, (int)max_rows, (int)(n1 / 2),
-                                                    (int8_t *)q2, scale2);
+    p.rowmax = (uint32_t *)(sgl_ws + (int64_t)p.max_rows * (n1 / 2));
+    if (!rowmax_cleared) fill_u32_kernel<<<(unsigned)((p.max_rows + 255) / 256), 256, 0, st>>>(p.rowmax, p.max_rows, 0u);
+    const int32_t rc = mode == MODE_W8A8 ? launch_dma<MODE_W8A8, true, ZDT_BF16>(p, n_tiles, st)
+                                         : launch_dma<MODE_W4A8, true, ZDT_BF16>(p, n_tiles, st);
+    if (rc != ZBALHIP_OK) return rc;
+    const int rb = p.max_rows < 16384 ? p.max_rows : 16384;
+    requant_rows_kernel<<<(unsigned)rb, kRequantThreads, 0, st>>>(sgl_ws, p.rowmax, row_off, p.experts, shared ? p.shared_row : p.max_rows,
+                                                                  p.max_rows, (int)(n1 / 2), (int8_t *)q2, scale2);
     return zbalhip_check_launch();
 }
 
-extern "C" int32_t zbalhip_gmm2_dequant(const void *a, const float *a_scale, const void *w2, const void *wscale,
-                                        int32_t wscale_dtype, const int32_t *row_off, int64_t experts,
-                                        int64_t max_rows, int64_t k, int64_t n, int32_t mode, int32_t out_dtype,
-                                        void *y, void *stream)
+extern "C" int32_t zbalhip_gmm1_swiglu_quant(const void *a, const float *a_scale, const void *w1, const void *w1scale,
+                                             const int32_t *row_off, int64_t experts, int64_t max_rows, int64_t k,
+                                             int64_t n1, int32_t mode, void *q2, float *scale2, float *sgl_ws,
+                                             void *stream)
+{
+    return zbalhip_gmm1_swiglu_quant_shared(a, a_scale, w1, w1scale, row_off, experts, max_rows, k, n1, mode, q2, scale2, sgl_ws,
+                                            nullptr, stream);
+}
+
+extern "C" int32_t zbalhip_gmm2_dequant_shared(const void *a, const float *a_scale, const void *w2, const void *wscale,
+                                               int32_t wscale_dtype, const int32_t *row_off, int64_t experts,
+                                               int64_t max_rows, int64_t k, int64_t n, int32_t mode, int32_t out_dtype,
+                                               void *y, const zbalhip_shared_expert_t *shared, void *stream)
 {
     const int w_is_list = (mode & ZBALHIP_WEIGHTS_AS_LISTS) != 0;
     mode &= ~ZBALHIP_WEIGHTS_AS_LISTS;
@@ -1177,6 +1206,7 @@ extern "C" int32_t zbalhip_gmm2_dequant(const void *a, const float *a_scale, con
     if (experts <= 0 || experts > 1024 || max_rows < 0 || k <= 0 || k % 128 != 0 || k > 128 * 256 || n <= 0 || n % BN != 0)
         return ZBALHIP_INVALID;
     if (mode == MODE_W8A8 && wscale_dtype != ZDT_FP32 && wscale_dtype != ZDT_BF16) return ZBALHIP_INVALID;
+    if (!shared_is_valid(shared, experts, true)) return ZBALHIP_INVALID;
     if (max_rows == 0) return ZBALHIP_OK;
     hipStream_t st = (hipStream_t)stream;
     GemmParams p = {};
@@ -1185,6 +1215,7 @@ extern "C" int32_t zbalhip_gmm2_dequant(const void *a, const float *a_scale, con
     p.wscale_is_bf16 = (wscale_dtype == ZDT_BF16);
     p.w_is_list = w_is_list;
     p.out = y;
+    with_shared(p, shared, n * 2);
     const int n_tiles = (int)(n / BN);
     const bool bf = out_dtype == ZDT_BF16;
     if (mode == MODE_W8A8)
@@ -1192,6 +1223,15 @@ extern "C" int32_t zbalhip_gmm2_dequant(const void *a, const float *a_scale, con
     if (mode == MODE_FP8)
         return bf ? launch_dma<MODE_FP8, false, ZDT_BF16>(p, n_tiles, st) : launch_dma<MODE_FP8, false, ZDT_FP16>(p, n_tiles, st);
     return bf ? launch_dma<MODE_W4A8, false, ZDT_BF16>(p, n_tiles, st) : launch_dma<MODE_W4A8, false, ZDT_FP16>(p, n_tiles, st);
+}
+
+extern "C" int32_t zbalhip_gmm2_dequant(const void *a, const float *a_scale, const void *w2, const void *wscale,
+                                        int32_t wscale_dtype, const int32_t *row_off, int64_t experts,
+                                        int64_t max_rows, int64_t k, int64_t n, int32_t mode, int32_t out_dtype,
+                                        void *y, void *stream)
+{
+    return zbalhip_gmm2_dequant_shared(a, a_scale, w2, wscale, wscale_dtype, row_off, experts, max_rows, k, n, mode, out_dtype, y,
+                                       nullptr, stream);
 }
 
 extern "C" int32_t zbalhip_gemm_prepare(void)

@@ -88,11 +88,13 @@ grouped_gemm_stream_kernel(GemmParams p)
      * tiles each left the XCDs of the popular experts, whose row tiles share weights in the L2, idle early); the row tiles
      * of a column follow each other on its XCD. Every wave works the tile out for itself, without a barrier.
      */
+    auto nth_expert = [&](int i) { return p.shared_index < 0 ? i : (i == 0 ? p.shared_index : i - 1); };      /* a shared expert has the most rows: first */
     auto rows_of = [&](int base, int &lo, int &hi) {
         lo = hi = 0;
-        if (base + lane < E) { lo = p.row_off[base + lane]; hi = p.row_off[base + lane + 1]; }
+        const int e = nth_expert(base + lane);
+        if (base + lane < E) { lo = first_row_of(p, e); hi = p.row_off[e + 1]; }
     };
-    int lo[2], hi[2];                                              /* experts 0 .. 127, one per lane each: one round trip for all of them */
+    int lo[2], hi[2];                                              /* the first 128 experts, one per lane each: one round trip for all of them */
     rows_of(0, lo[0], hi[0]);
     rows_of(64, lo[1], hi[1]);
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -115,7 +117,7 @@ grouped_gemm_stream_kernel(GemmParams p)
         const uint64_t past = __ballot(tiles + incl > slot);
         if (past) {
             const int src = __ffsll((long long)past) - 1;
-            expert = base + src;
+            expert = nth_expert(base + src);
             mt_e = __builtin_amdgcn_readlane(m, src);
             first_row = __builtin_amdgcn_readlane(l, src);
             end_row = __builtin_amdgcn_readlane(h, src);
@@ -135,7 +137,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     const int last_rel = row_end - 1 - row_begin;
 
     /* the wave's two 16-channel sub-tiles: block rows r0, r0 + 16 .. of one 128-channel block, or the same rows of a gate and an up block */
-    const uint8_t *wb = expert_base<uint8_t>(p.w, p.w_is_list, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
+    const uint8_t *wb = weights_of<uint8_t>(p, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
     const int col0 = GMM1 ? n_tile : n_tile * 2, col1 = GMM1 ? I / 128 + n_tile : n_tile * 2 + 1;
     const uint8_t *w_src[NT];
 #pragma unroll
@@ -193,7 +195,7 @@ grouped_gemm_stream_kernel(GemmParams p)
                     lds_addr(lds_sa) + (b * S::SA_FLOATS + s * 64) * 4);
         }
         if (MODE == MODE_W4A8) {
-            const uint16_t *gs = expert_base<uint16_t>(p.wscale, p.w_is_list, expert, (int64_t)KB * p.N);
+            const uint16_t *gs = scales_of<uint16_t>(p, expert, (int64_t)KB * p.N);
             const int sg = (wave >> 1) & (PF - 1);
             gs += (int64_t)(kb0 + sg) * p.N + ((wave & 1) ? col1 : col0) * 128;
             dma4_sv(reinterpret_cast<const float *>(gs), lane_x * 4u, lds_addr(lds_gs) + b * S::GS_BYTES + sg * (BN * 2) + (wave & 1) * 256);
@@ -210,17 +212,17 @@ grouped_gemm_stream_kernel(GemmParams p)
         if (wave >= 4) {
             const int w4 = wave - 4;
             if (GMM1 || !p.wscale_is_bf16) {
-                const float *wsb = expert_base<float>(p.wscale, p.w_is_list, expert, p.N);
+                const float *wsb = scales_of<float>(p, expert, p.N);
                 const float *src = !GMM1 ? wsb + n_tile * BN + w4 * 64 : (w4 < 2 ? wsb + n_tile * 128 + w4 * 64 : wsb + I + n_tile * 128 + (w4 - 2) * 64);
                 dma4_sv(src, lane * 4u, dst0 + w4 * 256);
             } else if (w4 < 2) {
-                const uint16_t *wsb = expert_base<uint16_t>(p.wscale, p.w_is_list, expert, p.N);
+                const uint16_t *wsb = scales_of<uint16_t>(p, expert, p.N);
                 dma4_sv(reinterpret_cast<const float *>(wsb + n_tile * BN + w4 * 128), lane * 4u, dst0 + w4 * 256);
             }
         }
     } else if constexpr (MODE == MODE_FP8) {
         const int sw_stride = p.N / 128;
-        const float *base = expert_base<float>(p.wscale, p.w_is_list, expert, (int64_t)KB * sw_stride);
+        const float *base = scales_of<float>(p, expert, (int64_t)KB * sw_stride);
         for (int b = (wave & 3) * 64; b < KB; b += 256) {
             if (b + lane < KB)
                 dma4_sv(base + (wave < 4 ? col0 : col1), (uint32_t)(b + lane) * (uint32_t)sw_stride * 4u,

@@ -32,6 +32,14 @@ struct GemmParams {
     float *out_scale;        /* GMM1: scale2 (fp8 mode) */
     float *sgl_ws;           /* GMM1 int8 modes: fp32 SwiGLU values [rows, N/2] */
     uint32_t *rowmax;        /* GMM1 int8 modes: per-row absmax bits */
+    /*
+     * A shared expert in the same launch: the last of `experts`, with tensors of its own. Its rows start at shared_row,
+     * behind all rows that the routed experts can have, and end at row_off[experts]. shared_index is -1 without one.
+     */
+    int shared_index, shared_row;
+    const uint8_t *shared_w;
+    const void *shared_wscale;
+    void *shared_out;        /* GMM2: where row 0 would be if row shared_row is the first */
 };
 
 /*
@@ -46,6 +54,21 @@ __device__ __forceinline__ const T *expert_base(const void *base, int is_list, i
         return (const T *)(uintptr_t)((table_t)(uintptr_t)base)[expert];
     }
     return (const T *)base + (int64_t)expert * stride_elems;
+}
+
+template <typename T> __device__ __forceinline__ const T *weights_of(const GemmParams &p, int expert, int64_t stride)
+{
+    if (expert == p.shared_index) return (const T *)p.shared_w;
+    return expert_base<T>(p.w, p.w_is_list, expert, stride);
+}
+template <typename T> __device__ __forceinline__ const T *scales_of(const GemmParams &p, int expert, int64_t stride)
+{
+    if (expert == p.shared_index) return (const T *)p.shared_wscale;
+    return expert_base<T>(p.wscale, p.w_is_list, expert, stride);
+}
+__device__ __forceinline__ int first_row_of(const GemmParams &p, int expert)
+{
+    return expert == p.shared_index ? p.shared_row : p.row_off[expert];
 }
 
 struct TileCoord {
@@ -91,7 +114,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
     const int I = p.N / 2;
     const int q8 = (lane >> 4) * 8;
     if constexpr (!GMM1) {
-        uint16_t *y = (uint16_t *)p.out;
+        uint16_t *y = (uint16_t *)(tc.expert == p.shared_index ? p.shared_out : p.out);
 #pragma unroll
         for (int mt = 0; mt < MTM; ++mt) {
             const int row = row_begin + (RG * mt + wm) * 16 + frag_row;
