@@ -971,27 +971,43 @@ template <int MODE, bool GMM1> struct FewRows {
     static constexpr int STAGES_64 = MODE == MODE_W4A8 ? 4 : 3;
 };
 
-/* row tile of the streaming kernel; fp8's block scales leave no registers for a fourth row sub-tile */
-template <int MODE> constexpr int kStreamRows = MODE == MODE_FP8 ? 48 : 64;
+/*
+ * Row tiles of the streaming kernel: the lower one while most experts' rows fit it (four slabs of weights in flight, as the
+ * memory wants it), the taller one beyond (two; the L2 serves the row tiles of an expert together). The registers end them:
+ * fp8's block scales leave no room for a fourth sub-tile in the lower one, W8A8's second GEMM has room for eight.
+ */
+template <int MODE, bool GMM1> struct StreamRows {
+    static constexpr int LOW = MODE == MODE_FP8 ? 48 : 64;
+    static constexpr int TALL = MODE == MODE_W8A8 && !GMM1 ? 128 : 96;
+};
 
 /*
- * Where the streaming kernel takes over from the kernel below (K in whole chunks of its four slabs only). W4A8: always. The
- * 8-bit modes: while most experts' rows fit one tile of it, as a second one reads the weights again; layers in us with it
- * against without, uniform / Zipf(1.2) routing:
- *   - W8A8 first GEMM, rows per expert on average: 50 -18 / -32, 56 -20 / -36 (7168 x 4096: +20 / -20), 62 +12 / -37;
- *     second 56 -2 / -15, 62 +10 / -13;
- *   - fp8 first GEMM 28 -15 / -10, 37 -6 / -13, 56 -3 / -11 (2048 x 2048; 7168 x 4096 at 48: +28 / -21); second 28 0 / -4, 37 +5 / -6.
- * Long K loops whose tiles fill whole rounds of CUs run at the memory's rate in both kernels (7168 x 4096, 32 experts: 512
- * tiles, 6.6 TB/s), and there popular experts of up to 128 rows are one tile in the other: Zipf 128 tokens W8A8 +11.
+ * Where the streaming kernel takes over from the kernel above (K in whole chunks of its four slabs only), by rows per
+ * expert on average; 0: it does not. Layers in us with it against without, uniform / Zipf(1.2) routing, 128 experts of
+ * 4096 x 3072 / 1536 x 4096 (M), 64 of 2048 x 2048 / 1024 x 2048 (S), 32 of 7168 x 4096 / 2048 x 7168 (W):
+ *   - W4A8: always (M 128 rows -12 / -190, 250 -81 / -184; 64 rows against 96: 512 rows 3 / -199 and 13 / -206, 1024 +80 and -64);
+ *   - W8A8 first GEMM, 96 rows: 75 M -23 / -52, W -7 / -20, 128 M -35 / -23, W -17 / -4, 187 M +3 / -64, S -8 / -41,
+ *     250 M +35 / -46, W +22 / -27, 375 S -9 / -33, 512 M +90 / +17; second, 128 rows: 75 M -12 / -37, 128 M -27 / -32,
+ *     250 W -13 / -18, 375 M -25 / -21, 512 M +14 / -24;
+ *   - fp8 first GEMM: 75 W -7 / -29, 128 W -21 / -13, 187 S +2 / -27, 250 W +39 / -37, 375 S 0 / -23, 768 S +27 / 0; second:
+ *     75 W -10 / -25, 250 W -13 / -29, 500 W +9 / +17, 768 S -3 / -17.
+ * Beyond, the many-row shapes' arithmetic intensity wins, the sooner the longer K is. Long K loops whose tiles fill whole
+ * rounds of CUs run at the memory's rate in both kernels (W, 512 tiles: 6.6 TB/s), and there popular experts of up to 128
+ * rows are one tile in the other: 128 tokens Zipf W8A8 +11.
  */
 template <int MODE, bool GMM1>
-inline bool stream_pays(const GemmParams &p, int n_tiles)
+inline int stream_rows(const GemmParams &p, int n_tiles)
 {
+    using R = StreamRows<MODE, GMM1>;
     const int64_t rows = p.max_rows, e = p.experts, tiles = e * n_tiles, round = (tiles + 255) / 256 * 256;
-    if (p.K % 512 != 0) return false;
-    if (MODE == MODE_W4A8) return true;
-    if (GMM1 && p.K >= 6144 && rows <= 40 * e && tiles * 8 >= round * 7) return false;
-    return rows <= (MODE == MODE_W8A8 ? (GMM1 ? 54 : 60) : (GMM1 ? 40 : 36)) * e;
+    if (p.K % 512 != 0) return 0;
+    if (MODE == MODE_W4A8) return rows <= 640 * e ? R::LOW : R::TALL;
+    if (GMM1 && p.K >= 6144 && rows <= 40 * e && tiles * 8 >= round * 7) return 0;
+    const int64_t low = MODE == MODE_W8A8 ? 48 : 36;
+    int64_t tall = 400;
+    if (GMM1 && p.K > 2048) tall = MODE == MODE_W8A8 ? 200 : 160;
+    if (MODE == MODE_FP8 && !GMM1 && p.K <= 1024) tall = 800;
+    return rows <= low * e ? R::LOW : (rows <= tall * e ? R::TALL : 0);
 }
 
 /* every shape a launch of (MODE, GMM1, OUT_DT) can take */
@@ -1003,9 +1019,9 @@ int32_t prepare_mode()
     int32_t rc = prepare_shape<MODE, GMM1, OUT_DT, 256, 2, 4, false>(nullptr, &n);
     if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG, false>(nullptr, &n);
     if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 64, F::STAGES_64, F::RG, true>(nullptr, &n);
-    if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, kStreamRows<MODE>>(nullptr, &n);
+    if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, StreamRows<MODE, GMM1>::LOW>(nullptr, &n);
+    if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, StreamRows<MODE, GMM1>::TALL>(nullptr, &n);
     if constexpr (MODE == MODE_W4A8) {
-        if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, 96>(nullptr, &n);
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, 2, false>(nullptr, &n);
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 192, 3, 2, false>(nullptr, &n);
     } else {
@@ -1075,11 +1091,6 @@ int32_t launch_w4a8(const GemmParams &p, int n_tiles, hipStream_t st)
 {
     using F = FewRows<MODE_W4A8, GMM1>;
     const int64_t rows = p.max_rows, e = p.experts;
-    if (stream_pays<MODE_W4A8, GMM1>(p, n_tiles)) {
-        /* 64 rows, 96 from where an expert's tiles are many (16384 tokens on 128 experts 3911 / 3749 us; 8192 equal, 4000 1020 / 1025) */
-        if (rows <= 640 * e) return launch_stream<MODE_W4A8, GMM1, OUT_DT, kStreamRows<MODE_W4A8>>(p, n_tiles, st);
-        return launch_stream<MODE_W4A8, GMM1, OUT_DT, 96>(p, n_tiles, st);
-    }
     if (rows <= 48 * e && p.K >= 128 * (F::STAGES_64 - 1))
         return launch_dma_shape<MODE_W4A8, GMM1, OUT_DT, 64, F::STAGES_64, F::RG, true>(p, n_tiles, st);
     if (p.K >= 256) {
@@ -1093,12 +1104,15 @@ int32_t launch_w4a8(const GemmParams &p, int n_tiles, hipStream_t st)
 template <int MODE, bool GMM1, int OUT_DT>
 int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
 {
+    using R = StreamRows<MODE, GMM1>;
+    const int stream = stream_rows<MODE, GMM1>(p, n_tiles);
+    if (stream == R::LOW) return launch_stream<MODE, GMM1, OUT_DT, R::LOW>(p, n_tiles, st);
+    if (stream == R::TALL) return launch_stream<MODE, GMM1, OUT_DT, R::TALL>(p, n_tiles, st);
     if constexpr (MODE == MODE_W4A8) {
         return launch_w4a8<GMM1, OUT_DT>(p, n_tiles, st);
     } else {
         using F = FewRows<MODE, GMM1>;
         const int64_t rows = p.max_rows, e = p.experts;
-        if (stream_pays<MODE, GMM1>(p, n_tiles)) return launch_stream<MODE, GMM1, OUT_DT, kStreamRows<MODE>>(p, n_tiles, st);
         if (rows <= few_rows_limit<MODE, GMM1>(p, n_tiles) * e && p.K >= 256) {
             /*
              * Where nearly every expert has a single row tile its weight slabs are read once: they are requested with the

@@ -1,5 +1,5 @@
 /*
- * The grouped GEMM as a weight stream: the kernel for experts with few rows each, and for int4 weights with any number.
+ * The grouped GEMM as a weight stream: the kernel for experts with few or moderately many rows, and for int4 weights with any number.
  *
  * A weight byte is wanted by one wave only, so the weights do not go through LDS: a wave keeps the fragments of the next
  * four slabs (128 K each) of its own 32 channels in flight in registers, in exactly the order the pre-pack stores them
@@ -19,6 +19,7 @@
  * weights on every pass: W8A8, 128 experts of 4096 x 3072 / 1536 x 4096, top-8, 509 tokens 487 -> 461 us, Zipf(1.2)
  * routing 508 -> 457; 64 of 2048 x 2048 / 1024 x 2048, top-6, 200 tokens 111 -> 97. W4A8, 128 experts: 20 tokens 188 -> 166,
  * 509 tokens 320 -> 271, Zipf 397 -> 294, 2048 Zipf 842 -> 562, 16384 (96 rows) 3913 -> 3749.
+ * The taller tiles: W8A8, 128 experts, 2048 tokens 720 -> 657, 1200 tokens Zipf 647 -> 558; fp8, 32 experts, 512 tokens 424 -> 384.
  */
 #ifndef ZBAL_GEMM_STREAM_H_
 #define ZBAL_GEMM_STREAM_H_
@@ -28,15 +29,16 @@
 namespace {
 
 template <int MODE, int TM> struct StreamShape {
-    /* at many rows per expert (TM = 96) the L2 serves the weights: two slabs of look-ahead do, and leave room for six row sub-tiles */
-    static constexpr int PF = TM > 64 ? 2 : 4;                  /* slabs in flight, and slabs per activation chunk */
+    /* in the taller tiles the L2 serves the weights: two slabs of look-ahead do, and leave registers for six or eight row sub-tiles */
+    static constexpr int PF = TM > (MODE == MODE_FP8 ? 48 : 64) ? 2 : 4;                  /* slabs in flight, and slabs per activation chunk */
     static constexpr int MT_STEP = 4 / PF;                      /* row sub-tiles come in ones, or in twos: then two slabs of them are one transfer of every wave */
     static constexpr int NW = 8, NT = 2, THREADS = NW * 64;
     static constexpr int MTM = TM / 16;
     static constexpr int LOADS = MODE == MODE_W4A8 ? 1 : 2;     /* 16-byte loads per lane, sub-tile and slab */
     static constexpr int WRB = MODE == MODE_W4A8 ? 64 : 128;    /* bytes of a weight row per slab */
     static constexpr int A_BYTES = PF * TM * BKB;               /* one chunk: [slab][row][128 bytes, swizzled] */
-    static constexpr int SA_FLOATS = MODE == MODE_FP8 ? PF * 64 : 0;      /* one chunk's block scales, [slab][64 rows] */
+    static constexpr int SA_ROWS = TM > 64 ? 128 : 64;
+    static constexpr int SA_FLOATS = MODE == MODE_FP8 ? PF * SA_ROWS : 0; /* one chunk's block scales, [slab][row] */
     static constexpr int GS_BYTES = MODE == MODE_W4A8 ? PF * BN * 2 : 0;  /* one chunk's fp16 group scales, [slab][channel] */
     static constexpr int ES_FLOATS = MODE == MODE_W8A8 ? 256 + (TM + 63) / 64 * 64 : (MODE == MODE_FP8 ? 2 * 256 : 0);
     static constexpr int LDS_BYTES = 2 * (A_BYTES + SA_FLOATS * 4 + GS_BYTES) + ES_FLOATS * 4 + NW * TM * 4;
@@ -188,11 +190,10 @@ grouped_gemm_stream_kernel(GemmParams p)
             dma16_sv(p.a + (int64_t)row_begin * K + (int64_t)(kb0 + s) * BKB, (uint32_t)rel * (uint32_t)K + chunk16,
                      lds_a0 + b * S::A_BYTES + s * (TM * BKB) + rb * 1024);
         }
-        static_assert(MODE != MODE_FP8 || TM <= 64, "one lane per row");
-        if (MODE == MODE_FP8) {                                    /* waves s and s + 4 bring the same */
-            const int rel = lane_x > last_rel ? last_rel : lane_x;
+        if (MODE == MODE_FP8) {                                    /* 64 rows of slab s; several waves bring the same ones */
+            const int row = (TM > 64 ? (wave / PF & 1) * 64 : 0) + lane_x, rel = row > last_rel ? last_rel : row;
             dma4_sv(p.a_scale + (int64_t)row_begin * KB + kb0 + s, (uint32_t)rel * (uint32_t)KB * 4u,
-                    lds_addr(lds_sa) + (b * S::SA_FLOATS + s * 64) * 4);
+                    lds_addr(lds_sa) + (b * S::SA_FLOATS + s * S::SA_ROWS + (TM > 64 ? (wave / PF & 1) * 64 : 0)) * 4);
         }
         if (MODE == MODE_W4A8) {
             const uint16_t *gs = scales_of<uint16_t>(p, expert, (int64_t)KB * p.N);
@@ -205,7 +206,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     /* what the epilogue (W8A8) or the K loop (fp8) needs of the tile's scales; older than everything else, so there first */
     if constexpr (MODE == MODE_W8A8) {
         const uint32_t dst0 = lds_addr(lds_es);
-        if (wave < (TM + 63) / 64) {
+        if (wave < (TM + 63) / 64) {                               /* 64 token scales each */
             const int rel = wave * 64 + lane > last_rel ? last_rel : wave * 64 + lane;
             dma4_sv(p.a_scale + row_begin, (uint32_t)rel * 4u, dst0 + 1024 + wave * 256);
         }
@@ -289,7 +290,7 @@ grouped_gemm_stream_kernel(GemmParams p)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 const i32x8 a = load_a(mt);
-                const float sa = lds_sa[b * S::SA_FLOATS + s * 64 + mt * 16 + frag_row];
+                const float sa = lds_sa[b * S::SA_FLOATS + s * S::SA_ROWS + mt * 16 + frag_row];
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
                     const f32x4 part = mfma_fp8_16x16x128(w[nt], a);

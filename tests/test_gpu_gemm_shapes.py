@@ -53,7 +53,7 @@ def test_w4a8_shapes_bit_exact(buf, edges, K, N):
     assert np.array_equal(host(s2).view(np.uint32), r_s2.view(np.uint32)) and np.array_equal(host(q2), r_q2)
 
 
-@pytest.mark.parametrize("edges", ["few", "47", "53", "64", "100", "sparse"])
+@pytest.mark.parametrize("edges", ["few", "47", "53", "64", "100", "160", "sparse"])
 @pytest.mark.parametrize("K,N", [(256, 512), (640, 1280)] + STREAM_SHAPES)
 def test_8_bit_shapes(buf, edges, K, N):
     counts = np.array(EDGES[edges], dtype=np.int64)
