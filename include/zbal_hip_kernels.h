@@ -332,6 +332,20 @@ ZBALHIP_API int32_t zbalhip_gmm2_dequant(const void *a, const float *a_scale, co
                              int64_t k, int64_t n, int32_t mode, int32_t out_dtype, void *y, void *stream);
 
 /*
+ * zbalhip_dispatch_notify and zbalhip_dispatch_normal in one launch, for a group of one rank and at least one token.
+ */
+typedef struct {
+    const int32_t *tokens_per_expert;
+    int32_t *recv_data, *put_offset, *total_recv;
+    int64_t *recv_tokens_per_expert;
+    int32_t *balance_matrix;
+} zbalhip_notify_t;
+ZBALHIP_API int32_t zbalhip_dispatch_normal_notified(const void *x, int32_t x_dtype, const int32_t *topk_idx,
+                                    const int32_t *send_token_idx, const zbalhip_notify_t *notify, int64_t tokens,
+                                    int64_t hidden, int64_t topk, int64_t experts, int32_t quant_mode, void *dest,
+                                    float *dest_scale, int64_t dest_rows, void *stream);
+
+/*
  * The stages of the fused operator with a shared expert riding along (same K and N as the routed experts, same scale
  * types): its tokens are one expert's rows more, so its weights stream in the same launches. Its rows lie behind the
  * max_rows = tokens * topk rows that the routed experts can have, `rows` = tokens of them in token order; q1, xs, q2,

@@ -204,6 +204,17 @@ int32_t zbal_dispatch_normal_notify_end(zbal_pending_counts_t *pending, int64_t 
                                         zbal_comm_t comm, aclrtStream stream, int64_t flags);
 
 /*
+ * extension: zbal_dispatch_normal_notify and zbal_dispatch_normal as one call, which on a group of one rank is one launch.
+ */
+int32_t zbal_dispatch_normal_notified(const zbal_tensor_info_t *srcTokens, const zbal_tensor_info_t *topkIndex,
+                                      const zbal_tensor_info_t *sendTokensIndex, const zbal_tensor_info_t *sendTokensPerExpert,
+                                      int64_t expertNum, int64_t topKNum, const zbal_tensor_info_t *recvBuff,
+                                      const zbal_tensor_info_t *totalRecvTokens, const zbal_tensor_info_t *recvTokensPerExpert,
+                                      const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,
+                                      zbal_quant_mode_t quantMode, const zbal_tensor_info_t *destTokens,
+                                      const zbal_tensor_info_t *destScale, zbal_comm_t comm, aclrtStream stream, int64_t flags);
+
+/*
  * extension: softmax + top-k router. logits [T, E] fp32 -> topkIndex [T, K]
  * (int64, the type zbal_dispatch_normal_layout takes, or int32, the type
  * the dispatch and fused operators take: the descriptor's dataType says

@@ -128,6 +128,8 @@ SIGNATURES = {
     "zbal_dispatch_normal_notify_begin": (_i32, [_TI, _i64, _i64, _TI, _TI, _TI, _TI, _TI, ctypes.POINTER(PendingCounts), _vp,
                                                  _vp, _i64]),
     "zbal_dispatch_normal_notify_end": (_i32, [ctypes.POINTER(PendingCounts), _i64, _vp, _vp, _vp, _i64]),
+    "zbal_dispatch_normal_notified": (_i32, [_TI, _TI, _TI, _TI, _i64, _i64, _TI, _TI, _TI, _TI, _TI, _i32, _TI, _TI,
+                                             _vp, _vp, _i64]),
     "zbal_dispatch_normal": (_i32, [_TI, _TI, _TI, _TI, _TI, _i64, _i32, _TI, _TI, _vp, _vp, _i64]),
     "zbal_combine_normal": (_i32, [_TI, _TI, _TI, _TI, _TI, _TI, _u16, _TI, _vp, _vp, _i64]),
     "zbal_dispatch_low_latency": (_i32, [_TI, _TI, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _TI, _TI, _TI, _TI, _TI,
@@ -162,6 +164,7 @@ SIGNATURES = {
                                            _vp, _i64, _vp, _i32, _vp]),
     "zbalhip_dispatch_low_latency_ranks": (_i32, [_vp, _i32, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _vp, _vp, _i32, _i32, _i64,
                                                   _vp, _vp, _vp, _vp, _vp]),
+    "zbalhip_dispatch_normal_notified": (_i32, [_vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _i64, _vp]),
     "zbalhip_fused_permute_quant_shared": (_i32, [_vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp,
                                                   _vp, _i64, _vp, _i32, _vp, _vp]),
     "zbalhip_gmm1_swiglu_quant_shared": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp]),

@@ -363,6 +363,17 @@ public:
                                  const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,
                                  aclrtStream stream, int64_t, zbal_pending_counts_t *pending) override
     {
+        return Notify(sendTokensPerExpert, sendCount, topKNum, recvBuff, totalRecvTokens, recvTokensPerExpert, pushTargetOffset,
+                      balanceMatrix, stream, pending, nullptr);
+    }
+
+    /* checks a notify's arguments and launches it, or leaves its operands in `later` for a launch that does its work too */
+    int32_t Notify(const zbal_tensor_info_t *sendTokensPerExpert, int64_t sendCount, int64_t topKNum,
+                   const zbal_tensor_info_t *recvBuff, const zbal_tensor_info_t *totalRecvTokens,
+                   const zbal_tensor_info_t *recvTokensPerExpert, const zbal_tensor_info_t *pushTargetOffset,
+                   const zbal_tensor_info_t *balanceMatrix, aclrtStream stream, zbal_pending_counts_t *pending,
+                   zbalhip_notify_t *later)
+    {
         const char *op = "NotifyDispatch";
         const int64_t R = info_.groupSize, me = info_.myGroupRank;
         const int64_t E = sendCount; /* one count per expert, zbal_deepep.cpp:325-326 */
@@ -378,6 +389,11 @@ public:
         /* the counts of the other ranks are read where they lie: at the same offset in each rank's window */
         const void *counts[ZBALHIP_MAX_REDUCE_PEERS];
         if (!PeerCopies(op, sendTokensPerExpert->data, (size_t)E * 4, counts)) return Z_INVALID_PARAM;
+        if (later) {
+            *later = {(const int32_t *)sendTokensPerExpert->data, (int32_t *)recvBuff->data, (int32_t *)pushTargetOffset->data,
+                      (int32_t *)totalRecvTokens->data, (int64_t *)recvTokensPerExpert->data, (int32_t *)balanceMatrix->data};
+            return Z_OK;
+        }
         if (pending) {
             pending->block = countsBlocks_.Take();
             ZBAL_VALIDATE_RETURN(pending->block != nullptr, op << " failed as no pinned memory is left", Z_ERROR);
@@ -423,6 +439,33 @@ public:
                            const zbal_tensor_info_t *destTokens, const zbal_tensor_info_t *destScale,
                            aclrtStream stream, int64_t) override
     {
+        return Dispatch(srcTokens, topkIndex, sendTokensIndex, pushTargetOffset, expertNum, quantMode, destTokens, destScale, stream,
+                        nullptr);
+    }
+
+    int32_t DispatchNormalNotified(const zbal_tensor_info_t *srcTokens, const zbal_tensor_info_t *topkIndex,
+                                   const zbal_tensor_info_t *sendTokensIndex, const zbal_tensor_info_t *sendTokensPerExpert,
+                                   int64_t expertNum, int64_t topKNum, const zbal_tensor_info_t *recvBuff,
+                                   const zbal_tensor_info_t *totalRecvTokens, const zbal_tensor_info_t *recvTokensPerExpert,
+                                   const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,
+                                   zbal_quant_mode_t quantMode, const zbal_tensor_info_t *destTokens,
+                                   const zbal_tensor_info_t *destScale, aclrtStream stream) override
+    {
+        /* several ranks' counts have to be there before any offset is known, and a batch without tokens has no dispatch launch */
+        const bool together = info_.groupSize == 1 && srcTokens->dim == 2 && srcTokens->shape[0] > 0;
+        zbalhip_notify_t note = {};
+        const int32_t rc = Notify(sendTokensPerExpert, expertNum, topKNum, recvBuff, totalRecvTokens, recvTokensPerExpert,
+                                  pushTargetOffset, balanceMatrix, stream, nullptr, together ? &note : nullptr);
+        if (rc != Z_OK) return rc;
+        return Dispatch(srcTokens, topkIndex, sendTokensIndex, pushTargetOffset, expertNum, quantMode, destTokens, destScale, stream,
+                        together ? &note : nullptr);
+    }
+
+    int32_t Dispatch(const zbal_tensor_info_t *srcTokens, const zbal_tensor_info_t *topkIndex, const zbal_tensor_info_t *sendTokensIndex,
+                     const zbal_tensor_info_t *pushTargetOffset, int64_t expertNum, zbal_quant_mode_t quantMode,
+                     const zbal_tensor_info_t *destTokens, const zbal_tensor_info_t *destScale, aclrtStream stream,
+                     const zbalhip_notify_t *note)
+    {
         const char *op = "DispatchNormal";
         const int64_t R = info_.groupSize, me = info_.myGroupRank;
         ZBAL_VALIDATE_RETURN(R <= ZBALHIP_MAX_REDUCE_PEERS && expertNum % R == 0,
@@ -466,6 +509,11 @@ public:
         const void *dest[ZBALHIP_MAX_REDUCE_PEERS], *scale[ZBALHIP_MAX_REDUCE_PEERS] = {};
         if (!PeerCopies(op, destTokens->data, (size_t)destRows * rowBytes, dest)) return Z_INVALID_PARAM;
         if (scalesPerRow > 0 && !PeerCopies(op, destScale->data, (size_t)destRows * scalesPerRow * 4, scale)) return Z_INVALID_PARAM;
+        if (note)
+            return Launched(op, zbalhip_dispatch_normal_notified(srcTokens->data, srcTokens->dataType, (const int32_t *)topkIndex->data,
+                                                                 (const int32_t *)sendTokensIndex->data, note, T, H, K, expertNum,
+                                                                 (int32_t)quantMode | IdsFlag(topkIndex), (void *)dest[0],
+                                                                 scalesPerRow > 0 ? (float *)scale[0] : nullptr, destRows, stream));
         return Launched(op, zbalhip_dispatch_normal(srcTokens->data, srcTokens->dataType, (const int32_t *)topkIndex->data,
                                                     (const int32_t *)sendTokensIndex->data,
                                                     (const int32_t *)pushTargetOffset->data, T, H, K, expertNum,

@@ -166,6 +166,14 @@ public:
                                    const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,
                                    int64_t expertNum, zbal_quant_mode_t quantMode, const zbal_tensor_info_t *destTokens,
                                    const zbal_tensor_info_t *destScale, aclrtStream stream, int64_t flags) = 0;
+    virtual int32_t DispatchNormalNotified(const zbal_tensor_info_t *srcTokens, const zbal_tensor_info_t *topkIndex,
+                                           const zbal_tensor_info_t *sendTokensIndex,
+                                           const zbal_tensor_info_t *sendTokensPerExpert, int64_t expertNum, int64_t topKNum,
+                                           const zbal_tensor_info_t *recvBuff, const zbal_tensor_info_t *totalRecvTokens,
+                                           const zbal_tensor_info_t *recvTokensPerExpert,
+                                           const zbal_tensor_info_t *pushTargetOffset, const zbal_tensor_info_t *balanceMatrix,
+                                           zbal_quant_mode_t quantMode, const zbal_tensor_info_t *destTokens,
+                                           const zbal_tensor_info_t *destScale, aclrtStream stream) = 0;
     virtual int32_t CombineNormal(const zbal_tensor_info_t *srcTokens, const zbal_tensor_info_t *srcTokensPerEp,
                                   const zbal_tensor_info_t *topKWeight, const zbal_tensor_info_t *topkIndex,
                                   const zbal_tensor_info_t *sendTokensIndex, const zbal_tensor_info_t *balanceMatrix,

@@ -32,6 +32,7 @@ struct Library {
     decltype(&zbal_moe_topk_route) topk_route;
     decltype(&zbal_dispatch_normal_layout_in_rank) layout;
     decltype(&zbal_dispatch_normal_notify) notify;
+    decltype(&zbal_dispatch_normal_notified) notified;
     decltype(&zbal_dispatch_normal_notify_begin) notify_begin;
     decltype(&zbal_dispatch_normal_notify_end) notify_end;
     decltype(&zbal_dispatch_normal) dispatch;
@@ -292,28 +293,24 @@ struct Note {
     at::Tensor recv_data, recv_per_expert, put_offset, balance, total;
 };
 
-/* pending: the counts are wanted on the host as well */
-Note notify_call(const Frame &f, const at::Tensor &per_expert, int64_t topk, zbal_pending_counts_t *pending)
+Note notify_outputs(const Frame &f, int64_t E)
 {
-    const int64_t E = per_expert.size(0);
     Outputs out(f.dev);
     const size_t o0 = out.plan(E, at::kInt), o1 = out.plan(E, at::kLong), o2 = out.plan(E, at::kInt), o3 = out.plan(2, at::kInt),
                  o4 = out.plan(1, at::kInt);
-    Note n{out.make(o0, {1, E}, at::kInt), out.make(o1, {E}, at::kLong), out.make(o2, {1, E}, at::kInt),
-           out.make(o3, {1, 2}, at::kInt), out.make(o4, {1}, at::kInt)};
-    const Info i0(per_expert), i1(n.recv_data), i2(n.total), i3(n.recv_per_expert), i4(n.put_offset), i5(n.balance);
-    check("zbal_dispatch_normal_notify", unlocked([&] {
-              return pending ? L.notify_begin(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, pending, f.comm, f.stream, 0)
-                             : L.notify(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, f.comm, f.stream, 0);
-          }));
-    return n;
+    return {out.make(o0, {1, E}, at::kInt), out.make(o1, {E}, at::kLong), out.make(o2, {1, E}, at::kInt),
+            out.make(o3, {1, 2}, at::kInt), out.make(o4, {1}, at::kInt)};
 }
 
 /* (comm, dev, per_expert, topk) -> (recv_data, recv_per_expert, put_offset, balance_matrix, total_recv) */
 PyObject *notify(PyObject *const *args, Py_ssize_t nargs)
 {
     const Frame f(args, nargs, 4);
-    Note n = notify_call(f, f.t(2), f.n(3), nullptr);
+    const at::Tensor &per_expert = f.t(2);
+    const int64_t E = per_expert.size(0), topk = f.n(3);
+    const Note n = notify_outputs(f, E);
+    const Info i0(per_expert), i1(n.recv_data), i2(n.total), i3(n.recv_per_expert), i4(n.put_offset), i5(n.balance);
+    check("zbal_dispatch_normal_notify", unlocked([&] { return L.notify(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, f.comm, f.stream, 0); }));
     return tuple_of(wrap(n.recv_data), wrap(n.recv_per_expert), wrap(n.put_offset), wrap(n.balance), wrap(n.total));
 }
 
@@ -333,23 +330,20 @@ void receive(Outputs &out, int64_t qm, const at::Tensor &x, int64_t rows, at::Te
     }
 }
 
-void dispatch_call(const Frame &f, const at::Tensor &x, const at::Tensor &ids, const at::Tensor &send, const at::Tensor &put_offset,
-                   const at::Tensor &balance, int64_t E, int64_t qm, int64_t rows, at::Tensor *recv, at::Tensor *scales)
-{
-    Outputs out(f.dev);
-    receive(out, qm, x, rows, recv, scales);
-    const Info i0(x), i1(ids), i2(send), i3(put_offset), i4(balance), i5(*recv), i6(*scales);
-    check("zbal_dispatch_normal", unlocked([&] {
-              return L.dispatch(*i0, *i1, *i2, *i3, *i4, E, (zbal_quant_mode_t)qm, *i5, *i6, f.comm, f.stream, 0);
-          }));
-}
-
 /* (comm, dev, x, ids, send_idx, put_offset, balance_matrix, experts, quant_mode, rows) -> (recv, scales) */
 PyObject *dispatch(PyObject *const *args, Py_ssize_t nargs)
 {
     const Frame f(args, nargs, 10);
+    const at::Tensor &x = f.t(2);
+    const at::Tensor ids = expert_ids(f.t(3));
+    const int64_t E = f.n(7), qm = f.n(8);
     at::Tensor recv, scales;
-    dispatch_call(f, f.t(2), expert_ids(f.t(3)), f.t(4), f.t(5), f.t(6), f.n(7), f.n(8), f.n(9), &recv, &scales);
+    Outputs out(f.dev);
+    receive(out, qm, x, f.n(9), &recv, &scales);
+    const Info i0(x), i1(ids), i2(f.t(4)), i3(f.t(5)), i4(f.t(6)), i5(recv), i6(scales);
+    check("zbal_dispatch_normal", unlocked([&] {
+              return L.dispatch(*i0, *i1, *i2, *i3, *i4, E, (zbal_quant_mode_t)qm, *i5, *i6, f.comm, f.stream, 0);
+          }));
     return tuple_of(wrap(recv), wrap(scales));
 }
 
@@ -366,22 +360,29 @@ PyObject *dispatch_counts(PyObject *const *args, Py_ssize_t nargs)
     const at::Tensor &x = f.t(2), &per_expert = f.t(5);
     const at::Tensor ids = expert_ids(f.t(3));
     const int64_t worst = f.n(7), E = per_expert.size(0), qm = f.n(6), most = ids.numel() > 0 ? ids.numel() : 1;
-    zbal_pending_counts_t pending = {};
-    const Note n = notify_call(f, per_expert, ids.size(1), worst > 0 ? nullptr : &pending);
+    const Note n = notify_outputs(f, E);
     at::Tensor recv, scales;
-    std::vector<int64_t> counts;
+    Outputs out(f.dev);
+    receive(out, qm, x, worst > 0 ? worst : most, &recv, &scales);
+    std::vector<int64_t> counts(worst > 0 ? 0 : (size_t)E);
+    const Info i0(x), i1(ids), i2(f.t(4)), i3(per_expert), i4(n.recv_data), i5(n.total), i6(n.recv_per_expert), i7(n.put_offset),
+        i8(n.balance), i9(recv), i10(scales);
+    const zbal_quant_mode_t mode = (zbal_quant_mode_t)qm;
     if (worst > 0) {
-        dispatch_call(f, x, ids, f.t(4), n.put_offset, n.balance, E, qm, worst, &recv, &scales);
+        check("zbal_dispatch_normal", unlocked([&] {
+                  return L.notified(*i0, *i1, *i2, *i3, E, ids.size(1), *i4, *i5, *i6, *i7, *i8, mode, *i9, *i10, f.comm, f.stream, 0);
+              }));
     } else {
-        counts.resize((size_t)E);
-        auto wait = [&] { return L.notify_end(&pending, E, counts.data(), f.comm, f.stream, 0); };
-        try {
-            dispatch_call(f, x, ids, f.t(4), n.put_offset, n.balance, E, qm, most, &recv, &scales);
-        } catch (...) {
-            (void)wait();
-            throw;
-        }
-        check("zbal_dispatch_normal_notify", unlocked(wait));
+        zbal_pending_counts_t pending = {};
+        int32_t dispatched = 0;
+        check("zbal_dispatch_normal_notify", unlocked([&] {
+                  int32_t rc = L.notify_begin(*i3, E, ids.size(1), *i4, *i5, *i6, *i7, *i8, &pending, f.comm, f.stream, 0);
+                  if (rc != 0) return rc;
+                  dispatched = L.dispatch(*i0, *i1, *i2, *i7, *i8, E, mode, *i9, *i10, f.comm, f.stream, 0);
+                  rc = L.notify_end(&pending, E, counts.data(), f.comm, f.stream, 0);
+                  return dispatched != 0 ? 0 : rc;
+              }));
+        check("zbal_dispatch_normal", dispatched);
     }
     int64_t total = 0;
     for (const int64_t c : counts) total += c;
@@ -628,7 +629,8 @@ PyObject *bind(PyObject *const *args, Py_ssize_t nargs)
     void *h = dlopen(path, RTLD_NOW | RTLD_LOCAL);
     if (h == nullptr) fail(PyExc_RuntimeError, dlerror());
     if (!find(h, "zbal_moe_topk_route", &L.topk_route) || !find(h, "zbal_dispatch_normal_layout_in_rank", &L.layout) ||
-        !find(h, "zbal_dispatch_normal_notify", &L.notify) || !find(h, "zbal_dispatch_normal_notify_begin", &L.notify_begin) ||
+        !find(h, "zbal_dispatch_normal_notify", &L.notify) || !find(h, "zbal_dispatch_normal_notified", &L.notified) ||
+        !find(h, "zbal_dispatch_normal_notify_begin", &L.notify_begin) ||
         !find(h, "zbal_dispatch_normal_notify_end", &L.notify_end) ||
         !find(h, "zbal_dispatch_normal", &L.dispatch) || !find(h, "zbal_combine_normal", &L.combine) ||
         !find(h, "zbal_dispatch_low_latency", &L.ll_dispatch) || !find(h, "zbal_combine_low_latency", &L.ll_combine) ||
