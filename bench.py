@@ -224,11 +224,10 @@ def bench_moe(args, torch, np, capi, buf, workload):
     out_fused = out.clone()
 
     # ---- the same stages one by one through the inner kernel ABI, with events between them -----------------
-    off = {k: int(v) for k, v in plan_workspace(lib, T, H, K, E, N1, mode).items()}
-    base = ws.data_ptr()
-    q1, xs, eidx, row_off, q2, sc2, y = (base + off[k] for k in ("q1", "xs", "expand_idx", "row_off", "q2", "scale2", "y"))
-    lscratch = base + off["layout_scratch"]
-    sgl = base + off["sgl"] if mode != 2 else None
+    stage = {k: torch.empty(n, dtype=torch.uint8, device=dev) for k, n in stage_buffers(T, H, K, E, N1, mode).items()}
+    q1, xs, eidx, row_off, q2, sc2, y, lscratch = (
+        stage[k].data_ptr() for k in ("q1", "xs", "expand_idx", "row_off", "q2", "scale2", "y", "layout_scratch"))
+    sgl = stage["sgl"].data_ptr() if mode != 2 else None
     rowmax = sgl + rows * I * 4 if sgl else None      # int modes: row maxima behind the fp32 SwiGLU values; the permute launch clears them
     names = ["route", "permute_quant", "gmm1_swiglu_quant", "gmm2_dequant", "combine"]
     s2dt = {1: capi.DT_BF16, 2: capi.DT_FP32, 3: capi.DT_FP16}[mode]
@@ -395,33 +394,15 @@ def bench_reduce(args, torch, np, capi, buf):
     return line
 
 
-def plan_workspace(lib, T, H, K, E, N1, qmode):
-    """Offsets of the fused operator's workspace regions; mirrors PlanFusedWorkspace in the host layer
-    (csrc/host/zbal_gpu_communicator.cpp) and is cross-checked against the size the library reports."""
-    rows = max(T * K, 1)
-    I = N1 // 2
-    fp8 = qmode == 2
-    off = {}
-    cur = 0
-
-    def take(name, nbytes):
-        nonlocal cur
-        off[name] = cur
-        cur = (cur + nbytes + 255) & ~255
-
-    take("q1", rows * H)
-    take("xs", rows * (H // 128 if fp8 else 1) * 4)
-    take("expand_idx", rows * 4)
-    take("counts", E * 8)
-    take("row_off", (E + 1) * 4)
-    take("layout_scratch", 50 * E * 4)
-    take("q2", rows * I)
-    take("scale2", rows * ((I + 127) // 128 if fp8 else 1) * 4)
+def stage_buffers(T, H, K, E, N1, mode):
+    """Bytes of every buffer that the stages hand on, as include/zbal_hip_kernels.h states them for the calls above
+    (expand_idx [T,K], row_off [E+1], 50 rows of layout scratch, the row maxima behind the SwiGLU values)."""
+    rows, I, fp8 = T * K, N1 // 2, mode == 2
+    sizes = {"q1": rows * H, "xs": rows * (H // 128 if fp8 else 1) * 4, "expand_idx": rows * 4, "row_off": (E + 1) * 4,
+             "layout_scratch": 50 * E * 4, "q2": rows * I, "scale2": rows * (I // 128 if fp8 else 1) * 4, "y": rows * H * 2}
     if not fp8:
-        take("sgl", rows * (I + 1) * 4)
-    take("y", rows * H * 2)
-    assert cur == lib.zbal_fused_deep_moe_workspace_size(T, H, K, E, N1, 0, qmode), "workspace plan out of sync"
-    return off
+        sizes["sgl"] = rows * (I + 1) * 4
+    return sizes
 
 
 if __name__ == "__main__":
