@@ -164,10 +164,12 @@ int32_t zbal_fused_deep_moe(const zbal_tensor_info_t *x, const zbal_tensor_info_
 
 /*
  * extension: bytes of workspace zbal_fused_deep_moe needs for a batch of
- * `tokens` rows. Takes the place of the size computation the reference keeps
+ * `tokens` rows, or of fewer. Takes the place of the size computation the reference keeps
  * in its adaptor and host launcher (zbal_deepep.cpp:42-84,
  * zbal_kernel_fused_deep_moe_host.cpp:59-132). shareGmm1HLen is 0 without a
- * shared expert. Returns 0 on invalid input.
+ * shared expert; with one of the routed experts' width the size is what lets
+ * it run in their launches (with less it takes turns with them). Returns 0 on
+ * invalid input.
  */
 uint64_t zbal_fused_deep_moe_workspace_size(int64_t tokens, int64_t hidden, int64_t topk, int64_t moeExpertNum,
                                             int64_t gmm1HLen, int64_t shareGmm1HLen, int64_t quantMode);

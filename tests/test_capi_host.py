@@ -251,6 +251,32 @@ def test_a_workspace_sized_by_the_reference_is_large_enough(lib, tokens, hidden,
             assert 0 < ours <= want, (share_n1, quant_mode, ours, want)
 
 
+def regions_side_by_side(tokens, hidden, topk, experts, n1, fp8):
+    """The workspace regions of a layer without a shared expert, none on top of another."""
+    rows, inter = max(tokens * topk, 1), n1 // 2
+    sizes = [rows * hidden, rows * (hidden // 128 if fp8 else 1) * 4, rows * 4, experts * 8, (experts + 2) * 4, 50 * experts * 4,
+             rows * inter, rows * ((inter + 127) // 128 if fp8 else 1) * 4, 0 if fp8 else rows * (inter + 1) * 4, rows * hidden * 2]
+    return sum((n + 255) // 256 * 256 for n in sizes)
+
+
+@pytest.mark.parametrize("hidden,topk,experts,n1", [(7168, 8, 32, 4096), (4096, 8, 128, 3072), (2048, 6, 64, 2048), (4096, 2, 8, 28672),
+                                                    (7168, 8, 256, 4096)])
+def test_the_workspace_of_a_layer_is_what_its_regions_need(lib, hidden, topk, experts, n1):
+    """Room for the rows of a shared expert in the routed experts' launches costs a caller without one nothing: the
+    workspace is at most the regions of the routed rows laid side by side. A workspace for the largest batch serves every
+    smaller one, either side of where the shared expert stops riding (640 routed rows per expert)."""
+    f, last = lib.zbal_fused_deep_moe_workspace_size, 640 * experts // topk
+    for mode in (0, 2, 3):
+        for share in (0, n1, 256):
+            sizes = [f(t, hidden, topk, experts, n1, share, mode) for t in sorted((0, 1, 7, 128, last // 2, last - 1, last, last + 1,
+                                                                                   2 * last, 16384 + last))]
+            assert sizes[0] > 0 and sizes == sorted(sizes), (mode, share)
+        for t in (0, 1, 128, last, last + 1):
+            side = regions_side_by_side(t, hidden, topk, experts, n1, mode == 2)
+            assert f(t, hidden, topk, experts, n1, 0, mode) <= side, (mode, t)
+            assert f(t, hidden, topk, experts, n1, n1, mode) <= side * (topk + 1) // topk + 2560, (mode, t)
+
+
 def test_kernel_seam_types_and_exports():
     """CommGroupInfo keeps the reference's layout (zbal_comm_host_device_struct.h:133-151: 2160 bytes,
     peerGroupRank2WorldRank at 64) and the nine launcher functions of zbal_npu_operators.h are exported with C++
