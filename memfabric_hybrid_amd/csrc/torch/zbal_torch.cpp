@@ -350,46 +350,43 @@ PyObject *dispatch(PyObject *const *args, Py_ssize_t nargs)
 /*
  * Notify and dispatch in one call. (comm, dev, x, ids, send_idx, per_expert, quant_mode, worst_rows, running) ->
  * (recv, scales, list of received counts, put_offset, balance_matrix). worst_rows > 0: that many rows, an empty list
- * and no wait for the GPU; else the counts are read back, recv has their sum of rows (one at least), and the list holds
- * them, or their running sums. The read-back does not hold the GPU up: the dispatch goes into tensors with a row for
- * every pick and is queued before the counts are waited for; what is returned are the rows that there are.
+ * and no wait for the GPU; else the counts are read back, recv and scales are allocated for their sum of rows (one at
+ * least), and the list holds them, or their running sums. The GPU waits for the host in between: dispatching into
+ * tensors with a row for every pick before the counts are known saves 3 % (4096 tokens bf16 217 -> 211 us), but leaves
+ * the caller with all of those rows however few there are.
  */
 PyObject *dispatch_counts(PyObject *const *args, Py_ssize_t nargs)
 {
     const Frame f(args, nargs, 9);
     const at::Tensor &x = f.t(2), &per_expert = f.t(5);
     const at::Tensor ids = expert_ids(f.t(3));
-    const int64_t worst = f.n(7), E = per_expert.size(0), qm = f.n(6), most = ids.numel() > 0 ? ids.numel() : 1;
+    const int64_t worst = f.n(7), E = per_expert.size(0), qm = f.n(6), K = ids.size(1);
     const Note n = notify_outputs(f, E);
     at::Tensor recv, scales;
     Outputs out(f.dev);
-    receive(out, qm, x, worst > 0 ? worst : most, &recv, &scales);
     std::vector<int64_t> counts(worst > 0 ? 0 : (size_t)E);
     const Info i0(x), i1(ids), i2(f.t(4)), i3(per_expert), i4(n.recv_data), i5(n.total), i6(n.recv_per_expert), i7(n.put_offset),
-        i8(n.balance), i9(recv), i10(scales);
+        i8(n.balance);
     const zbal_quant_mode_t mode = (zbal_quant_mode_t)qm;
     if (worst > 0) {
+        receive(out, qm, x, worst, &recv, &scales);
+        const Info i9(recv), i10(scales);
         check("zbal_dispatch_normal", unlocked([&] {
-                  return L.notified(*i0, *i1, *i2, *i3, E, ids.size(1), *i4, *i5, *i6, *i7, *i8, mode, *i9, *i10, f.comm, f.stream, 0);
+                  return L.notified(*i0, *i1, *i2, *i3, E, K, *i4, *i5, *i6, *i7, *i8, mode, *i9, *i10, f.comm, f.stream, 0);
               }));
     } else {
-        zbal_pending_counts_t pending = {};
-        int32_t dispatched = 0;
         check("zbal_dispatch_normal_notify", unlocked([&] {
-                  int32_t rc = L.notify_begin(*i3, E, ids.size(1), *i4, *i5, *i6, *i7, *i8, &pending, f.comm, f.stream, 0);
-                  if (rc != 0) return rc;
-                  dispatched = L.dispatch(*i0, *i1, *i2, *i7, *i8, E, mode, *i9, *i10, f.comm, f.stream, 0);
-                  rc = L.notify_end(&pending, E, counts.data(), f.comm, f.stream, 0);
-                  return dispatched != 0 ? 0 : rc;
+                  zbal_pending_counts_t pending = {};
+                  const int32_t rc = L.notify_begin(*i3, E, K, *i4, *i5, *i6, *i7, *i8, &pending, f.comm, f.stream, 0);
+                  return rc != 0 ? rc : L.notify_end(&pending, E, counts.data(), f.comm, f.stream, 0);
               }));
-        check("zbal_dispatch_normal", dispatched);
-    }
-    int64_t total = 0;
-    for (const int64_t c : counts) total += c;
-    const int64_t rows = total == 0 ? 1 : total;
-    if (worst <= 0 && rows < most) {
-        recv = recv.narrow(0, 0, rows);
-        if (qm != NO_QUANT) scales = scales.narrow(0, 0, rows);
+        int64_t total = 0;
+        for (const int64_t c : counts) total += c;
+        receive(out, qm, x, total == 0 ? 1 : total, &recv, &scales);
+        const Info i9(recv), i10(scales);
+        check("zbal_dispatch_normal", unlocked([&] {
+                  return L.dispatch(*i0, *i1, *i2, *i7, *i8, E, mode, *i9, *i10, f.comm, f.stream, 0);
+              }));
     }
     PyObject *list = PyList_New((Py_ssize_t)counts.size());
     const bool running = f.n(8) != 0;
