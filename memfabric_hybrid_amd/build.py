@@ -70,7 +70,7 @@ def build_torch_adaptor(force=False):
          ["-shared", "-DUSE_ROCM", "-I" + os.path.join(ROOT, "include"), "-isystem", inc, "-isystem",
           os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", os.path.join(ROCM, "include"),
           "-I" + sysconfig.get_paths()["include"], src, "-o", TORCH_LIB, "-L" + os.path.join(torch_dir, "lib"),
-          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-ldl"])
+          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-ldl"])
     return TORCH_LIB
 
 

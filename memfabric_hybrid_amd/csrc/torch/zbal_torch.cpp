@@ -4,8 +4,8 @@
  * operators.py and buffer.py keep the signatures and return tuples on top of it.
  *
  * Small batches are bound by the host: with ctypes descriptors built field by field in Python a low-latency dispatch
- * and its combine took 55-60 us of host time for 16 us of kernels. Here a call costs its launches, one or two
- * allocations and about a microsecond.
+ * and its combine took 55-60 us of host time for 16 us of kernels. Here a call costs its launches, an allocation per
+ * output and about a microsecond.
  *
  * The library is the one capi.py has loaded (bind() gets its path): one libzbal.so per process.
  */
@@ -13,8 +13,8 @@
 
 #include <ATen/ATen.h>
 #include <ATen/Context.h>
+#include <ATen/ops/empty_cuda_dispatch.h>
 #include <c10/core/DeviceGuard.h>
-#include <c10/core/StorageImpl.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -152,22 +152,19 @@ at::Tensor expert_ids(const at::Tensor &t)
 /* ---- outputs ----------------------------------------------------------------------------------------------------- */
 
 /*
- * The outputs of one call. Large ones have an allocation each; the small ones (indices, counts, offsets) share one:
- * several tensors over one storage, each at a 256-byte boundary. (An allocation is 0.8 us of host time; a tensor kept
- * for long pins only what it shares the storage with, hence the limit.)
+ * An output: an allocation of its own, so that it can be freed, saved and kept by itself. (The device's own entry, not the
+ * dispatcher's: a low-latency dispatch has six; 7 tokens with their combine 15.4 -> 13.6 us.)
  */
-constexpr int64_t kShareBytes = 1 << 20;
+at::Tensor empty(c10::Device dev, at::IntArrayRef sizes, at::ScalarType t)
+{
+    return at::cuda::empty(sizes, t, at::kStrided, dev, false, std::nullopt);
+}
 
-class Outputs {
+/* What a call writes and nobody gets to see: pieces of one allocation, each at a 256-byte boundary. */
+class Scratch {
 public:
-    explicit Outputs(c10::Device dev) : dev_(dev) {}
+    explicit Scratch(c10::Device dev) : dev_(dev) {}
 
-    at::Tensor big(at::IntArrayRef sizes, at::ScalarType t)
-    {
-        return at::empty(sizes, at::TensorOptions().dtype(t).device(dev_));
-    }
-
-    /* room for a small output; its tensor comes from make() after all of them have been announced */
     size_t plan(int64_t numel, at::ScalarType t)
     {
         const size_t at = bytes_;
@@ -175,23 +172,22 @@ public:
         return at;
     }
 
-    at::Tensor make(size_t offset, at::IntArrayRef sizes, at::ScalarType t)
+    /* after every piece has been planned */
+    Info info(size_t offset, int64_t numel, at::ScalarType t)
     {
-        if (!storage_) {
-            const at::Tensor whole = big({(int64_t)(bytes_ ? bytes_ : 1)}, at::kByte);
-            storage_ = whole.storage();
-        }
-        at::Tensor r = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(storage_), c10::DispatchKeySet(c10::DispatchKey::CUDA),
-                                                                c10::scalarTypeToTypeMeta(t));
-        r.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
-        r.unsafeGetTensorImpl()->set_storage_offset((int64_t)(offset / c10::elementSize(t)));
+        if (!whole_.defined()) whole_ = empty(dev_, {(int64_t)bytes_}, at::kByte);
+        Info r;
+        r.ti.data = static_cast<uint8_t *>(whole_.data_ptr()) + offset;
+        r.ti.dataType = datatype(t);
+        r.ti.dim = 1;
+        r.ti.shape[0] = (uint32_t)numel;
         return r;
     }
 
 private:
     c10::Device dev_;
     size_t bytes_ = 0;
-    c10::Storage storage_;
+    at::Tensor whole_;
 };
 
 PyObject *wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
@@ -264,9 +260,7 @@ PyObject *topk_route(PyObject *const *args, Py_ssize_t nargs)
     const at::Tensor &logits = f.t(2);
     const int64_t T = logits.size(0), K = f.n(3);
     const at::ScalarType it = f.n(4) ? at::kLong : at::kInt;
-    Outputs out(f.dev);
-    const size_t oi = out.plan(T * K, it), ow = out.plan(T * K, at::kFloat);
-    const at::Tensor idx = out.make(oi, {T, K}, it), w = out.make(ow, {T, K}, at::kFloat);
+    const at::Tensor idx = empty(f.dev, {T, K}, it), w = empty(f.dev, {T, K}, at::kFloat);
     const Info il(logits), ii(idx), iw(w);
     check("zbal_moe_topk_route", unlocked([&] { return L.topk_route(*il, K, *ii, *iw, f.comm, f.stream, 0); }));
     return tuple_of(wrap(idx), wrap(w));
@@ -278,28 +272,13 @@ PyObject *layout(PyObject *const *args, Py_ssize_t nargs)
     const Frame f(args, nargs, 4);
     const at::Tensor &idx = f.t(2);
     const int64_t T = idx.size(0), K = idx.size(1), E = f.n(3);
-    Outputs out(f.dev);
-    const size_t o0 = out.plan(1, at::kInt), o1 = out.plan(E, at::kInt), o2 = out.plan(T * K, at::kInt), o3 = out.plan(T, at::kInt);
-    const at::Tensor per_rank = out.make(o0, {1}, at::kInt), per_expert = out.make(o1, {E}, at::kInt),
-                     send = out.make(o2, {T, K}, at::kInt), in_rank = out.make(o3, {T, 1}, at::kInt);
+    const at::Tensor per_rank = empty(f.dev, {1}, at::kInt), per_expert = empty(f.dev, {E}, at::kInt),
+                     send = empty(f.dev, {T, K}, at::kInt), in_rank = empty(f.dev, {T, 1}, at::kInt);
     const Info i0(idx), i1(per_rank), i2(per_expert), i3(send), i4(in_rank);
     check("zbal_dispatch_normal_layout", unlocked([&] {
               return L.layout(*i0, T, E, K, *i1, *i2, *i3, *i4, f.comm, f.stream, 0);
           }));
     return tuple_of(wrap(per_rank), wrap(per_expert), wrap(send), wrap(in_rank));
-}
-
-struct Note {
-    at::Tensor recv_data, recv_per_expert, put_offset, balance, total;
-};
-
-Note notify_outputs(const Frame &f, int64_t E)
-{
-    Outputs out(f.dev);
-    const size_t o0 = out.plan(E, at::kInt), o1 = out.plan(E, at::kLong), o2 = out.plan(E, at::kInt), o3 = out.plan(2, at::kInt),
-                 o4 = out.plan(1, at::kInt);
-    return {out.make(o0, {1, E}, at::kInt), out.make(o1, {E}, at::kLong), out.make(o2, {1, E}, at::kInt),
-            out.make(o3, {1, 2}, at::kInt), out.make(o4, {1}, at::kInt)};
 }
 
 /* (comm, dev, per_expert, topk) -> (recv_data, recv_per_expert, put_offset, balance_matrix, total_recv) */
@@ -308,25 +287,27 @@ PyObject *notify(PyObject *const *args, Py_ssize_t nargs)
     const Frame f(args, nargs, 4);
     const at::Tensor &per_expert = f.t(2);
     const int64_t E = per_expert.size(0), topk = f.n(3);
-    const Note n = notify_outputs(f, E);
-    const Info i0(per_expert), i1(n.recv_data), i2(n.total), i3(n.recv_per_expert), i4(n.put_offset), i5(n.balance);
+    const at::Tensor recv_data = empty(f.dev, {1, E}, at::kInt), recv_per_expert = empty(f.dev, {E}, at::kLong),
+                     put_offset = empty(f.dev, {1, E}, at::kInt), balance = empty(f.dev, {1, 2}, at::kInt),
+                     total = empty(f.dev, {1}, at::kInt);
+    const Info i0(per_expert), i1(recv_data), i2(total), i3(recv_per_expert), i4(put_offset), i5(balance);
     check("zbal_dispatch_normal_notify", unlocked([&] { return L.notify(*i0, E, topk, *i1, *i2, *i3, *i4, *i5, f.comm, f.stream, 0); }));
-    return tuple_of(wrap(n.recv_data), wrap(n.recv_per_expert), wrap(n.put_offset), wrap(n.balance), wrap(n.total));
+    return tuple_of(wrap(recv_data), wrap(recv_per_expert), wrap(put_offset), wrap(balance), wrap(total));
 }
 
 /* the receive tensors of `rows` rows for one quantisation mode: rows, scales (one unused scale without quantisation) */
-void receive(Outputs &out, int64_t qm, const at::Tensor &x, int64_t rows, at::Tensor *recv, at::Tensor *scales)
+void receive(const Frame &f, int64_t qm, const at::Tensor &x, int64_t rows, at::Tensor *recv, at::Tensor *scales)
 {
     const int64_t H = x.size(1);
     if (qm == NO_QUANT) {
-        *recv = out.big({rows, H}, x.scalar_type());
-        *scales = out.big({1}, at::kFloat);
+        *recv = empty(f.dev, {rows, H}, x.scalar_type());
+        *scales = empty(f.dev, {1}, at::kFloat);
     } else if (qm == QUANT_BF16_2_INT8) {
-        *recv = out.big({rows, H}, at::kChar);
-        *scales = out.big({rows}, at::kFloat);
+        *recv = empty(f.dev, {rows, H}, at::kChar);
+        *scales = empty(f.dev, {rows}, at::kFloat);
     } else {
-        *recv = out.big({rows, H}, at::kFloat8_e4m3fn);
-        *scales = out.big({rows, H / 128}, at::kFloat);
+        *recv = empty(f.dev, {rows, H}, at::kFloat8_e4m3fn);
+        *scales = empty(f.dev, {rows, H / 128}, at::kFloat);
     }
 }
 
@@ -338,8 +319,7 @@ PyObject *dispatch(PyObject *const *args, Py_ssize_t nargs)
     const at::Tensor ids = expert_ids(f.t(3));
     const int64_t E = f.n(7), qm = f.n(8);
     at::Tensor recv, scales;
-    Outputs out(f.dev);
-    receive(out, qm, x, f.n(9), &recv, &scales);
+    receive(f, qm, x, f.n(9), &recv, &scales);
     const Info i0(x), i1(ids), i2(f.t(4)), i3(f.t(5)), i4(f.t(6)), i5(recv), i6(scales);
     check("zbal_dispatch_normal", unlocked([&] {
               return L.dispatch(*i0, *i1, *i2, *i3, *i4, E, (zbal_quant_mode_t)qm, *i5, *i6, f.comm, f.stream, 0);
@@ -361,15 +341,16 @@ PyObject *dispatch_counts(PyObject *const *args, Py_ssize_t nargs)
     const at::Tensor &x = f.t(2), &per_expert = f.t(5);
     const at::Tensor ids = expert_ids(f.t(3));
     const int64_t worst = f.n(7), E = per_expert.size(0), qm = f.n(6), K = ids.size(1);
-    const Note n = notify_outputs(f, E);
     at::Tensor recv, scales;
-    Outputs out(f.dev);
+    const at::Tensor put_offset = empty(f.dev, {1, E}, at::kInt), balance = empty(f.dev, {1, 2}, at::kInt);
+    Scratch tmp(f.dev);
+    const size_t o4 = tmp.plan(E, at::kInt), o5 = tmp.plan(1, at::kInt), o6 = tmp.plan(E, at::kLong);
     std::vector<int64_t> counts(worst > 0 ? 0 : (size_t)E);
-    const Info i0(x), i1(ids), i2(f.t(4)), i3(per_expert), i4(n.recv_data), i5(n.total), i6(n.recv_per_expert), i7(n.put_offset),
-        i8(n.balance);
+    const Info i0(x), i1(ids), i2(f.t(4)), i3(per_expert), i4 = tmp.info(o4, E, at::kInt), i5 = tmp.info(o5, 1, at::kInt),
+               i6 = tmp.info(o6, E, at::kLong), i7(put_offset), i8(balance);
     const zbal_quant_mode_t mode = (zbal_quant_mode_t)qm;
     if (worst > 0) {
-        receive(out, qm, x, worst, &recv, &scales);
+        receive(f, qm, x, worst, &recv, &scales);
         const Info i9(recv), i10(scales);
         check("zbal_dispatch_normal", unlocked([&] {
                   return L.notified(*i0, *i1, *i2, *i3, E, K, *i4, *i5, *i6, *i7, *i8, mode, *i9, *i10, f.comm, f.stream, 0);
@@ -382,7 +363,7 @@ PyObject *dispatch_counts(PyObject *const *args, Py_ssize_t nargs)
               }));
         int64_t total = 0;
         for (const int64_t c : counts) total += c;
-        receive(out, qm, x, total == 0 ? 1 : total, &recv, &scales);
+        receive(f, qm, x, total == 0 ? 1 : total, &recv, &scales);
         const Info i9(recv), i10(scales);
         check("zbal_dispatch_normal", unlocked([&] {
                   return L.dispatch(*i0, *i1, *i2, *i7, *i8, E, mode, *i9, *i10, f.comm, f.stream, 0);
@@ -395,7 +376,7 @@ PyObject *dispatch_counts(PyObject *const *args, Py_ssize_t nargs)
         run = running ? run + counts[e] : counts[e];
         PyList_SET_ITEM(list, (Py_ssize_t)e, PyLong_FromLongLong(run));
     }
-    return tuple_of(wrap(recv), wrap(scales), list, wrap(n.put_offset), wrap(n.balance));
+    return tuple_of(wrap(recv), wrap(scales), list, wrap(put_offset), wrap(balance));
 }
 
 /* (comm, dev, x, put_offset, weights, ids, send_idx, balance_matrix, experts) -> out */
@@ -404,8 +385,7 @@ PyObject *combine(PyObject *const *args, Py_ssize_t nargs)
     const Frame f(args, nargs, 9);
     const at::Tensor &x = f.t(2);
     const at::Tensor ids = expert_ids(f.t(5));
-    Outputs o(f.dev);
-    const at::Tensor out = o.big({ids.size(0), x.size(1)}, x.scalar_type());
+    const at::Tensor out = empty(f.dev, {ids.size(0), x.size(1)}, x.scalar_type());
     const Info i0(x), i1(f.t(3)), i2(f.t(4)), i3(ids), i4(f.t(6)), i5(f.t(7)), i6(out);
     const int64_t E = f.n(8);
     check("zbal_combine_normal", unlocked([&] {
@@ -432,19 +412,15 @@ PyObject *ll_dispatch(PyObject *const *args, Py_ssize_t nargs)
     const at::Tensor &x = f.t(2);
     const at::Tensor ids = expert_ids(f.t(3));
     const int64_t T = x.size(0), K = ids.size(1), H = x.size(1), rows = T * K > 0 ? T * K : 1, E = f.n(5), qm = f.n(6), most = f.n(4),
-                  type = token_nums_type(), blocks = qm == QUANT_BF16_2_FP8E4M3_B128 ? H / 128 : 1;
+                  type = token_nums_type();
     const at::ScalarType rt = qm == NO_QUANT ? x.scalar_type() : qm == QUANT_BF16_2_INT8 ? at::kChar : at::kFloat8_e4m3fn;
-    Outputs out(f.dev);
-    const bool share = rows * H * (int64_t)c10::elementSize(rt) <= kShareBytes;
-    const size_t orecv = share ? out.plan(rows * H, rt) : 0, oscale = out.plan(rows * blocks, at::kFloat);
-    const size_t o0 = out.plan(rows, at::kInt), o1 = out.plan(E, at::kInt), o2 = out.plan(E, at::kLong), o3 = out.plan(E, at::kInt),
-                 o4 = out.plan(E, at::kFloat);
-    const at::Tensor expand_idx = out.make(o0, {rows}, at::kInt), ep_recv = out.make(o1, {E}, at::kInt),
-                     nums = out.make(o2, {E}, at::kLong), put_offset = out.make(o3, {E}, at::kInt),
-                     status = out.make(o4, {E}, at::kFloat);
-    const at::Tensor recv = share ? out.make(orecv, {rows, H}, rt) : out.big({rows, H}, rt),
-                     scales = qm == QUANT_BF16_2_FP8E4M3_B128 ? out.make(oscale, {rows, blocks}, at::kFloat) : out.make(oscale, {rows}, at::kFloat);
-    const Info i0(x), i1(ids), i2(recv), i3(scales), i4(expand_idx), i5(nums), i6(ep_recv), i7(put_offset), i8(status);
+    const at::Tensor recv = empty(f.dev, {rows, H}, rt),
+                     scales = qm == QUANT_BF16_2_FP8E4M3_B128 ? empty(f.dev, {rows, H / 128}, at::kFloat) : empty(f.dev, {rows}, at::kFloat),
+                     expand_idx = empty(f.dev, {rows}, at::kInt), ep_recv = empty(f.dev, {E}, at::kInt), nums = empty(f.dev, {E}, at::kLong);
+    Scratch tmp(f.dev);
+    const size_t o7 = tmp.plan(E, at::kInt), o8 = tmp.plan(E, at::kFloat);
+    const Info i0(x), i1(ids), i2(recv), i3(scales), i4(expand_idx), i5(nums), i6(ep_recv), i7 = tmp.info(o7, E, at::kInt),
+               i8 = tmp.info(o8, E, at::kFloat);
     check("zbal_dispatch_low_latency", unlocked([&] {
               return L.ll_dispatch(*i0, *i1, E, 1, 0, qm, T > most ? T : most, 0, type, *i2, *i3, *i4, *i5, *i6, *i7, *i8, f.comm,
                                    f.stream, 0);
@@ -459,8 +435,7 @@ PyObject *ll_combine(PyObject *const *args, Py_ssize_t nargs)
     const at::Tensor &x = f.t(2);
     const at::Tensor ids = expert_ids(f.t(3));
     const int64_t T = ids.size(0), K = ids.size(1), E = f.n(7);
-    Outputs o(f.dev);
-    const at::Tensor out = o.big({T, x.size(1)}, x.scalar_type());
+    const at::Tensor out = empty(f.dev, {T, x.size(1)}, x.scalar_type());
     Info i2(f.t(4));
     i2.shape2(T, K);
     const Info i0(x), i1(ids), i3(f.t(5)), i4(f.t(6)), i5(out);
@@ -569,18 +544,17 @@ PyObject *fused(PyObject *const *args, Py_ssize_t nargs)
     }
     const Info wt(f.t(8)), smooth = info_or_null(args[11]), ssmooth = info_or_null(args[16]), mask = info_or_null(args[17]);
 
-    Outputs o(f.dev);
     at::Tensor workspace, out, share_out;
     if (args[18] == Py_None) {
         const uint64_t bytes = L.fused_workspace(T, H, K, E, n1, sn1, qm);
         if (bytes == 0) fail(PyExc_ValueError, "invalid fused MoE shape");
-        workspace = o.big({(int64_t)bytes}, at::kByte);
+        workspace = empty(f.dev, {(int64_t)bytes}, at::kByte);
     } else {
         workspace = f.t(18);
     }
-    out = args[19] == Py_None ? o.big({T, H}, x.scalar_type()) : f.t(19);
-    if (shared) share_out = args[20] == Py_None ? o.big({T, H}, x.scalar_type()) : f.t(20);
-    const at::Tensor nums = o.big({E}, at::kLong);
+    out = args[19] == Py_None ? empty(f.dev, {T, H}, x.scalar_type()) : f.t(19);
+    if (shared) share_out = args[20] == Py_None ? empty(f.dev, {T, H}, x.scalar_type()) : f.t(20);
+    const at::Tensor nums = empty(f.dev, {E}, at::kLong);
     const Info iout(out), inums(nums), iws(workspace);
     Info ishare;
     if (shared) ishare = Info(share_out);
