@@ -46,7 +46,7 @@ def _newer(target, sources):
 
 def _headers():
     hs = []
-    for d in (os.path.join(ROOT, "include"), os.path.join(CSRC, "kernels"), os.path.join(CSRC, "host")):
+    for d in [os.path.join(ROOT, "include")] + [os.path.join(CSRC, d) for d in ("kernels", "host", "torch")]:
         hs += [os.path.join(d, f) for f in os.listdir(d) if f.endswith(".h")]
     return hs
 

@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "zbal.h"
+#include "zbal_py_result.h"
 
 namespace {
 
@@ -53,9 +54,6 @@ template <typename F> bool find(void *h, const char *name, F *f)
     if (*f == nullptr) PyErr_Format(PyExc_RuntimeError, "libzbal.so has no symbol %s", name);
     return *f != nullptr;
 }
-
-/* a Python exception is set */
-struct PyFail {};
 
 [[noreturn]] void fail(PyObject *type, const char *text)
 {
@@ -190,21 +188,7 @@ private:
     at::Tensor whole_;
 };
 
-PyObject *wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
-
-template <typename... T> PyObject *tuple_of(T... items)
-{
-    PyObject *all[] = {items...};
-    PyObject *r = PyTuple_New(sizeof...(items));
-    for (size_t i = 0; i < sizeof...(items); ++i) {
-        if (all[i] == nullptr) {
-            Py_XDECREF(r);
-            throw PyFail{};
-        }
-        PyTuple_SET_ITEM(r, (Py_ssize_t)i, all[i]);
-    }
-    return r;
-}
+Owned wrap(at::Tensor t) { return checked(THPVariable_Wrap(std::move(t))); }
 
 /* ---- the frame of a call --------------------------------------------------------------------------------------- */
 
@@ -369,14 +353,7 @@ PyObject *dispatch_counts(PyObject *const *args, Py_ssize_t nargs)
                   return L.dispatch(*i0, *i1, *i2, *i7, *i8, E, mode, *i9, *i10, f.comm, f.stream, 0);
               }));
     }
-    PyObject *list = PyList_New((Py_ssize_t)counts.size());
-    const bool running = f.n(8) != 0;
-    int64_t run = 0;
-    for (size_t e = 0; e < counts.size(); ++e) {
-        run = running ? run + counts[e] : counts[e];
-        PyList_SET_ITEM(list, (Py_ssize_t)e, PyLong_FromLongLong(run));
-    }
-    return tuple_of(wrap(recv), wrap(scales), list, wrap(put_offset), wrap(balance));
+    return tuple_of(wrap(recv), wrap(scales), list_of(counts, f.n(8) != 0), wrap(put_offset), wrap(balance));
 }
 
 /* (comm, dev, x, put_offset, weights, ids, send_idx, balance_matrix, experts) -> out */
@@ -391,7 +368,7 @@ PyObject *combine(PyObject *const *args, Py_ssize_t nargs)
     check("zbal_combine_normal", unlocked([&] {
               return L.combine(*i0, *i1, *i2, *i3, *i4, *i5, (uint16_t)E, *i6, f.comm, f.stream, 0);
           }));
-    return wrap(out);
+    return wrap(out).release();
 }
 
 /* MOE_EXPERT_TOKEN_NUMS_TYPE (zbal_deepep.cpp:497), 1 where it is not set */
@@ -442,7 +419,7 @@ PyObject *ll_combine(PyObject *const *args, Py_ssize_t nargs)
     check("zbal_combine_low_latency", unlocked([&] {
               return L.ll_combine(*i0, *i1, *i2, *i3, *i4, *i5, E, f.comm, f.stream, 0);
           }));
-    return wrap(out);
+    return wrap(out).release();
 }
 
 /* ---- the fused layer --------------------------------------------------------------------------------------------- */
@@ -487,10 +464,7 @@ Info list_info(PyObject *seq, int64_t experts, PyObject *tables, c10::Device dev
         memcpy(table.data_ptr(), addresses.data(), (size_t)experts * 8);
         table = table.to(dev);
     }
-    PyObject *wrapped = wrap(table);
-    if (wrapped == nullptr) throw PyFail{};
-    Release release_table{wrapped};
-    if (PyDict_SetItem(tables, key, wrapped) != 0) throw PyFail{};
+    if (PyDict_SetItem(tables, key, wrap(table).get()) != 0) throw PyFail{};
     while (PyDict_Size(tables) > kMostTables) {
         Py_ssize_t pos = 0;
         PyObject *oldest = nullptr, *value = nullptr;
@@ -562,10 +536,8 @@ PyObject *fused(PyObject *const *args, Py_ssize_t nargs)
               return L.fused(*i0, *i1, *w1, *s1, *w2, *s2, *wt, *smooth, *sw1, *ss1, *sw2, *ss2, *ssmooth, *mask, *iout, *ishare,
                              *inums, *iws, E, qm, 0, n1, sn1, lists ? 1 : 0, f.comm, f.stream, 0);
           }));
-    PyObject *share = Py_None;
-    if (shared) share = wrap(share_out);
-    else Py_INCREF(share);
-    return tuple_of(wrap(out), share, wrap(nums));
+    if (!shared) Py_INCREF(Py_None);
+    return tuple_of(wrap(out), shared ? wrap(share_out) : Owned(Py_None), wrap(nums));
 }
 
 /* (tensors,) -> whether every one of them is marked as pre-packed */
