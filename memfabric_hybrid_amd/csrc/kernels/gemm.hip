@@ -885,6 +885,18 @@ inline unsigned grid_for(int64_t max_rows, int64_t experts, int n_tiles, int til
     return (unsigned)((g + 7) / 8 * 8);
 }
 
+/* CUs of the current device (a partition of the GPU has fewer than 256); 0 if it cannot be asked */
+inline int cu_count()
+{
+    static std::atomic<int> cus[64];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    n = cus[dev].load(std::memory_order_relaxed);
+    if (n == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+        cus[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
+
 /*
  * The kernels need more dynamic LDS than the default limit: raised once per kernel instantiation and device, which
  * cannot be recorded into a graph. zbalhip_gemm_prepare does it for every instantiation ahead of time (the host layer
@@ -994,19 +1006,42 @@ template <int MODE, bool GMM1> struct StreamRows {
  * Beyond, the many-row shapes' arithmetic intensity wins, the sooner the longer K is. Long K loops whose tiles fill whole
  * rounds of CUs run at the memory's rate in both kernels (W, 512 tiles: 6.6 TB/s), and there popular experts of up to 128
  * rows are one tile in the other: 128 tokens Zipf W8A8 +11.
+ * With every expert as popular as the next, row counts just past a tile's height cost: two tiles of 50 rows where the other
+ * kernel has one of 128 (or 320). Both GEMMs of nine shapes, 8 to 256 experts, 2048 to 8192 wide, 1024 to 14336 deep,
+ * 8 to 400 rows, both kernels in turn in one process, uniform / Zipf(0.6) / Zipf(1.2) routing, per cent:
+ *   - first GEMM, K > 2048: 84 rows 0 / -11 / -15; 88-108 rows W8A8 +6 (up to +31) / -9 / -12, 88-112 fp8 +12 (+34) / -7 / -13:
+ *     left to the other; 120-160 rows W8A8 -4 / -12 / -18, fp8 -3 / -12 / -22; W8A8 190-200 rows +5 (+15) / -11 / -22: hence 184;
+ *   - many tiles (256 experts: 4096 in the first GEMM, 7168 in the second), where both run at the memory's rate longer: first
+ *     fp8 GEMM 112-150 rows +10 / -2 / -20, second GEMM 200-320 rows W8A8 +7 / +1 / -16, fp8 +13 / +3 / -22;
+ *   - second fp8 GEMM, K 14336, 8 experts: 160-190 rows +34 / +25 / +33 (a third row tile on a few CUs, and K is long); from
+ *     200 to 350, where the other kernel's tile is 320 rows, -27 / -25 / -25, 400 rows (a fifth row tile) +27 / -14 / -12;
+ *   - W4A8 -2 ... -50 throughout.
  */
 template <int MODE, bool GMM1>
 inline int stream_rows(const GemmParams &p, int n_tiles)
 {
     using R = StreamRows<MODE, GMM1>;
-    const int64_t rows = p.max_rows, e = p.experts, tiles = e * n_tiles, round = (tiles + 255) / 256 * 256;
+    const int64_t rows = p.max_rows, e = p.experts, tiles = e * n_tiles;
     if (p.K % 512 != 0) return 0;
     if (MODE == MODE_W4A8) return rows <= 640 * e ? R::LOW : R::TALL;
-    if (GMM1 && p.K >= 6144 && rows <= 40 * e && tiles * 8 >= round * 7) return 0;
+    const bool many_tiles = tiles >= 4096;
     const int64_t low = MODE == MODE_W8A8 ? 48 : 36;
-    int64_t tall = 400;
-    if (GMM1 && p.K > 2048) tall = MODE == MODE_W8A8 ? 200 : 160;
-    if (MODE == MODE_FP8 && !GMM1 && p.K <= 1024) tall = 800;
+    int64_t tall = many_tiles && !GMM1 ? 192 : 400;
+    if (GMM1 && p.K > 2048) {
+        if (p.K >= 6144 && rows <= 40 * e) {
+            const int64_t cus = cu_count(), round = cus > 0 ? (tiles + cus - 1) / cus * cus : tiles;
+            if (tiles * 8 >= round * 7) return 0;
+        }
+        if (rows > 87 * e && rows <= (MODE == MODE_W8A8 ? 108 : 112) * e) return 0;
+        tall = MODE == MODE_W8A8 ? 184 : (many_tiles ? 87 : 160);
+    }
+    if (MODE == MODE_FP8 && !GMM1) {
+        if (p.K > 8192) {
+            if (rows > 150 * e && rows <= 192 * e) return 0;
+            tall = 352;
+        }
+        if (p.K <= 1024 && !many_tiles) tall = 800;
+    }
     return rows <= low * e ? R::LOW : (rows <= tall * e ? R::TALL : 0);
 }
 

@@ -79,3 +79,52 @@ def test_8_bit_shapes(buf, edges, K, N):
     assert np.allclose(host(s2), r_s2, rtol=1e-4)
     assert_requant_close(zo.e4m3_to_f32(host(q2)).reshape(blocks) * host(s2)[:, :, None],
                          zo.e4m3_to_f32(r_q2).reshape(blocks) * r_s2[:, :, None], host(q2), r_q2)
+
+
+# averages either side of the lines that `stream_rows` draws by K and rows per expert; the second GEMM runs with the shorter K too
+LINES = [(2560, 87), (2560, 88), (2560, 108), (2560, 109), (2560, 112), (2560, 113), (2560, 160), (2560, 184), (2560, 185), (8704, 150),
+         (8704, 151), (8704, 192), (8704, 193), (8704, 352), (8704, 353)]
+
+
+@pytest.mark.parametrize("K,avg", LINES)
+def test_8_bit_lines_of_the_dispatch(buf, K, avg):
+    N, counts = 512, np.array([avg - 40, avg + 40, 2 * avg, 0], dtype=np.int64)
+    E, rows = len(counts), int(counts.sum())
+    assert rows == avg * E
+    a = rng(1).integers(-127, 128, (rows, K)).astype(np.int8)
+    xs = rng(2).uniform(0.005, 0.05, rows).astype(np.float32)
+    w = rng(3).integers(-128, 128, (E, K, N)).astype(np.int8)
+    ws = rng(4).uniform(0.0015, 0.0045, (E, N)).astype(np.float32)
+    packed = buf.prepack_weight(dev(w))
+    q2, s2, _ = gmm1(buf, dev(a), dev(xs), packed, dev(ws), counts, K, N, 1)
+    r_q2, r_s2 = zo.gmm1_swiglu_quant_w8a8(a, xs, w, ws, counts)[:2]
+    assert np.array_equal(host(s2).view(np.uint32), r_s2.view(np.uint32)) and np.array_equal(host(q2), r_q2)
+
+    a, sa, w, sw = fp8_operands(E, K, N, rows, 20)
+    packed = buf.prepack_weight(dev(w))
+    y = gmm2(buf, dev(a), dev(sa), packed, dev(sw), capi.DT_FP32, counts, K, N, 2)
+    assert_fp8_close(zo.bf16_to_f32(host(y)), zo.bf16_to_f32(zo.gmm2_fp8(a, sa, w, sw, counts)), "fp8 GEMM", FP8_GEMM_ELEM_TOL)
+    q2, s2, _ = gmm1(buf, dev(a), dev(sa), packed, dev(sw), counts, K, N, 2)
+    r_q2, r_s2, _ = zo.gmm1_swiglu_quant_fp8(a, sa, w, sw, counts)
+    blocks = (rows, N // 256, 128)
+    assert np.allclose(host(s2), r_s2, rtol=1e-4)
+    assert_requant_close(zo.e4m3_to_f32(host(q2)).reshape(blocks) * host(s2)[:, :, None],
+                         zo.e4m3_to_f32(r_q2).reshape(blocks) * r_s2[:, :, None], host(q2), r_q2)
+
+
+@pytest.mark.parametrize("avg", [192, 193])
+def test_many_tiles_are_the_same_rows_as_few(buf, avg):
+    """1024 experts of four channel tiles are many tiles, 64 are not: the second GEMM gives the same bits either way."""
+    K, N, E, part = 512, 1024, 1024, 64
+    counts = rng(5).multinomial(avg * part, np.full(part, 1.0 / part), size=E // part).reshape(-1).astype(np.int64)
+    rows = int(counts.sum())
+    a = torch.randint(-127, 128, (rows, K), dtype=torch.int8, device="cuda")
+    xs = torch.rand((rows,), device="cuda") + 0.5
+    w = torch.randint(-128, 128, (E, N, K), dtype=torch.int8, device="cuda")         # any bytes are a pre-packed weight
+    ws = torch.rand((E, N), device="cuda") + 0.5
+    whole = gmm2(buf, a, xs, w, ws, capi.DT_FP32, counts, K, N, 1)
+    off = np.concatenate([[0], np.cumsum(counts)])
+    for e in range(0, E, part):
+        r = slice(int(off[e]), int(off[e + part]))
+        got = gmm2(buf, a[r].contiguous(), xs[r].contiguous(), w[e:e + part], ws[e:e + part], capi.DT_FP32, counts[e:e + part], K, N, 1)
+        assert torch.equal(whole[r].view(torch.int16), got.view(torch.int16))
