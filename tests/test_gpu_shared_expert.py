@@ -1,6 +1,7 @@
 """A shared expert of the routed experts' width runs in their launches: every way the layout is worked out (inside the
 permute launch, from range histograms, from a launch of its own), x_active_mask, smooth scales and tensor lists, against
-the oracle, which runs it as a one-expert layer. A workspace without room for its rows gives the same results."""
+the oracle, which runs it as a one-expert layer; so does every kernel shape that its rows can bring a launch to. A
+workspace without room for its rows gives the same results."""
 import numpy as np
 import pytest
 import torch
@@ -26,6 +27,26 @@ def buf():
                                                       (1200, 256, 4, 8, 128, None, False), (1200, 256, 4, 8, 128, 0, True),
                                                       (1100, 256, 4, 8, 128, 1001, True), (600, 256, 8, 300, 128, 555, False)])
 def test_shared_expert_in_the_routed_launches(buf, mode, T, H, K, E, I, active, smooth):
+    check_shared_expert(buf, mode, T, H, K, E, I, active, smooth)
+
+
+# both tall tiles of the weight stream (150 and 711 rows per expert, the shared one's among them) and the staged kernel's
+# 320-row tile with the K of a prefill layer in both GEMMs (480 rows)
+@pytest.mark.parametrize("mode,T,H,K,E,I,active,smooth", [(0, 300, 512, 4, 8, 512, None, False), (2, 300, 512, 4, 8, 512, 200, False),
+                                                           (3, 300, 512, 4, 8, 512, None, True), (3, 1280, 512, 4, 8, 512, 1200, False),
+                                                           (0, 800, 7168, 2, 4, 2048, None, False), (2, 800, 7168, 2, 4, 2048, 777, False)])
+def test_shared_expert_in_tall_tiles(buf, mode, T, H, K, E, I, active, smooth):
+    check_shared_expert(buf, mode, T, H, K, E, I, active, smooth)
+
+
+@pytest.mark.parametrize("mode", [0, 2, 3])
+@pytest.mark.parametrize("T,active,smooth", [(1, None, False), (70, 37, True), (300, None, False)])
+def test_shared_expert_with_tensor_lists(buf, mode, T, active, smooth):
+    """The routed experts' operands as lists of tensors, the shared expert's a tensor each."""
+    check_shared_expert(buf, mode, T, 512, 4, 8, 512, active, smooth, lists=True)
+
+
+def check_shared_expert(buf, mode, T, H, K, E, I, active, smooth, lists=False):
     smooth = smooth and mode != 2
     x, ids, es, w1, s1, w2, s2 = fused_inputs(T, H, K, E, I, mode, 200 + mode)
     _, _, _, sw1, ss1, sw2, ss2 = fused_inputs(T, H, 1, 1, I, mode, 210 + mode)
@@ -41,7 +62,11 @@ def test_shared_expert_in_the_routed_launches(buf, mode, T, H, K, E, I, active, 
     if smooth:
         more.update(expert_smooth_scales=dev(sm), share_smooth_scales=dev(ssm[0]))
     seven = lambda: torch.full((T, H), 7.0, dtype=torch.bfloat16, device="cuda")
-    args = (dev(x, torch.bfloat16), dev(ids), pack(w1), dev(s1, sdt1), pack(w2), dev(s2, sdt2), dev(es), E)
+    routed = (pack(w1), dev(s1, sdt1), pack(w2), dev(s2, sdt2))
+    if lists:
+        routed = [[t[e].clone() for e in range(E)] for t in routed]
+        more["is_tensor_list"] = True
+    args = (dev(x, torch.bfloat16), dev(ids), *routed, dev(es), E)
     share = dict(share_gmm1_weight=pack(sw1), share_gmm1_scale=dev(ss1, sdt1), share_gmm2_weight=pack(sw2), share_gmm2_scale=dev(ss2, sdt2))
     out, shared, nums = buf.fused_deep_moe(*args, quant_mode=mode, out=seven(), share_out=seven(), **share, **more)
     untouched = host(torch.full((T - n, H), 7.0, dtype=torch.bfloat16))

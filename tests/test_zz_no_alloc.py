@@ -1,12 +1,13 @@
-"""The layout entry point that allocates nothing (zbalhip_dispatch_layout_static) against the one that takes
-the caller's scratch (zbalhip_dispatch_layout): same outputs, bit for bit, on two calls in a row, the second
-on a smaller input, so that whatever the first call left in the library's static scratch must not matter.
-Both are called through the C ABI (ctypes)."""
+"""The layout entry point without a scratch argument (zbalhip_dispatch_layout_static) against the one that takes the
+caller's scratch, as the reference does (zbalhip_dispatch_layout), and against the oracle: same outputs, bit for bit, on
+two calls in a row, the second on a smaller input. Neither keeps anything between calls, so calls on different streams
+need no order. Both are called through the C ABI (ctypes)."""
 import numpy as np
 import pytest
 import torch
 
 from memfabric_hybrid_amd import capi
+from oracle import oracle as zo
 from zbal_testlib import rng
 
 pytestmark = pytest.mark.gpu
@@ -15,7 +16,7 @@ MAX_BLOCKS = 50          # ZBALHIP_LAYOUT_MAX_BLOCKS
 
 
 def _layout_pair(lib, idx, experts, ranks):
-    """(with caller scratch, with the static scratch): each a tuple of the three outputs as numpy arrays"""
+    """(with the caller's scratch, without one): each a tuple of the three outputs as numpy arrays"""
     T, K = idx.shape
     d_idx = torch.from_numpy(idx).cuda()
     is64 = 1 if idx.dtype == np.int64 else 0
@@ -46,6 +47,8 @@ def test_static_layout_matches_scratch_layout_twice():
         want, got = _layout_pair(lib, idx, E, R)
         for w, g, name in zip(want, got, ("tokens_per_rank", "tokens_per_expert", "send_token_idx")):
             assert np.array_equal(w, g), name
+        for w, g, name in zip(zo.dispatch_layout(idx, E, R), got, ("tokens_per_rank", "tokens_per_expert", "send_token_idx")):
+            assert np.array_equal(w, g), name
         valid = (idx >= 0) & (idx < E)
         assert got[1].sum() == valid.sum()
         assert np.array_equal(got[2][~valid], np.full((~valid).sum(), -1, dtype=np.int32))
@@ -63,8 +66,8 @@ def test_static_layout_refuses_what_the_scratch_cannot_hold():
 
 
 def test_static_layout_calls_on_two_streams_take_turns():
-    """Calls issued back to back on two streams share the one static scratch: the library queues each behind the
-    one before (an event per GPU), so both give the caller-scratch results although their streams are not ordered."""
+    """Calls issued back to back on two streams that nothing orders give the same as one after the other: the layout has
+    no memory of its own that they could share."""
     lib = capi.load()
     torch.cuda.set_device(0)
     cases = []
