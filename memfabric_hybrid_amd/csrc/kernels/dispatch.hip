@@ -313,8 +313,8 @@ enum { LM_GIVEN = 0, LM_INLINE = 1, LM_TABLE = 2, LM_COUNTS = 3 };     /* where 
  * Notify and dispatch of a group of one rank in one launch: the offsets are the running sum of at most 1024 counts, which
  * every wave of the permute kernel works out for itself while its row is on its way (a launch of its own in front took
  * 2-5 us of the GPU and 3 us of the host: 24.3 -> 21.5 us for the whole exchange of 64 to 512 tokens). The first wave of
- * all writes what a notify launch would. Where the host waits for the counts a launch of its own still has them there
- * sooner (28 against 26 us).
+ * all writes what a notify launch would. Where the host waits for the counts, a launch of its own has them there sooner
+ * (26 us for that exchange, 28 with the notify riding along), and it is what runs then.
  */
 struct NotifyOut {
     const int32_t *counts;        /* [experts] */

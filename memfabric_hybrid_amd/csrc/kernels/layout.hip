@@ -688,7 +688,7 @@ extern "C" int32_t zbalhip_dispatch_layout_static(const void *topk_idx, int32_t 
 {
     if (!topk_idx || !tokens_per_rank || !tokens_per_expert || !send_token_idx) return ZBALHIP_INVALID;
     if (experts > ZBALHIP_LAYOUT_STATIC_MAX_EXPERTS) {
-        zbalhip_set_last_error("zbalhip_dispatch_layout_static: more experts than the static scratch holds (1024)");
+        zbalhip_set_last_error("zbalhip_dispatch_layout_static: more than 1024 experts (the limit of the static scratch that the layout once had)");
         return ZBALHIP_INVALID;
     }
     return zbalhip_dispatch_layout_in_rank(topk_idx, idx_is_i64, tokens, experts, topk, ranks, tokens_per_rank,
