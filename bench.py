@@ -64,8 +64,8 @@ def parse():
     ap.add_argument("--tokens", type=int, default=4096, help="development only; the reported workload is 4096")
     ap.add_argument("--cpu-sample-tokens", type=int, default=2560)
     ap.add_argument("--workload", choices=["prefill", "prefill_w8a8", "decode", "qwen_w4a8", "reduce"], default="prefill",
-                    help="prefill = the headline fp8 MoE layer (default); prefill_w8a8 = the same shape in W8A8 (profiling: no "
-                         "BASELINE configuration); decode = 128-token W8A8 layer with Zipf routing; qwen_w4a8 = 16384-token "
+                    help="prefill = the headline fp8 MoE layer (default); prefill_w8a8 = the same shape in W8A8 "
+                         "(profiling); decode = 128-token W8A8 layer with Zipf routing; qwen_w4a8 = 16384-token "
                          "W4A8 layer; reduce = the 8 x 256 MiB local reduction")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--equal-rows", action="store_true",
@@ -110,7 +110,7 @@ def other_workloads(args, torch, np, capi, buf):
     out = []
     red = bench_reduce(args, torch, np, capi, buf)
     for name, v in red["variants"].items():
-        out.append({"workload": "local reduce-scatter shard, 8 x 256 MiB %s (BASELINE configs[3])" % name, "ms": v["ms"],
+        out.append({"workload": "local reduce-scatter shard, 8 x 256 MiB %s" % name, "ms": v["ms"],
                     "achieved": v["gbs"], "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": v["gbs"] / PEAK_HBM_GBS,
                     "exact": v["exact"]})
     torch.cuda.empty_cache()
@@ -128,14 +128,14 @@ def other_workloads(args, torch, np, capi, buf):
 
 # mode: zbal_fused_deep_moe quantMode (1 = W8A8, 2 = fp8 block-scaled, 3 = W4A8)
 MOE_WORKLOADS = {
-    "prefill": dict(name="DeepSeek-V3-style prefill share (BASELINE configs[1])", T=4096, H=7168, E=32, K=8, I=2048,
+    "prefill": dict(name="DeepSeek-V3-style prefill share", T=4096, H=7168, E=32, K=8, I=2048,
                     mode=2, zipf=None, quant="fp8 e4m3, act 1x128, weight 128x128", dtype="fp8_e4m3"),
-    "prefill_w8a8": dict(name="the prefill share's shape in W8A8 (profiling; not a BASELINE configuration)", T=4096, H=7168, E=32,
+    "prefill_w8a8": dict(name="the prefill share's shape in W8A8 (profiling)", T=4096, H=7168, E=32,
                          K=8, I=2048, mode=1, zipf=None, quant="W8A8 int8, per-token act, per-channel weight scales",
                          dtype="int8"),
-    "decode": dict(name="low-latency decode share (BASELINE configs[2])", T=128, H=7168, E=32, K=8, I=2048,
+    "decode": dict(name="low-latency decode share", T=128, H=7168, E=32, K=8, I=2048,
                    mode=1, zipf=1.2, quant="W8A8 int8, per-token act, per-channel weight scales", dtype="int8"),
-    "qwen_w4a8": dict(name="Qwen3-MoE-style W4A8 layer (BASELINE configs[4])", T=16384, H=4096, E=128, K=8, I=1536,
+    "qwen_w4a8": dict(name="Qwen3-MoE-style W4A8 layer", T=16384, H=4096, E=128, K=8, I=1536,
                       mode=3, zipf=None, quant="W4A8: int8 per-token act, int4 g128 weights, fp16 group scales",
                       dtype="int8"),
 }
@@ -278,7 +278,8 @@ def bench_moe(args, torch, np, capi, buf, workload):
                     "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": wbytes1 / t1 / 1e9 / PEAK_HBM_GBS, "traffic": None,
                     "experts_with_tokens": touched}
     else:
-        kname = "grouped_gemm_dma_kernel<%s, gmm1>" % {1: "int8", 2: "fp8", 3: "w4a8"}[mode]
+        kname = {1: "grouped_gemm_dma_kernel<int8, gmm1>", 2: "grouped_gemm_dma_kernel<fp8, gmm1>",
+                 3: "grouped_gemm_stream_kernel<w4a8, gmm1>"}[mode]
         routed = workload in ("prefill", "qwen_w4a8") and T == cfg["T"] and not args.equal_rows
         roofline = {"kernel": kname, "bound": "mfma", "achieved": flops1 / t1 / 1e12,
                     "peak": PEAK_FP8_TFLOPS, "unit": "TFLOP/s" if mode == 2 else "TOP/s",
@@ -340,7 +341,7 @@ def bench_moe(args, torch, np, capi, buf, workload):
 
 
 def bench_reduce(args, torch, np, capi, buf):
-    """one rank's reduce-scatter shard, 8 peer buffers of 256 MiB held as local HBM
+    """One rank's reduce-scatter shard, 8 peer buffers of 256 MiB held as local HBM
     allocations, through zbal_reduce_scatter. Algorithmic bytes = (8 + 1) x 256 MiB = 2.416 GB per launch."""
     from memfabric_hybrid_amd.operators import create_group, destroy_group
     lib = buf.lib
@@ -386,7 +387,7 @@ def bench_reduce(args, torch, np, capi, buf):
     line = {"metric": "local N-buffer reduce GB/s at 1 GPU", "value": b["gbs"], "unit": "GB/s", "n_gpus": 1,
             "steps": args.steps, "warmup": args.warmup, "ms_per_step": b["ms"], "higher_is_better": True,
             "scaling": "weak", "vs_baseline": None, "dtype": "bf16 in, fp32 accumulate, bf16 out", "data": "synthetic",
-            "config": {"workload": "local reduce-scatter shard (BASELINE configs[3])", "buffers": R,
+            "config": {"workload": "local reduce-scatter shard", "buffers": R,
                        "bytes_per_buffer": nbytes},
             "roofline": {"kernel": "reduce_kernel<bf16, sum, 8>", "bound": "hbm", "achieved": b["gbs"], "peak": PEAK_HBM_GBS,
                          "unit": "GB/s", "frac": b["gbs"] / PEAK_HBM_GBS, "traffic": measured_traffic("reduce_8x256MiB_bf16")},

@@ -116,7 +116,7 @@ __device__ __forceinline__ int32_t zb_rint_i8(float v)
 /*
  * exp() of the SwiGLU epilogue: Cody-Waite reduction by ln2, a degree-6
  * polynomial in fmaf form and scaling by two exact powers of two. The same
- * operation sequence is what the CPU checker evaluates, so both sides agree
+ * operation sequence is what the CPU oracle evaluates, so both sides agree
  * bit for bit (the hardware v_exp_f32 is an approximation and would not).
  */
 __device__ __forceinline__ float zb_expf(float x)

@@ -1,7 +1,7 @@
 /*
  * TEST INFRASTRUCTURE — CPU restatement of the zbal MoE / reduce hot path.
  *
- * This file is the checker that the parity tests, the smoke test and the
+ * This file is the oracle that the parity tests, the smoke test and the
  * cpu_baseline leg of the benchmark compare the HIP library against. Nothing
  * in the shipped library includes, links or calls it.
  *

@@ -3,7 +3,7 @@
 W8A8 and W4A8: the integer contraction is exact and the epilogues evaluate the oracle's operation
 sequence, so quantised bytes, scales and bf16 rows must match bit for bit. fp8 block-scaled: the MFMA's
 internal summation order differs from the oracle's, so outputs are compared within max relative error
-2e-2 (north star) and quantised bytes after dequantisation."""
+2e-2 and quantised bytes after dequantisation."""
 import ctypes
 
 import numpy as np
@@ -390,7 +390,7 @@ def test_fused_moe_fp8(buf, T, H, K, E, I):
     assert np.array_equal(nums, counts)
     f, r = zo.bf16_to_f32(out), zo.bf16_to_f32(ref)
     assert np.abs(r).max() > 1e-3                        # the comparison is not vacuous
-    print("fp8 errors (max-normalised, element-wise):", assert_fp8_close(f, r, layer=True))     # north star tolerance
+    print("fp8 errors (max-normalised, element-wise):", assert_fp8_close(f, r, layer=True))
     assert calc_diff(f, r) < 1e-4
 
 
@@ -791,7 +791,7 @@ def test_w8a8_gemms_random_row_counts_bit_exact(buf, seed):
             assert np.array_equal(host(y), zo.grouped_gemm_w8a8_dequant(a, xs, w, ws, counts)), what
 
 
-# ---- BASELINE configuration 1 end to end --------------------------------------------------------------------------------
+# ---- the small CPU-reference layer end to end --------------------------------------------------------------------------------
 
 def test_config1_small_moe_layer(buf):
     """256 tokens x 1024, 8 experts, softmax top-2 router, int8 per-token activations, one int8 GEMM 1024->2048

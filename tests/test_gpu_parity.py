@@ -34,7 +34,7 @@ def test_router(buf, T, E, K):
     idx, w = buf.topk_route(dev(logits), K)
     ridx, rw = zo.topk_route(logits, K)
     assert np.array_equal(host(idx), ridx)
-    assert np.allclose(host(w), rw, rtol=1e-6, atol=0)     # north star: weights within 1e-6 relative
+    assert np.allclose(host(w), rw, rtol=1e-6, atol=0)     # weights within 1e-6 relative
 
 
 @pytest.mark.parametrize("T,E,K,style", [(1000, 100, 32, "ties"), (1000, 129, 30, "ties"), (3000, 31, 24, "spread"),
@@ -379,7 +379,7 @@ def test_reduce_full_size_sampled_windows(buf):
 
 
 def test_reduce_scatter_and_all_reduce_over_peer_windows(buf):
-    """cfg4 shape in miniature: 8 'ranks' as local windows, this rank reduces its slice of every peer's buffer."""
+    """the 8 x 256 MiB reduction in miniature: 8 'ranks' as local windows, this rank reduces its slice of every peer's buffer."""
     from memfabric_hybrid_amd.operators import create_group, destroy_group
     lib = buf.lib
     R, me = 8, 5
@@ -406,7 +406,7 @@ def test_reduce_scatter_and_all_reduce_over_peer_windows(buf):
             assert lib.zbal_all_reduce(wins[me].data_ptr(), full.data_ptr(), tmp.data_ptr(), R * n, dt, capi.REDUCE_SUM,
                                        comm, capi.stream_ptr()) == 0
             assert np.array_equal(host(full), zo.reduce(ins, dt, capi.REDUCE_SUM))
-            if dt == capi.DT_FP32:     # north star: fp32 within 1e-6 relative of the exact sum
+            if dt == capi.DT_FP32:     # fp32 within 1e-6 relative of the exact sum
                 exact = np.sum(np.stack(ins).astype(np.float64), 0)
                 assert np.allclose(host(full), exact, rtol=1e-6, atol=1e-6)
             # a send buffer outside this rank's window is refused
