@@ -94,7 +94,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     auto rows_of = [&](int base, int &lo, int &hi) {
         lo = hi = 0;
         const int e = nth_expert(base + lane);
-        if (base + lane < E) { lo = first_row_of(p, e); hi = p.row_off[e + 1]; }
+        if (base + lane < E) { lo = first_row_of<SHARED_IN_REGISTERS>(p, e); hi = p.row_off[e + 1]; }
     };
     int lo[2], hi[2];                                              /* the first 128 experts, one per lane each: one round trip for all of them */
     rows_of(0, lo[0], hi[0]);
@@ -139,7 +139,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     const int last_rel = row_end - 1 - row_begin;
 
     /* the wave's two 16-channel sub-tiles: block rows r0, r0 + 16 .. of one 128-channel block, or the same rows of a gate and an up block */
-    const uint8_t *wb = weights_of<uint8_t>(p, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
+    const uint8_t *wb = weights_of<uint8_t, SHARED_IN_REGISTERS>(p, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
     const int col0 = GMM1 ? n_tile : n_tile * 2, col1 = GMM1 ? I / 128 + n_tile : n_tile * 2 + 1;
     const uint8_t *w_src[NT];
 #pragma unroll
@@ -196,7 +196,7 @@ grouped_gemm_stream_kernel(GemmParams p)
                     lds_addr(lds_sa) + (b * S::SA_FLOATS + s * S::SA_ROWS + (TM > 64 ? (wave / PF & 1) * 64 : 0)) * 4);
         }
         if (MODE == MODE_W4A8) {
-            const uint16_t *gs = scales_of<uint16_t>(p, expert, (int64_t)KB * p.N);
+            const uint16_t *gs = scales_of<uint16_t, SHARED_IN_REGISTERS>(p, expert, (int64_t)KB * p.N);
             const int sg = (wave >> 1) & (PF - 1);
             gs += (int64_t)(kb0 + sg) * p.N + ((wave & 1) ? col1 : col0) * 128;
             dma4_sv(reinterpret_cast<const float *>(gs), lane_x * 4u, lds_addr(lds_gs) + b * S::GS_BYTES + sg * (BN * 2) + (wave & 1) * 256);
@@ -213,17 +213,17 @@ grouped_gemm_stream_kernel(GemmParams p)
         if (wave >= 4) {
             const int w4 = wave - 4;
             if (GMM1 || !p.wscale_is_bf16) {
-                const float *wsb = scales_of<float>(p, expert, p.N);
+                const float *wsb = scales_of<float, SHARED_IN_REGISTERS>(p, expert, p.N);
                 const float *src = !GMM1 ? wsb + n_tile * BN + w4 * 64 : (w4 < 2 ? wsb + n_tile * 128 + w4 * 64 : wsb + I + n_tile * 128 + (w4 - 2) * 64);
                 dma4_sv(src, lane * 4u, dst0 + w4 * 256);
             } else if (w4 < 2) {
-                const uint16_t *wsb = scales_of<uint16_t>(p, expert, p.N);
+                const uint16_t *wsb = scales_of<uint16_t, SHARED_IN_REGISTERS>(p, expert, p.N);
                 dma4_sv(reinterpret_cast<const float *>(wsb + n_tile * BN + w4 * 128), lane * 4u, dst0 + w4 * 256);
             }
         }
     } else if constexpr (MODE == MODE_FP8) {
         const int sw_stride = p.N / 128;
-        const float *base = scales_of<float>(p, expert, (int64_t)KB * sw_stride);
+        const float *base = scales_of<float, SHARED_IN_REGISTERS>(p, expert, (int64_t)KB * sw_stride);
         for (int b = (wave & 3) * 64; b < KB; b += 256) {
             if (b + lane < KB)
                 dma4_sv(base + (wave < 4 ? col0 : col1), (uint32_t)(b + lane) * (uint32_t)sw_stride * 4u,
@@ -401,7 +401,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     tc.n_tile = n_tile;
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));               /* as in the other kernel: nothing of the epilogue's stays live across the K loop */
-    epilogue<MODE, GMM1, OUT_DT, 1, MTM, NT>(p, tc, accf, acci, row_begin, row_end, 0, wave, lane_e, lds_rowmax, TM, lds_es);
+    epilogue<MODE, GMM1, OUT_DT, 1, MTM, NT, SHARED_IN_REGISTERS>(p, tc, accf, acci, row_begin, row_end, 0, wave, lane_e, lds_rowmax, TM, lds_es);
 }
 
 } // namespace

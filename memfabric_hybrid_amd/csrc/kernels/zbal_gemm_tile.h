@@ -56,19 +56,41 @@ __device__ __forceinline__ const T *expert_base(const void *base, int is_list, i
     return (const T *)base + (int64_t)expert * stride_elems;
 }
 
-template <typename T> __device__ __forceinline__ const T *weights_of(const GemmParams &p, int expert, int64_t stride)
+/*
+ * How a kernel knows of a shared expert. The staged kernel's K loop takes all scalar registers, and the shared expert's
+ * tensors, kept in some through it, pushed others out into lanes of vector registers (9 to 31 more of them; fp8 2048 rows, 256-row
+ * shape: first GEMM +3.5 %, second +1.5 %): it reads them where a tile of the shared expert needs them, from the launch's
+ * arguments in memory. The streaming kernel has registers left, and its one tile would wait for the reads (W4A8 +0.5 %).
+ */
+enum Shared { SHARED_NONE, SHARED_ON_DEMAND, SHARED_IN_REGISTERS };
+
+/* GemmParams is the kernels' only parameter */
+using LaunchArgs = const GemmParams __attribute__((address_space(4))) *;
+__device__ __forceinline__ LaunchArgs launch_args()
 {
-    if (expert == p.shared_index) return (const T *)p.shared_w;
+    auto *args = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));                     /* not hoisted */
+    return (LaunchArgs)args;
+}
+
+template <Shared SH> __device__ __forceinline__ bool is_shared(const GemmParams &p, int expert)
+{
+    return SH != SHARED_NONE && expert == p.shared_index;
+}
+template <typename T, Shared SH> __device__ __forceinline__ const T *weights_of(const GemmParams &p, int expert, int64_t stride)
+{
+    if (is_shared<SH>(p, expert)) return (const T *)(SH == SHARED_ON_DEMAND ? launch_args()->shared_w : p.shared_w);
     return expert_base<T>(p.w, p.w_is_list, expert, stride);
 }
-template <typename T> __device__ __forceinline__ const T *scales_of(const GemmParams &p, int expert, int64_t stride)
+template <typename T, Shared SH> __device__ __forceinline__ const T *scales_of(const GemmParams &p, int expert, int64_t stride)
 {
-    if (expert == p.shared_index) return (const T *)p.shared_wscale;
+    if (is_shared<SH>(p, expert)) return (const T *)(SH == SHARED_ON_DEMAND ? launch_args()->shared_wscale : p.shared_wscale);
     return expert_base<T>(p.wscale, p.w_is_list, expert, stride);
 }
-__device__ __forceinline__ int first_row_of(const GemmParams &p, int expert)
+template <Shared SH> __device__ __forceinline__ int first_row_of(const GemmParams &p, int expert)
 {
-    return expert == p.shared_index ? p.shared_row : p.row_off[expert];
+    if constexpr (SH == SHARED_ON_DEMAND) return is_shared<SH>(p, expert) ? launch_args()->shared_row : p.row_off[expert];
+    else return is_shared<SH>(p, expert) ? p.shared_row : p.row_off[expert];
 }
 
 struct TileCoord {
@@ -96,7 +118,7 @@ __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float 
  * A wave's NT channel sub-tiles are 16 * NT consecutive channels (GMM1: 8 * NT gate and the matching 8 * NT up columns).
  * `lds_rowmax` is [16 / NT][tile_rows] floats of scratch for the row maxima of the waves' channel ranges (GMM1 only).
  */
-template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT>
+template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT, Shared SH>
 __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &tc, f32x4 (&accf)[MTM][NT],
                                          i32x4 (&acci)[MTM][NT], int row_begin, int row_end, int wm, int wn, int lane,
                                          float *lds_rowmax, int tile_rows, const float *es)
@@ -114,7 +136,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
     const int I = p.N / 2;
     const int q8 = (lane >> 4) * 8;
     if constexpr (!GMM1) {
-        uint16_t *y = (uint16_t *)(tc.expert == p.shared_index ? p.shared_out : p.out);
+        uint16_t *y = (uint16_t *)p.out;
+        if (is_shared<SH>(p, tc.expert)) y = (uint16_t *)(SH == SHARED_ON_DEMAND ? launch_args()->shared_out : p.shared_out);
 #pragma unroll
         for (int mt = 0; mt < MTM; ++mt) {
             const int row = row_begin + (RG * mt + wm) * 16 + frag_row;

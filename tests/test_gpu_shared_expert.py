@@ -2,13 +2,16 @@
 permute launch, from range histograms, from a launch of its own), x_active_mask, smooth scales and tensor lists, against
 the oracle, which runs it as a one-expert layer; so does every kernel shape that its rows can bring a launch to. A
 workspace without room for its rows gives the same results."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+from memfabric_hybrid_amd import capi
 from memfabric_hybrid_amd.operators import OperatorBuffer
 from oracle import oracle as zo
-from test_gpu_gemm import fused_inputs
+from test_gpu_gemm import fp8_operands, fused_inputs, gmm1, gmm2, row_off_dev
 from zbal_testlib import dev, host, max_rel_err, rng
 
 pytestmark = pytest.mark.gpu
@@ -86,3 +89,37 @@ def check_shared_expert(buf, mode, T, H, K, E, I, active, smooth, lists=False):
     ws = torch.empty((tight,), dtype=torch.uint8, device="cuda")
     out2, shared2, _ = buf.fused_deep_moe(*args, quant_mode=mode, out=seven(), share_out=seven(), workspace=ws, **share, **more)
     assert np.array_equal(host(out2), host(out)) and np.array_equal(host(shared2), host(shared))
+
+
+class SharedExpert(ctypes.Structure):
+    """zbalhip_shared_expert_t"""
+    _fields_ = [("weight", ctypes.c_void_p), ("scale", ctypes.c_void_p), ("rows", ctypes.c_int64), ("out", ctypes.c_void_p)]
+
+
+@pytest.mark.parametrize("R,S", [(2000, 1600), (1601, 1537)])
+def test_shared_expert_in_the_256_row_shape(buf, R, S):
+    """More than 1536 rows per expert fp8, which only a caller of the kernel ABI brings there with a shared expert: the
+    kernel that knows of one gives the bits of the kernel that does not, run for either expert by itself."""
+    K, N = 384, 512
+    a, sa, w, sw = fp8_operands(2, K, N, R + S, 40)
+    a, sa, w, sw = dev(a), dev(sa), buf.prepack_weight(dev(w)), dev(sw)
+    off = row_off_dev([R, S])
+    alone = [(slice(0, R), 0), (slice(R, R + S), 1)]
+    y, y_shared = torch.empty((R, N), dtype=torch.bfloat16, device="cuda"), torch.empty((S, N), dtype=torch.bfloat16, device="cuda")
+    sh = SharedExpert(w[1].data_ptr(), sw[1].data_ptr(), S, y_shared.data_ptr())
+    capi.check("gmm2", buf.lib.zbalhip_gmm2_dequant_shared(
+        a.data_ptr(), sa.data_ptr(), w.data_ptr(), sw.data_ptr(), capi.DT_FP32, off.data_ptr(), 1, R, K, N, 2, capi.DT_BF16,
+        y.data_ptr(), ctypes.byref(sh), capi.stream_ptr()))
+    q2 = torch.empty((R + S, N // 2), dtype=torch.uint8, device="cuda")
+    s2 = torch.empty((R + S, N // 256), dtype=torch.float32, device="cuda")
+    sh.out = None
+    capi.check("gmm1", buf.lib.zbalhip_gmm1_swiglu_quant_shared(
+        a.data_ptr(), sa.data_ptr(), w.data_ptr(), sw.data_ptr(), off.data_ptr(), 1, R, K, N, 2, q2.data_ptr(), s2.data_ptr(), None,
+        ctypes.byref(sh), capi.stream_ptr()))
+    for (r, e), got in zip(alone, (y, y_shared)):
+        n = r.stop - r.start
+        one = (buf, a[r].contiguous(), sa[r].contiguous(), w[e:e + 1], sw[e:e + 1])
+        want = gmm2(*one, capi.DT_FP32, [n], K, N, 2)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+        want_q2, want_s2, _ = gmm1(*one, [n], K, N, 2)
+        assert torch.equal(q2[r], want_q2) and torch.equal(s2[r], want_s2)
