@@ -777,7 +777,7 @@ public:
             activeMask = (const uint8_t *)xActiveMask->data;
         }
         FusedWorkspace ws;
-        ZBAL_VALIDATE_RETURN(PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, false, &ws), op << " failed as the shapes are invalid",
+        ZBAL_VALIDATE_RETURN(PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, false, true, &ws), op << " failed as the shapes are invalid",
                              Z_INVALID_PARAM);
         ZBAL_VALIDATE_RETURN(workspace->data != nullptr && (reinterpret_cast<uintptr_t>(workspace->data) & 255u) == 0,
                              op << " failed as the workspace is null or not 256-byte aligned", Z_INVALID_PARAM);
@@ -796,8 +796,10 @@ public:
         FusedWorkspace along;
         const bool ride = shared && T <= MostRidingTokens(K, E) && SN1 == N1 && shareWscale2Dt == wscale2Dt &&
                           (smooth != nullptr) == (shareSmooth != nullptr) &&
-                          PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, true, &along) && wsBytes >= along.total;
+                          PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, true, true, &along) && wsBytes >= along.total;
         if (ride) ws = along;
+        FusedWorkspace apart;
+        if (PlanFusedWorkspace(T, H, K, E, N1, SN1, quantMode, ride, false, &apart) && wsBytes >= apart.total) ws = apart;
         uint8_t *base = (uint8_t *)workspace->data;
         const int64_t rows = T * K, allRows = rows + (ride ? T : 0);
         void *q1 = base + ws.q1;
@@ -910,7 +912,7 @@ CommunicatorPtr MakeGpuCommunicator(const GroupInfo &info) { return std::make_sh
 
 
 bool PlanFusedWorkspace(int64_t tokens, int64_t hidden, int64_t topk, int64_t experts, int64_t n1, int64_t shareN1,
-                        int64_t quantMode, bool ridesAlong, FusedWorkspace *ws)
+                        int64_t quantMode, bool ridesAlong, bool packed, FusedWorkspace *ws)
 {
     if (tokens < 0 || hidden <= 0 || topk <= 0 || experts <= 0 || n1 <= 0 || shareN1 < 0 || quantMode < 0 || quantMode > 3)
         return false;
@@ -930,17 +932,19 @@ bool PlanFusedWorkspace(int64_t tokens, int64_t hidden, int64_t topk, int64_t ex
     ws->layout_scratch = take((uint64_t)ZBALHIP_LAYOUT_MAX_BLOCKS * E * 4);
     ws->q2 = take(both(all * I, T * SI));
     ws->scale2 = take(both(all * (fp8 ? (I + 127) / 128 : 1), T * (fp8 ? (SI + 127) / 128 : 1)) * 4);
-    /*
-     * y is first written by the second GEMM, when the first GEMM's inputs and the requantisation's fp32 values have had
-     * their last reader: it takes their place. (16384 tokens x 8 picks, 4096 -> 1536, W4A8: 1.55 GB instead of 2.62 side by side.)
-     */
-    ws->y = off;
-    ws->endY = Align256(off + rows * H * 2);
     ws->q1 = take(all * H);
     ws->xs = take(all * (fp8 ? H / 128 : 1) * 4);
+    /*
+     * y is first written by the second GEMM, when the requantisation has had the first GEMM's fp32 values: packed, it takes
+     * their place (128 tokens x 8 picks of 7168, W8A8: 24.1 MB instead of 32.5). Its stores are then 0.6 us slower for one token and
+     * 1.2 for 509, so that is for workspaces without room for both.
+     */
+    const uint64_t start = off;
     ws->sgl = fp8 ? off : take(both(all * (I + 1), T * (SI + 1)) * 4);
-    ws->end1 = off;
-    ws->total = std::max(ws->end1, ws->endY);
+    const uint64_t end = off;
+    if (packed) off = start;
+    ws->y = take(rows * H * 2);
+    ws->total = std::max(off, end);
     return true;
 }
 
@@ -955,14 +959,11 @@ uint64_t FusedWorkspaceBytes(int64_t tokens, int64_t hidden, int64_t topk, int64
                              int64_t quantMode)
 {
     FusedWorkspace ws, along;
-    if (!PlanFusedWorkspace(tokens, hidden, topk, experts, n1, shareN1, quantMode, false, &ws)) return 0;
+    if (!PlanFusedWorkspace(tokens, hidden, topk, experts, n1, shareN1, quantMode, false, false, &ws)) return 0;
     const int64_t most = MostRidingTokens(topk, experts), riding = tokens < most ? tokens : most;
-    if (riding <= 0 || (shareN1 != 0 && shareN1 != n1) ||
-        !PlanFusedWorkspace(riding, hidden, topk, experts, n1, shareN1, quantMode, true, &along) || along.total <= ws.total)
-        return ws.total;
-    /* with no shared expert named, the room for one comes out of what y shares with the first GEMM's regions, or is left out */
-    const uint64_t shared = std::min(ws.end1, ws.endY) - ws.y;
-    return shareN1 == 0 && along.total - ws.total > shared ? ws.total : along.total;
+    if (shareN1 == n1 && riding > 0 && PlanFusedWorkspace(riding, hidden, topk, experts, n1, shareN1, quantMode, true, true, &along))
+        return std::max(ws.total, along.total);
+    return ws.total;
 }
 
 } // namespace zbal

@@ -246,21 +246,21 @@ bool SharedExpertArgsConsistent(const char *op, const zbal_tensor_info_t *shareG
 /* Layout of the fused operator's workspace; one function so that sizing and carving cannot diverge. */
 struct FusedWorkspace {
     uint64_t q1, xs, expand_idx, counts, row_off, layout_scratch, q2, scale2, sgl, y, total;
-    uint64_t end1, endY;      /* q1, xs and sgl lie in [y, end1), y in [y, endY) */
 };
 /*
  * shareN1 = output width of the shared expert's first GEMM, 0 without a shared expert.
  * ridesAlong: with room for a shared expert's rows behind the routed ones (shareN1 == n1), so that it runs in the routed
  * experts' launches. Without: it takes turns with them in the same regions.
+ * packed: y in the place of the int modes' fp32 values.
  */
 bool PlanFusedWorkspace(int64_t tokens, int64_t hidden, int64_t topk, int64_t experts, int64_t n1, int64_t shareN1,
-                        int64_t quantMode, bool ridesAlong, FusedWorkspace *ws);
+                        int64_t quantMode, bool ridesAlong, bool packed, FusedWorkspace *ws);
 /* the largest batch whose shared expert runs in the routed experts' launches (up to 640 routed rows per expert) */
 int64_t MostRidingTokens(int64_t topk, int64_t experts);
 /*
- * What a caller is told to provide: enough for this batch and for every smaller one with its shared expert riding along
- * where it does. With shareN1 == 0 that room is there as well where it takes no more than the regions laid side by side
- * would (a caller may size its workspace before it knows of the shared expert). 0 on invalid input.
+ * What a caller is told to provide: the regions of the routed rows side by side, which hold a riding shared expert's rows too
+ * when packed (int modes; T rows more in fp8, if the shared expert is named), for this batch and for every smaller one. 0 on
+ * invalid input.
  */
 uint64_t FusedWorkspaceBytes(int64_t tokens, int64_t hidden, int64_t topk, int64_t experts, int64_t n1, int64_t shareN1,
                              int64_t quantMode);

@@ -43,13 +43,19 @@ def test_shared_expert_in_tall_tiles(buf, mode, T, H, K, E, I, active, smooth):
 
 
 @pytest.mark.parametrize("mode", [0, 2, 3])
+@pytest.mark.parametrize("T,active,smooth", [(1, None, False), (70, 37, True), (300, None, False), (1200, 1100, False)])
+def test_shared_expert_in_the_smallest_workspace(buf, mode, T, active, smooth):
+    check_shared_expert(buf, mode, T, 512, 4, 8, 256, active, smooth, smallest=True)
+
+
+@pytest.mark.parametrize("mode", [0, 2, 3])
 @pytest.mark.parametrize("T,active,smooth", [(1, None, False), (70, 37, True), (300, None, False)])
 def test_shared_expert_with_tensor_lists(buf, mode, T, active, smooth):
     """The routed experts' operands as lists of tensors, the shared expert's a tensor each."""
     check_shared_expert(buf, mode, T, 512, 4, 8, 512, active, smooth, lists=True)
 
 
-def check_shared_expert(buf, mode, T, H, K, E, I, active, smooth, lists=False):
+def check_shared_expert(buf, mode, T, H, K, E, I, active, smooth, lists=False, smallest=False):
     smooth = smooth and mode != 2
     x, ids, es, w1, s1, w2, s2 = fused_inputs(T, H, K, E, I, mode, 200 + mode)
     _, _, _, sw1, ss1, sw2, ss2 = fused_inputs(T, H, 1, 1, I, mode, 210 + mode)
@@ -84,11 +90,26 @@ def check_shared_expert(buf, mode, T, H, K, E, I, active, smooth, lists=False):
                 assert max_rel_err(zo.bf16_to_f32(host(got)[:n]), zo.bf16_to_f32(want)) < 2e-2
             else:
                 assert np.array_equal(host(got)[:n], want)
-    # no room for its rows: it takes turns with the routed experts
+    # a byte less: packed more tightly, or without room for its rows, when it takes turns with the routed experts
     tight = buf.fused_workspace_bytes(T, H, K, E, 2 * I, mode, 2 * I) - 1
-    ws = torch.empty((tight,), dtype=torch.uint8, device="cuda")
-    out2, shared2, _ = buf.fused_deep_moe(*args, quant_mode=mode, out=seven(), share_out=seven(), workspace=ws, **share, **more)
+    run = lambda ws: buf.fused_deep_moe(*args, quant_mode=mode, out=seven(), share_out=seven(), workspace=ws, **share, **more)
+    out2, shared2, _ = run(torch.empty((tight,), dtype=torch.uint8, device="cuda"))
     assert np.array_equal(host(out2), host(out)) and np.array_equal(host(shared2), host(shared))
+    if not smallest:
+        return
+    # the smallest that is accepted: turns, in every mode
+    whole, low, high = torch.empty((tight,), dtype=torch.uint8, device="cuda"), 0, tight
+    while high - low > 1:
+        mid = (low + high) // 2
+        try:
+            out3, shared3, _ = run(whole[:mid])
+            high = mid
+        except capi.ZbalError:
+            low = mid
+    out3, shared3, _ = run(whole[:high])
+    assert np.array_equal(host(out3), host(out)) and np.array_equal(host(shared3), host(shared))
+    # no room for its rows in q1 and q2 (each rounded up to 256 bytes)
+    assert high <= buf.fused_workspace_bytes(T, H, K, E, 2 * I, mode, 2 * I) - T * (H + I) + 2 * 255
 
 
 class SharedExpert(ctypes.Structure):
