@@ -142,6 +142,35 @@ __device__ __forceinline__ float zb_expf(float x)
 }
 
 /*
+ * g / (1 + zb_expf(-g)) for |g| <= 80, bit for bit (compared for every such float on gfx950; only -0 comes out as +0): the
+ * same reduction and polynomial, where exp(-g) is a normal number, so one addition to the exponent scales it, rounding to
+ * an integer is adding and subtracting 1.5 * 2^23, and the quotient needs neither range scaling nor a second correction.
+ * 17 vector instructions without a branch, so the four values of a lane overlap; the general form takes about 50, and its
+ * three range checks are branches that run one value after the other. Layers: W4A8 16384 tokens over 128 experts of
+ * 4096 x 3072 3.60 -> 3.53 ms, W8A8 8192 tokens 1.65 -> 1.61; W8A8 4096 tokens over 32 of 7168 x 4096 1.61 -> 1.59.
+ */
+constexpr float kSiluNear = 80.0f;
+__device__ __forceinline__ float zb_silu_near(float g)
+{
+    constexpr float MAGIC = 12582912.0f;
+    const float t = g * -1.44269504088896341f + MAGIC;
+    const float n = t - MAGIC;
+    float r = __builtin_fmaf(n, -0.693145751953125f, -g);
+    r = __builtin_fmaf(n, -1.42860682030941723e-06f, r);
+    float p = 1.3888889e-03f;
+    p = __builtin_fmaf(p, r, 8.3333333e-03f);
+    p = __builtin_fmaf(p, r, 4.1666668e-02f);
+    p = __builtin_fmaf(p, r, 1.6666667e-01f);
+    p = __builtin_fmaf(p, r, 0.5f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    const float d = 1.0f + __uint_as_float((__float_as_uint(t) << 23) + __float_as_uint(p));
+    const float y = __builtin_amdgcn_rcpf(d);
+    const float q = g * y;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, g), y, q);
+}
+
+/*
  * Expert ids, read where the caller has them: an int32 array (stride 1) or an int64 one (stride 2), so that int64 ids
  * need no converting launch in front of the kernel. IDS_FULL: an int64 id outside of int32 is no expert (-1);
  * otherwise its low word counts, which is what converting the array first would have left.

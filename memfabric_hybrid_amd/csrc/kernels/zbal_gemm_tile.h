@@ -218,16 +218,32 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
 #pragma unroll
                     for (int i = 0; i < 4; ++i) { g[i] = accf[mt][nt][i] * xs; u[i] = accf[mt][nt + UP][i] * xs; }
                 }
+                /*
+                 * The int modes' exact exp and division: a wave whose values are all of ordinary size takes the short form
+                 * (any NaN, infinity or |g| > 80 in it: the general one).
+                 */
+                bool far = false;
+                if constexpr (MODE != MODE_FP8) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) far |= !(fabsf(g[i]) <= kSiluNear);
+                    far = __builtin_amdgcn_ballot_w64(far) != 0;
+                }
+                float left[4];
+                if (MODE != MODE_FP8 && far) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) left[i] = g[i] / (1.0f + zb_expf(-g[i]));
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        /* fp8: e4m3 keeps 3 mantissa bits, the hardware exp2 / reciprocal approximations (1 ulp) are ample */
+                        if constexpr (MODE == MODE_FP8)
+                            left[i] = g[i] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g[i] * -1.44269504088896341f));
+                        else left[i] = zb_silu_near(g[i]);
+                    }
+                }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    float left;
-                    if constexpr (MODE == MODE_FP8) {
-                        /* e4m3 keeps 3 mantissa bits: the hardware exp2 / reciprocal approximations (1 ulp) are ample */
-                        left = g[i] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g[i] * -1.44269504088896341f));
-                    } else {
-                        left = g[i] / (1.0f + zb_expf(-g[i]));
-                    }
-                    const float s = left * u[i];
+                    const float s = left[i] * u[i];
                     sg[mt][nt][i] = s;
                     rmax[mt] = fmaxf(rmax[mt], fabsf(s));
                 }

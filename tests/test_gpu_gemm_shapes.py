@@ -128,3 +128,26 @@ def test_many_tiles_are_the_same_rows_as_few(buf, avg):
         r = slice(int(off[e]), int(off[e + part]))
         got = gmm2(buf, a[r].contiguous(), xs[r].contiguous(), w[e:e + part], ws[e:e + part], capi.DT_FP32, counts[e:e + part], K, N, 1)
         assert torch.equal(whole[r].view(torch.int16), got.view(torch.int16))
+
+
+@pytest.mark.parametrize("mode", [1, 3])
+@pytest.mark.parametrize("spread", [0.2, 30.0, 70.0, 400.0])
+@pytest.mark.parametrize("avg", [20, 500])
+def test_swiglu_either_side_of_the_short_form(buf, mode, spread, avg):
+    """Gate values (standard deviation `spread`) that stay within the short form's 80, straddle it and leave exp()'s range; both kernels."""
+    K, N, counts = 512, 512, np.array([avg, 0, avg + 17, avg - 17], dtype=np.int64)
+    E, rows = len(counts), int(counts.sum())
+    a = rng(1).integers(-127, 128, (rows, K)).astype(np.int8)
+    a[5] = 0                                                       # gate and up are 0
+    xs = rng(2).uniform(0.5, 1.5, rows).astype(np.float32)
+    lo, hi = (-128, 128) if mode == 1 else (-8, 8)
+    w = rng(3).integers(lo, hi, (E, K, N)).astype(np.int8)
+    per_unit = spread / (73.0 * (hi - lo) * 0.29 * K ** 0.5)
+    if mode == 1:
+        ws = rng(4).uniform(0.5 * per_unit, 1.5 * per_unit, (E, N)).astype(np.float32)
+        want = zo.gmm1_swiglu_quant_w8a8(a, xs, w, ws, counts)[:2]
+    else:
+        ws = rng(4).uniform(0.5 * per_unit, 1.5 * per_unit, (E, K // 128, N)).astype(np.float16).view(np.uint16)
+        want = zo.gmm1_swiglu_quant_w4a8(a, xs, w, ws, counts)[:2]
+    q2, s2, _ = gmm1(buf, dev(a), dev(xs), buf.prepack_weight(dev(w), int4=mode == 3), dev(ws), counts, K, N, mode)
+    assert np.array_equal(host(s2).view(np.uint32), want[1].view(np.uint32)) and np.array_equal(host(q2), want[0])
