@@ -14,7 +14,7 @@
  * scales 16-byte vectors, gate/up pairs of the SwiGLU sit in the same lane,
  * and results leave as 8-element vectors.
  *
- * Workgroup tile: 64 to 320 token rows x 256 output channels x 128 K-bytes per
+ * Workgroup tile: 64 to 256 token rows x 256 output channels x 128 K-bytes per
  * step, eight waves; in the 256-row shape each wave has 64 rows x 128 channels
  * = 4x8 MFMA tiles (128 accumulator registers). For GMM1 the 256 channels are 128 gate
  * columns j and the matching 128 up columns I+j, so the SwiGLU product and,
@@ -36,6 +36,7 @@
 
 #include "zbal_device.h"
 #include "zbal_gemm_stream.h"
+#include "zbal_gemm_tall.h"
 #include "zbal_gemm_tile.h"
 #include "zbal_hip_kernels.h"
 
@@ -55,9 +56,8 @@ namespace {
  * pairs, so the read is free of bank conflicts whether the LDS serves 8 or 16 lanes per pass; plain
  * row-major storage would put all 16 rows on the same slot.
  *
- * TM = 256 and TM = 320 with two stages of 64 / 72 KiB (the slab for step k+1 is in flight while step k is
- * multiplied) have the arithmetic intensity that many-row experts need; the 320-row shape gives every wave a fifth
- * sub-tile. TM = 128 and TM = 64 with three or four stages are for few-row experts, where the job is to stream every
+ * TM = 256 with two stages of 64 KiB (the slab for step k+1 is in flight while step k is multiplied) has the arithmetic
+ * intensity that many-row experts need, where the 8-bit modes cannot take the kernel of zbal_gemm_tall.h. TM = 128 and TM = 64 with three or four stages are for few-row experts, where the job is to stream every
  * weight byte once at HBM speed: two weight slabs or more stay in flight per CU, and the MFMAs of sub-tiles past the
  * expert's end are skipped; W4A8, bound by its vector instructions, also has a 192-row shape. The few-row shapes and
  * that one split a tile over one or two row groups of waves instead of four (FewRows, launch_w4a8).
@@ -78,19 +78,19 @@ struct DmaShape {
     static constexpr int ROW_GROUPS = RG;
     static constexpr int COL_GROUPS = NW / RG;             /* the waves of a row group split the tile's 256 channels */
     static constexpr int NT = 16 / COL_GROUPS;             /* 16-channel sub-tiles per wave: 8 or 4 */
-    static constexpr int MTM = (TM / 16 + ROW_GROUPS - 1) / ROW_GROUPS;   /* 16-row sub-tiles per wave, at most: 2, 4, or 5 in the 320-row shape */
+    static constexpr int MTM = (TM / 16 + ROW_GROUPS - 1) / ROW_GROUPS;   /* 16-row sub-tiles per wave, at most: 2, 4 or 6 */
     static constexpr int THREADS = NW * 64;
     static constexpr int A_BYTES = TM * BKB;
     static constexpr int W_BYTES = BN * WRB;
     static constexpr int STAGE_BYTES = A_BYTES + W_BYTES;
     static constexpr int HALF_BLOCKS = 128 * WRB / 1024;   /* 1 KiB blocks per 128-channel half: 16 or 8 */
-    static constexpr int MAX_EXPERTS = TM > 256 ? 512 : D_MAX_EXPERTS;   /* what the lookup tables hold: the 320-row shape has 160 KiB of LDS less 144 KiB of stages for everything else */
+    static constexpr int MAX_EXPERTS = D_MAX_EXPERTS;       /* what the lookup tables hold */
     static constexpr int A_PARTS = (A_BYTES / 1024 + NW - 1) / NW;   /* 1 KiB blocks of the A tile per wave: 2, 4 or 5 */
     static constexpr int W_PARTS = W_BYTES / 1024 / NW;    /* 1 KiB blocks of the W tile per wave (2, 4 or 8) */
     static constexpr int PARTS = W_PARTS > A_PARTS ? W_PARTS : A_PARTS;
     static constexpr bool TWO_PHASE = TM == 256;            /* the tiles of short experts run after all the others (see the kernel) */
     /* two buffers of per-tile scales, floats each: fp8 2 x D_MAX_KB weight block scales; W8A8 256 channel + TM token scales */
-    static constexpr int SW_STRIDE = WRB == 64 ? 0 : (TM > 256 ? 576 : 2 * D_MAX_KB);      /* W4A8 has its own (lds_gs) */
+    static constexpr int SW_STRIDE = WRB == 64 ? 0 : 2 * D_MAX_KB;      /* W4A8 has its own (lds_gs) */
     static constexpr int SW_BYTES = 2 * SW_STRIDE * 4;
     static_assert(WRB == 64 || (SW_STRIDE >= 2 * D_MAX_KB && SW_STRIDE >= 256 + TM), "scale buffer too small");
     static constexpr int SA_FLOATS = WRB == 64 ? 0 : NSTAGE * TM;      /* the fp8 mode's activation block scales */
@@ -371,7 +371,7 @@ grouped_gemm_dma_kernel(GemmParams p)
      * out afresh for every transfer from a copy of the lane number that the K loop makes opaque once per step (kept
      * across the loop they were spilled, and a reload waits for the slabs in flight).
      */
-    constexpr bool FRESH_OFFSETS = TM > 256 || (MODE == MODE_W4A8 && TM >= 192);
+    constexpr bool FRESH_OFFSETS = MODE == MODE_W4A8 && TM >= 192;
     int lane_dma = lane;
     /* part j of a slab: the wave's j-th block of the W tile (j < W_PARTS), of the A tile (j < A_PARTS) and, with part 0, the scales */
     auto issue_part = [&](const Tile &t, int kb, int stage, int j) __attribute__((always_inline)) {
@@ -561,14 +561,10 @@ grouped_gemm_dma_kernel(GemmParams p)
             };
 
             if constexpr (MT > 0) {
-                /* five row sub-tiles in the fp8 mode: two passes over the weight fragments, see below */
-                constexpr bool TWO_PASS = MODE == MODE_FP8 && MT == 5;
-                constexpr bool AF_PER_PASS = TWO_PASS && GMM1;
-                constexpr int AFN = AF_PER_PASS ? 3 : MT;
-                i32x8 af[AFN];
+                i32x8 af[MT];
                 i32x8 wf_first = {};
 #pragma unroll
-                for (int mt = 0; mt < AFN; ++mt) {
+                for (int mt = 0; mt < MT; ++mt) {
                     const uint8_t *ab = sb + ((RG * mt + wm) * 16) * BKB;
                     const u32x4 lo = *reinterpret_cast<const u32x4 *>(ab + off_lo);
                     const u32x4 hi = *reinterpret_cast<const u32x4 *>(ab + off_hi);
@@ -592,121 +588,37 @@ grouped_gemm_dma_kernel(GemmParams p)
                      * matrix unit.
                      */
                     const float sw0 = sw_cur[kb], sw1 = sw_cur[D_MAX_KB + kb];
-                    if constexpr (MT == 5) {
-                        /*
-                         * Five row sub-tiles: 160 accumulators leave no room for five activation fragments beside the
-                         * weight fragment fetched ahead and the block-scale products. The step goes over the eight
-                         * weight fragments twice, first for row sub-tiles 0-2, then for 3-4, whose activation
-                         * fragments take the registers of the first three (the weight fragments are read again: LDS
-                         * reads are cheap here, registers are not). Each pass is the pipeline of the loop below.
-                         */
-                        auto pass = [&](auto lo_tag, auto n_tag) __attribute__((always_inline)) {
-                            constexpr int M0 = decltype(lo_tag)::value, MN = decltype(n_tag)::value;
-                            constexpr int A0 = AF_PER_PASS ? 0 : M0;       /* where the pass's fragments sit in af */
-                            if constexpr (!AF_PER_PASS) {
-                                /*
-                                 * Second GEMM: a wave's channels share one weight block scale, so one product per row
-                                 * sub-tile does; that leaves room for all five activation fragments from the start, and
-                                 * the weight fragment is read where it is used (measured against the form below on one
-                                 * GPU, 4096 tokens over 32 experts: 0.563 against 0.590 ms; the first GEMM the other way
-                                 * round, 1.16 against 1.00 ms).
-                                 */
-                                const float swx = wn >= COL_GROUPS / 2 ? sw1 : sw0;
-                                float sc[MN];
+                    float s0[MT], s1[MT];
 #pragma unroll
-                                for (int m = 0; m < MN; ++m)
-                                    sc[m] = lds_sa[cur_stage * TM + (RG * (M0 + m) + wm) * 16 + frag_row] * swx;
+                    for (int mt = 0; mt < MT; ++mt) {
+                        const float sa = lds_sa[cur_stage * TM + (RG * mt + wm) * 16 + frag_row];
+                        s0[mt] = sa * sw0;
+                        s1[mt] = sa * sw1;
+                    }
+                    i32x8 wf = wf_first;
+                    f32x4 part = mfma_fp8_16x16x128(wf, af[0]);
 #pragma unroll
-                                for (int nt = 0; nt < NT; ++nt) {
-                                    const i32x8 wfj = (M0 == 0 && nt == 0) ? wf_first : load_w(nt);
-                                    if (M0 == 0 && more && (nt == 0 || nt == 2)) { issue_quarter(nt); issue_quarter(nt + 1); }
-                                    f32x4 part = mfma_fp8_16x16x128(wfj, af[A0]);
+                    for (int nt = 0; nt < NT; ++nt) {
+                        i32x8 wf_n = wf;
+                        if (nt + 1 < NT) wf_n = load_w(nt + 1);
+                        /* the 256-row fp8 loop hands the slab out in two halves (0.6 % faster, measured against quarters on one GPU; the other loops are slower that way) */
+                        if (TM == 256) {
+                            if (more && (nt == 0 || nt == 2)) { issue_quarter(nt); issue_quarter(nt + 1); }
+                        } else if (more) {
+                            issue_at(nt);
+                        }
+                        const bool second = GMM1 ? (nt >= NT / 2) : (wn >= COL_GROUPS / 2);
 #pragma unroll
-                                    for (int m = 0; m < MN; ++m) {
-                                        f32x4 nxt_part = part;
-                                        if (m + 1 < MN) nxt_part = mfma_fp8_16x16x128(wfj, af[A0 + m + 1]);
-#pragma unroll
-                                        for (int i = 0; i < 4; ++i) accf[M0 + m][nt][i] = __builtin_fmaf(part[i], sc[m], accf[M0 + m][nt][i]);
-                                        part = nxt_part;
-                                    }
-                                }
-                                return;
-                            }
-                            i32x8 wf = wf_first;
-                            if (M0 != 0) {
-                                asm volatile("" ::: "memory");        /* not before the first pass is through with af */
-#pragma unroll
-                                for (int m = 0; m < MN; ++m) {
-                                    const uint8_t *ab = sb + ((RG * (M0 + m) + wm) * 16) * BKB;
-                                    const u32x4 lo = *reinterpret_cast<const u32x4 *>(ab + off_lo);
-                                    const u32x4 hi = *reinterpret_cast<const u32x4 *>(ab + off_hi);
-                                    af[m] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-                                    if (m == 0) wf = load_w(0);
-                                }
-                            }
-                            float s0[MN], s1[MN];
-#pragma unroll
-                            for (int m = 0; m < MN; ++m) {
-                                const float sa = lds_sa[cur_stage * TM + (RG * (M0 + m) + wm) * 16 + frag_row];
-                                s0[m] = sa * sw0;
-                                s1[m] = sa * sw1;
-                            }
-                            f32x4 part = mfma_fp8_16x16x128(wf, af[0]);
-#pragma unroll
-                            for (int nt = 0; nt < NT; ++nt) {
-                                i32x8 wf_n = wf;
-                                if (nt + 1 < NT) wf_n = load_w(nt + 1);
-                                if (M0 == 0 && more && (nt == 0 || nt == 2)) { issue_quarter(nt); issue_quarter(nt + 1); }
-                                const bool second = GMM1 ? (nt >= NT / 2) : (wn >= COL_GROUPS / 2);
-#pragma unroll
-                                for (int m = 0; m < MN; ++m) {
-                                    f32x4 nxt_part = part;
-                                    if (m + 1 < MN) nxt_part = mfma_fp8_16x16x128(wf, af[m + 1]);
-                                    else if (nt + 1 < NT) nxt_part = mfma_fp8_16x16x128(wf_n, af[0]);
-                                    const float sc = second ? s1[m] : s0[m];
-#pragma unroll
-                                    for (int i = 0; i < 4; ++i) accf[M0 + m][nt][i] = __builtin_fmaf(part[i], sc, accf[M0 + m][nt][i]);
-                                    part = nxt_part;
-                                }
-                                wf = wf_n;
-                            }
-                        };
-                        pass(std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
-                        pass(std::integral_constant<int, 3>{}, std::integral_constant<int, 2>{});
-                    } else {
-
-                        float s0[MT], s1[MT];
-    #pragma unroll
                         for (int mt = 0; mt < MT; ++mt) {
-                            const float sa = lds_sa[cur_stage * TM + (RG * mt + wm) * 16 + frag_row];
-                            s0[mt] = sa * sw0;
-                            s1[mt] = sa * sw1;
+                            f32x4 nxt_part = part;
+                            if (mt + 1 < MT) nxt_part = mfma_fp8_16x16x128(wf, af[mt + 1]);
+                            else if (nt + 1 < NT) nxt_part = mfma_fp8_16x16x128(wf_n, af[0]);
+                            const float sc = second ? s1[mt] : s0[mt];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(part[i], sc, accf[mt][nt][i]);
+                            part = nxt_part;
                         }
-                        i32x8 wf = wf_first;
-                        f32x4 part = mfma_fp8_16x16x128(wf, af[0]);
-    #pragma unroll
-                        for (int nt = 0; nt < NT; ++nt) {
-                            i32x8 wf_n = wf;
-                            if (nt + 1 < NT) wf_n = load_w(nt + 1);
-                            /* the 256-row fp8 loop hands the slab out in two halves (0.6 % faster, measured against quarters on one GPU; the other loops are slower that way) */
-                            if (TM == 256) {
-                                if (more && (nt == 0 || nt == 2)) { issue_quarter(nt); issue_quarter(nt + 1); }
-                            } else if (more) {
-                                issue_at(nt);
-                            }
-                            const bool second = GMM1 ? (nt >= NT / 2) : (wn >= COL_GROUPS / 2);
-    #pragma unroll
-                            for (int mt = 0; mt < MT; ++mt) {
-                                f32x4 nxt_part = part;
-                                if (mt + 1 < MT) nxt_part = mfma_fp8_16x16x128(wf, af[mt + 1]);
-                                else if (nt + 1 < NT) nxt_part = mfma_fp8_16x16x128(wf_n, af[0]);
-                                const float sc = second ? s1[mt] : s0[mt];
-    #pragma unroll
-                                for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(part[i], sc, accf[mt][nt][i]);
-                                part = nxt_part;
-                            }
-                            wf = wf_n;
-                        }
+                        wf = wf_n;
                     }
                 } else if constexpr (MODE == MODE_W4A8) {
                     /*
@@ -942,7 +854,27 @@ int32_t prepare_stream(hipStream_t st, int *n_cus)
     return prepare_kernel<&grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM>, StreamShape<MODE, TM>::LDS_BYTES>(st, n_cus);
 }
 
+template <int MODE, bool GMM1, int OUT_DT>
+int32_t prepare_tall(hipStream_t st, int *n_cus)
+{
+    return prepare_kernel<&grouped_gemm_tall_kernel<MODE, GMM1, OUT_DT>, TallShape<MODE>::LDS_BYTES>(st, n_cus);
+}
+
 /* launched with one persistent workgroup per CU, or fewer when there are not that many tiles */
+template <int MODE, bool GMM1, int OUT_DT>
+int32_t launch_tall(const GemmParams &p, int n_tiles, hipStream_t st)
+{
+    using S = TallShape<MODE>;
+    int n_cus = 0;
+    const int32_t rc = prepare_tall<MODE, GMM1, OUT_DT>(st, &n_cus);
+    if (rc != ZBALHIP_OK) return rc;
+    unsigned grid = grid_for(p.max_rows, p.experts, n_tiles, S::TM);
+    const unsigned resident = (unsigned)(n_cus + 7) / 8 * 8;
+    if (grid > resident) grid = resident;
+    grouped_gemm_tall_kernel<MODE, GMM1, OUT_DT><<<grid, S::THREADS, S::LDS_BYTES, st>>>(p);
+    return zbalhip_check_launch();
+}
+
 template <int MODE, bool GMM1, int OUT_DT, int TM, int NSTAGE, int RG, bool WSTREAM = false, Shared SH = SHARED_ON_DEMAND>
 int32_t launch_dma_shape(const GemmParams &p, int n_tiles, hipStream_t st)
 {
@@ -1061,7 +993,7 @@ int32_t prepare_mode()
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 192, 3, 2, false>(nullptr, &n);
     } else {
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 256, 2, 4, false, SHARED_NONE>(nullptr, &n);
-        if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 320, 2, 4, false>(nullptr, &n);
+        if (rc == ZBALHIP_OK) rc = prepare_tall<MODE, GMM1, OUT_DT>(nullptr, &n);
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG, true>(nullptr, &n);
     }
     return rc;
@@ -1088,25 +1020,6 @@ inline int64_t few_rows_limit(const GemmParams &p, int n_tiles)
     const bool few_tiles = (int64_t)p.experts * n_tiles <= 1024;
     return (MODE == MODE_FP8 && !few_tiles) ? 128 : 192;
 }
-
-/*
- * Two thirds of a two-stage tile's time does not depend on its rows (weight fragments, barrier, slab transfers), so
- * the fewer row tiles an expert has the better, and an expert whose rows just miss a multiple of 256 pays for a whole
- * tile more. The tall shape (five sub-tiles per wave; first built 288 rows high, then 320, which is the same loop and
- * 1.5 % faster even on the same tiles) cuts an expert into ceil(rows / 320) even tiles: where that is as many as
- * ceil(rows / 256) they are the same tiles as the 256-row shape's (and cost 1-4 % more in this kernel), where it is
- * fewer the expert is a tile's fixed cost shorter. Measured against the 256-row shape on 32 experts of 7168 x 4096 /
- * 2048 x 7168, random routing, first / second GEMM, rows per expert on average:
- *   - fp8: 256 rows -29 % / -15 %, 512 rows -16 % / -9 %, 1024 rows -8 % / -5 % (the 288-row build; 320 rows another
- *     -2 % / 0 %), 1500 rows 0 / +3 %, 2048 rows +2 % / +2 %, 3072 rows +2 % / +4 %, 4096 rows +2 % / +3 %: its
- *     five-sub-tile loop goes over the weight fragments twice and gives back what the saved tiles bring, hence the limit;
- *   - W8A8: 256 rows -26 % / -17 %, 1024 rows -9 % / -5 %, 1500 rows -5 % / -5 %, 2048 rows -4.5 % / -8 %, 3072 rows
- *     -3 % / -6 %, 4096 rows -5 % / -9 %: no limit;
- *   - with exactly 1024 rows for every expert fp8 +3 % / +4.6 % (the 288-row build).
- * W4A8 has no such shape (its loop has no registers for a fifth row sub-tile). The tall shape's LDS leaves room for
- * lookup tables of 512 experts; launches with more take the 256-row shape.
- */
-constexpr int64_t kTallRowsLimitFp8 = 1536;
 
 /*
  * W4A8 where the streaming kernel does not run (K no multiple of 512): the smaller the slab (16 KiB of weights), the more a step's own work shows, and the compute-bound sizes are
@@ -1167,9 +1080,13 @@ int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
             if (rows <= stream_limit * e) return launch_dma_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG, true>(p, n_tiles, st);
             return launch_dma_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG>(p, n_tiles, st);
         }
-        using Tall = DmaShape<320, 2, 128, 4>;
-        const bool tall_pays = MODE == MODE_W8A8 || rows <= kTallRowsLimitFp8 * e;
-        if (tall_pays && e <= Tall::MAX_EXPERTS) return launch_dma_shape<MODE, GMM1, OUT_DT, 320, 2, 4>(p, n_tiles, st);
+        /*
+         * Many rows: at every count against what ran there before (320-row tiles on four row groups of waves, fp8 beyond 1536 rows
+         * per expert the 256-row shape below), both GEMMs, 32 experts of 7168 x 4096 / 2048 x 7168, 64 of 2048 x 2048 /
+         * 1024 x 2048, 8 of 4096 x 28672 / 14336 x 4096, 250 to 2300 rows per expert: fp8 -8 / -11 % (0 ... -21), W8A8
+         * -10 / -8 % (+1 ... -15). 1024 rows of the first: fp8 1047 / 596 -> 935 / 543 us, W8A8 974 / 519 -> 905 / 468.
+         */
+        if (tall_accepts<MODE>(p)) return launch_tall<MODE, GMM1, OUT_DT>(p, n_tiles, st);
         /*
          * This shape's K loop has no scalar register to spare for a shared expert's tensors, and with this many rows per
          * expert the fused layer's takes turns with the routed ones: 2048 rows fp8, first GEMM 2.01 ms with the shared

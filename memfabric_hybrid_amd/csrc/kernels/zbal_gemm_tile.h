@@ -104,6 +104,9 @@ __device__ __forceinline__ f32x4 mfma_fp8_16x16x128(const i32x8 &wfrag, const i3
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wfrag, afrag, zero, 0, 0, 0, 0, 0, 0);
 }
 
+/* a barrier for what is in LDS: __syncthreads() would also wait for the slabs in flight */
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 /* four consecutive bytes -> one dword store helpers */
 __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float d)
 {
@@ -116,9 +119,10 @@ __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float 
  * are dealt round-robin over the row groups, so a tile that is not full leaves every SIMD the same share). The pre-pack put channels 32*(nt/2) + 8*(lane/16) + 4*(nt%2) + i in
  * those rows (zb_block_row_channel), so the sub-tiles nt = 2s and 2s+1 together are eight consecutive channels.
  * A wave's NT channel sub-tiles are 16 * NT consecutive channels (GMM1: 8 * NT gate and the matching 8 * NT up columns).
- * `lds_rowmax` is [16 / NT][tile_rows] floats of scratch for the row maxima of the waves' channel ranges (GMM1 only).
+ * `lds_rowmax` is [16 / NT][tile_rows] floats of scratch for the row maxima of the waves' channel ranges (GMM1 only);
+ * ONE_MAX: [tile_rows], zero before, which takes the maximum over the channel ranges itself.
  */
-template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT, Shared SH>
+template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT, Shared SH, bool ONE_MAX = false>
 __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &tc, f32x4 (&accf)[MTM][NT],
                                          i32x4 (&acci)[MTM][NT], int row_begin, int row_end, int wm, int wn, int lane,
                                          float *lds_rowmax, int tile_rows, const float *es)
@@ -251,16 +255,20 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             /* the four lane groups (lane/16) hold different columns of the same row */
             rmax[mt] = fmaxf(rmax[mt], __shfl_xor(rmax[mt], 16, 64));
             rmax[mt] = fmaxf(rmax[mt], __shfl_xor(rmax[mt], 32, 64));
-            if (lane < 16) lds_rowmax[wn * tile_rows + (RG * mt + wm) * 16 + lane] = rmax[mt];
+            if (lane < 16) {
+                float *at = lds_rowmax + (RG * mt + wm) * 16 + lane;
+                if (ONE_MAX) atomicMax(reinterpret_cast<uint32_t *>(at), __float_as_uint(rmax[mt]));      /* not negative, no NaN: ordered as integers */
+                else at[wn * tile_rows] = rmax[mt];
+            }
         }
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int mt = 0; mt < MTM; ++mt) {
             const int lr = (RG * mt + wm) * 16 + frag_row;
             const int row = row_begin + lr;
             float amax_tile = lds_rowmax[lr];
 #pragma unroll
-            for (int g = 1; g < COL_GROUPS; ++g) amax_tile = fmaxf(amax_tile, lds_rowmax[g * tile_rows + lr]);
+            for (int g = 1; g < (ONE_MAX ? 1 : COL_GROUPS); ++g) amax_tile = fmaxf(amax_tile, lds_rowmax[g * tile_rows + lr]);
             if (row >= row_end) continue;
             if constexpr (MODE == MODE_FP8) {
                 const float amax = fmaxf(amax_tile, 1e-4f);

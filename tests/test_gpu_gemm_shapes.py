@@ -151,3 +151,46 @@ def test_swiglu_either_side_of_the_short_form(buf, mode, spread, avg):
         want = zo.gmm1_swiglu_quant_w4a8(a, xs, w, ws, counts)[:2]
     q2, s2, _ = gmm1(buf, dev(a), dev(xs), buf.prepack_weight(dev(w), int4=mode == 3), dev(ws), counts, K, N, mode)
     assert np.array_equal(host(s2).view(np.uint32), want[1].view(np.uint32)) and np.array_equal(host(q2), want[0])
+
+
+# K slabs of the many-row kernel: scales of four steps in whole groups (4, 8), with two and three steps left over (6, 11), with one (5: the 256-row shape)
+@pytest.mark.parametrize("slabs", [4, 5, 6, 8, 11])
+@pytest.mark.parametrize("avg", [200, 900])
+def test_many_rows_fp8(buf, slabs, avg):
+    K, N = 128 * slabs, 768
+    counts = np.array([avg + 21, 0, 1, 320, 321, 3 * avg, avg + 60, 257], dtype=np.int64)
+    E, rows = len(counts), int(counts.sum())
+    counts[0] += max(0, 900 * E - rows) if avg == 900 else max(0, 200 * E - rows)      # more than any line to the kernels for fewer rows
+    rows = int(counts.sum())
+    a, sa, w, sw = fp8_operands(E, K, N, rows, 20 + slabs)
+    packed = buf.prepack_weight(dev(w))
+    y = gmm2(buf, dev(a), dev(sa), packed, dev(sw), capi.DT_FP32, counts, K, N, 2)
+    assert_fp8_close(zo.bf16_to_f32(host(y)), zo.bf16_to_f32(zo.gmm2_fp8(a, sa, w, sw, counts)), "fp8 GEMM", FP8_GEMM_ELEM_TOL)
+    q2, s2, _ = gmm1(buf, dev(a), dev(sa), packed, dev(sw), counts, K, N, 2)
+    r_q2, r_s2, _ = zo.gmm1_swiglu_quant_fp8(a, sa, w, sw, counts)
+    blocks = (rows, N // 256, 128)
+    assert np.allclose(host(s2), r_s2, rtol=1e-4)
+    assert_requant_close(zo.e4m3_to_f32(host(q2)).reshape(blocks) * host(s2)[:, :, None],
+                         zo.e4m3_to_f32(r_q2).reshape(blocks) * r_s2[:, :, None], host(q2), r_q2)
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+def test_many_tiles_per_workgroup_are_the_same_rows(buf, mode):
+    """More tiles than a workgroup works out at once (32 of them): the same bits as expert by expert, where it has a few."""
+    K, N, E, avg = 512, 16384, 32, 1300
+    counts = np.array([avg - 16 * e if e % 2 else avg + 16 * e for e in range(E)], dtype=np.int64)
+    rows = int(counts.sum())
+    assert (rows // 320) * (N // 256) > 32 * 256
+    a = torch.randint(0, 256, (rows, K), dtype=torch.uint8, device="cuda")
+    w = torch.randint(0, 256, (E, N, K), dtype=torch.uint8, device="cuda")           # any bytes are a pre-packed weight
+    if mode == 2:
+        a, w = a & 0x77, w & 0x77                                                    # no NaN codes
+        xs, ws = torch.rand((rows, K // 128), device="cuda") + 0.5, torch.rand((E, K // 128, N // 128), device="cuda") + 0.5
+    else:
+        xs, ws = torch.rand((rows,), device="cuda") + 0.5, torch.rand((E, N), device="cuda") + 0.5
+    whole = gmm2(buf, a, xs, w, ws, capi.DT_FP32, counts, K, N, mode)
+    off = np.concatenate([[0], np.cumsum(counts)])
+    for e in range(E):
+        r = slice(int(off[e]), int(off[e + 1]))
+        got = gmm2(buf, a[r].contiguous(), xs[r].contiguous(), w[e:e + 1], ws[e:e + 1], capi.DT_FP32, counts[e:e + 1], K, N, mode)
+        assert torch.equal(whole[r].view(torch.int16), got.view(torch.int16)), e
