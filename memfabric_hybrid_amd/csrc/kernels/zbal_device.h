@@ -236,6 +236,15 @@ __device__ __forceinline__ int32_t zb_wave_sum_dpp(int32_t x)
     return __builtin_amdgcn_readlane(x, 63);
 }
 
+/* max over the lanes l, l ^ 16, l ^ 32 and l ^ 48, in all of them: the swaps leave every lane with both values of a pair */
+__device__ __forceinline__ float zb_max_of_rows(float v)
+{
+    u32x2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 /* max over groups of 2^LOG2 consecutive lanes */
 template <int LOG2> __device__ __forceinline__ float zb_group_max(float v)
 {

@@ -251,10 +251,14 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
                     sg[mt][nt][i] = s;
                     rmax[mt] = fmaxf(rmax[mt], fabsf(s));
                 }
+                if constexpr (MODE != MODE_FP8) {
+                    if (row < row_end)
+                        *reinterpret_cast<f32x4 *>(p.sgl_ws + (int64_t)row * I + tc.n_tile * 128 + jl) =
+                            f32x4{sg[mt][nt][0], sg[mt][nt][1], sg[mt][nt][2], sg[mt][nt][3]};
+                }
             }
             /* the four lane groups (lane/16) hold different columns of the same row */
-            rmax[mt] = fmaxf(rmax[mt], __shfl_xor(rmax[mt], 16, 64));
-            rmax[mt] = fmaxf(rmax[mt], __shfl_xor(rmax[mt], 32, 64));
+            rmax[mt] = zb_max_of_rows(rmax[mt]);
             if (lane < 16) {
                 float *at = lds_rowmax + (RG * mt + wm) * 16 + lane;
                 if (ONE_MAX) atomicMax(reinterpret_cast<uint32_t *>(at), __float_as_uint(rmax[mt]));      /* not negative, no NaN: ordered as integers */
@@ -262,6 +266,12 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             }
         }
         lds_barrier();
+        /*
+         * One wave per row group raises the rows' maxima; the others, whose values are stored already, are done. (All of them
+         * reduced the maxima and stored after the barrier before: first GEMM at 1024 rows per expert, 128 experts of 4096 x 3072,
+         * W8A8 1781 -> 1715 us, W4A8 2199 -> 2158.)
+         */
+        if (MODE != MODE_FP8 && wn != 0) return;
 #pragma unroll
         for (int mt = 0; mt < MTM; ++mt) {
             const int lr = (RG * mt + wm) * 16 + frag_row;
@@ -288,13 +298,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
                 }
                 if (wn == 0 && lane < 16) p.out_scale[(int64_t)row * (I / 128) + tc.n_tile] = amax * (1.0f / 448.0f);
             } else {
-#pragma unroll
-                for (int nt = 0; nt < UP; ++nt) {
-                    const int t = wn * UP + nt, j = tc.n_tile * 128 + (t >> 1) * 32 + q8 + (t & 1) * 4;
-                    const f32x4 v = f32x4{sg[mt][nt][0], sg[mt][nt][1], sg[mt][nt][2], sg[mt][nt][3]};
-                    *reinterpret_cast<f32x4 *>(p.sgl_ws + (int64_t)row * I + j) = v;
-                }
-                if (wn == 0 && lane < 16) atomicMax(&p.rowmax[row], __float_as_uint(amax_tile));
+                if (lane < 16) atomicMax(&p.rowmax[row], __float_as_uint(amax_tile));
             }
         }
     }
