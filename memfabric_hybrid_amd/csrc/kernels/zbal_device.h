@@ -30,6 +30,7 @@
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef int32_t i32x2 __attribute__((ext_vector_type(2)));
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -234,6 +235,18 @@ __device__ __forceinline__ int32_t zb_wave_sum_dpp(int32_t x)
     x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
     x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
     return __builtin_amdgcn_readlane(x, 63);
+}
+
+/* inclusive sum over the lanes up to this one */
+__device__ __forceinline__ int32_t zb_wave_scan_dpp(int32_t x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);     /* row_shr:1, 2, 4, 8 */
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);     /* row_bcast:15 into rows 1 and 3 */
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);     /* row_bcast:31 into rows 2 and 3 */
+    return x;
 }
 
 /* max over the lanes l, l ^ 16, l ^ 32 and l ^ 48, in all of them: the swaps leave every lane with both values of a pair */

@@ -110,12 +110,7 @@ grouped_gemm_stream_kernel(GemmParams p)
         const uint64_t busy = __ballot(m > 0);
         const int c0 = (used + __builtin_amdgcn_mbcnt_hi((uint32_t)(busy >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)busy, 0))) * n_tiles;
         const int mine = (columns_before(c0 + n_tiles) - columns_before(c0)) * m;
-        int incl = mine;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int o = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += o;
-        }
+        const int incl = zb_wave_scan_dpp(mine);
         const uint64_t past = __ballot(tiles + incl > slot);
         if (past) {
             const int src = __ffsll((long long)past) - 1;
