@@ -40,7 +40,7 @@ template <int MODE, int TM> struct StreamShape {
     static constexpr int SA_ROWS = TM > 64 ? 128 : 64;
     static constexpr int SA_FLOATS = MODE == MODE_FP8 ? PF * SA_ROWS : 0; /* one chunk's block scales, [slab][row] */
     static constexpr int GS_BYTES = MODE == MODE_W4A8 ? PF * BN * 2 : 0;  /* one chunk's fp16 group scales, [slab][channel] */
-    static constexpr int ES_FLOATS = MODE == MODE_W8A8 ? 256 + (TM + 63) / 64 * 64 : (MODE == MODE_FP8 ? 2 * 256 : 0);
+    static constexpr int ES_FLOATS = MODE == MODE_FP8 ? 2 * 256 : (MODE == MODE_W8A8 ? 256 : 0) + (TM + 63) / 64 * 64;
     static constexpr int LDS_BYTES = 2 * (A_BYTES + SA_FLOATS * 4 + GS_BYTES) + ES_FLOATS * 4 + NW * TM * 4;
     static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
 };
@@ -198,14 +198,17 @@ grouped_gemm_stream_kernel(GemmParams p)
         }
     };
 
-    /* what the epilogue (W8A8) or the K loop (fp8) needs of the tile's scales; older than everything else, so there first */
-    if constexpr (MODE == MODE_W8A8) {
+    /*
+     * What the epilogue (int modes) or the K loop (fp8) needs of the tile's scales; older than everything else, so there first.
+     * (W4A8's epilogue loaded its token scales itself, one round trip per row sub-tile: 4.3 us of a tile's 27 in the second GEMM.)
+     */
+    if constexpr (MODE != MODE_FP8) {
         const uint32_t dst0 = lds_addr(lds_es);
         if (wave < (TM + 63) / 64) {                               /* 64 token scales each */
             const int rel = wave * 64 + lane > last_rel ? last_rel : wave * 64 + lane;
-            dma4_sv(p.a_scale + row_begin, (uint32_t)rel * 4u, dst0 + 1024 + wave * 256);
+            dma4_sv(p.a_scale + row_begin, (uint32_t)rel * 4u, dst0 + (MODE == MODE_W8A8 ? 1024 : 0) + wave * 256);
         }
-        if (wave >= 4) {
+        if (MODE == MODE_W8A8 && wave >= 4) {
             const int w4 = wave - 4;
             if (GMM1 || !p.wscale_is_bf16) {
                 const float *wsb = scales_of<float, SHARED_IN_REGISTERS>(p, expert, p.N);
@@ -402,7 +405,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     tc.n_tile = n_tile;
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));               /* as in the other kernel: nothing of the epilogue's stays live across the K loop */
-    epilogue<MODE, GMM1, OUT_DT, 1, MTM, NT, SHARED_IN_REGISTERS>(p, tc, accf, acci, row_begin, row_end, 0, wave, lane_e, lds_rowmax, TM, lds_es);
+    epilogue<MODE, GMM1, OUT_DT, 1, MTM, NT, SHARED_IN_REGISTERS, false, MODE != MODE_FP8>(p, tc, accf, acci, row_begin, row_end, 0, wave, lane_e, lds_rowmax, TM, lds_es);
 }
 
 } // namespace

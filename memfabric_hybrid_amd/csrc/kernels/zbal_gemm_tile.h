@@ -122,7 +122,7 @@ __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float 
  * `lds_rowmax` is [16 / NT][tile_rows] floats of scratch for the row maxima of the waves' channel ranges (GMM1 only);
  * ONE_MAX: [tile_rows], zero before, which takes the maximum over the channel ranges itself.
  */
-template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT, Shared SH, bool ONE_MAX = false>
+template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT, Shared SH, bool ONE_MAX = false, bool ROW_SCALES = MODE == MODE_W8A8>
 __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &tc, f32x4 (&accf)[MTM][NT],
                                          i32x4 (&acci)[MTM][NT], int row_begin, int row_end, int wm, int wn, int lane,
                                          float *lds_rowmax, int tile_rows, const float *es)
@@ -131,11 +131,19 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
      * W8A8: `es` is this tile's scales in LDS, brought there by DMA while the tile was multiplied: [0, 256) the
      * channel scales of the tile's 256 weight rows (fp32, or 256 bf16 in the first 512 bytes), [256, 256 +
      * tile_rows) the per-token scales of its rows. A global load here is waited for with a count that also waits
-     * for the next tile's slabs, which are already in flight (decode: 5-6 % of both GEMMs). The W4A8 mode, whose
-     * channel scales travel with the slabs, still loads its per-token scale here: its kernel has no registers to
-     * spare, and a spill costs more than the wait.
+     * for the next tile's slabs, which are already in flight (decode: 5-6 % of both GEMMs). ROW_SCALES: the per-token scales
+     * are there. The W4A8 mode of the staged kernel, whose channel scales travel with the slabs and which has no registers to
+     * spare, loads its per-token scales here, all of them before it uses the first.
      */
-    const float *es_row = es + 256;
+    float xs_loaded[MTM];
+    if constexpr (MODE == MODE_W4A8 && !ROW_SCALES) {
+#pragma unroll
+        for (int mt = 0; mt < MTM; ++mt) {
+            const int row = row_begin + (RG * mt + wm) * 16 + (lane & 15);
+            xs_loaded[mt] = p.a_scale[row < p.max_rows ? row : p.max_rows - 1];
+        }
+    }
+    const float *es_row = es + (MODE == MODE_W8A8 ? 256 : 0);
     const int frag_row = lane & 15;
     const int I = p.N / 2;
     const int q8 = (lane >> 4) * 8;
@@ -147,8 +155,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             const int row = row_begin + (RG * mt + wm) * 16 + frag_row;
             if (row >= row_end) continue;
             float xs = 1.0f;
-            if (MODE == MODE_W8A8) xs = es_row[(RG * mt + wm) * 16 + frag_row];
-            else if (MODE == MODE_W4A8) xs = p.a_scale[row];
+            if (ROW_SCALES) xs = es_row[(RG * mt + wm) * 16 + frag_row];
+            else if (MODE == MODE_W4A8) xs = xs_loaded[mt];
 #pragma unroll
             for (int s = 0; s < NT / 2; ++s) {    /* sub-tiles 2s and 2s+1: eight consecutive channels from n */
                 const int nl = wn * (16 * NT) + s * 32 + q8;       /* within the tile */
@@ -200,8 +208,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             if ((RG * mt + wm) * 16 >= row_end - row_begin) continue;
             const int row = row_begin + (RG * mt + wm) * 16 + frag_row;
             float xs = 1.0f;
-            if (MODE == MODE_W8A8) xs = es_row[(RG * mt + wm) * 16 + frag_row];
-            else if (MODE == MODE_W4A8) xs = p.a_scale[row < p.max_rows ? row : p.max_rows - 1];
+            if (ROW_SCALES) xs = es_row[(RG * mt + wm) * 16 + frag_row];
+            else if (MODE == MODE_W4A8) xs = xs_loaded[mt];
             rmax[mt] = 0.0f;
 #pragma unroll
             for (int nt = 0; nt < UP; ++nt) {
