@@ -9,12 +9,18 @@
 
 /*
  * Stable ranks of the picks [p0, p1) of one block: `run[e]` holds the number of earlier picks of expert e on entry
- * and the number up to p1 on return. Picks are taken 64 per wave at a time; lanes holding the same expert find
+ * and, with TOTALS, the number up to p1 on return; `first` is this thread's first pick (first_pick), which the caller
+ * may have asked for early. Picks are taken 64 per wave at a time; lanes holding the same expert find
  * each other by intersecting one ballot per index bit. The waves do not take turns: each leaves the size of its
  * groups in `cnt` (one byte per wave and expert, a group has at most 64 members) and a pick's rank is the running
  * count plus the groups of the waves before its own. Ends on a barrier.
  */
-__device__ __forceinline__ void rank_picks(const ExpertIds &idx, int64_t p0, int64_t p1, int experts, int nbits,
+__device__ __forceinline__ int first_pick(const ExpertIds &idx, int64_t p0, int64_t p1)
+{
+    return p0 + threadIdx.x < p1 ? idx[p0 + threadIdx.x] : -1;
+}
+template <bool TOTALS = true>
+__device__ __forceinline__ void rank_picks(const ExpertIds &idx, int64_t p0, int64_t p1, int first, int experts, int nbits,
                                            int32_t *run, uint8_t *cnt /* [waves][experts rounded up to 4] */,
                                            int32_t *__restrict__ send_token_idx)
 {
@@ -27,7 +33,7 @@ __device__ __forceinline__ void rank_picks(const ExpertIds &idx, int64_t p0, int
 
     for (int it = 0; it < iters; ++it) {
         const int64_t i = p0 + (int64_t)it * threads + threadIdx.x;
-        const int e = (i < p1) ? idx[i] : -1;
+        const int e = it == 0 ? first : (i < p1 ? idx[i] : -1);
         for (int j = threadIdx.x; j < nwaves * pad / 4; j += threads) reinterpret_cast<uint32_t *>(cnt)[j] = 0u;
         const bool valid = (e >= 0 && e < experts);
         uint64_t peers = __ballot(valid);
@@ -49,6 +55,7 @@ __device__ __forceinline__ void rank_picks(const ExpertIds &idx, int64_t p0, int
         } else if (i < p1) {
             send_token_idx[i] = -1;
         }
+        if (!TOTALS && it + 1 == iters) break;
         __syncthreads();
         for (int e2 = threadIdx.x; e2 < experts; e2 += threads) {
             int32_t sum = 0;

@@ -56,6 +56,25 @@ def test_layout_in_one_launch(buf, T, K, E, R, npdt):
     assert T == 0 or np.array_equal(host(in_rank), want_in)
 
 
+# whole tokens per wave: 64, 21, 10, one, one, and more picks than a wave has lanes; tokens either side of a block's eight steps of them
+@pytest.mark.parametrize("K", [1, 3, 6, 33, 64, 65])
+@pytest.mark.parametrize("T", [1, 127, 128, 129, 1345])
+@pytest.mark.parametrize("npdt", [np.int64, np.int32])
+def test_tokens_of_one_rank(buf, T, K, npdt):
+    E = 40
+    idx = rng(T + K).integers(-1, E + 1, size=(T, K)).astype(npdt)
+    idx[::3] = E                                                                # tokens without a valid pick
+    idx[::6, K - 1] = E - 1                                                     # or with the last one only
+    d = dev(idx)
+    per_rank, per_expert, send, in_rank = (torch.full(s, -7, dtype=torch.int32, device="cuda") for s in ((1,), (E,), (T, K), (T, 1)))
+    assert buf.lib.zbalhip_dispatch_layout_in_rank(d.data_ptr(), int(npdt == np.int64), T, E, K, 1, per_rank.data_ptr(),
+                                                   per_expert.data_ptr(), send.data_ptr(), in_rank.data_ptr(), capi.stream_ptr()) == 0
+    want = ((idx >= 0) & (idx < E)).any(axis=1)
+    assert np.array_equal(host(in_rank)[:, 0], want.astype(np.int32)) and host(per_rank)[0] == want.sum()
+    _, want_expert, want_send = zo.dispatch_layout(idx.astype(np.int64), E, 1)
+    assert np.array_equal(host(per_expert), want_expert) and np.array_equal(host(send), want_send)
+
+
 @pytest.mark.parametrize("E", [1, 63, 64, 65, 1024])
 def test_counts_read_back_by_the_notify_kernel(buf, E):
     """Several calls in a row, with work queued in front and behind, give the counts of that call."""
