@@ -948,6 +948,10 @@ template <int MODE, bool GMM1> struct StreamRows {
  *   - second fp8 GEMM, K 14336, 8 experts: 160-190 rows +34 / +25 / +33 (a third row tile on a few CUs, and K is long); from
  *     200 to 350, where the other kernel's tile is 320 rows, -27 / -25 / -25, 400 rows (a fifth row tile) +27 / -14 / -12;
  *   - W4A8 -2 ... -50 throughout.
+ * Against the many-row kernel of zbal_gemm_tall.h (nine shapes, 112 to 600 rows, uniform / Zipf(0.6) / Zipf(1.2), per cent that it
+ * takes more): the lines lie where it wins with every routing. First GEMM 200 rows W8A8 -16 / +1 / +13, fp8 -24 / 0 / +18,
+ * 400 rows -10 / -9 / +2, -16 / -12 / +2; second 300 rows W8A8 -3 / -2 / +13, fp8 -11 / -9 / +10, 400 rows fp8 -15 / -11 / +2;
+ * K 1024, 64 experts, fp8: 500 rows -16 / -5 / +11, 600 rows -10 / -12 / -5, 800 rows Zipf(1.2) -13 (until then the line was 800).
  */
 template <int MODE, bool GMM1>
 inline int stream_rows(const GemmParams &p, int n_tiles)
@@ -972,7 +976,7 @@ inline int stream_rows(const GemmParams &p, int n_tiles)
             if (rows > 150 * e && rows <= 192 * e) return 0;
             tall = 352;
         }
-        if (p.K <= 1024 && !many_tiles) tall = 800;
+        if (p.K <= 1024 && !many_tiles) tall = 520;
     }
     return rows <= low * e ? R::LOW : (rows <= tall * e ? R::TALL : 0);
 }

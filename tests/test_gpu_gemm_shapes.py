@@ -83,7 +83,7 @@ def test_8_bit_shapes(buf, edges, K, N):
 
 # averages either side of the lines that `stream_rows` draws by K and rows per expert; the second GEMM runs with the shorter K too
 LINES = [(2560, 87), (2560, 88), (2560, 108), (2560, 109), (2560, 112), (2560, 113), (2560, 160), (2560, 184), (2560, 185), (8704, 150),
-         (8704, 151), (8704, 192), (8704, 193), (8704, 352), (8704, 353)]
+         (8704, 151), (8704, 192), (8704, 193), (8704, 352), (8704, 353), (1024, 520), (1024, 521)]
 
 
 @pytest.mark.parametrize("K,avg", LINES)
