@@ -918,18 +918,24 @@ template <int MODE, bool GMM1> struct FewRows {
 /*
  * Row tiles of the streaming kernel: the lower one while most experts' rows fit it (four slabs of weights in flight, as the
  * memory wants it), the taller one beyond (two; the L2 serves the row tiles of an expert together). The registers end them:
- * fp8's block scales leave no room for a fourth sub-tile in the lower one, W8A8's second GEMM has room for eight.
+ * fp8's block scales leave no room for a fourth sub-tile in the lower one, W8A8's second GEMM and W4A8 have room for eight.
+ * W4A8 is bound by vector issue, and a weight unpacked for 128 rows instead of 96 is a tenth of a row's instructions less: 1024 rows
+ * per expert, 128 experts of 4096 x 3072 / 1536 x 4096, 2050 -> 1984 / 1008 -> 964 us.
  */
 template <int MODE, bool GMM1> struct StreamRows {
     static constexpr int LOW = MODE == MODE_FP8 ? 48 : 64;
-    static constexpr int TALL = MODE == MODE_W8A8 && !GMM1 ? 128 : 96;
+    static constexpr int TALL = (MODE == MODE_W8A8 && !GMM1) || MODE == MODE_W4A8 ? 128 : 96;
 };
 
 /*
  * Where the streaming kernel takes over from the kernel above (K in whole chunks of its four slabs only), by rows per
  * expert on average; 0: it does not. Layers in us with it against without, uniform / Zipf(1.2) routing, 128 experts of
  * 4096 x 3072 / 1536 x 4096 (M), 64 of 2048 x 2048 / 1024 x 2048 (S), 32 of 7168 x 4096 / 2048 x 7168 (W):
- *   - W4A8: always (M 128 rows -12 / -190, 250 -81 / -184; 64 rows against 96: 512 rows 3 / -199 and 13 / -206, 1024 +80 and -64);
+ *   - W4A8: always (M 128 rows -12 / -190, 250 -81 / -184). 128 rows against 64, uniform / Zipf(0.6) / Zipf(1.2), both GEMMs, per
+ *     cent: M 80 rows -9 / +3 / +6, 112 -7 / -4 / +1, 200 -7 / -5 / -3, 640 -5 / -6 / -8, 1024 -8 / -8 / -8; S 64 rows -9 / +20 / +9,
+ *     200 -6 / +4 / +2, 250 -1 / -1 / +1, 375 -2 / -4 / -3, 640 -7 / -7 / -8; W 128 rows +4 / 0 / +5, 200 -6 / -3 / -3; 8 experts of
+ *     14336 x 4096 200 rows +8 / - / +33: from where its tiles, rows * n_tiles / 128, fill the chip (two workgroups per CU)
+ *     twice, and once with many rows (8 experts 650 rows against 96-row tiles -1 / -3; 2 of 4096 x 3072, 70 tiles, +16);
  *   - W8A8 first GEMM, 96 rows: 75 M -23 / -52, W -7 / -20, 128 M -35 / -23, W -17 / -4, 187 M +3 / -64, S -8 / -41,
  *     250 M +35 / -46, W +22 / -27, 375 S -9 / -33, 512 M +90 / +17; second, 128 rows: 75 M -12 / -37, 128 M -27 / -32,
  *     250 W -13 / -18, 375 M -25 / -21, 512 M +14 / -24;
@@ -959,7 +965,7 @@ inline int stream_rows(const GemmParams &p, int n_tiles)
     using R = StreamRows<MODE, GMM1>;
     const int64_t rows = p.max_rows, e = p.experts, tiles = e * n_tiles;
     if (p.K % 512 != 0) return 0;
-    if (MODE == MODE_W4A8) return rows <= 640 * e ? R::LOW : R::TALL;
+        if (MODE == MODE_W4A8) return rows > 112 * e && rows * n_tiles >= (rows > 640 * e ? 65536 : 128000) ? R::TALL : R::LOW;
     const bool many_tiles = tiles >= 4096;
     const int64_t low = MODE == MODE_W8A8 ? 48 : 36;
     int64_t tall = many_tiles && !GMM1 ? 192 : 400;

@@ -27,7 +27,7 @@ EDGES = {"few": [0, 1, 15, 16, 17, 2, 8, 5, 0, 3], "64": [1, 0, 16, 31, 33, 63, 
          "100": [0, 96, 97, 127, 128, 129, 112, 64, 1, 200], "160": [191, 192, 193, 176, 177, 0, 30, 160, 161, 256],
          "47": [47, 48, 49, 33, 32, 31, 0, 17, 64, 1], "53": [63, 64, 65, 49, 48, 128, 50, 0, 20, 33],
          "sparse": [0] * 63 + [5, 70] + [0] * 66 + [16, 1] + [0] * 60 + [33, 2], "1000": [1000, 769, 96, 97, 1151, 1153, 767, 800, 0, 700],
-         "224": [128, 129, 256, 257, 192, 255, 0, 144, 300, 250], "640": [384, 385, 192, 577, 1, 0, 600, 383, 500, 191]}
+         "900": [128, 129, 127, 112, 113, 1024, 1025, 3001, 2945, 1], "224": [128, 129, 256, 257, 192, 255, 0, 144, 300, 250], "640": [384, 385, 192, 577, 1, 0, 600, 383, 500, 191]}
 
 
 # whole chunks of the streaming kernel's slabs, channel tiles in eighths and not
