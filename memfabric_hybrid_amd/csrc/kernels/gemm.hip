@@ -848,10 +848,10 @@ int32_t prepare_shape(hipStream_t st, int *n_cus)
     return prepare_kernel<&grouped_gemm_dma_kernel<MODE, GMM1, OUT_DT, TM, NSTAGE, RG, WSTREAM, SH>, S::LDS_BYTES>(st, n_cus);
 }
 
-template <int MODE, bool GMM1, int OUT_DT, int TM>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1>
 int32_t prepare_stream(hipStream_t st, int *n_cus)
 {
-    return prepare_kernel<&grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM>, StreamShape<MODE, TM>::LDS_BYTES>(st, n_cus);
+    return prepare_kernel<&grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT>, StreamShape<MODE, TM, SPLIT>::LDS_BYTES>(st, n_cus);
 }
 
 template <int MODE, bool GMM1, int OUT_DT>
@@ -890,16 +890,16 @@ int32_t launch_dma_shape(const GemmParams &p, int n_tiles, hipStream_t st)
 }
 
 /* the streaming kernel: every XCD gets a workgroup for each tile it can have (a partial row tile per expert with rows at most) */
-template <int MODE, bool GMM1, int OUT_DT, int TM>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1>
 int32_t launch_stream(const GemmParams &p, int n_tiles, hipStream_t st)
 {
-    using S = StreamShape<MODE, TM>;
+    using S = StreamShape<MODE, TM, SPLIT>;
     int n_cus = 0;
-    const int32_t rc = prepare_stream<MODE, GMM1, OUT_DT, TM>(st, &n_cus);
+    const int32_t rc = prepare_stream<MODE, GMM1, OUT_DT, TM, SPLIT>(st, &n_cus);
     if (rc != ZBALHIP_OK) return rc;
     const int64_t partial = p.max_rows < p.experts ? p.max_rows : p.experts;
-    const int64_t per_xcd = (p.max_rows / TM + partial) * ((n_tiles + 7) / 8);
-    grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM><<<(unsigned)(8 * per_xcd), S::THREADS, S::LDS_BYTES, st>>>(p);
+    const int64_t per_xcd = (p.max_rows / TM + partial) * ((n_tiles * SPLIT + 7) / 8);
+    grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT><<<(unsigned)(8 * per_xcd), S::THREADS, S::LDS_BYTES, st>>>(p);
     return zbalhip_check_launch();
 }
 
@@ -987,6 +987,22 @@ inline int stream_rows(const GemmParams &p, int n_tiles)
     return rows <= low * e ? R::LOW : (rows <= tall * e ? R::TALL : 0);
 }
 
+/*
+ * A token or two: where the experts that can have rows make tiles for half of the CUs at most, two workgroups share each of
+ * them, four waves and half of the channels to either, because what one CU takes from memory (30 GB/s) is the limit then.
+ * Tiles of 16 rows, since there are hardly more. Rows in all, us for whole tiles -> halves (quarters):
+ *   - 8 of 32 experts, 7168 x 4096, 128 tiles: W8A8 first GEMM 49.7 -> 41.9 (43.1); second, 224 tiles of 2048 x 7168: 19.3 (19.5);
+ *   - 8 of 128, 4096 x 3072 / 1536 x 4096, 96 / 128 tiles: W8A8 30.7 -> 22.9 (24.7) / 11.8 -> 10.2 (10.4), W4A8 19.9 -> 18.1
+ *     (20.4) / 7.9 -> 6.8 (7.4); 16 rows, 192 / 256 tiles: W8A8 36.6 (37.9) / 17.4 (17.1), W4A8 23.5 (24.8) / 10.3 (10.2);
+ *   - 6 of 64, 2048 x 2048 / 1024 x 2048, 48 tiles: W8A8 18.5 -> 14.6 (14.0) / 8.0 -> 6.0 (5.1), W4A8 14.4 -> 14.0 (14.9) /
+ *     5.9 -> 5.1 (5.0), fp8 second 8.2 -> 6.0 (5.5); 12 rows, 96 tiles: fp8 second 8.6 -> 6.9, W4A8 14.4 (14.5) / 6.2 -> 5.3.
+ */
+inline bool few_tiles(const GemmParams &p, int n_tiles)
+{
+    const int64_t rows = p.max_rows, e = p.experts, busy = rows < e ? rows : e;
+    return p.K % 512 == 0 && busy * n_tiles * 2 <= cu_count() && (rows <= 16 || rows <= 8 * e);
+}
+
 /* every shape a launch of (MODE, GMM1, OUT_DT) can take */
 template <int MODE, bool GMM1, int OUT_DT>
 int32_t prepare_mode()
@@ -998,6 +1014,9 @@ int32_t prepare_mode()
     if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 64, F::STAGES_64, F::RG, true>(nullptr, &n);
     if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, StreamRows<MODE, GMM1>::LOW>(nullptr, &n);
     if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, StreamRows<MODE, GMM1>::TALL>(nullptr, &n);
+    if constexpr (!(MODE == MODE_FP8 && GMM1)) {
+        if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, 16, 2>(nullptr, &n);
+    }
     if constexpr (MODE == MODE_W4A8) {
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, 2, false>(nullptr, &n);
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 192, 3, 2, false>(nullptr, &n);
@@ -1065,6 +1084,9 @@ int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
 {
     using R = StreamRows<MODE, GMM1>;
     const int stream = stream_rows<MODE, GMM1>(p, n_tiles);
+    if constexpr (!(MODE == MODE_FP8 && GMM1)) {
+        if (few_tiles(p, n_tiles)) return launch_stream<MODE, GMM1, OUT_DT, 16, 2>(p, n_tiles, st);
+    }
     if (stream == R::LOW) return launch_stream<MODE, GMM1, OUT_DT, R::LOW>(p, n_tiles, st);
     if (stream == R::TALL) return launch_stream<MODE, GMM1, OUT_DT, R::TALL>(p, n_tiles, st);
     if constexpr (MODE == MODE_W4A8) {

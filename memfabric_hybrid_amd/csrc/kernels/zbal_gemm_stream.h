@@ -19,6 +19,7 @@
  * weights on every pass: W8A8, 128 experts of 4096 x 3072 / 1536 x 4096, top-8, 509 tokens 487 -> 461 us, Zipf(1.2)
  * routing 508 -> 457; 64 of 2048 x 2048 / 1024 x 2048, top-6, 200 tokens 111 -> 97. W4A8, 128 experts: 20 tokens 188 -> 166,
  * 509 tokens 320 -> 271, Zipf 397 -> 294, 2048 Zipf 842 -> 562, 16384 (96 rows) 3913 -> 3749.
+ * A token or two: the tiles are halved between two workgroups of four waves (SPLIT, see few_tiles in gemm.hip).
  * The taller tiles: W8A8, 128 experts, 2048 tokens 720 -> 657, 1200 tokens Zipf 647 -> 558; fp8, 32 experts, 512 tokens 424 -> 384.
  */
 #ifndef ZBAL_GEMM_STREAM_H_
@@ -28,11 +29,11 @@
 
 namespace {
 
-template <int MODE, int TM> struct StreamShape {
+template <int MODE, int TM, int SPLIT = 1> struct StreamShape {
     /* in the taller tiles the L2 serves the weights: two slabs of look-ahead do, and leave registers for six or eight row sub-tiles */
     static constexpr int PF = TM > (MODE == MODE_FP8 ? 48 : 64) ? 2 : 4;                  /* slabs in flight, and slabs per activation chunk */
     static constexpr int MT_STEP = 4 / PF;                      /* row sub-tiles come in ones, or in twos: then two slabs of them are one transfer of every wave */
-    static constexpr int NW = 8, NT = 2, THREADS = NW * 64;
+    static constexpr int NW = 8 / SPLIT, NT = 2, THREADS = NW * 64;      /* SPLIT workgroups share a tile's channels */
     static constexpr int MTM = TM / 16;
     static constexpr int LOADS = MODE == MODE_W4A8 ? 1 : 2;     /* 16-byte loads per lane, sub-tile and slab */
     static constexpr int WRB = MODE == MODE_W4A8 ? 64 : 128;    /* bytes of a weight row per slab */
@@ -40,6 +41,7 @@ template <int MODE, int TM> struct StreamShape {
     static constexpr int SA_ROWS = TM > 64 ? 128 : 64;
     static constexpr int SA_FLOATS = MODE == MODE_FP8 ? PF * SA_ROWS : 0; /* one chunk's block scales, [slab][row] */
     static constexpr int GS_BYTES = MODE == MODE_W4A8 ? PF * BN * 2 : 0;  /* one chunk's fp16 group scales, [slab][channel] */
+    static constexpr int SA_LOADS = PF > NW ? PF / NW : 1;
     static constexpr int ES_FLOATS = MODE == MODE_FP8 ? 2 * 256 : (MODE == MODE_W8A8 ? 256 : 0) + (TM + 63) / 64 * 64;
     static constexpr int LDS_BYTES = 2 * (A_BYTES + SA_FLOATS * 4 + GS_BYTES) + ES_FLOATS * 4 + NW * TM * 4;
     static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
@@ -66,11 +68,12 @@ template <int N> __device__ __forceinline__ void wait_w(u32x4 (&w)[2][2])
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]) : "n"(N));
 }
 
-template <int MODE, bool GMM1, int OUT_DT, int TM>
-__global__ void __launch_bounds__(512, 4)
+template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1>
+__global__ void __launch_bounds__(512 / SPLIT, 4)
 grouped_gemm_stream_kernel(GemmParams p)
 {
-    using S = StreamShape<MODE, TM>;
+    static_assert(SPLIT == 1 || MODE != MODE_FP8 || !GMM1, "fp8's first GEMM requantises 128 columns, which are one workgroup's");
+    using S = StreamShape<MODE, TM, SPLIT>;
     constexpr int PF = S::PF, NT = S::NT, MTM = S::MTM, LOADS = S::LOADS, NW = S::NW, WRB = S::WRB;
     constexpr int W_BLOCK_BYTES = 128 * WRB;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -81,11 +84,11 @@ grouped_gemm_stream_kernel(GemmParams p)
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n_tiles = GMM1 ? (p.N / 2) / 128 : p.N / BN;
+    const int n_tiles = (GMM1 ? (p.N / 2) / 128 : p.N / BN) * SPLIT;
     const int K = p.K, KB = K / 128, I = p.N / 2, E = p.experts;
 
     /*
-     * This workgroup's tile. A column is one expert with rows and 256 of its channels: the weights one row tile streams. The
+     * This workgroup's tile. A column is one expert with rows and 256 / SPLIT of its channels: the weights one row tile streams. The
      * columns are dealt to the XCDs in turn, so every XCD streams the same bytes whatever the routing (a contiguous run of
      * tiles each left the XCDs of the popular experts, whose row tiles share weights in the L2, idle early); the row tiles
      * of a column follow each other on its XCD. Every wave works the tile out for itself, without a barrier.
@@ -128,6 +131,8 @@ grouped_gemm_stream_kernel(GemmParams p)
         used += __popcll(busy);
     }
     if (expert < 0) return;
+    const int part = SPLIT == 1 ? 0 : n_tile % SPLIT, chan = part * NW + wave;      /* which 32 of the tile's 256 channels are this wave's */
+    n_tile /= SPLIT;
     const int height = ((end_row - first_row + mt_e - 1) / mt_e + 15) & ~15;      /* even tiles, as in the other kernel */
     const int row_begin = first_row + m_tile * height;
     const int row_end = row_begin + height < end_row ? row_begin + height : end_row;
@@ -139,8 +144,8 @@ grouped_gemm_stream_kernel(GemmParams p)
     const uint8_t *w_src[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        const int r = GMM1 ? wave * 16 : (wave & 3) * 32 + nt * 16;
-        const int col = GMM1 ? (nt == 0 ? col0 : col1) : (wave < 4 ? col0 : col1);
+        const int r = GMM1 ? chan * 16 : (chan & 3) * 32 + nt * 16;
+        const int col = GMM1 ? (nt == 0 ? col0 : col1) : (chan < 4 ? col0 : col1);
         w_src[nt] = uniform_ptr(wb + (int64_t)col * KB * W_BLOCK_BYTES + r * WRB);
     }
     const int frag_row = lane & 15;
@@ -175,10 +180,9 @@ grouped_gemm_stream_kernel(GemmParams p)
         int lane_x = lane;
         asm volatile("" : "+v"(lane_x));           /* the lane offsets are worked out afresh: there is no register to keep them in */
         const int r = lane_x >> 3;
-        const int s = wave & (PF - 1);
 #pragma unroll
-        for (int j = 0; j < MT / S::MT_STEP; ++j) {                /* slab s of row block wave / PF + j * (8 / PF) */
-            const int rb = wave / PF + j * (NW / PF);
+        for (int j = 0; j < MT * SPLIT / S::MT_STEP; ++j) {        /* slab s of row block rb */
+            const int s = (wave + j * NW) & (PF - 1), rb = (wave + j * NW) / PF;
             int rel = rb * 8 + r;
             const uint32_t chunk16 = ((lane_x & 7) ^ (r ^ (rb & 1))) * 16;
             if (rel > last_rel) rel = last_rel;
@@ -186,15 +190,22 @@ grouped_gemm_stream_kernel(GemmParams p)
                      lds_a0 + b * S::A_BYTES + s * (TM * BKB) + rb * 1024);
         }
         if (MODE == MODE_FP8) {                                    /* 64 rows of slab s; several waves bring the same ones */
-            const int row = (TM > 64 ? (wave / PF & 1) * 64 : 0) + lane_x, rel = row > last_rel ? last_rel : row;
-            dma4_sv(p.a_scale + (int64_t)row_begin * KB + kb0 + s, (uint32_t)rel * (uint32_t)KB * 4u,
-                    lds_addr(lds_sa) + (b * S::SA_FLOATS + s * S::SA_ROWS + (TM > 64 ? (wave / PF & 1) * 64 : 0)) * 4);
+#pragma unroll
+            for (int j = 0; j < S::SA_LOADS; ++j) {
+                const int s = (wave + j * NW) & (PF - 1);
+                const int row = (TM > 64 ? (wave / PF & 1) * 64 : 0) + lane_x, rel = row > last_rel ? last_rel : row;
+                dma4_sv(p.a_scale + (int64_t)row_begin * KB + kb0 + s, (uint32_t)rel * (uint32_t)KB * 4u,
+                        lds_addr(lds_sa) + (b * S::SA_FLOATS + s * S::SA_ROWS + (TM > 64 ? (wave / PF & 1) * 64 : 0)) * 4);
+            }
         }
         if (MODE == MODE_W4A8) {
             const uint16_t *gs = scales_of<uint16_t, SHARED_IN_REGISTERS>(p, expert, (int64_t)KB * p.N);
-            const int sg = (wave >> 1) & (PF - 1);
-            gs += (int64_t)(kb0 + sg) * p.N + ((wave & 1) ? col1 : col0) * 128;
-            dma4_sv(reinterpret_cast<const float *>(gs), lane_x * 4u, lds_addr(lds_gs) + b * S::GS_BYTES + sg * (BN * 2) + (wave & 1) * 256);
+#pragma unroll
+            for (int j = 0; j < SPLIT; ++j) {                      /* 128 of the tile's 256 channels of slab sg */
+                const int t = wave + j * NW, sg = (t >> 1) & (PF - 1);
+                dma4_sv(reinterpret_cast<const float *>(gs + (int64_t)(kb0 + sg) * p.N + ((t & 1) ? col1 : col0) * 128), lane_x * 4u,
+                        lds_addr(lds_gs) + b * S::GS_BYTES + sg * (BN * 2) + (t & 1) * 256);
+            }
         }
     };
 
@@ -204,28 +215,36 @@ grouped_gemm_stream_kernel(GemmParams p)
      */
     if constexpr (MODE != MODE_FP8) {
         const uint32_t dst0 = lds_addr(lds_es);
-        if (wave < (TM + 63) / 64) {                               /* 64 token scales each */
-            const int rel = wave * 64 + lane > last_rel ? last_rel : wave * 64 + lane;
-            dma4_sv(p.a_scale + row_begin, (uint32_t)rel * 4u, dst0 + (MODE == MODE_W8A8 ? 1024 : 0) + wave * 256);
-        }
-        if (MODE == MODE_W8A8 && wave >= 4) {
-            const int w4 = wave - 4;
-            if (GMM1 || !p.wscale_is_bf16) {
-                const float *wsb = scales_of<float, SHARED_IN_REGISTERS>(p, expert, p.N);
-                const float *src = !GMM1 ? wsb + n_tile * BN + w4 * 64 : (w4 < 2 ? wsb + n_tile * 128 + w4 * 64 : wsb + I + n_tile * 128 + (w4 - 2) * 64);
-                dma4_sv(src, lane * 4u, dst0 + w4 * 256);
-            } else if (w4 < 2) {
-                const uint16_t *wsb = scales_of<uint16_t, SHARED_IN_REGISTERS>(p, expert, p.N);
-                dma4_sv(reinterpret_cast<const float *>(wsb + n_tile * BN + w4 * 128), lane * 4u, dst0 + w4 * 256);
+#pragma unroll
+        for (int j = 0; j < SPLIT; ++j) {
+            const int t = wave + j * NW;
+            if (t < (TM + 63) / 64) {                              /* 64 token scales each */
+                const int rel = t * 64 + lane > last_rel ? last_rel : t * 64 + lane;
+                dma4_sv(p.a_scale + row_begin, (uint32_t)rel * 4u, dst0 + (MODE == MODE_W8A8 ? 1024 : 0) + t * 256);
+            }
+            if (MODE == MODE_W8A8 && t >= 4) {
+                const int w4 = t - 4;
+                if (GMM1 || !p.wscale_is_bf16) {
+                    const float *wsb = scales_of<float, SHARED_IN_REGISTERS>(p, expert, p.N);
+                    const float *src = !GMM1 ? wsb + n_tile * BN + w4 * 64 : (w4 < 2 ? wsb + n_tile * 128 + w4 * 64 : wsb + I + n_tile * 128 + (w4 - 2) * 64);
+                    dma4_sv(src, lane * 4u, dst0 + w4 * 256);
+                } else if (w4 < 2) {
+                    const uint16_t *wsb = scales_of<uint16_t, SHARED_IN_REGISTERS>(p, expert, p.N);
+                    dma4_sv(reinterpret_cast<const float *>(wsb + n_tile * BN + w4 * 128), lane * 4u, dst0 + w4 * 256);
+                }
             }
         }
     } else if constexpr (MODE == MODE_FP8) {
         const int sw_stride = p.N / 128;
         const float *base = scales_of<float, SHARED_IN_REGISTERS>(p, expert, (int64_t)KB * sw_stride);
-        for (int b = (wave & 3) * 64; b < KB; b += 256) {
-            if (b + lane < KB)
-                dma4_sv(base + (wave < 4 ? col0 : col1), (uint32_t)(b + lane) * (uint32_t)sw_stride * 4u,
-                        lds_addr(lds_es) + ((wave < 4 ? 0 : 256) + b) * 4);
+#pragma unroll
+        for (int j = 0; j < SPLIT; ++j) {
+            const int t = wave + j * NW;
+            for (int b = (t & 3) * 64; b < KB; b += 256) {
+                if (b + lane < KB)
+                    dma4_sv(base + (t < 4 ? col0 : col1), (uint32_t)(b + lane) * (uint32_t)sw_stride * 4u,
+                            lds_addr(lds_es) + ((t < 4 ? 0 : 256) + b) * 4);
+            }
         }
     }
 
@@ -292,7 +311,7 @@ grouped_gemm_stream_kernel(GemmParams p)
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
                     const f32x4 part = mfma_fp8_16x16x128(w[nt], a);
-                    const float sc = sa * ((GMM1 ? nt == 1 : wave >= 4) ? sw1 : sw0);
+                    const float sc = sa * ((GMM1 ? nt == 1 : chan >= 4) ? sw1 : sw0);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(part[i], sc, accf[mt][nt][i]);
                 }
@@ -310,7 +329,7 @@ grouped_gemm_stream_kernel(GemmParams p)
                 const u32x4 pk = wr[s][nt][0];
                 w0[nt] = i32x4{lo4(pk[0]), hi4(pk[0]), lo4(pk[1]), hi4(pk[1])};
                 w1[nt] = i32x4{lo4(pk[2]), hi4(pk[2]), lo4(pk[3]), hi4(pk[3])};
-                const int r = GMM1 ? nt * 128 + wave * 16 : wave * 32 + nt * 16;
+                const int r = GMM1 ? nt * 128 + chan * 16 : chan * 32 + nt * 16;
                 const u32x2 g = *reinterpret_cast<const u32x2 *>(lds_gs + (b * PF + s) * BN + (lane >> 4) * 8 + zb_block_row_channel(r));
                 gs[nt][0] = zb_fp16_to_f32(g[0] & 0xffffu);
                 gs[nt][1] = zb_fp16_to_f32(g[0] >> 16);
@@ -370,7 +389,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     auto k_loop = [&](auto mt_tag, auto stream_tag) __attribute__((always_inline)) {
         constexpr int MT = decltype(mt_tag)::value;
         constexpr int L = NT * LOADS;                                   /* loads per slab */
-        constexpr int D = MT / S::MT_STEP + (MODE == MODE_W8A8 ? 0 : 1);      /* transfers per chunk */
+        constexpr int D = MT * SPLIT / S::MT_STEP + (MODE == MODE_W8A8 ? 0 : (MODE == MODE_FP8 ? S::SA_LOADS : SPLIT));      /* transfers per chunk */
         Slabs wr;
         issue_chunk(mt_tag, 0, 0);
 #pragma unroll
@@ -406,13 +425,14 @@ grouped_gemm_stream_kernel(GemmParams p)
     };
     auto k_loop_mt = [&](auto stream_tag) __attribute__((always_inline)) {
         constexpr int ST = S::MT_STEP;
-        if (MTM >= 4 * ST && mt_act > 3 * ST) k_loop(std::integral_constant<int, MTM >= 4 * ST ? 4 * ST : MTM>{}, stream_tag);
+        if constexpr (MTM == 1) k_loop(std::integral_constant<int, 1>{}, stream_tag);
+        else if (MTM >= 4 * ST && mt_act > 3 * ST) k_loop(std::integral_constant<int, MTM >= 4 * ST ? 4 * ST : MTM>{}, stream_tag);
         else if (MTM >= 3 * ST && mt_act > 2 * ST) k_loop(std::integral_constant<int, MTM >= 3 * ST ? 3 * ST : MTM>{}, stream_tag);
         else if (MTM >= 2 * ST && mt_act > ST) k_loop(std::integral_constant<int, MTM >= 2 * ST ? 2 * ST : MTM>{}, stream_tag);
         else k_loop(std::integral_constant<int, ST>{}, stream_tag);
     };
     /* weights that the other row tiles of the column want too stay in the L2 for them; the others leave no trace in it */
-    if (mt_e == 1) k_loop_mt(std::true_type{});
+    if (MTM == 1 || mt_e == 1) k_loop_mt(std::true_type{});
     else k_loop_mt(std::false_type{});
     if constexpr (MODE == MODE_W4A8) {
 #pragma unroll
@@ -428,7 +448,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     tc.n_tile = n_tile;
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));               /* as in the other kernel: nothing of the epilogue's stays live across the K loop */
-    epilogue<MODE, GMM1, OUT_DT, 1, MTM, NT, SHARED_IN_REGISTERS, false, MODE != MODE_FP8>(p, tc, accf, acci, row_begin, row_end, 0, wave, lane_e, lds_rowmax, TM, lds_es);
+    epilogue<MODE, GMM1, OUT_DT, 1, MTM, NT, SHARED_IN_REGISTERS, false, MODE != MODE_FP8, NW>(p, tc, accf, acci, row_begin, row_end, 0, chan, lane_e, lds_rowmax, TM, lds_es);
 }
 
 } // namespace

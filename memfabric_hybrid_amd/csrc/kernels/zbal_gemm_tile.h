@@ -119,10 +119,12 @@ __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float 
  * are dealt round-robin over the row groups, so a tile that is not full leaves every SIMD the same share). The pre-pack put channels 32*(nt/2) + 8*(lane/16) + 4*(nt%2) + i in
  * those rows (zb_block_row_channel), so the sub-tiles nt = 2s and 2s+1 together are eight consecutive channels.
  * A wave's NT channel sub-tiles are 16 * NT consecutive channels (GMM1: 8 * NT gate and the matching 8 * NT up columns).
- * `lds_rowmax` is [16 / NT][tile_rows] floats of scratch for the row maxima of the waves' channel ranges (GMM1 only);
+ * `lds_rowmax` is [COL_GROUPS][tile_rows] floats of scratch for the row maxima of the workgroup's channel ranges (GMM1 only;
+ * all of the tile's but where several workgroups share it);
  * ONE_MAX: [tile_rows], zero before, which takes the maximum over the channel ranges itself.
  */
-template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT, Shared SH, bool ONE_MAX = false, bool ROW_SCALES = MODE == MODE_W8A8>
+template <int MODE, bool GMM1, int OUT_DT, int RG, int MTM, int NT, Shared SH, bool ONE_MAX = false, bool ROW_SCALES = MODE == MODE_W8A8,
+          int COL_GROUPS = 16 / NT>
 __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &tc, f32x4 (&accf)[MTM][NT],
                                          i32x4 (&acci)[MTM][NT], int row_begin, int row_end, int wm, int wn, int lane,
                                          float *lds_rowmax, int tile_rows, const float *es)
@@ -195,7 +197,8 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
         }
     } else {
         /* SwiGLU on gate sub-tile nt and up sub-tile nt + NT/2: columns j = n_tile*128 + 32*(t/2) + q8 + 4*(t%2) + i with t = wn*NT/2 + nt */
-        constexpr int UP = NT / 2, COL_GROUPS = 16 / NT;
+        constexpr int UP = NT / 2;
+        const int group = wn % COL_GROUPS;         /* of this workgroup's */
         float sg[MTM][UP][4];
         float rmax[MTM];
 #pragma unroll
@@ -270,7 +273,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
             if (lane < 16) {
                 float *at = lds_rowmax + (RG * mt + wm) * 16 + lane;
                 if (ONE_MAX) atomicMax(reinterpret_cast<uint32_t *>(at), __float_as_uint(rmax[mt]));      /* not negative, no NaN: ordered as integers */
-                else at[wn * tile_rows] = rmax[mt];
+                else at[group * tile_rows] = rmax[mt];
             }
         }
         lds_barrier();
@@ -279,7 +282,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const TileCoord &t
          * reduced the maxima and stored after the barrier before: first GEMM at 1024 rows per expert, 128 experts of 4096 x 3072,
          * W8A8 1781 -> 1715 us, W4A8 2199 -> 2158.)
          */
-        if (MODE != MODE_FP8 && wn != 0) return;
+        if (MODE != MODE_FP8 && group != 0) return;
 #pragma unroll
         for (int mt = 0; mt < MTM; ++mt) {
             const int lr = (RG * mt + wm) * 16 + frag_row;

@@ -194,3 +194,35 @@ def test_many_tiles_per_workgroup_are_the_same_rows(buf, mode):
         r = slice(int(off[e]), int(off[e + 1]))
         got = gmm2(buf, a[r].contiguous(), xs[r].contiguous(), w[e:e + 1], ws[e:e + 1], capi.DT_FP32, counts[e:e + 1], K, N, mode)
         assert torch.equal(whole[r].view(torch.int16), got.view(torch.int16)), e
+
+
+@pytest.mark.parametrize("counts", [[1], [16], [0, 17, 1], [0] * 20 + [1] + [0] * 50 + [2, 1] + [0] * 57, [3, 0, 8, 33]])
+@pytest.mark.parametrize("K,N", STREAM_SHAPES)
+def test_tiles_shared_by_two_workgroups(buf, counts, K, N):
+    """A handful of rows: every mode, channel scales of either type, experts without rows and just past a tile's 16."""
+    counts = np.array(counts, dtype=np.int64)
+    E, rows = len(counts), int(counts.sum())
+    a = rng(1).integers(-128, 128, (rows, K)).astype(np.int8)
+    xs = rng(2).uniform(0.005, 0.05, rows).astype(np.float32)
+    w = rng(3).integers(-128, 128, (E, K, N)).astype(np.int8)
+    ws = rng(4).uniform(0.0015, 0.0045, (E, N)).astype(np.float32)
+    packed = buf.prepack_weight(dev(w))
+    for dt, s in ((capi.DT_FP32, ws), (capi.DT_BF16, zo.f32_to_bf16(ws))):
+        assert np.array_equal(host(gmm2(buf, dev(a), dev(xs), packed, dev(s), dt, counts, K, N, 1)),
+                              zo.grouped_gemm_w8a8_dequant(a, xs, w, s, counts))
+    q2, s2, _ = gmm1(buf, dev(a), dev(xs), packed, dev(ws), counts, K, N, 1)
+    r_q2, r_s2 = zo.gmm1_swiglu_quant_w8a8(a, xs, w, ws, counts)[:2]
+    assert np.array_equal(host(s2).view(np.uint32), r_s2.view(np.uint32)) and np.array_equal(host(q2), r_q2)
+
+    w = rng(5).integers(-8, 8, (E, K, N)).astype(np.int8)
+    gs = rng(6).uniform(0.001, 0.01, (E, K // 128, N)).astype(np.float16).view(np.uint16)
+    packed = buf.prepack_weight(dev(w), int4=True)
+    assert np.array_equal(host(gmm2(buf, dev(a), dev(xs), packed, dev(gs), capi.DT_FP16, counts, K, N, 3)),
+                          zo.gmm2_w4a8(a, xs, w, gs, counts))
+    q2, s2, _ = gmm1(buf, dev(a), dev(xs), packed, dev(gs), counts, K, N, 3)
+    r_q2, r_s2, _ = zo.gmm1_swiglu_quant_w4a8(a, xs, w, gs, counts)
+    assert np.array_equal(host(s2).view(np.uint32), r_s2.view(np.uint32)) and np.array_equal(host(q2), r_q2)
+
+    a, sa, w, sw = fp8_operands(E, K, N, rows, 20)
+    y = gmm2(buf, dev(a), dev(sa), buf.prepack_weight(dev(w)), dev(sw), capi.DT_FP32, counts, K, N, 2)
+    assert_fp8_close(zo.bf16_to_f32(host(y)), zo.bf16_to_f32(zo.gmm2_fp8(a, sa, w, sw, counts)), "fp8 GEMM", FP8_GEMM_ELEM_TOL)
