@@ -182,6 +182,23 @@ def test_combine_normal_exact_and_round_trip(buf, T, H, K, E):
     assert calc_diff(zo.bf16_to_f32(host(out)), zo.bf16_to_f32(x) * wv) < 5e-5
 
 
+@pytest.mark.parametrize("E", [63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("T", [1, 200, 2048])
+def test_combine_at_the_limits_of_its_expert_bases(buf, T, E):
+    """Every expert has rows once there are enough picks, the last ones among them; exclusive bases and running sums."""
+    H, K = 64, 3
+    x = bf16_normal((T, H), 51)
+    idx = distinct_topk(T, E, K, 52)
+    idx[0] = [E - 1, 0, E // 2]
+    w = rng(53).uniform(0.05, 1.0, (T, K)).astype(np.float32)
+    recv, _, h, r_dest, _, rows, put, r_send = run_dispatch(buf, x, zo.DT_BF16, idx, E, capi.NO_QUANT)
+    assert np.array_equal(host(buf.combine(recv, h, dev(w))), zo.combine(r_dest, zo.DT_BF16, put, w, idx.astype(np.int32), r_send, E))
+    recv, _, _, h = buf.low_latency_dispatch(dev(x), dev(idx), T, E, use_fp8=False)
+    r_ex, _, r_eidx, _, r_counts = zo.dispatch_low_latency(x, zo.DT_BF16, idx.astype(np.int32), E, 0, T * K)
+    assert np.array_equal(host(buf.low_latency_combine(recv, dev(w), h)),
+                          zo.combine_low_latency(r_ex, zo.DT_BF16, idx.astype(np.int32), r_eidx, r_counts, w, E))
+
+
 def test_combine_fp16(buf):
     T, H, K, E = 20, 256, 4, 8
     x = zo.f32_to_fp16(rng(14).standard_normal((T, H)).astype(np.float32))
