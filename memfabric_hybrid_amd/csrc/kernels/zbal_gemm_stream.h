@@ -308,12 +308,20 @@ grouped_gemm_stream_kernel(GemmParams p)
             for (int mt = 0; mt < MT; ++mt) {
                 const i32x8 a = load_a(mt);
                 const float sa = lds_sa[b * S::SA_FLOATS + s * S::SA_ROWS + mt * 16 + frag_row];
+                /*
+                 * As in the W4A8 loop below, the MFMAs first: 150 rows per expert, 32 of 7168 x 4096 / 2048 x 7168, 264 -> 260 / 133 ->
+                 * 132 us; 400 rows, 64 of 2048 x 2048 / 1024 x 2048, 168 -> 166 / 88.6 -> 86.4. (W8A8, which has nothing to convert: 0 / +1 %.)
+                 */
+                f32x4 part[NT];
+                __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) part[nt] = mfma_fp8_16x16x128(w[nt], a);
+                __builtin_amdgcn_s_setprio(0);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
-                    const f32x4 part = mfma_fp8_16x16x128(w[nt], a);
                     const float sc = sa * ((GMM1 ? nt == 1 : chan >= 4) ? sw1 : sw0);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(part[i], sc, accf[mt][nt][i]);
+                    for (int i = 0; i < 4; ++i) accf[mt][nt][i] = __builtin_fmaf(part[nt][i], sc, accf[mt][nt][i]);
                 }
                 asm volatile("" ::: "memory");
             }
