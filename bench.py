@@ -278,7 +278,7 @@ def bench_moe(args, torch, np, capi, buf, workload):
                     "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": wbytes1 / t1 / 1e9 / PEAK_HBM_GBS, "traffic": None,
                     "experts_with_tokens": touched}
     else:
-        kname = {1: "grouped_gemm_dma_kernel<int8, gmm1>", 2: "grouped_gemm_dma_kernel<fp8, gmm1>",
+        kname = {1: "grouped_gemm_tall_kernel<int8, gmm1>", 2: "grouped_gemm_tall_kernel<fp8, gmm1>",
                  3: "grouped_gemm_stream_kernel<w4a8, gmm1>"}[mode]
         routed = workload in ("prefill", "qwen_w4a8") and T == cfg["T"] and not args.equal_rows
         roofline = {"kernel": kname, "bound": "mfma", "achieved": flops1 / t1 / 1e12,
