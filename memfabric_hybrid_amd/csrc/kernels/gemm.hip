@@ -854,24 +854,24 @@ int32_t prepare_stream(hipStream_t st, int *n_cus)
     return prepare_kernel<&grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT>, StreamShape<MODE, TM, SPLIT>::LDS_BYTES>(st, n_cus);
 }
 
-template <int MODE, bool GMM1, int OUT_DT>
+template <int MODE, bool GMM1, int OUT_DT, bool ANY_K = false>
 int32_t prepare_tall(hipStream_t st, int *n_cus)
 {
-    return prepare_kernel<&grouped_gemm_tall_kernel<MODE, GMM1, OUT_DT>, TallShape<MODE>::LDS_BYTES>(st, n_cus);
+    return prepare_kernel<&grouped_gemm_tall_kernel<MODE, GMM1, OUT_DT, ANY_K>, TallShape<MODE>::LDS_BYTES>(st, n_cus);
 }
 
 /* launched with one persistent workgroup per CU, or fewer when there are not that many tiles */
-template <int MODE, bool GMM1, int OUT_DT>
+template <int MODE, bool GMM1, int OUT_DT, bool ANY_K = false>
 int32_t launch_tall(const GemmParams &p, int n_tiles, hipStream_t st)
 {
     using S = TallShape<MODE>;
     int n_cus = 0;
-    const int32_t rc = prepare_tall<MODE, GMM1, OUT_DT>(st, &n_cus);
+    const int32_t rc = prepare_tall<MODE, GMM1, OUT_DT, ANY_K>(st, &n_cus);
     if (rc != ZBALHIP_OK) return rc;
     unsigned grid = grid_for(p.max_rows, p.experts, n_tiles, S::TM);
     const unsigned resident = (unsigned)(n_cus + 7) / 8 * 8;
     if (grid > resident) grid = resident;
-    grouped_gemm_tall_kernel<MODE, GMM1, OUT_DT><<<grid, S::THREADS, S::LDS_BYTES, st>>>(p);
+    grouped_gemm_tall_kernel<MODE, GMM1, OUT_DT, ANY_K><<<grid, S::THREADS, S::LDS_BYTES, st>>>(p);
     return zbalhip_check_launch();
 }
 
@@ -1023,6 +1023,9 @@ int32_t prepare_mode()
     } else {
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 256, 2, 4, false, SHARED_NONE>(nullptr, &n);
         if (rc == ZBALHIP_OK) rc = prepare_tall<MODE, GMM1, OUT_DT>(nullptr, &n);
+        if constexpr (MODE == MODE_FP8) {
+            if (rc == ZBALHIP_OK) rc = prepare_tall<MODE, GMM1, OUT_DT, true>(nullptr, &n);
+        }
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, F::RG, true>(nullptr, &n);
     }
     return rc;
@@ -1116,9 +1119,15 @@ int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
          * Many rows: at every count against what ran there before (320-row tiles on four row groups of waves, fp8 beyond 1536 rows
          * per expert the 256-row shape below), both GEMMs, 32 experts of 7168 x 4096 / 2048 x 7168, 64 of 2048 x 2048 /
          * 1024 x 2048, 8 of 4096 x 28672 / 14336 x 4096, 250 to 2300 rows per expert: fp8 -8 / -11 % (0 ... -21), W8A8
-         * -10 / -8 % (+1 ... -15). 1024 rows of the first: fp8 1047 / 596 -> 935 / 543 us, W8A8 974 / 519 -> 905 / 468.
+         * -10 / -8 % (+1 ... -15). 1024 rows of the first: fp8 1047 / 596 -> 935 / 543 us, W8A8 974 / 519 -> 905 / 468. The kernel for
+         * any fp8 K, 256 to 1800 rows of twelve such K from 256 to 32768: -11 % (+5 ... -25).
          */
-        if (tall_accepts<MODE>(p)) return launch_tall<MODE, GMM1, OUT_DT>(p, n_tiles, st);
+        if (tall_accepts<MODE>(p)) {
+            if constexpr (MODE == MODE_FP8) {
+                if (tall_wants_any_k(p.K / 128)) return launch_tall<MODE, GMM1, OUT_DT, true>(p, n_tiles, st);
+            }
+            return launch_tall<MODE, GMM1, OUT_DT>(p, n_tiles, st);
+        }
         /*
          * This shape's K loop has no scalar register to spare for a shared expert's tensors, and with this many rows per
          * expert the fused layer's takes turns with the routed ones: 2048 rows fp8, first GEMM 2.01 ms with the shared

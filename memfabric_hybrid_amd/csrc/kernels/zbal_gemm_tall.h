@@ -33,29 +33,39 @@ template <int MODE> struct TallShape {
     static constexpr int TM = 320, THREADS = 512, RG = 2, COL_GROUPS = 4, NT = 4, MTM = 10;
     static constexpr int HALF = 4;                              /* sub-tiles per wave in the first part: 128 rows of the tile */
     static constexpr int A_BYTES = TM * BKB, STAGE_BYTES = A_BYTES + BN * 128;
-    static constexpr int MAX_KB = 128, MAX_EXPERTS = 512, TABLE = 32;
+    static constexpr int MAX_KB = 256, MAX_EXPERTS = 512, TABLE = 32;
     static constexpr int SA_FLOATS = MODE == MODE_FP8 ? TM * 4 : 0;                      /* four steps' block scales, [row][step] */
-    static constexpr int SC_FLOATS = MODE == MODE_FP8 ? 2 * MAX_KB : 256 + TM;           /* fp8: weight block scales; W8A8: channel and token scales */
+    static constexpr int SC_FLOATS = MODE == MODE_FP8 ? MAX_KB : 256 + TM;               /* fp8: weight block scales, twice 128; W8A8: channel and token scales */
     static constexpr int LDS_BYTES = 2 * (STAGE_BYTES + SA_FLOATS * 4 + SC_FLOATS * 4) + TM * 4 + TABLE * 16 + (MAX_EXPERTS + 1) * 4;
     static_assert(LDS_BYTES <= 160 * 1024, "tile does not fit the LDS");
 };
 
 /*
- * fp8's scales travel as four steps of a row, and a tile's last step on its own (KB % 4 = 1) would want a third buffer for
- * them; the tables end the number of experts and fp8's K.
+ * The tables end the number of experts. fp8's scales travel as four steps of a row: rows of fewer are read along with a
+ * neighbour's, which wants a tile without the first or the last row of all.
  */
 template <int MODE> inline bool tall_accepts(const GemmParams &p)
 {
     const int kb = p.K / 128;
     if (kb < 2 || p.experts > TallShape<MODE>::MAX_EXPERTS) return false;
-    return MODE != MODE_FP8 || (kb >= 4 && kb % 4 != 1 && kb <= TallShape<MODE>::MAX_KB);
+    return MODE != MODE_FP8 || (kb <= TallShape<MODE>::MAX_KB && (kb >= 4 || p.max_rows > TallShape<MODE>::TM));
 }
 
-template <int MODE, bool GMM1, int OUT_DT>
+/*
+ * fp8: K whose steps leave one over from groups of four, make less than one group, or are more than the weight block scales have
+ * room for twice, take a kernel of their own (ANY_K), because what it asks in every step costs the others: 1024 rows per expert,
+ * 32 experts of 7168 x 4096 / 2048 x 7168, 990 -> 1010 / 532 -> 550 us. Those K in the 256-row shape -> in ANY_K, first GEMM 4096 wide,
+ * second 7168: 32 experts, K 1152, 256 rows 73 -> 57 us, 512 rows 113 -> 100, 1800 rows 338 -> 325; K 5248, 256 rows 335 -> 223, 1024
+ * rows 818 -> 757; K 256, 512 rows 51 -> 44; second, K 640, 512 rows 157 -> 126, K 384 126 -> 98; 8 experts, K 17408, 300 rows 454 -> 278.
+ */
+inline bool tall_wants_any_k(int kb) { return kb < 4 || kb % 4 == 1 || kb > 128; }
+
+template <int MODE, bool GMM1, int OUT_DT, bool ANY_K = false>
 __global__ void __launch_bounds__(512, 2)
 grouped_gemm_tall_kernel(GemmParams p)
 {
     static_assert(MODE == MODE_W8A8 || MODE == MODE_FP8, "8-bit modes");
+    static_assert(!ANY_K || MODE == MODE_FP8, "W8A8 has no scales by step");
     using S = TallShape<MODE>;
     constexpr Shared SH = SHARED_ON_DEMAND;
     constexpr int TM = S::TM, RG = S::RG, NT = S::NT, MTM = S::MTM, H = S::HALF, A_BYTES = S::A_BYTES, STAGE_BYTES = S::STAGE_BYTES;
@@ -101,13 +111,22 @@ grouped_gemm_tall_kernel(GemmParams p)
     const int id0 = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
     const int id_end = ((int)(blockIdx.x & 7) + 1) * chunk < total ? ((int)(blockIdx.x & 7) + 1) * chunk : total;
     if (id0 >= id_end) return;
+    /* ANY_K has no registers for what the compiler would work out of `lane` ahead of the loops */
+    auto fresh_lane = [&]() __attribute__((always_inline)) {
+        int l = lane;
+        if constexpr (ANY_K) asm volatile("" : "+v"(l));
+        return l;
+    };
     /* tiles `from` .. `from` + 31 of this workgroup's sequence, one per lane of wave 0 */
     auto make_table = [&](int from) __attribute__((always_inline)) {
-        const int id = id0 + (from + lane) * slots;
-        if (wave != 0 || lane >= S::TABLE) return;
+        const int lane_t = fresh_lane();
+        int n_tiles_t = n_tiles;
+        if constexpr (ANY_K) asm volatile("" : "+s"(n_tiles_t));
+        const int id = id0 + (from + lane_t) * slots;
+        if (wave != 0 || lane_t >= S::TABLE) return;
         int expert = -1, n_tile = 0, row_begin = 0, row_end = 0;
         if (id < id_end) {
-            const int q = id / n_tiles;
+            const int q = id / n_tiles_t;
             int lo = 0, hi = E;                                       /* mtp[lo] <= q < mtp[hi] */
             while (hi - lo > 1) {
                 const int mid = (lo + hi) >> 1;
@@ -115,7 +134,7 @@ grouped_gemm_tall_kernel(GemmParams p)
                 else hi = mid;
             }
             expert = lo;
-            const int first = lds_mtp[lo], mt_e = lds_mtp[lo + 1] - first, l = id - first * n_tiles;
+            const int first = lds_mtp[lo], mt_e = lds_mtp[lo + 1] - first, l = id - first * n_tiles_t;
             int group_n = slots / mt_e;
             group_n = group_n < 1 ? 1 : (group_n > GROUP_N ? GROUP_N : group_n);
             const int per_group = mt_e * group_n, ng = l / per_group, r = l - ng * per_group;
@@ -125,7 +144,7 @@ grouped_gemm_tall_kernel(GemmParams p)
             row_begin = first_row + r % mt_e * height;
             row_end = row_begin + height < end_row ? row_begin + height : end_row;
         }
-        *reinterpret_cast<i32x4 *>(lds_tiles + lane * 4) = i32x4{expert, n_tile, row_begin, row_end};
+        *reinterpret_cast<i32x4 *>(lds_tiles + lane_t * 4) = i32x4{expert, n_tile, row_begin, row_end};
     };
     struct Tile {
         int expert, n_tile, row_begin, row_end, last_rel;
@@ -168,22 +187,43 @@ grouped_gemm_tall_kernel(GemmParams p)
         if (rel > (uint32_t)t.last_rel) rel = t.last_rel;
         dma16_sv(t.a + (int64_t)kb * BKB, __umul24(rel, (uint32_t)K) + t_chunk, lds0 + stage * STAGE_BYTES + j * 8192);
     };
-    /* fp8: the scales of steps kb .. kb + 3 (the last four where there are fewer), 64 rows per wave, by waves 0-4 */
+    /*
+     * fp8's activation scales come in groups of four steps, to two buffers in turn. The last group of a tile brings the row's
+     * last four values, whatever it uses of them. It starts at step `tail`; where four would leave one step over, the last two
+     * groups have three and two, because the group after the next may not come before this one has been used up. A row of two
+     * or three values comes with the end of the row before it, in the tile of the very first row with the start of the one behind.
+     */
+    const int tail = !ANY_K ? 0 : (KB % 4 == 1 ? KB - 2 : (KB - 1) & ~3);
+    auto starts_group = [&](int kb) __attribute__((always_inline)) { return ANY_K ? kb == tail || (kb < tail && (kb & 3) == 0) : (kb & 3) == 0; };
+    /* a step's place among its group's four values */
+    auto place = [&](const Tile &t, int kb) __attribute__((always_inline)) {
+        return kb < tail ? kb & 3 : (KB < 4 && t.row_begin == 0 ? kb : kb - (KB - 4));
+    };
+    /* the group that starts with step kb, 64 rows per wave, by waves 0-4 */
     auto bring_sa = [&](const Tile &t, int kb, int half) __attribute__((always_inline)) {
         if (MODE != MODE_FP8 || wave >= TM / 64) return;
-        uint32_t rel = wave * 64 + lane;
+        uint32_t rel = wave * 64 + fresh_lane();
         if (rel > (uint32_t)t.last_rel) rel = t.last_rel;
-        dma16_sv(reinterpret_cast<const uint8_t *>(t.sa + (kb + 4 > KB ? KB - 4 : kb)), __umul24(rel, (uint32_t)KB * 4u), lds_addr(lds_sa) + (half * S::SA_FLOATS + wave * 256) * 4);
+        const int from = ANY_K ? kb - place(t, kb) : (kb + 4 > KB ? KB - 4 : kb);
+        dma16_sv(reinterpret_cast<const uint8_t *>(t.sa + from), __umul24(rel, (uint32_t)KB * 4u), lds_addr(lds_sa) + (half * S::SA_FLOATS + wave * 256) * 4);
     };
-    /* fp8: the weight block scales of every step; W8A8: what the epilogue scales with (channels at 0, tokens at 256) */
-    auto bring_scales = [&](const Tile &t, int buf) __attribute__((always_inline)) {
+    /*
+     * fp8: the weight block scales of up to 128 steps, for either 128 of the channels, to one of two buffers in turn. With more
+     * steps the two are one: the second 128 (`upper`) come beside the tile's first step, the next tile's first 128 once all
+     * of this one's have been used. W8A8: what the epilogue scales with (channels at 0, tokens at 256).
+     */
+    int bufs = ANY_K && KB > 128 ? 1 : 2;
+    if constexpr (ANY_K) asm volatile("" : "+s"(bufs));                 /* or the compiler keeps `buf` in a vector register */
+    const int second = ANY_K && KB > 128 ? 256 : 128;                   /* where the second 128 channels' start */
+    auto bring_scales = [&](const Tile &t, int buf, bool upper = false) __attribute__((always_inline)) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr(lds_sc) + buf * S::SC_FLOATS * 4);
         if constexpr (MODE == MODE_FP8) {
             const int stride = p.N / 128;
             const float *base = scales_of<float, SH>(p, t.expert, (int64_t)KB * stride) +
                                 (wave < 4 ? (GMM1 ? t.n_tile : t.n_tile * 2) : (GMM1 ? I / 128 + t.n_tile : t.n_tile * 2 + 1));
             const int b = (wave & 3) * 64;
-            if (b + lane < KB) dma4_sv(base, (uint32_t)(b + lane) * (uint32_t)stride * 4u, dst + ((wave < 4 ? 0 : S::MAX_KB) + b) * 4);
+            const int step = b + fresh_lane();
+            if ((!ANY_K || (b >= 128) == upper) && step < KB) dma4_sv(base, (uint32_t)step * (uint32_t)stride * 4u, dst + ((wave < 4 ? 0 : second) + b) * 4);
         } else {
             if (wave < TM / 64) {
                 const int rel = wave * 64 + lane > t.last_rel ? t.last_rel : wave * 64 + lane;
@@ -246,7 +286,7 @@ grouped_gemm_tall_kernel(GemmParams p)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) wf[nt] = load_w(nt);
     a[0] = load_a(0);
-    sa[0] = load_sa(0, 0);
+    sa[0] = load_sa(0, ANY_K ? place(cur, 0) : 0);
 
     while (true) {
         if ((++seq & (S::TABLE - 1)) == 0) {
@@ -267,7 +307,7 @@ grouped_gemm_tall_kernel(GemmParams p)
             }
         const int mt_act = (((cur.row_end - cur.row_begin + 15) >> 4) - wm + RG - 1) / RG;
         /* GMM1: gate and up have a weight block each; GMM2: the wave's channels are in one */
-        const float *sw0_at = lds_sc + buf * S::SC_FLOATS + (!GMM1 && wn >= 2 ? S::MAX_KB : 0), *sw1_at = lds_sc + buf * S::SC_FLOATS + S::MAX_KB;
+        const float *sw0_at = lds_sc + buf * S::SC_FLOATS + (!GMM1 && wn >= 2 ? second : 0), *sw1_at = lds_sc + buf * S::SC_FLOATS + second;
         float sw0 = 0.0f, sw1 = 0.0f;
         if constexpr (MODE == MODE_FP8) {
             sw0 = sw0_at[0];
@@ -317,7 +357,7 @@ grouped_gemm_tall_kernel(GemmParams p)
             const bool in2 = kb + 1 < KB, in1 = kb + 2 < KB;
             const Tile &t2 = in2 ? cur : nxt, &t1 = in1 ? cur : nxt;        /* whose slabs the two parts that are asked for in this step belong to */
             const int kb2 = in2 ? kb + 1 : 0, kb1 = in1 ? kb + 2 : kb + 2 - KB;
-            const int st = stage, k4 = kb + 4 - (kb & 3) > KB ? kb - (KB - 4) : kb & 3;      /* this step's place among the four */
+            const int st = stage, k4 = ANY_K ? place(cur, kb) : (kb + 4 - (kb & 3) > KB ? kb - (KB - 4) : kb & 3);
             int act = mt_act;
             asm volatile("" : "+s"(act));       /* compared where it is asked for: ten conditions in scalar registers push others out */
             i32x8 az;
@@ -327,8 +367,14 @@ grouped_gemm_tall_kernel(GemmParams p)
                 if (mt == H - 1) {
                     landed();
                     if (kb == 0) {             /* everybody is past the last tile's epilogue */
-                        if (more) bring_scales(nxt, buf ^ 1);
-                        if (GMM1 && tid < TM) lds_rowmax[tid] = 0.0f;
+                        if (!ANY_K && more) bring_scales(nxt, buf ^ 1);
+                        if constexpr (ANY_K) {
+                            if (GMM1 && wave < TM / 64) lds_rowmax[wave * 64 + fresh_lane()] = 0.0f;
+                        } else if (GMM1 && tid < TM) lds_rowmax[tid] = 0.0f;
+                    }
+                    if (ANY_K && (kb == 0 || (KB > 128 && kb == 127))) {
+                        const bool upper = KB > 128 && kb == 0;
+                        if (upper || more) bring_scales(upper ? cur : nxt, buf ^ (bufs - 1), upper);
                     }
                     az = load_a(H);
                     saz = load_sa(H, k4);
@@ -356,7 +402,7 @@ grouped_gemm_tall_kernel(GemmParams p)
                 if (mt == FIRST) { bring_w(t1, kb1, st, 0); bring_w(t1, kb1, st, 1); }
                 if (mt == FIRST + 1) { bring_w(t1, kb1, st, 2); bring_w(t1, kb1, st, 3); }
                 if (mt == FIRST + 2) { bring_a(t1, kb1, st, 0); bring_a(t1, kb1, st, 1); }
-                if (mt == FIRST + 3 && MODE == MODE_FP8 && (kb1 & 3) == 0) bring_sa(t1, kb1, half ^ 1);
+                if (mt == FIRST + 3 && MODE == MODE_FP8 && starts_group(kb1)) bring_sa(t1, kb1, half ^ 1);
                 if (mt < act) {
                     if (mt + 1 < MTM) {
                         a[b ^ 1] = load_a(mt + 1);
@@ -367,10 +413,10 @@ grouped_gemm_tall_kernel(GemmParams p)
                 __builtin_amdgcn_sched_barrier(0);
             }
             stage ^= 1;
-            if (k4 == 3) half ^= 1;                        /* and the last four of a tile end with its last step */
+            if (ANY_K ? starts_group(kb2) : k4 == 3) half ^= 1;        /* the last group of a tile ends with its last step */
             landed();
             a[0] = load_a(0);
-            sa[0] = load_sa(0, kb2 + 4 - (kb2 & 3) > KB ? kb2 - (KB - 4) : kb2 & 3);
+            sa[0] = load_sa(0, ANY_K ? place(t2, kb2) : (kb2 + 4 - (kb2 & 3) > KB ? kb2 - (KB - 4) : kb2 & 3));
             sub_tile(H, az, saz, std::true_type{});
             sw0 = sw0_n;
             sw1 = sw1_n;
@@ -386,7 +432,7 @@ grouped_gemm_tall_kernel(GemmParams p)
                                                             lds_sc + buf * S::SC_FLOATS);
         if (!more) break;
         cur = nxt;
-        buf ^= 1;
+        buf ^= bufs - 1;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       /* the LDS goes to another workgroup */
 }

@@ -1,0 +1,61 @@
+"""Which shapes the grouped GEMM's kernel for many rows takes, asked of the rule itself (no GPU needed: it is host code)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from memfabric_hybrid_amd import build
+
+HIPCC = os.path.join(build.ROCM, "bin", "hipcc")
+
+PROGRAM = r"""
+#include <cstdio>
+#include <hip/hip_runtime.h>
+#include <type_traits>
+#include "zbal_gemm_tall.h"
+
+int main()
+{
+    int mode, slabs, experts, rows;
+    while (scanf("%d %d %d %d", &mode, &slabs, &experts, &rows) == 4) {
+        GemmParams p = {};
+        p.K = slabs * 128;
+        p.experts = experts;
+        p.max_rows = rows;
+        printf("%d\n", mode == MODE_FP8 ? tall_accepts<MODE_FP8>(p) : tall_accepts<MODE_W8A8>(p));
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def accepts(tmp_path_factory):
+    if not (os.path.exists(HIPCC) or shutil.which("hipcc")):
+        pytest.skip("hipcc not available")
+    d = tmp_path_factory.mktemp("dispatch")
+    (d / "accepts.hip").write_text(PROGRAM)
+    cmd = [HIPCC] + build.HIP_FLAGS + build.INCLUDES + [str(d / "accepts.hip"), "-o", str(d / "accepts")]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0, r.stdout
+
+    def ask(cases):
+        out = subprocess.run([str(d / "accepts")], input="".join("%d %d %d %d\n" % c for c in cases), capture_output=True, text=True)
+        assert out.returncode == 0, out.stderr
+        return [v == "1" for v in out.stdout.split()]
+    return ask
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+def test_the_many_row_kernel_takes_every_k(accepts, mode):
+    """Two to 256 steps of 128 (the entry points take no more), at any number of experts that its tables hold."""
+    cases = [(mode, kb, e, 256 * e) for kb in range(2, 257) for e in (2, 32, 512)]
+    got = accepts(cases)
+    assert len(got) == len(cases) and all(got), [c for c, ok in zip(cases, got) if not ok][:5]
+
+
+def test_the_many_row_kernel_refuses_what_it_has_no_room_for(accepts):
+    # a single step; more experts than the tables hold; fp8 rows of two or three scales where one tile has all rows
+    refused = [(1, 1, 8, 4096), (2, 1, 8, 4096), (1, 8, 513, 1 << 20), (2, 8, 513, 1 << 20), (2, 2, 1, 320), (2, 3, 1, 320)]
+    taken = [(1, 2, 1, 320), (2, 2, 1, 321), (2, 3, 1, 321), (2, 4, 1, 320)]
+    assert accepts(refused + taken) == [False] * len(refused) + [True] * len(taken)

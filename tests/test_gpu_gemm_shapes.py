@@ -153,16 +153,21 @@ def test_swiglu_either_side_of_the_short_form(buf, mode, spread, avg):
     assert np.array_equal(host(s2).view(np.uint32), want[1].view(np.uint32)) and np.array_equal(host(q2), want[0])
 
 
-# K slabs of the many-row kernel: scales of four steps in whole groups (4, 8), with two and three steps left over (6, 11), with one (5: the 256-row shape)
-@pytest.mark.parametrize("slabs", [4, 5, 6, 8, 11])
+# K slabs of the many-row kernel: scales of four steps in whole groups (4, 8), with two and three steps left over (6, 11), with one,
+# which makes the last two groups of three and two (5, 9), and rows of less than one group (2, 3)
+@pytest.mark.parametrize("slabs", [2, 3, 4, 5, 6, 8, 9, 11])
 @pytest.mark.parametrize("avg", [200, 900])
 def test_many_rows_fp8(buf, slabs, avg):
     K, N = 128 * slabs, 768
     counts = np.array([avg + 21, 0, 1, 320, 321, 3 * avg, avg + 60, 257], dtype=np.int64)
     E, rows = len(counts), int(counts.sum())
     counts[0] += max(0, 900 * E - rows) if avg == 900 else max(0, 200 * E - rows)      # more than any line to the kernels for fewer rows
-    rows = int(counts.sum())
-    a, sa, w, sw = fp8_operands(E, K, N, rows, 20 + slabs)
+    check_fp8_gemms(buf, counts, K, N, 20 + slabs)
+
+
+def check_fp8_gemms(buf, counts, K, N, seed):
+    E, rows = len(counts), int(counts.sum())
+    a, sa, w, sw = fp8_operands(E, K, N, rows, seed)
     packed = buf.prepack_weight(dev(w))
     y = gmm2(buf, dev(a), dev(sa), packed, dev(sw), capi.DT_FP32, counts, K, N, 2)
     assert_fp8_close(zo.bf16_to_f32(host(y)), zo.bf16_to_f32(zo.gmm2_fp8(a, sa, w, sw, counts)), "fp8 GEMM", FP8_GEMM_ELEM_TOL)
@@ -172,6 +177,15 @@ def test_many_rows_fp8(buf, slabs, avg):
     assert np.allclose(host(s2), r_s2, rtol=1e-4)
     assert_requant_close(zo.e4m3_to_f32(host(q2)).reshape(blocks) * host(s2)[:, :, None],
                          zo.e4m3_to_f32(r_q2).reshape(blocks) * r_s2[:, :, None], host(q2), r_q2)
+
+
+# weight block scales of 128 steps in turns of tiles, of more than that from where the last tile's were
+@pytest.mark.parametrize("slabs", [128, 129, 131, 256])
+def test_many_rows_fp8_long_k(buf, slabs):
+    K, N, counts = 128 * slabs, 512, np.array([401, 0, 700], dtype=np.int64)
+    E, rows = len(counts), int(counts.sum())
+    assert rows > 352 * E
+    check_fp8_gemms(buf, counts, K, N, 30)
 
 
 @pytest.mark.parametrize("mode", [1, 2])

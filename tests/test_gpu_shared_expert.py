@@ -117,11 +117,13 @@ class SharedExpert(ctypes.Structure):
     _fields_ = [("weight", ctypes.c_void_p), ("scale", ctypes.c_void_p), ("rows", ctypes.c_int64), ("out", ctypes.c_void_p)]
 
 
+# a K of one slab: the 256-row shape; of three: the many-row kernel
+@pytest.mark.parametrize("K", [128, 384])
 @pytest.mark.parametrize("R,S", [(2000, 1600), (1601, 1537)])
-def test_shared_expert_in_the_256_row_shape(buf, R, S):
-    """More than 1536 rows per expert fp8, which only a caller of the kernel ABI brings there with a shared expert: the
-    kernel that knows of one gives the bits of the kernel that does not, run for either expert by itself."""
-    K, N = 384, 512
+def test_shared_expert_in_many_rows(buf, R, S, K):
+    """More rows than the fused layer brings there with a shared expert: the bits are those of a launch for either expert by
+    itself, which in the 256-row shape is a kernel that knows of no shared expert."""
+    N = 512
     a, sa, w, sw = fp8_operands(2, K, N, R + S, 40)
     a, sa, w, sw = dev(a), dev(sa), buf.prepack_weight(dev(w)), dev(sw)
     off = row_off_dev([R, S])
