@@ -931,11 +931,7 @@ template <int MODE, bool GMM1> struct StreamRows {
  * Where the streaming kernel takes over from the kernel above (K in whole chunks of its four slabs only), by rows per
  * expert on average; 0: it does not. Layers in us with it against without, uniform / Zipf(1.2) routing, 128 experts of
  * 4096 x 3072 / 1536 x 4096 (M), 64 of 2048 x 2048 / 1024 x 2048 (S), 32 of 7168 x 4096 / 2048 x 7168 (W):
- *   - W4A8: always (M 128 rows -12 / -190, 250 -81 / -184). 128 rows against 64, uniform / Zipf(0.6) / Zipf(1.2), both GEMMs, per
- *     cent: M 80 rows -9 / +3 / +6, 112 -7 / -4 / +1, 200 -7 / -5 / -3, 640 -5 / -6 / -8, 1024 -8 / -8 / -8; S 64 rows -9 / +20 / +9,
- *     200 -6 / +4 / +2, 250 -1 / -1 / +1, 375 -2 / -4 / -3, 640 -7 / -7 / -8; W 128 rows +4 / 0 / +5, 200 -6 / -3 / -3; 8 experts of
- *     14336 x 4096 200 rows +8 / - / +33: from where its tiles, rows * n_tiles / 128, fill the chip (two workgroups per CU)
- *     twice, and once with many rows (8 experts 650 rows against 96-row tiles -1 / -3; 2 of 4096 x 3072, 70 tiles, +16);
+ *   - W4A8: always (M 128 rows -12 / -190, 250 -81 / -184), see w4a8_taller_tile;
  *   - W8A8 first GEMM, 96 rows: 75 M -23 / -52, W -7 / -20, 128 M -35 / -23, W -17 / -4, 187 M +3 / -64, S -8 / -41,
  *     250 M +35 / -46, W +22 / -27, 375 S -9 / -33, 512 M +90 / +17; second, 128 rows: 75 M -12 / -37, 128 M -27 / -32,
  *     250 W -13 / -18, 375 M -25 / -21, 512 M +14 / -24;
@@ -965,7 +961,7 @@ inline int stream_rows(const GemmParams &p, int n_tiles)
     using R = StreamRows<MODE, GMM1>;
     const int64_t rows = p.max_rows, e = p.experts, tiles = e * n_tiles;
     if (p.K % 512 != 0) return 0;
-        if (MODE == MODE_W4A8) return rows > 112 * e && rows * n_tiles >= (rows > 640 * e ? 65536 : 128000) ? R::TALL : R::LOW;
+    if (MODE == MODE_W4A8) return w4a8_taller_tile(rows, e, n_tiles, cu_count()) ? R::TALL : R::LOW;
     const bool many_tiles = tiles >= 4096;
     const int64_t low = MODE == MODE_W8A8 ? 48 : 36;
     int64_t tall = many_tiles && !GMM1 ? 192 : 400;
@@ -1120,7 +1116,7 @@ int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
          * per expert the 256-row shape below), both GEMMs, 32 experts of 7168 x 4096 / 2048 x 7168, 64 of 2048 x 2048 /
          * 1024 x 2048, 8 of 4096 x 28672 / 14336 x 4096, 250 to 2300 rows per expert: fp8 -8 / -11 % (0 ... -21), W8A8
          * -10 / -8 % (+1 ... -15). 1024 rows of the first: fp8 1047 / 596 -> 935 / 543 us, W8A8 974 / 519 -> 905 / 468. The kernel for
-         * any fp8 K, 256 to 1800 rows of twelve such K from 256 to 32768: -11 % (+5 ... -25).
+         * any fp8 K, 256 to 1800 rows per expert, thirty shapes with K from 256 to 32768: -10 % (+5 ... -24).
          */
         if (tall_accepts<MODE>(p)) {
             if constexpr (MODE == MODE_FP8) {

@@ -48,6 +48,19 @@ template <int MODE, int TM, int SPLIT = 1> struct StreamShape {
 };
 
 /*
+ * W4A8: tiles of 128 rows instead of 64. Shapes as at stream_rows, uniform / Zipf(0.6) / Zipf(1.2) routing, both GEMMs, per cent
+ * that 128 rows take more: M 80 rows -9 / +3 / +6, 112 -7 / -4 / +1, 200 -7 / -5 / -3, 640 -5 / -6 / -8, 1024 -8 / -8 / -8; S 64 rows
+ * -9 / +20 / +9, 200 -6 / +4 / +2, 250 -1 / -1 / +1, 375 -2 / -4 / -3, 640 -7 / -7 / -8; W 128 rows +4 / 0 / +5, 200 -6 / -3 / -3; 8 experts of
+ * 14336 x 4096 200 rows +8 / - / +33; 2 of 4096 x 3072, 70 tiles, +16: from where the taller tiles all but fill the chip (two
+ * workgroups per CU) twice, which S does at 250 rows, and once with many rows. Below that 64 rows are no worse than the 96 that ran there before: 700 rows per expert, first /
+ * second GEMM, 8 experts of S 48.5 -> 44.8 / 21.5 -> 22.1 us, 8 of M 110.5 -> 111.0 / 48.0 -> 46.1; 900 rows, 8 of S 69.5 -> 55.4 / 30.7 -> 27.4.
+ */
+inline bool w4a8_taller_tile(int64_t rows, int64_t experts, int n_tiles, int64_t cus)
+{
+    return rows > 112 * experts && rows * n_tiles >= (rows > 640 * experts ? 2 * 128 : 500) * (cus > 0 ? cus : 256);
+}
+
+/*
  * A weight load whose wait is counted by hand. The compiler counts its own loads exactly, but not the LDS-DMA transfers
  * issued from inline asm, so its waits reach that many loads too far: half of what an int4 wave has in flight. The value
  * may only be touched after a wait_w() that names it (tests/test_kernel_asm_checks.py reads the generated code for that);

@@ -1,4 +1,4 @@
-"""Which shapes the grouped GEMM's kernel for many rows takes, asked of the rule itself (no GPU needed: it is host code)."""
+"""Which kernel the grouped GEMMs take, asked of the rules themselves (no GPU needed: they are host code)."""
 import os
 import shutil
 import subprocess
@@ -13,12 +13,19 @@ PROGRAM = r"""
 #include <cstdio>
 #include <hip/hip_runtime.h>
 #include <type_traits>
+#include "zbal_gemm_stream.h"
 #include "zbal_gemm_tall.h"
 
 int main()
 {
     int mode, slabs, experts, rows;
     while (scanf("%d %d %d %d", &mode, &slabs, &experts, &rows) == 4) {
+        if (mode == MODE_W4A8) {
+            int n_tiles, cus;
+            if (scanf("%d %d", &n_tiles, &cus) != 2) return 1;
+            printf("%d\n", w4a8_taller_tile(rows, experts, n_tiles, cus));
+            continue;
+        }
         GemmParams p = {};
         p.K = slabs * 128;
         p.experts = experts;
@@ -40,7 +47,7 @@ def accepts(tmp_path_factory):
     assert r.returncode == 0, r.stdout
 
     def ask(cases):
-        out = subprocess.run([str(d / "accepts")], input="".join("%d %d %d %d\n" % c for c in cases), capture_output=True, text=True)
+        out = subprocess.run([str(d / "accepts")], input="".join(" ".join(map(str, c)) + "\n" for c in cases), capture_output=True, text=True)
         assert out.returncode == 0, out.stderr
         return [v == "1" for v in out.stdout.split()]
     return ask
@@ -59,3 +66,16 @@ def test_the_many_row_kernel_refuses_what_it_has_no_room_for(accepts):
     refused = [(1, 1, 8, 4096), (2, 1, 8, 4096), (1, 8, 513, 1 << 20), (2, 8, 513, 1 << 20), (2, 2, 1, 320), (2, 3, 1, 320)]
     taken = [(1, 2, 1, 320), (2, 2, 1, 321), (2, 3, 1, 321), (2, 4, 1, 320)]
     assert accepts(refused + taken) == [False] * len(refused) + [True] * len(taken)
+
+
+@pytest.mark.parametrize("cus", [256, 128, 64, 32])
+def test_the_taller_w4a8_tile_wants_a_full_chip(accepts, cus):
+    """rows * channel tiles from 500 per CU on, from 256 with more than 640 rows per expert; none up to 112 rows. Unknown: as on a whole GPU."""
+    case = lambda rows, experts, n_tiles, cus=cus: (3, 4, experts, rows, n_tiles, cus)
+    low = [case(112 * 64, 64, 1000), case(500 * 8, 8, cus // 8 - 1), case(640 * 8, 8, (500 * cus - 1) // 5120), case(641 * 8, 8, 256 * cus // 5128),
+           case(256 * cus - 1, 1, 1)]
+    tall = [case(113 * 64, 64, 1000), case(500 * 8, 8, cus // 8), case(640 * 8, 8, (500 * cus - 1) // 5120 + 1), case(641 * 8, 8, 256 * cus // 5128 + 1),
+            case(256 * cus, 1, 1)]
+    assert accepts(low + tall) == [False] * len(low) + [True] * len(tall)
+    if cus == 256:
+        assert accepts([c[:5] + (0,) for c in low + tall]) == [False] * len(low) + [True] * len(tall)

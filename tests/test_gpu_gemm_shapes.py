@@ -130,6 +130,33 @@ def test_many_tiles_are_the_same_rows_as_few(buf, avg):
         assert torch.equal(whole[r].view(torch.int16), got.view(torch.int16))
 
 
+# either side of 112 rows per expert, of the tiles that all but fill the chip twice (up to 640 rows) and once; experts whose tiles have
+# one to eight sub-tiles of 16 rows, five and six (65 to 96 rows) among them, and none
+@pytest.mark.parametrize("E,avg,N", [(64, 112, 4864), (64, 113, 4864), (8, 640, 6144), (8, 640, 6400), (8, 641, 3072), (8, 641, 3328)])
+def test_w4a8_lines_of_the_dispatch(buf, E, avg, N):
+    """The same bits as expert by expert, where the tiles are of 64 rows."""
+    K, rows = 512, avg * E
+    edges = [0, 70, 161, 192] if E == 8 else [0, 70, 161, 192, 1, 96, 127, 128]
+    counts = np.array(edges + [(rows - sum(edges)) // (E - len(edges))] * (E - len(edges)), dtype=np.int64)
+    counts[-1] += rows - counts.sum()
+    assert (counts >= 0).all() and counts.max() * (N // 256) < 65536
+    a = torch.randint(-128, 128, (rows, K), dtype=torch.int8, device="cuda")
+    xs = torch.rand((rows,), device="cuda") + 0.5
+    w = torch.randint(-128, 128, (E, N, K // 2), dtype=torch.int8, device="cuda")      # any bytes are a pre-packed weight
+    gs = ((torch.rand((E, K // 128, N), device="cuda") + 0.5) * 1e-3).to(torch.float16)
+    whole = gmm2(buf, a, xs, w, gs, capi.DT_FP16, counts, K, N, 3)
+    q2, s2, _ = gmm1(buf, a, xs, w, gs, counts, K, N, 3)
+    off = np.concatenate([[0], np.cumsum(counts)])
+    for e in range(E):
+        r = slice(int(off[e]), int(off[e + 1]))
+        if counts[e] == 0:
+            continue
+        one = (buf, a[r].contiguous(), xs[r].contiguous(), w[e:e + 1], gs[e:e + 1])
+        assert torch.equal(whole[r].view(torch.int16), gmm2(*one, capi.DT_FP16, counts[e:e + 1], K, N, 3).view(torch.int16)), e
+        want_q2, want_s2, _ = gmm1(*one, counts[e:e + 1], K, N, 3)
+        assert torch.equal(q2[r], want_q2) and torch.equal(s2[r], want_s2), e
+
+
 @pytest.mark.parametrize("mode", [1, 3])
 @pytest.mark.parametrize("spread", [0.2, 30.0, 70.0, 400.0])
 @pytest.mark.parametrize("avg", [20, 500])

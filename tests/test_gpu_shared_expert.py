@@ -33,10 +33,11 @@ def test_shared_expert_in_the_routed_launches(buf, mode, T, H, K, E, I, active, 
     check_shared_expert(buf, mode, T, H, K, E, I, active, smooth)
 
 
-# both tall tiles of the weight stream (150 and 711 rows per expert, the shared one's among them) and the staged kernel's
-# 320-row tile with the K of a prefill layer in both GEMMs (480 rows)
+# the tall tiles of the weight stream (150 rows per expert, the shared one's among them; W4A8's want the chip full: 711 rows), the
+# lower W4A8 ones with as many rows, and the many-row kernel with the K of a prefill layer in both GEMMs (480 rows)
 @pytest.mark.parametrize("mode,T,H,K,E,I,active,smooth", [(0, 300, 512, 4, 8, 512, None, False), (2, 300, 512, 4, 8, 512, 200, False),
                                                            (3, 300, 512, 4, 8, 512, None, True), (3, 1280, 512, 4, 8, 512, 1200, False),
+                                                           (3, 1280, 3072, 4, 8, 1536, 1200, False),
                                                            (0, 800, 7168, 2, 4, 2048, None, False), (2, 800, 7168, 2, 4, 2048, 777, False)])
 def test_shared_expert_in_tall_tiles(buf, mode, T, H, K, E, I, active, smooth):
     check_shared_expert(buf, mode, T, H, K, E, I, active, smooth)
