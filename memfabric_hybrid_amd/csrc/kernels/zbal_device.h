@@ -143,7 +143,7 @@ __device__ __forceinline__ float zb_expf(float x)
 }
 
 /*
- * g / (1 + zb_expf(-g)) for |g| <= 80, bit for bit (compared for every such float on gfx950; only -0 comes out as +0): the
+ * g / (1 + zb_expf(-g)) for |g| <= 80, bit for bit (tests/test_gpu_gemm_shapes.py compares every such float; only -0 comes out as +0): the
  * same reduction and polynomial, where exp(-g) is a normal number, so one addition to the exponent scales it, rounding to
  * an integer is adding and subtracting 1.5 * 2^23, and the quotient needs neither range scaling nor a second correction.
  * 17 vector instructions without a branch, so the four values of a lane overlap; the general form takes about 50, and its

@@ -180,6 +180,36 @@ def test_swiglu_either_side_of_the_short_form(buf, mode, spread, avg):
     assert np.array_equal(host(s2).view(np.uint32), want[1].view(np.uint32)) and np.array_equal(host(q2), want[0])
 
 
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_swiglu_short_form_over_every_float(buf, sign):
+    """Every gate value of at most 80: a dot product of 1 and an up value that is a power of two leave the SwiGLU of channel scale
+    times token scale, mantissa times 2^e. The launch is made twice, the second time with an infinity in every sixteenth row, which
+    sends its wave to the general form: the same bits, and of the two only the general one keeps the sign of -0."""
+    K, I, rows = 128, 1 << 20, 16
+    a = torch.zeros((rows, K), dtype=torch.int8, device="cuda")
+    a[:, 0] = 1
+    w = torch.zeros((1, K, 2 * I), dtype=torch.int8, device="cuda")
+    w[:, 0] = 1
+    packed = buf.prepack_weight(w)
+    # subnormal values, then fifteen exponents at a time
+    groups = [(None, [-126] * 15)] + [(e, list(range(e, e + 15))) for e in range(-126, 7, 15)]
+    for lowest, exponents in groups:
+        xs = torch.tensor([2.0 ** min(e, 6) for e in exponents] + [1.0], dtype=torch.float32, device="cuda")
+        far = xs.clone()
+        far[-1] = float("inf")
+        for m in range(0, 1 << 23, I):
+            ws = torch.empty((1, 2 * I), dtype=torch.float32, device="cuda")
+            ws[0, :I] = torch.arange(m, m + I, device="cuda", dtype=torch.float32) * 2.0 ** -23 + (0.0 if lowest is None else 1.0)
+            ws[0, :I] *= sign
+            ws[0, I:] = 2.0 ** -(-126 if lowest is None else lowest)                     # an up value of 1 in the first row
+            short, general = [gmm1(buf, a, x, packed, ws, [rows], K, 2 * I, 1)[2][:15 * I].view(torch.int32) for x in (xs, far)]
+            if lowest is None and m == 0:
+                zeros = slice(0, 15 * I, I)
+                assert (short[zeros] == 0).all() and (general[zeros] == (0 if sign > 0 else -2 ** 31)).all()
+                general[zeros] = 0
+            assert torch.equal(short, general), (lowest, m)
+
+
 # K slabs of the many-row kernel: scales of four steps in whole groups (4, 8), with two and three steps left over (6, 11), with one,
 # which makes the last two groups of three and two (5, 9), and rows of less than one group (2, 3)
 @pytest.mark.parametrize("slabs", [2, 3, 4, 5, 6, 8, 9, 11])
