@@ -109,10 +109,10 @@ def test_gmm1_w8a8_bit_exact(buf, E, K, N1, rows):
     assert np.array_equal(host(q2), r_q2)
 
 
-# experts with no rows, with only a short tile, with exactly full tiles of either two-stage shape (256 and 320 rows), one
-# row more than those, 17 to 20 sub-tiles of 16 rows (five per wave in some or all row groups of the 320-row shape), and
-# with short tails of both classes (up to a quarter and up to half of a tile): the 256-row shape runs the short tails
-# after all other tiles, the longer class first
+# experts with no rows, with only a short tile, with exactly full tiles (256 rows, and 320 in the many-row kernel), one row
+# more than those, 17 to 20 sub-tiles of 16 rows (nine or ten per wave in the many-row kernel), and with short tails of both
+# classes (up to a quarter and up to half of a tile): the 256-row shape runs the short tails after all other tiles, the longer
+# class first
 TILE_ORDER_COUNTS = np.array([0, 5, 256, 257, 300, 320, 321, 384, 385, 1024, 1030, 130, 64, 0, 512 + 128, 511, 1, 288, 289, 273,
                               576, 305, 641], dtype=np.int64)
 
@@ -123,7 +123,7 @@ def test_gemms_w8a8_tile_order_with_short_tails_bit_exact(buf, N, big):
     counts, K = TILE_ORDER_COUNTS.copy(), 384
     counts[9] = big
     E, rows = len(counts), int(counts.sum())
-    assert rows > 192 * E                                     # beyond the few-row shape: W8A8 takes the 320-row shape
+    assert rows > 192 * E                                     # beyond the few-row shape: the many-row kernel
     a = rng(61).integers(-127, 128, (rows, K)).astype(np.int8)
     xs = rng(62).uniform(0.005, 0.05, rows).astype(np.float32)
     w = rng(63).integers(-16, 16, (E, K, N)).astype(np.int8)
@@ -136,12 +136,15 @@ def test_gemms_w8a8_tile_order_with_short_tails_bit_exact(buf, N, big):
     assert np.array_equal(host(q2), r_q2)
 
 
-@pytest.mark.parametrize("big", [1024, 40000])           # rows of one expert: the average selects the 320-row / the 256-row shape
-def test_gemms_fp8_tile_order_with_short_tails(buf, big):
-    counts, K, N = TILE_ORDER_COUNTS.copy(), 256, 512
+# one K slab: the 256-row shape; the others: the many-row kernel, with less than a group of four slabs' scales, one over from
+# such groups, two and three
+@pytest.mark.parametrize("K", [128, 256, 640, 768, 896])
+@pytest.mark.parametrize("big", [1024, 40000])           # rows of one expert: a few tiles, or more than a hundred
+def test_gemms_fp8_tile_order_with_short_tails(buf, big, K):
+    counts, N = TILE_ORDER_COUNTS.copy(), 512
     counts[9] = big
     E, rows = len(counts), int(counts.sum())
-    assert (128 * E < rows <= 1536 * E) if big == 1024 else (rows > 1536 * E)
+    assert rows > 128 * E
     a, sa, w, sw = fp8_operands(E, K, N, rows, 70)
     y = gmm2(buf, dev(a), dev(sa), buf.prepack_weight(dev(w)), dev(sw), capi.DT_FP32, counts, K, N, 2)
     ref = zo.gmm2_fp8(a, sa, w, sw, counts)
@@ -172,7 +175,7 @@ def test_gemms_w8a8_even_row_tiles_in_the_few_row_shape_bit_exact(buf):
     assert np.array_equal(host(q2), r_q2)
 
 
-@pytest.mark.parametrize("rows", [40000, 200000])      # few rows per expert (128-row shape) / many (256-row shape: more experts than the 320-row shape's tables hold)
+@pytest.mark.parametrize("rows", [40000, 200000])      # few and many rows per expert: with one K slab both take the 256-row shape
 def test_gmm2_w8a8_largest_expert_count_bit_exact(buf, rows):
     """1024 experts, the most the kernel's lookup tables hold: the tile lookup, the cost prefix and the list of short
     experts all run over sixteen 64-expert chunks. Skewed counts leave many experts empty or short."""
@@ -237,12 +240,14 @@ def test_gmm1_fp8(buf, E, K, N1, rows):
 
 # ---- either side of the launcher's shape limits -------------------------------------------------------------
 
-@pytest.mark.parametrize("rows_per_expert", [96, 97, 128, 129, 192, 193, 1536, 1537])
-def test_gemms_at_the_shape_limits(buf, rows_per_expert):
-    """The launcher picks the 128-row, the 320-row or the 256-row shape from rows / experts (few rows: up to 96 .. 192
-    by mode and GEMM; fp8 takes 320-row tiles up to 1536 rows): the same operands either side of every limit, W8A8
-    bit exact and fp8 within its tolerance."""
-    E, K, N = 4, 256, 512
+# 4 experts: the streaming hint and the 128-row shape end at 84 .. 192 rows per expert by mode and GEMM, the many-row kernel
+# follows; its tables hold 512 experts, the 256-row shape takes more; one expert in one tile of it, whose fp8 rows of two
+# scales have no neighbours to be read along with
+@pytest.mark.parametrize("E,rows_per_expert,N", [(4, n, 512) for n in (84, 85, 96, 97, 100, 101, 128, 129, 192, 193)] +
+                         [(512, 200, 256), (513, 200, 256), (1, 320, 512), (1, 321, 512)])
+def test_gemms_at_the_shape_limits(buf, E, rows_per_expert, N):
+    """The same operands either side of every limit, W8A8 bit exact and fp8 within its tolerance."""
+    K = 256
     rows = rows_per_expert * E
     counts = ragged_counts(E, rows, 7 * rows_per_expert)
     a = rng(81).integers(-127, 128, (rows, K)).astype(np.int8)
@@ -268,7 +273,7 @@ def test_gemms_at_the_shape_limits(buf, rows_per_expert):
 
 # ---- both workgroup shapes, with more tiles than workgroups ------------------------------------------------------
 
-@pytest.mark.parametrize("E,K,N,rows", [(8, 256, 2304, 8192),     # 1024 rows per expert: 320-row tiles, 2 stages, ~300 tiles
+@pytest.mark.parametrize("E,K,N,rows", [(8, 256, 2304, 8192),     # 1024 rows per expert: the many-row kernel, ~300 tiles
                                         (64, 256, 1024, 8000),    # <= 128 on average: 128-row tiles, 3 stages, ~400 tiles
                                         (4, 128, 256, 3000)])     # a single K slab
 def test_gmm2_w8a8_many_tiles_per_workgroup(buf, E, K, N, rows):
@@ -303,9 +308,9 @@ def test_gmm1_fp8_many_tiles_per_workgroup(buf, E, K, N1, rows):
 
 # ---- W4A8 ----------------------------------------------------------------------------------------------------------
 
-# 96 rows per expert is the last size that takes the 128-row shape in this mode
-@pytest.mark.parametrize("E,K,N,rows", [(4, 256, 256, 300), (16, 1024, 512, 200), (4, 256, 256, 384), (4, 256, 256, 388),
-                                        (2, 256, 512, 700)])
+# with two K slabs 48 and 100 rows per expert are the last of the 64-row and of the lower 128-row shape in this mode
+@pytest.mark.parametrize("E,K,N,rows", [(4, 256, 256, 300), (16, 1024, 512, 200), (4, 256, 256, 384), (4, 256, 256, 388), (4, 384, 256, 192),
+                                        (4, 384, 256, 196), (4, 256, 256, 400), (4, 256, 256, 404), (2, 256, 512, 700)])
 def test_w4a8_bit_exact(buf, E, K, N, rows):
     counts = ragged_counts(E, rows, E + K)
     a = rng(41).integers(-127, 128, (rows, K)).astype(np.int8)
