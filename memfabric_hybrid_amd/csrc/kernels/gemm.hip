@@ -57,7 +57,8 @@ namespace {
  * row-major storage would put all 16 rows on the same slot.
  *
  * TM = 256 with two stages of 64 KiB (the slab for step k+1 is in flight while step k is multiplied) has the arithmetic
- * intensity that many-row experts need, where the 8-bit modes cannot take the kernel of zbal_gemm_tall.h. TM = 128 and TM = 64 with three or four stages are for few-row experts, where the job is to stream every
+ * intensity that many-row experts need, for W4A8 and where the 8-bit modes cannot take the kernel of zbal_gemm_tall.h (a single
+ * slab, more than 512 experts). TM = 128 and TM = 64 with three or four stages are for few-row experts, where the job is to stream every
  * weight byte once at HBM speed: two weight slabs or more stay in flight per CU, and the MFMAs of sub-tiles past the
  * expert's end are skipped; W4A8, bound by its vector instructions, also has a 192-row shape. The few-row shapes and
  * that one split a tile over one or two row groups of waves instead of four (FewRows, launch_w4a8).
@@ -78,14 +79,14 @@ struct DmaShape {
     static constexpr int ROW_GROUPS = RG;
     static constexpr int COL_GROUPS = NW / RG;             /* the waves of a row group split the tile's 256 channels */
     static constexpr int NT = 16 / COL_GROUPS;             /* 16-channel sub-tiles per wave: 8 or 4 */
-    static constexpr int MTM = (TM / 16 + ROW_GROUPS - 1) / ROW_GROUPS;   /* 16-row sub-tiles per wave, at most: 2, 4 or 6 */
+    static constexpr int MTM = (TM / 16 + ROW_GROUPS - 1) / ROW_GROUPS;   /* 16-row sub-tiles per wave, at most: 2, 4, 6 or 8 */
     static constexpr int THREADS = NW * 64;
     static constexpr int A_BYTES = TM * BKB;
     static constexpr int W_BYTES = BN * WRB;
     static constexpr int STAGE_BYTES = A_BYTES + W_BYTES;
     static constexpr int HALF_BLOCKS = 128 * WRB / 1024;   /* 1 KiB blocks per 128-channel half: 16 or 8 */
     static constexpr int MAX_EXPERTS = D_MAX_EXPERTS;       /* what the lookup tables hold */
-    static constexpr int A_PARTS = (A_BYTES / 1024 + NW - 1) / NW;   /* 1 KiB blocks of the A tile per wave: 2, 4 or 5 */
+    static constexpr int A_PARTS = (A_BYTES / 1024 + NW - 1) / NW;   /* 1 KiB blocks of the A tile per wave: 1 to 4 */
     static constexpr int W_PARTS = W_BYTES / 1024 / NW;    /* 1 KiB blocks of the W tile per wave (2, 4 or 8) */
     static constexpr int PARTS = W_PARTS > A_PARTS ? W_PARTS : A_PARTS;
     static constexpr bool TWO_PHASE = TM == 256;            /* the tiles of short experts run after all the others (see the kernel) */
@@ -1030,8 +1031,8 @@ int32_t prepare_mode()
 /*
  * Shape choice from what the host knows (the row counts themselves live on the device). With few rows per expert the
  * GEMM is a weight-streaming job and takes the three-stage 128-row shape (which needs two K slabs to fill its
- * pipeline); with many it needs the arithmetic intensity of a two-stage shape, 320 or 256 rows high. The shapes were
- * timed against each other on 7168 x 4096 / 2048 x 7168 experts (W4A8: 4096 x 3072 / 1536 x 4096, 128 experts) with 32
+ * pipeline); with many it needs the arithmetic intensity of taller tiles. The 128-row shape was timed against the 320-row one (of
+ * four row groups of waves) that the many-row kernel has replaced, on 7168 x 4096 / 2048 x 7168 experts (W4A8: 4096 x 3072 / 1536 x 4096, 128 experts) with 32
  * and with 256 experts, random routing; rows per expert on average, first / second GEMM, 128-row against tall
  * (W4A8: 256-row) shape in ms:
  *   - fp8, 32 experts: 128 rows 0.247 / 0.136 against 0.256 / 0.145; 192 rows 0.298 / 0.160 against 0.278 / 0.166;

@@ -184,8 +184,8 @@ grouped_gemm_stream_kernel(GemmParams p)
     };
 
     /*
-     * The activations (and what scales them) of slabs kb0 .. kb0 + 3, to buffer b: MT + (scales ? 1 : 0) operations of every
-     * wave. Rows past the tile's end repeat its last one.
+     * The activations (and what scales them) of a chunk's PF slabs from kb0 on, to buffer b, in the same number of operations of
+     * every wave: D in k_loop, whose waits count them. Rows past the tile's end repeat its last one.
      */
     const uint32_t lds_a0 = lds_addr(smem);
     auto issue_chunk = [&](auto mt_tag, int kb0, int b) __attribute__((always_inline)) {

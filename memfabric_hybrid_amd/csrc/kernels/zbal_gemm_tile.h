@@ -104,7 +104,10 @@ __device__ __forceinline__ f32x4 mfma_fp8_16x16x128(const i32x8 &wfrag, const i3
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wfrag, afrag, zero, 0, 0, 0, 0, 0, 0);
 }
 
-/* a barrier for what is in LDS: __syncthreads() would also wait for the slabs in flight */
+/*
+ * A barrier for what is in LDS, with the slabs in flight left alone whatever the compiler takes a barrier to wait for (its
+ * __syncthreads() waits for no more on gfx950, and the staged kernel's step has one).
+ */
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 /* four consecutive bytes -> one dword store helpers */
