@@ -33,8 +33,8 @@ struct PeerSource {
  * U chunks per lane and pass. Every wave resolves the token's picks itself, one lane per pick, and takes them from
  * there as scalars: no LDS, no barrier between the loads of a pick's address and the row loads. BASES: one rank of at most 64 *
  * BASES experts, whose bases are asked for one per lane beside the picks and taken from the lane that has them, instead of by a
- * load that depends on the pick (0: such a load). The kernel alone, hidden 7168, 32 experts: 7 tokens 4.8 -> 3.9 us, 128 tokens
- * 5.2 -> 4.7; 4096 tokens 94.0 -> 92.5.
+ * load that depends on the pick (0: such a load). The kernel alone, hidden 7168, 32 experts, rows in the cache / from memory: 7 tokens
+ * 4.0 -> 3.8 / 4.8 -> 4.8 us, 128 tokens 4.5 -> 4.2 / 6.4 -> 5.8, 4096 tokens 91.3 -> 90.4 / 93.4 -> 92.2.
  */
 template <int DT, int U, int BASES>
 __global__ void __launch_bounds__(kThreads)

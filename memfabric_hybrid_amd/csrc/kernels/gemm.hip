@@ -989,6 +989,8 @@ inline int stream_rows(const GemmParams &p, int n_tiles)
  * them, four waves and half of the channels to either, because what one CU takes from memory (30 GB/s) is the limit then.
  * Tiles of 16 rows, since there are hardly more. Rows in all, us for whole tiles -> halves (quarters):
  *   - 8 of 32 experts, 7168 x 4096, 128 tiles: W8A8 first GEMM 49.7 -> 41.9 (43.1); second, 224 tiles of 2048 x 7168: 19.3 (19.5);
+ *     beyond the half of the CUs (one token with a shared expert is 9 of 33): 144 tiles 50.3 -> 57.7, 160 52.2 -> 59.2; second, 140 tiles
+ *     14.2 -> 15.3, fp8 14.5 -> 15.3; W4A8, 4096 x 3072 / 1536 x 4096, 144 tiles 20.7 -> 21.9 / 7.3 -> 7.9;
  *   - 8 of 128, 4096 x 3072 / 1536 x 4096, 96 / 128 tiles: W8A8 30.7 -> 22.9 (24.7) / 11.8 -> 10.2 (10.4), W4A8 19.9 -> 18.1
  *     (20.4) / 7.9 -> 6.8 (7.4); 16 rows, 192 / 256 tiles: W8A8 36.6 (37.9) / 17.4 (17.1), W4A8 23.5 (24.8) / 10.3 (10.2);
  *   - 6 of 64, 2048 x 2048 / 1024 x 2048, 48 tiles: W8A8 18.5 -> 14.6 (14.0) / 8.0 -> 6.0 (5.1), W4A8 14.4 -> 14.0 (14.9) /

@@ -587,7 +587,10 @@ topk_route_kernel(const float *__restrict__ logits, int tokens, int experts, int
         if ((bidx & 63) == lane) used |= 1u << (bidx >> 6);
         if (lane == k) { picked = best; myidx = bidx; }
     }
-    /* one exp and one quotient for all picks, summed in their order (16384 tokens, 128 experts, top-8 15.5 us; in every round 20.5) */
+    /*
+     * One exp and one quotient for all picks, summed in their order: the kernel alone, 16384 tokens, 128 experts, top-8, logits in
+     * the cache / from memory 15.6 / 16.6 us; in every round 20.5 / 21.4 (17 to 19 between a layer's other kernels, on their clock).
+     */
     const float myw = zb_expf(picked - mx) / sum;
     float wsum = 0.0f;
     for (int k = 0; k < topk; ++k) wsum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myw), k));

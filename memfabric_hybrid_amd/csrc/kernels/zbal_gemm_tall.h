@@ -4,8 +4,9 @@
  *
  * What bounds it: no single unit. A step's MFMAs, the LDS reads that feed them and the transfers that refill the LDS each
  * take about half of it, and what is lost is lost where they wait for one another; the more they overlap, the lower the
- * clock that the power limit leaves (W8A8, 4096 tokens over 32 experts: MFMAs in 54 % of the cycles at 1.80 GHz, 49 % at 1.88
- * in the kernel this one replaced; without the transfers the first GEMM would take 767 instead of 935 us). Hence:
+ * clock that the power limit leaves (W8A8, 4096 tokens over 32 experts: MFMAs in 60 / 52 % of the cycles at 1.85 / 1.93 GHz, fp8 50 /
+ * 45 % at 1.88 / 1.95). As built / slabs always in the L2 / no transfers / no stores of the second GEMM's rows, us: fp8 965 / 879 / 863
+ * and 514 / 486 / 449 / 455, W8A8 893 / 812 / 760 and 461 / 423 / 382 / 388. Hence:
  *
  *  - The waves are two row groups x four channel ranges. A wave keeps the four weight fragments of a step in registers and
  *    streams its ten activation fragments past them, so that every fragment is read once (four row groups of five sub-tiles
