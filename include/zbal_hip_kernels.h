@@ -368,6 +368,16 @@ ZBALHIP_API int32_t zbalhip_gmm1_swiglu_quant_shared(const void *a, const float 
                                   const int32_t *row_off, int64_t experts, int64_t max_rows, int64_t k, int64_t n1,
                                   int32_t mode, void *q2, float *scale2, float *sgl_ws,
                                   const zbalhip_shared_expert_t *shared, void *stream);
+/*
+ * The same with memory for tiles that several workgroups share along K (8-bit modes with few rows per expert): `parts_bytes`
+ * at `parts`, 16-byte aligned, of which the first ZBALHIP_PART_WORDS 32-bit words are zero; null: no tile is shared. The more bytes,
+ * the more rows a shared tile may have. shared may be null.
+ */
+#define ZBALHIP_PART_WORDS 512
+ZBALHIP_API int32_t zbalhip_gmm1_swiglu_quant_parts(const void *a, const float *a_scale, const void *w1, const void *w1scale,
+                                  const int32_t *row_off, int64_t experts, int64_t max_rows, int64_t k, int64_t n1,
+                                  int32_t mode, void *q2, float *scale2, float *sgl_ws,
+                                  const zbalhip_shared_expert_t *shared, void *parts, int64_t parts_bytes, void *stream);
 ZBALHIP_API int32_t zbalhip_gmm2_dequant_shared(const void *a, const float *a_scale, const void *w2, const void *wscale,
                              int32_t wscale_dtype, const int32_t *row_off, int64_t experts, int64_t max_rows,
                              int64_t k, int64_t n, int32_t mode, int32_t out_dtype, void *y,

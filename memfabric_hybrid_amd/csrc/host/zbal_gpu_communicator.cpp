@@ -816,6 +816,15 @@ public:
         const int32_t gemmMode = mode | (isTensorList ? ZBALHIP_WEIGHTS_AS_LISTS : 0);
         /* int modes: the permute launch clears the row maxima the first GEMM accumulates into (no fill launch) */
         const int32_t clearedFlag = sgl ? ZBALHIP_ROWMAX_CLEARED : 0;
+        /*
+         * What the second GEMM's y takes up beyond the row maxima is nobody's during the first: there its workgroups exchange the
+         * sums of tiles that they share, behind words that the permute launch clears along with the row maxima.
+         */
+        uint32_t *clearFrom = sgl ? (uint32_t *)(sgl + allRows * I) : (uint32_t *)y;
+        uint32_t *parts = std::max((uint32_t *)y, (uint32_t *)(base + Align256(sgl ? ws.sgl + (uint64_t)allRows * (I + 1) * 4 : 0)));
+        int64_t clearCount = sgl ? allRows : 0, partsBytes = (uint8_t *)y + rows * H * 2 - (uint8_t *)parts;
+        if (mode == 3 || partsBytes <= ZBALHIP_PART_WORDS * 4 || parts - clearFrom > clearCount + 1024) parts = nullptr;
+        else clearCount = parts + ZBALHIP_PART_WORDS - clearFrom;
         if (T == 0) { /* nothing routed: counts are zero */
             return Launched(op, zbalhip_fused_permute_quant(x->data, x->dataType, (const int32_t *)expertIds->data, smooth,
                                                             nullptr, 0, H, K, E, qmode, q1, xs, expandIdx,
@@ -849,19 +858,19 @@ public:
                                       SI, H, mode, x->dataType, shareOutput->data, stream);
             if (rc != 0) return Launched(op, rc);
         }
-        uint32_t *rowMax = sgl ? (uint32_t *)(sgl + allRows * I) : nullptr;
+        uint32_t *clearWords = clearCount ? clearFrom : nullptr;
         const int32_t *ids = (const int32_t *)expertIds->data;
         const int32_t permuteMode = qmode | IdsFlag(expertIds);
         int64_t *counts = (int64_t *)expertTokenNums->data;
         rc = ride ? zbalhip_fused_permute_quant_shared(x->data, x->dataType, ids, smooth, activeMask, T, H, K, E, permuteMode, q1, xs,
-                                                       expandIdx, counts, rowOff, rowMax, sgl ? allRows : 0, layoutScratch,
+                                                       expandIdx, counts, rowOff, clearWords, clearCount, layoutScratch,
                                                        ZBALHIP_LAYOUT_MAX_BLOCKS, shareSmooth, stream)
                   : zbalhip_fused_permute_quant(x->data, x->dataType, ids, smooth, activeMask, T, H, K, E, permuteMode, q1, xs,
-                                                expandIdx, counts, rowOff, rowMax, sgl ? allRows : 0, layoutScratch,
+                                                expandIdx, counts, rowOff, clearWords, clearCount, layoutScratch,
                                                 ZBALHIP_LAYOUT_MAX_BLOCKS, stream);
         if (rc != 0) return Launched(op, rc);
-        rc = zbalhip_gmm1_swiglu_quant_shared(q1, xs, gmm1Weight->data, gmm1Scale->data, rowOff, E, rows, H, N1,
-                                              gemmMode | clearedFlag, q2, scale2, sgl, ride ? &along1 : nullptr, stream);
+        rc = zbalhip_gmm1_swiglu_quant_parts(q1, xs, gmm1Weight->data, gmm1Scale->data, rowOff, E, rows, H, N1,
+                                             gemmMode | clearedFlag, q2, scale2, sgl, ride ? &along1 : nullptr, parts, partsBytes, stream);
         if (rc != 0) return Launched(op, rc);
         rc = zbalhip_gmm2_dequant_shared(q2, scale2, gmm2Weight->data, gmm2Scale->data, wscale2Dt, rowOff, E, rows, I, H, gemmMode,
                                          x->dataType, y, ride ? &along2 : nullptr, stream);

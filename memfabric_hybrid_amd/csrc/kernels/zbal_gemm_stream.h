@@ -88,6 +88,8 @@ grouped_gemm_stream_kernel(GemmParams p)
     static_assert(SPLIT == 1 || MODE != MODE_FP8 || !GMM1, "fp8's first GEMM requantises 128 columns, which are one workgroup's");
     using S = StreamShape<MODE, TM, SPLIT>;
     constexpr int PF = S::PF, NT = S::NT, MTM = S::MTM, LOADS = S::LOADS, NW = S::NW, WRB = S::WRB;
+    constexpr int MAX_PARTS = 4;
+    constexpr bool SHARES_K = GMM1 && MODE != MODE_W4A8 && SPLIT == 1;
     constexpr int W_BLOCK_BYTES = 128 * WRB;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     float *lds_sa = reinterpret_cast<float *>(smem + 2 * S::A_BYTES);
@@ -115,17 +117,52 @@ grouped_gemm_stream_kernel(GemmParams p)
     int lo[2], hi[2];                                              /* the first 128 experts, one per lane each: one round trip for all of them */
     rows_of(0, lo[0], hi[0]);
     rows_of(64, lo[1], hi[1]);
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int xcd = blockIdx.x & 7;
+    int slot = blockIdx.x >> 3;
     auto columns_before = [&](int y) { return (y - xcd + 7) >> 3; };      /* of this XCD, among columns 0 .. y - 1 */
-    int expert = -1, n_tile = 0, m_tile = 0, mt_e = 1, first_row = 0, end_row = 0;
-    for (int base = 0, tiles = 0, used = 0; base < E; base += 64) {
-        int l = lo[0], h = hi[0];
-        if (base == 64) { l = lo[1]; h = hi[1]; }
-        else if (base > 64) rows_of(base, l, h);
-        const int m = (h - l + TM - 1) / TM;
-        const uint64_t busy = __ballot(m > 0);
-        const int c0 = (used + __builtin_amdgcn_mbcnt_hi((uint32_t)(busy >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)busy, 0))) * n_tiles;
-        const int mine = (columns_before(c0 + n_tiles) - columns_before(c0)) * m;
+    /* f for 64 experts at a time, one per lane: first of them, and the lane's first row, end row, row tiles, first column and tiles on this XCD; until it is true */
+    auto walk = [&](auto f) __attribute__((always_inline)) {
+        for (int base = 0, used = 0; base < E; base += 64) {
+            int l = lo[0], h = hi[0];
+            if (base == 64) { l = lo[1]; h = hi[1]; }
+            else if (base > 64) rows_of(base, l, h);
+            const int m = (h - l + TM - 1) / TM;
+            const uint64_t busy = __ballot(m > 0);
+            const int c0 = (used + __builtin_amdgcn_mbcnt_hi((uint32_t)(busy >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)busy, 0))) * n_tiles;
+            if (f(base, l, h, m, c0, (columns_before(c0 + n_tiles) - columns_before(c0)) * m)) break;
+            used += __popcll(busy);
+        }
+    };
+    /*
+     * The memory gives every CU the same, so what is over when all CUs have the same number of tiles (`rest`, at the end) runs on
+     * a few CUs, long after the others: fp8, 528 tiles of 7168 x 4096 on 256 CUs, 16 tiles alone for the last 30 of 168 us. Such
+     * tiles are shared along K by up to four workgroups each, which leave their sums in memory; the last of them to get there
+     * adds the parts up, in their order, whichever it is, and has the epilogue. Nobody waits for anybody. Layers with a shared
+     * expert, 32 experts of 7168 x 4096 / 2048 x 7168: fp8, 37 tokens 270 -> 254 us, 12 tokens 245 -> 239, W8A8, 20 tokens 274 -> 257,
+     * 60 tokens 287 -> 273 (up to eight: 254, 238, 261, 275). The words and sums go past the L2s, which are the XCDs' own.
+     */
+    int part_k = 0, parts = 1, piece = 0;
+    int64_t part_rows = 0;
+    if constexpr (SHARES_K) {
+        if (p.part_sums != nullptr) {
+            int tiles = 0;
+            walk([&](int, int, int, int, int, int mine) { tiles += __builtin_amdgcn_readlane(zb_wave_scan_dpp(mine), 63); return false; });
+            const int rest = tiles % p.part_cus, whole = tiles - rest;
+            if (rest > 0 && whole > 0 && slot >= whole) {
+                parts = p.part_cus / rest;
+                if (parts > KB / PF) parts = KB / PF;
+                if (parts > MAX_PARTS) parts = MAX_PARTS;
+                const int u = slot - whole;
+                part_k = u / rest;
+                if (part_k >= parts) return;
+                piece = u - part_k * rest;
+                slot = whole + piece;
+                part_rows = p.part_floats / (256 * rest * parts);
+            }
+        }
+    }
+    int expert = -1, n_tile = 0, m_tile = 0, mt_e = 1, first_row = 0, end_row = 0, tiles = 0;
+    walk([&](int base, int l, int h, int m, int c0, int mine) {
         const int incl = zb_wave_scan_dpp(mine);
         const uint64_t past = __ballot(tiles + incl > slot);
         if (past) {
@@ -138,11 +175,11 @@ grouped_gemm_stream_kernel(GemmParams p)
             m_tile = at - col * mt_e;
             const int first_col = __builtin_amdgcn_readlane(c0, src);
             n_tile = (columns_before(first_col) + col) * 8 + xcd - first_col;
-            break;
+            return true;
         }
         tiles += __builtin_amdgcn_readlane(incl, 63);
-        used += __popcll(busy);
-    }
+        return false;
+    });
     if (expert < 0) return;
     const int part = SPLIT == 1 ? 0 : n_tile % SPLIT, chan = part * NW + wave;      /* which 32 of the tile's 256 channels are this wave's */
     n_tile /= SPLIT;
@@ -150,6 +187,14 @@ grouped_gemm_stream_kernel(GemmParams p)
     const int row_begin = first_row + m_tile * height;
     const int row_end = row_begin + height < end_row ? row_begin + height : end_row;
     const int last_rel = row_end - 1 - row_begin;
+    if constexpr (SHARES_K) {
+        if (parts > 1 && last_rel >= part_rows) {              /* no room for its sums */
+            if (part_k > 0) return;
+            parts = 1;
+        }
+    }
+    /* slabs of this workgroup: whole chunks */
+    const int kb_from = SHARES_K ? KB / PF * part_k / parts * PF : 0, kb_to = SHARES_K ? KB / PF * (part_k + 1) / parts * PF : KB;
 
     /* the wave's two 16-channel sub-tiles: block rows r0, r0 + 16 .. of one 128-channel block, or the same rows of a gate and an up block */
     const uint8_t *wb = weights_of<uint8_t, SHARED_IN_REGISTERS>(p, expert, (int64_t)(p.N / 128) * KB * W_BLOCK_BYTES);
@@ -412,15 +457,15 @@ grouped_gemm_stream_kernel(GemmParams p)
         constexpr int L = NT * LOADS;                                   /* loads per slab */
         constexpr int D = MT * SPLIT / S::MT_STEP + (MODE == MODE_W8A8 ? 0 : (MODE == MODE_FP8 ? S::SA_LOADS : SPLIT));      /* transfers per chunk */
         Slabs wr;
-        issue_chunk(mt_tag, 0, 0);
+        issue_chunk(mt_tag, kb_from, 0);
 #pragma unroll
-        for (int s = 0; s < PF; ++s) load_w(stream_tag, wr, s, s);
+        for (int s = 0; s < PF; ++s) load_w(stream_tag, wr, s, kb_from + s);
         /* issued since chunk c's transfers: the fragments of its slabs, L each; since slab s's fragments: three more slabs, and D */
         auto begin_chunk = [&]() __attribute__((always_inline)) {
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(PF * L) : "memory");
         };
-        int b = 0, kb0 = 0;
-        for (; kb0 + PF < KB; kb0 += PF) {
+        int b = 0, kb0 = kb_from;
+        for (; kb0 + PF < kb_to; kb0 += PF) {
             begin_chunk();               /* chunk kb0's activations have landed for everybody, and nobody reads the other buffer any more */
             issue_chunk(mt_tag, kb0 + PF, b ^ 1);
 #pragma unroll
@@ -462,6 +507,52 @@ grouped_gemm_stream_kernel(GemmParams p)
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) accf[mt][nt][i] *= 0.0625f;
+    }
+    if constexpr (SHARES_K) {
+        if (parts > 1) {
+            /* [row][256] sums of a part; a wave has 32 of the channels, its lane 4 of either 16 */
+            int l = lane;
+            asm volatile("" : "+v"(l));
+            auto sums_at = [&](int part, int mt, int nt) {
+                return reinterpret_cast<uint64_t *>(p.part_sums + xcd * p.part_floats + (piece * parts + part) * part_rows * 256 +
+                                                    ((mt * 16 + (l & 15)) * 256 + wave * 32 + nt * 16 + (l >> 4) * 4));
+            };
+            auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+                for (int mt = 0; mt < MTM; ++mt)
+                    if (mt * 16 + (l & 15) <= last_rel) {
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt) f(mt, nt);
+                    }
+            };
+            each([&](int mt, int nt) __attribute__((always_inline)) {
+                const u32x4 v = MODE == MODE_FP8 ? __builtin_bit_cast(u32x4, accf[mt][nt]) : __builtin_bit_cast(u32x4, acci[mt][nt]);
+                uint64_t *at = sums_at(part_k, mt, nt);
+                __hip_atomic_store(at, (uint64_t)v[1] << 32 | v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(at + 1, (uint64_t)v[3] << 32 | v[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            });
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (threadIdx.x == 0)
+                *reinterpret_cast<uint32_t *>(lds_rowmax) = __hip_atomic_fetch_add(p.part_done + xcd * p.part_cus + piece, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<uint32_t *>(lds_rowmax)) != (uint32_t)parts - 1) return;
+            each([&](int mt, int nt) __attribute__((always_inline)) {
+                accf[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                acci[mt][nt] = i32x4{0, 0, 0, 0};
+            });
+            for (int part = 0; part < parts; ++part) {
+                each([&](int mt, int nt) __attribute__((always_inline)) {
+                    uint64_t *at = sums_at(part, mt, nt);
+                    const uint64_t v0 = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    const uint64_t v1 = __hip_atomic_load(at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    const u32x4 v = {(uint32_t)v0, (uint32_t)(v0 >> 32), (uint32_t)v1, (uint32_t)(v1 >> 32)};
+                    if (MODE == MODE_FP8) accf[mt][nt] += __builtin_bit_cast(f32x4, v);
+                    else acci[mt][nt] += __builtin_bit_cast(i32x4, v);
+                });
+            }
+            __syncthreads();               /* lds_rowmax goes to the epilogue */
+        }
     }
     TileCoord tc;
     tc.expert = expert;

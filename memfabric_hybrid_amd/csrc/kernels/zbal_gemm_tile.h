@@ -40,6 +40,14 @@ struct GemmParams {
     const uint8_t *shared_w;
     const void *shared_wscale;
     void *shared_out;        /* GMM2: where row 0 would be if row shared_row is the first */
+    /*
+     * For the streaming kernel's tiles that several workgroups share along K (8-bit modes' first GEMM; null: none do): 8 * part_cus
+     * words that are zero when the launch starts, and room for part_floats sums of every XCD's tiles.
+     */
+    uint32_t *part_done;
+    float *part_sums;
+    int64_t part_floats;
+    int part_cus;            /* CUs per XCD */
 };
 
 /*
