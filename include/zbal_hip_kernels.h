@@ -300,6 +300,15 @@ ZBALHIP_API int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, 
 #define ZBALHIP_ROWMAX_CLEARED 0x200
 
 /*
+ * OR-ed into `mode` of the GEMMs (int modes): the first one leaves its fp32 SwiGLU values and row maxima in sgl_ws as they are and
+ * writes neither q2 nor scale2; the second one has them as `a` (the values) and `a_scale` (the maxima, max_rows words behind the
+ * values), and makes the bytes of its rows itself. y may not lie on top of them. K of the second GEMM in whole multiples of 512.
+ * zbalhip_gmm2_takes_values: whether that is the faster way (one launch less, but every channel tile makes its rows' bytes).
+ */
+#define ZBALHIP_SWIGLU_VALUES 0x400
+ZBALHIP_API int32_t zbalhip_gmm2_takes_values(int64_t experts, int64_t max_rows, int64_t k, int32_t mode);
+
+/*
  * Grouped GEMM 1 with dequant + SwiGLU + requant epilogue (AIC loop
  * …swiglu_quant_multistage_workspace.h:603-833, epilogue
  * block_epilogue_per_token_dequant_swiglu.h:171-298, BlockQuant

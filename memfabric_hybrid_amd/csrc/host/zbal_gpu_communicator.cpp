@@ -825,6 +825,9 @@ public:
         int64_t clearCount = sgl ? allRows : 0, partsBytes = (uint8_t *)y + rows * H * 2 - (uint8_t *)parts;
         if (mode == 3 || partsBytes <= ZBALHIP_PART_WORDS * 4 || parts - clearFrom > clearCount + 1024) parts = nullptr;
         else clearCount = parts + ZBALHIP_PART_WORDS - clearFrom;
+        /* few rows: the second GEMM takes the first one's values, if y is not where they lie */
+        const int32_t valuesFlag = sgl && (uint8_t *)y >= (uint8_t *)(sgl + allRows * (I + 1)) &&
+                                   zbalhip_gmm2_takes_values(E + (ride ? 1 : 0), allRows, I, mode) ? ZBALHIP_SWIGLU_VALUES : 0;
         if (T == 0) { /* nothing routed: counts are zero */
             return Launched(op, zbalhip_fused_permute_quant(x->data, x->dataType, (const int32_t *)expertIds->data, smooth,
                                                             nullptr, 0, H, K, E, qmode, q1, xs, expandIdx,
@@ -870,9 +873,10 @@ public:
                                                 ZBALHIP_LAYOUT_MAX_BLOCKS, stream);
         if (rc != 0) return Launched(op, rc);
         rc = zbalhip_gmm1_swiglu_quant_parts(q1, xs, gmm1Weight->data, gmm1Scale->data, rowOff, E, rows, H, N1,
-                                             gemmMode | clearedFlag, q2, scale2, sgl, ride ? &along1 : nullptr, parts, partsBytes, stream);
+                                             gemmMode | clearedFlag | valuesFlag, q2, scale2, sgl, ride ? &along1 : nullptr, parts, partsBytes, stream);
         if (rc != 0) return Launched(op, rc);
-        rc = zbalhip_gmm2_dequant_shared(q2, scale2, gmm2Weight->data, gmm2Scale->data, wscale2Dt, rowOff, E, rows, I, H, gemmMode,
+        rc = zbalhip_gmm2_dequant_shared(valuesFlag ? (const void *)sgl : q2, valuesFlag ? sgl + allRows * I : scale2, gmm2Weight->data,
+                                         gmm2Scale->data, wscale2Dt, rowOff, E, rows, I, H, gemmMode | valuesFlag,
                                          x->dataType, y, ride ? &along2 : nullptr, stream);
         if (rc != 0) return Launched(op, rc);
         const void *ySrc[1] = {y};

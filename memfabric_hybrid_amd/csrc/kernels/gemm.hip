@@ -849,10 +849,10 @@ int32_t prepare_shape(hipStream_t st, int *n_cus)
     return prepare_kernel<&grouped_gemm_dma_kernel<MODE, GMM1, OUT_DT, TM, NSTAGE, RG, WSTREAM, SH>, S::LDS_BYTES>(st, n_cus);
 }
 
-template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1, bool VALUES = false>
 int32_t prepare_stream(hipStream_t st, int *n_cus)
 {
-    return prepare_kernel<&grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT>, StreamShape<MODE, TM, SPLIT>::LDS_BYTES>(st, n_cus);
+    return prepare_kernel<&grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT, VALUES>, StreamShape<MODE, TM, SPLIT, VALUES>::LDS_BYTES>(st, n_cus);
 }
 
 template <int MODE, bool GMM1, int OUT_DT, bool ANY_K = false>
@@ -891,16 +891,16 @@ int32_t launch_dma_shape(const GemmParams &p, int n_tiles, hipStream_t st)
 }
 
 /* the streaming kernel: every XCD gets a workgroup for each tile it can have (a partial row tile per expert with rows at most) */
-template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1, bool VALUES = false>
 int32_t launch_stream(const GemmParams &p, int n_tiles, hipStream_t st)
 {
-    using S = StreamShape<MODE, TM, SPLIT>;
+    using S = StreamShape<MODE, TM, SPLIT, VALUES>;
     int n_cus = 0;
-    const int32_t rc = prepare_stream<MODE, GMM1, OUT_DT, TM, SPLIT>(st, &n_cus);
+    const int32_t rc = prepare_stream<MODE, GMM1, OUT_DT, TM, SPLIT, VALUES>(st, &n_cus);
     if (rc != ZBALHIP_OK) return rc;
     const int64_t partial = p.max_rows < p.experts ? p.max_rows : p.experts;
     const int64_t per_xcd = (p.max_rows / TM + partial) * ((n_tiles * SPLIT + 7) / 8) + (p.part_sums ? p.part_cus : 0);
-    grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT><<<(unsigned)(8 * per_xcd), S::THREADS, S::LDS_BYTES, st>>>(p);
+    grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT, VALUES><<<(unsigned)(8 * per_xcd), S::THREADS, S::LDS_BYTES, st>>>(p);
     return zbalhip_check_launch();
 }
 
@@ -1015,6 +1015,10 @@ int32_t prepare_mode()
     if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, StreamRows<MODE, GMM1>::TALL>(nullptr, &n);
     if constexpr (!(MODE == MODE_FP8 && GMM1)) {
         if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, 16, 2>(nullptr, &n);
+    }
+    if constexpr (MODE != MODE_FP8 && !GMM1) {
+        if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, 16, 2, true>(nullptr, &n);
+        if (rc == ZBALHIP_OK) rc = prepare_stream<MODE, GMM1, OUT_DT, 32, 1, true>(nullptr, &n);
     }
     if constexpr (MODE == MODE_W4A8) {
         if (rc == ZBALHIP_OK) rc = prepare_shape<MODE, GMM1, OUT_DT, 128, 3, 2, false>(nullptr, &n);
@@ -1137,7 +1141,27 @@ int32_t launch_dma(const GemmParams &p, int n_tiles, hipStream_t st)
     }
 }
 
+/* the second GEMM of the int modes from the first one's fp32 values (zbalhip_gmm2_takes_values) */
+template <int MODE, int OUT_DT>
+int32_t launch_values(const GemmParams &p, int n_tiles, hipStream_t st)
+{
+    if (few_tiles(p, n_tiles)) return launch_stream<MODE, false, OUT_DT, 16, 2, true>(p, n_tiles, st);
+    return launch_stream<MODE, false, OUT_DT, 32, 1, true>(p, n_tiles, st);
+}
+
 } // namespace
+
+/*
+ * The requantisation launch is saved, but every channel tile of an expert makes its rows' bytes again, the more of them the
+ * longer a row and the more rows. Layers, us: 7168 x 4096 / 2048 x 7168, 32 experts, W8A8, 1 row per 4 experts 76.2 -> 73.7, 1 row per
+ * expert 188 -> 182, 2.3 rows 236 -> 232, 3 rows 238 -> 238, 8 rows 242.5 -> 243.5, Zipf(1.2) 242 -> 246; 128 of 4096 x 3072 /
+ * 1536 x 4096, W4A8, 1 token 37.9 -> 34.4, 3 rows 211 -> 207, 8 rows 226 -> 228; 64 of 2048 x 2048 / 1024 x 2048, W8A8, 1 token
+ * 32.3 -> 29.4, 2 rows 74.2 -> 71.7, 4.7 rows Zipf 76.8 -> 75.3.
+ */
+extern "C" int32_t zbalhip_gmm2_takes_values(int64_t experts, int64_t max_rows, int64_t k, int32_t mode)
+{
+    return (mode == MODE_W8A8 || mode == MODE_W4A8) && k > 0 && k % 512 == 0 && max_rows * k <= 5120 * experts;
+}
 
 /* the shared expert that rides along: one expert more, its rows from max_rows on (`shared` null: none) */
 static void with_shared(GemmParams &p, const zbalhip_shared_expert_t *shared, int64_t out_row_bytes)
@@ -1181,8 +1205,9 @@ extern "C" int32_t zbalhip_gmm1_swiglu_quant_parts(const void *a, const float *a
                                                    const zbalhip_shared_expert_t *shared, void *parts, int64_t parts_bytes, void *stream)
 {
     const int w_is_list = (mode & ZBALHIP_WEIGHTS_AS_LISTS) != 0;
-    const bool rowmax_cleared = (mode & ZBALHIP_ROWMAX_CLEARED) != 0;
-    mode &= ~(ZBALHIP_WEIGHTS_AS_LISTS | ZBALHIP_ROWMAX_CLEARED);
+    const bool rowmax_cleared = (mode & ZBALHIP_ROWMAX_CLEARED) != 0, values = (mode & ZBALHIP_SWIGLU_VALUES) != 0;
+    mode &= ~(ZBALHIP_WEIGHTS_AS_LISTS | ZBALHIP_ROWMAX_CLEARED | ZBALHIP_SWIGLU_VALUES);
+    if (values && mode == MODE_FP8) return ZBALHIP_INVALID;
     if (!a || !a_scale || !w1 || !w1scale || !row_off || !q2 || !scale2) return ZBALHIP_INVALID;
     if (mode < MODE_W8A8 || mode > MODE_W4A8) return ZBALHIP_INVALID;
     if (misaligned16(a) || misaligned16(w1) || misaligned16(w1scale) || misaligned16(q2) || misaligned16(sgl_ws)) return ZBALHIP_INVALID;
@@ -1206,7 +1231,7 @@ extern "C" int32_t zbalhip_gmm1_swiglu_quant_parts(const void *a, const float *a
     if (!rowmax_cleared) fill_u32_kernel<<<(unsigned)((p.max_rows + 255) / 256), 256, 0, st>>>(p.rowmax, p.max_rows, 0u);
     const int32_t rc = mode == MODE_W8A8 ? launch_dma<MODE_W8A8, true, ZDT_BF16>(p, n_tiles, st)
                                          : launch_dma<MODE_W4A8, true, ZDT_BF16>(p, n_tiles, st);
-    if (rc != ZBALHIP_OK) return rc;
+    if (rc != ZBALHIP_OK || values) return rc;
     const int rb = p.max_rows < 16384 ? p.max_rows : 16384;
     requant_rows_kernel<<<(unsigned)rb, kRequantThreads, 0, st>>>(sgl_ws, p.rowmax, row_off, p.experts, shared ? p.shared_row : p.max_rows,
                                                                   p.max_rows, (int)(n1 / 2), (int8_t *)q2, scale2);
@@ -1237,7 +1262,9 @@ extern "C" int32_t zbalhip_gmm2_dequant_shared(const void *a, const float *a_sca
                                                void *y, const zbalhip_shared_expert_t *shared, void *stream)
 {
     const int w_is_list = (mode & ZBALHIP_WEIGHTS_AS_LISTS) != 0;
-    mode &= ~ZBALHIP_WEIGHTS_AS_LISTS;
+    const bool values = (mode & ZBALHIP_SWIGLU_VALUES) != 0;
+    mode &= ~(ZBALHIP_WEIGHTS_AS_LISTS | ZBALHIP_SWIGLU_VALUES);
+    if (values && (mode == MODE_FP8 || k % 512 != 0)) return ZBALHIP_INVALID;
     if (!a || !a_scale || !w2 || !wscale || !row_off || !y) return ZBALHIP_INVALID;
     if (mode < MODE_W8A8 || mode > MODE_W4A8) return ZBALHIP_INVALID;
     if (misaligned16(a) || misaligned16(w2) || misaligned16(wscale) || misaligned16(y)) return ZBALHIP_INVALID;
@@ -1257,6 +1284,10 @@ extern "C" int32_t zbalhip_gmm2_dequant_shared(const void *a, const float *a_sca
     with_shared(p, shared, n * 2);
     const int n_tiles = (int)(n / BN);
     const bool bf = out_dtype == ZDT_BF16;
+    if (values) {
+        if (mode == MODE_W8A8) return bf ? launch_values<MODE_W8A8, ZDT_BF16>(p, n_tiles, st) : launch_values<MODE_W8A8, ZDT_FP16>(p, n_tiles, st);
+        return bf ? launch_values<MODE_W4A8, ZDT_BF16>(p, n_tiles, st) : launch_values<MODE_W4A8, ZDT_FP16>(p, n_tiles, st);
+    }
     if (mode == MODE_W8A8)
         return bf ? launch_dma<MODE_W8A8, false, ZDT_BF16>(p, n_tiles, st) : launch_dma<MODE_W8A8, false, ZDT_FP16>(p, n_tiles, st);
     if (mode == MODE_FP8)

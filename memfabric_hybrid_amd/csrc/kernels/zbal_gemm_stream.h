@@ -29,7 +29,7 @@
 
 namespace {
 
-template <int MODE, int TM, int SPLIT = 1> struct StreamShape {
+template <int MODE, int TM, int SPLIT = 1, bool VALUES = false> struct StreamShape {
     /* in the taller tiles the L2 serves the weights: two slabs of look-ahead do, and leave registers for six or eight row sub-tiles */
     static constexpr int PF = TM > (MODE == MODE_FP8 ? 48 : 64) ? 2 : 4;                  /* slabs in flight, and slabs per activation chunk */
     static constexpr int MT_STEP = 4 / PF;                      /* row sub-tiles come in ones, or in twos: then two slabs of them are one transfer of every wave */
@@ -43,7 +43,9 @@ template <int MODE, int TM, int SPLIT = 1> struct StreamShape {
     static constexpr int GS_BYTES = MODE == MODE_W4A8 ? PF * BN * 2 : 0;  /* one chunk's fp16 group scales, [slab][channel] */
     static constexpr int SA_LOADS = PF > NW ? PF / NW : 1;
     static constexpr int ES_FLOATS = MODE == MODE_FP8 ? 2 * 256 : (MODE == MODE_W8A8 ? 256 : 0) + (TM + 63) / 64 * 64;
-    static constexpr int LDS_BYTES = 2 * (A_BYTES + SA_FLOATS * 4 + GS_BYTES) + ES_FLOATS * 4 + NW * TM * 4;
+    /* VALUES, see k_loop: the activations of as many slabs as there is room for, [slab][rows of the sub-tiles that there are][128 bytes, swizzled] */
+    static constexpr int A_ALL = VALUES ? 2048 * TM : 2 * A_BYTES;
+    static constexpr int LDS_BYTES = A_ALL + 2 * (SA_FLOATS * 4 + GS_BYTES) + ES_FLOATS * 4 + NW * TM * 4;
     static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
 };
 
@@ -81,18 +83,19 @@ template <int N> __device__ __forceinline__ void wait_w(u32x4 (&w)[2][2])
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]) : "n"(N));
 }
 
-template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1>
+template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1, bool VALUES = false>
 __global__ void __launch_bounds__(512 / SPLIT, 4)
 grouped_gemm_stream_kernel(GemmParams p)
 {
+    static_assert(!VALUES || (!GMM1 && MODE != MODE_FP8 && StreamShape<MODE, TM, SPLIT>::PF == 4), "second GEMM of the int modes, lower tiles");
     static_assert(SPLIT == 1 || MODE != MODE_FP8 || !GMM1, "fp8's first GEMM requantises 128 columns, which are one workgroup's");
-    using S = StreamShape<MODE, TM, SPLIT>;
+    using S = StreamShape<MODE, TM, SPLIT, VALUES>;
     constexpr int PF = S::PF, NT = S::NT, MTM = S::MTM, LOADS = S::LOADS, NW = S::NW, WRB = S::WRB;
     constexpr int MAX_PARTS = 4;
     constexpr bool SHARES_K = GMM1 && MODE != MODE_W4A8 && SPLIT == 1;
     constexpr int W_BLOCK_BYTES = 128 * WRB;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    float *lds_sa = reinterpret_cast<float *>(smem + 2 * S::A_BYTES);
+    float *lds_sa = reinterpret_cast<float *>(smem + S::A_ALL);
     uint16_t *lds_gs = reinterpret_cast<uint16_t *>(lds_sa + 2 * S::SA_FLOATS);
     float *lds_es = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(lds_gs) + 2 * S::GS_BYTES);
     float *lds_rowmax = lds_es + S::ES_FLOATS;
@@ -239,7 +242,7 @@ grouped_gemm_stream_kernel(GemmParams p)
         asm volatile("" : "+v"(lane_x));           /* the lane offsets are worked out afresh: there is no register to keep them in */
         const int r = lane_x >> 3;
 #pragma unroll
-        for (int j = 0; j < MT * SPLIT / S::MT_STEP; ++j) {        /* slab s of row block rb */
+        for (int j = 0; j < (VALUES ? 0 : MT * SPLIT / S::MT_STEP); ++j) {        /* slab s of row block rb */
             const int s = (wave + j * NW) & (PF - 1), rb = (wave + j * NW) / PF;
             int rel = rb * 8 + r;
             const uint32_t chunk16 = ((lane_x & 7) ^ (r ^ (rb & 1))) * 16;
@@ -276,7 +279,7 @@ grouped_gemm_stream_kernel(GemmParams p)
 #pragma unroll
         for (int j = 0; j < SPLIT; ++j) {
             const int t = wave + j * NW;
-            if (t < (TM + 63) / 64) {                              /* 64 token scales each */
+            if (!VALUES && t < (TM + 63) / 64) {                   /* 64 token scales each */
                 const int rel = t * 64 + lane > last_rel ? last_rel : t * 64 + lane;
                 dma4_sv(p.a_scale + row_begin, (uint32_t)rel * 4u, dst0 + (MODE == MODE_W8A8 ? 1024 : 0) + t * 256);
             }
@@ -319,9 +322,10 @@ grouped_gemm_stream_kernel(GemmParams p)
     i32x4 magic = {0x4b400000, 0x4b400000, 0x4b400000, 0x4b400000};      /* W4A8: see multiply() */
     if constexpr (MODE == MODE_W4A8) asm volatile("" : "+v"(magic));
     /* one slab over the first MT row sub-tiles: fragments of slot s, activations of slab s of buffer b */
+    int values_from = 0;           /* VALUES: first slab of those in LDS */
     auto multiply = [&](auto mt_tag, const Slabs &wr, int s, int b, int kb) __attribute__((always_inline)) {
         constexpr int MT = decltype(mt_tag)::value;
-        const uint8_t *ab = smem + b * S::A_BYTES + s * (TM * BKB);
+        const uint8_t *ab = VALUES ? smem + (kb - values_from) * (MT * 2048) : smem + b * S::A_BYTES + s * (TM * BKB);
         auto load_a = [&](int mt) -> i32x8 {
             const u32x4 lo = *reinterpret_cast<const u32x4 *>(ab + mt * (16 * BKB) + off_lo);
             const u32x4 hi = *reinterpret_cast<const u32x4 *>(ab + mt * (16 * BKB) + off_hi);
@@ -455,11 +459,80 @@ grouped_gemm_stream_kernel(GemmParams p)
     auto k_loop = [&](auto mt_tag, auto stream_tag) __attribute__((always_inline)) {
         constexpr int MT = decltype(mt_tag)::value;
         constexpr int L = NT * LOADS;                                   /* loads per slab */
-        constexpr int D = MT * SPLIT / S::MT_STEP + (MODE == MODE_W8A8 ? 0 : (MODE == MODE_FP8 ? S::SA_LOADS : SPLIT));      /* transfers per chunk */
+        constexpr int D = (VALUES ? 0 : MT * SPLIT / S::MT_STEP) + (MODE == MODE_W8A8 ? 0 : (MODE == MODE_FP8 ? S::SA_LOADS : SPLIT));      /* transfers per chunk */
         Slabs wr;
-        issue_chunk(mt_tag, kb_from, 0);
+        /*
+         * VALUES: the int modes' second GEMM with few rows makes the bytes of its rows itself, of the first GEMM's fp32 values and the
+         * rows' maxima, instead of a launch between the two (4.7 us, in which nothing streams): a group of slabs at a time, as many as
+         * there is room for, the first behind its own requests for weights. See zbalhip_gmm2_takes_values.
+         */
+        constexpr int GROUP = S::A_ALL / (MT * 2048) / PF * PF, BATCH = MODE == MODE_W8A8 ? 4 : 8;
+        uint32_t row_max = 0;
+        auto request_values = [&](u32x4 (&v)[BATCH], int first, int from, int pieces, int total) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < PF; ++s) load_w(stream_tag, wr, s, kb_from + s);
+            for (int j = 0; j < BATCH; ++j) {
+                const int i = first + j * NW < total ? first + j * NW : total - 1, row = i / pieces;
+                load16_sv<false>(v[j], lane * 16, uniform_ptr(p.a + ((int64_t)(row_begin + row) * K + from * 128 + (i - row * pieces) * 256) * 4));
+            }
+        };
+        /* behind the wait, for the compiler */
+        auto touch = [&](u32x4 (&v)[BATCH]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) asm volatile("" : "+v"(v[j]));
+        };
+        auto store_values = [&](const u32x4 (&v)[BATCH], int first, int pieces, int total) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) {
+                const int i = first + j * NW;
+                if (i >= total) break;
+                const int row = i / pieces;
+                const float mx = __uint_as_float(__builtin_amdgcn_readlane(row_max, row)), inv = mx == 0.0f ? 0.0f : 1.0f / mx;
+                uint32_t q = 0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) q |= ((uint32_t)zb_rint_i8((__uint_as_float(v[j][u]) * 127.0f) * inv) & 0xffu) << (8 * u);
+                const int slab = (i - row * pieces) * 2 + (lane >> 5), slot = ((lane & 31) >> 2) ^ (row & 7) ^ ((row >> 3) & 1);
+                *reinterpret_cast<uint32_t *>(smem + slab * (MT * 2048) + row * BKB + slot * 16 + (lane & 3) * 4) = q;
+            }
+        };
+        auto bring_values = [&](int from, auto first_tag) __attribute__((always_inline)) {
+            constexpr bool FIRST = decltype(first_tag)::value;
+            const int slabs = from + GROUP < KB ? GROUP : KB - from, pieces = slabs / 2, total = (last_rel + 1) * pieces;
+            values_from = from;
+            u32x4 v[BATCH];
+            if constexpr (FIRST) {
+                const int row = lane <= last_rel ? lane : last_rel;
+                asm volatile("s_nop 4\n\tglobal_load_dword %0, %1, %2" : "=v"(row_max) : "v"((uint32_t)row * 4u), "s"(uniform_ptr((const uint8_t *)(p.a_scale + row_begin))));
+                request_values(v, wave, from, pieces, total);
+#pragma unroll
+                for (int s = 0; s < PF; ++s) load_w(stream_tag, wr, s, kb_from + s);
+                /* everything but the fragments has landed */
+                asm volatile("s_waitcnt vmcnt(%1)" : "+v"(row_max) : "n"(PF * L));
+                touch(v);
+                if (wave == 0 && lane < TM) lds_es[(MODE == MODE_W8A8 ? 256 : 0) + lane] = __uint_as_float(row_max) * (1.0f / 127.0f);
+                store_values(v, wave, pieces, total);
+            }
+            for (int first = wave + (FIRST ? BATCH * NW : 0); first < total; first += BATCH * NW) {
+                request_values(v, first, from, pieces, total);
+                asm volatile("s_waitcnt vmcnt(0)");
+                touch(v);
+                store_values(v, first, pieces, total);
+            }
+        };
+        issue_chunk(mt_tag, kb_from, 0);
+        if constexpr (VALUES) {
+            bring_values(0, std::true_type{});
+        } else {
+#pragma unroll
+            for (int s = 0; s < PF; ++s) load_w(stream_tag, wr, s, kb_from + s);
+        }
+        auto next_values = [&](int kb0) __attribute__((always_inline)) {      /* before chunk kb0, behind its barrier */
+            if constexpr (VALUES) {
+                if (kb0 - values_from == GROUP) {
+                    bring_values(kb0, std::false_type{});
+                    lds_barrier();
+                }
+            }
+        };
         /* issued since chunk c's transfers: the fragments of its slabs, L each; since slab s's fragments: three more slabs, and D */
         auto begin_chunk = [&]() __attribute__((always_inline)) {
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(PF * L) : "memory");
@@ -467,6 +540,7 @@ grouped_gemm_stream_kernel(GemmParams p)
         int b = 0, kb0 = kb_from;
         for (; kb0 + PF < kb_to; kb0 += PF) {
             begin_chunk();               /* chunk kb0's activations have landed for everybody, and nobody reads the other buffer any more */
+            next_values(kb0);
             issue_chunk(mt_tag, kb0 + PF, b ^ 1);
 #pragma unroll
             for (int s = 0; s < PF; ++s) {
@@ -478,6 +552,7 @@ grouped_gemm_stream_kernel(GemmParams p)
             b ^= 1;
         }
         begin_chunk();
+        next_values(kb0);
         if constexpr (PF == 4) {
             wait_w<3 * L>(wr[0]);
             multiply(mt_tag, wr, 0, b, kb0);
