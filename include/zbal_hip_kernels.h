@@ -305,7 +305,7 @@ ZBALHIP_API int32_t zbalhip_fused_permute_quant(const void *x, int32_t x_dtype, 
  * values), and makes the bytes of its rows itself. y may not lie on top of them. K of the second GEMM in whole multiples of 512.
  * zbalhip_gmm2_takes_values: whether that is the faster way (one launch less, but every channel tile makes its rows' bytes).
  */
-#define ZBALHIP_SWIGLU_VALUES 0x400
+#define ZBALHIP_SWIGLU_VALUES 0x800
 ZBALHIP_API int32_t zbalhip_gmm2_takes_values(int64_t experts, int64_t max_rows, int64_t k, int32_t mode);
 
 /*

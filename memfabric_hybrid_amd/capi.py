@@ -24,7 +24,7 @@ DT_UINT8, DT_UINT16, DT_UINT32, DT_FP8_E4M3, DT_INT4X2 = 9, 10, 11, 12, 13
 REDUCE_PROD, REDUCE_SUM, REDUCE_MAX, REDUCE_MIN = 0, 1, 2, 3
 # zbal_quant_mode_t
 NO_QUANT, QUANT_INT8, QUANT_FP8_B128, QUANT_W4A8_G128 = 0, 1, 2, 3
-SWIGLU_VALUES = 0x400    # ZBALHIP_SWIGLU_VALUES: OR-ed into the mode of both GEMMs
+SWIGLU_VALUES = 0x800    # ZBALHIP_SWIGLU_VALUES: OR-ed into the mode of both GEMMs
 ROWMAX_CLEARED = 0x200   # ZBALHIP_ROWMAX_CLEARED: OR-ed into the mode of zbalhip_gmm1_swiglu_quant
 # zbal_backend_t
 BACKEND_GPU, BACKEND_DUMMY = 0, 1

@@ -774,10 +774,10 @@ requant_rows_kernel(const float *__restrict__ sgl, const uint32_t *__restrict__ 
 #pragma unroll
             for (int u = 0; u < kRequantPieces; ++u) {
                 const int c = c0 + u * kRequantThreads + (int)threadIdx.x;
-                uint32_t w = 0;
+                float q[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w |= ((uint32_t)zb_rint_i8((v[u][i] * 127.0f) * inv) & 0xffu) << (8 * i);
-                if (c < vecs) dst[c] = w;
+                for (int i = 0; i < 4; ++i) q[i] = (v[u][i] * 127.0f) * inv;
+                if (c < vecs) dst[c] = zb_pack4_i8(q[0], q[1], q[2], q[3]);
             }
         }
     }

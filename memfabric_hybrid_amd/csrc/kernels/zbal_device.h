@@ -106,12 +106,17 @@ __device__ __forceinline__ uint32_t zb_cvt_pk_e4m3(float a, float b)
     return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) & 0xffffu;
 }
 
-/* round-half-even to int, clamped to int8 */
-__device__ __forceinline__ int32_t zb_rint_i8(float v)
+/*
+ * Four floats -> four int8 in a dword: clamped to [-128, 127], rounded to nearest even by the addition of 1.5 * 2^23, which leaves the
+ * integer in the low bits. A NaN gives -128 (the median of a NaN and two numbers is the smaller number).
+ */
+__device__ __forceinline__ uint32_t zb_pack4_i8(float a, float b, float c, float d)
 {
-    float r = __builtin_rintf(v);
-    r = fminf(fmaxf(r, -128.0f), 127.0f);
-    return (int32_t)r;
+    constexpr float MAGIC = 12582912.0f;
+    const uint32_t ai = __float_as_uint(__builtin_amdgcn_fmed3f(a, -128.0f, 127.0f) + MAGIC), bi = __float_as_uint(__builtin_amdgcn_fmed3f(b, -128.0f, 127.0f) + MAGIC);
+    const uint32_t ci = __float_as_uint(__builtin_amdgcn_fmed3f(c, -128.0f, 127.0f) + MAGIC), di = __float_as_uint(__builtin_amdgcn_fmed3f(d, -128.0f, 127.0f) + MAGIC);
+    const uint32_t ab = __builtin_amdgcn_perm(bi, ai, 0x0c0c0400), cd = __builtin_amdgcn_perm(di, ci, 0x04000c0c);
+    return ab | cd;
 }
 
 /*
@@ -187,6 +192,14 @@ struct ExpertIds {
         if (kind == IDS_I32) return p[i];
         const u32x2 w = reinterpret_cast<const u32x2 *>(p)[i];
         return of_words(w[0], w[1]);
+    }
+    /* ids i .. i + 3, one or two loads that need no more than the array's alignment */
+    __device__ __forceinline__ i32x4 four(int64_t i) const
+    {
+        typedef u32x4 __attribute__((aligned(4))) words_t;
+        if (kind == IDS_I32) return __builtin_bit_cast(i32x4, (u32x4)*reinterpret_cast<const words_t *>(p + i));
+        const u32x4 a = *reinterpret_cast<const words_t *>(p + 2 * i), b = *reinterpret_cast<const words_t *>(p + 2 * i + 4);
+        return i32x4{of_words(a[0], a[1]), of_words(a[2], a[3]), of_words(b[0], b[1]), of_words(b[2], b[3])};
     }
 };
 inline ExpertIds expert_ids(const void *p, bool is_i64, bool full = false)

@@ -487,11 +487,11 @@ grouped_gemm_stream_kernel(GemmParams p)
                 if (i >= total) break;
                 const int row = i / pieces;
                 const float mx = __uint_as_float(__builtin_amdgcn_readlane(row_max, row)), inv = mx == 0.0f ? 0.0f : 1.0f / mx;
-                uint32_t q = 0;
+                float q[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) q |= ((uint32_t)zb_rint_i8((__uint_as_float(v[j][u]) * 127.0f) * inv) & 0xffu) << (8 * u);
+                for (int u = 0; u < 4; ++u) q[u] = (__uint_as_float(v[j][u]) * 127.0f) * inv;
                 const int slab = (i - row * pieces) * 2 + (lane >> 5), slot = ((lane & 31) >> 2) ^ (row & 7) ^ ((row >> 3) & 1);
-                *reinterpret_cast<uint32_t *>(smem + slab * (MT * 2048) + row * BKB + slot * 16 + (lane & 3) * 4) = q;
+                *reinterpret_cast<uint32_t *>(smem + slab * (MT * 2048) + row * BKB + slot * 16 + (lane & 3) * 4) = zb_pack4_i8(q[0], q[1], q[2], q[3]);
             }
         };
         auto bring_values = [&](int from, auto first_tag) __attribute__((always_inline)) {
