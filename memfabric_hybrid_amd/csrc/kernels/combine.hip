@@ -190,7 +190,7 @@ extern "C" int32_t zbalhip_combine(const void *const *y, int32_t ranks, int32_t 
     const dim3 grid((unsigned)tokens, (unsigned)splits);
     hipStream_t st = (hipStream_t)stream;
 #define ZB_GO_BASES(DT, U, BASES)                                                                                     \
-    combine_kernel<DT, U, BASES><<<grid, threads, 0, st>>>(src, base, base_is_inclusive, w, ids, send_token_idx,       \
+    zb_launch(combine_kernel<DT, U, BASES>, grid, threads, 0, st, src, base, base_is_inclusive, w, ids, send_token_idx, \
                                                            (int)hidden, (int)topk, (int)experts, (uint16_t *)out)
 #define ZB_GO(DT, U)                                                                                                  \
     do {                                                                                                              \

@@ -722,7 +722,7 @@ int32_t launch_quant(const void *x, const ExpertIds &topk_idx, const int32_t *ra
     const NotifyOut no = ex.notify ? *ex.notify : NotifyOut{};
     constexpr bool NOTIFIES = !SMOOTH && QM != QM_INT8_NOEPS;      /* the quantisations of the normal-mode dispatch */
 #define ZB_LAUNCH_I(S, LMV)                                                                                       \
-    permute_quant_kernel<XDT, QM, S, SMOOTH, LMV><<<(unsigned)(tokens + (LMV == LM_INLINE ? 1 : 0)), threads, 0, st>>>( \
+    zb_launch(permute_quant_kernel<XDT, QM, S, SMOOTH, LMV>, (unsigned)(tokens + (LMV == LM_INLINE ? 1 : 0)), threads, 0, st,  \
         (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, smooth, (int)hidden, (int)topk,       \
         (int)experts, pr, il, rt, ex.shared, no, ex.clear_words, ex.clear_count)
 #define ZB_LAUNCH(S)                                                                                              \
@@ -763,15 +763,15 @@ static int32_t permute_launch(const void *x, int32_t x_dtype, const ExpertIds &t
         if (threads > kThreads) threads = kThreads;
         if (ex.inline_layout && tokens * topk > kCountByAll) threads = kThreads;
         if (ex.inline_layout)
-            permute_copy_kernel<LM_INLINE, 4><<<(unsigned)tokens + 1, threads, 0, st>>>(
+            zb_launch(permute_copy_kernel<LM_INLINE, 4>, (unsigned)tokens + 1, threads, 0, st,
                 (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, (int)hidden, (int)topk, (int)experts, pr,
                 *ex.inline_layout, NotifyOut{});
         else if (ex.notify)
-            permute_copy_kernel<LM_COUNTS, 4><<<(unsigned)tokens, threads, 0, st>>>(
+            zb_launch(permute_copy_kernel<LM_COUNTS, 4>, (unsigned)tokens, threads, 0, st,
                 (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, (int)hidden, (int)topk, (int)experts, pr,
                 InlineLayout{}, *ex.notify);
         else
-            permute_copy_kernel<LM_GIVEN, 4><<<(unsigned)tokens, threads, 0, st>>>(
+            zb_launch(permute_copy_kernel<LM_GIVEN, 4>, (unsigned)tokens, threads, 0, st,
                 (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, (int)hidden, (int)topk, (int)experts, pr,
                 InlineLayout{}, NotifyOut{});
         return zbalhip_check_launch();

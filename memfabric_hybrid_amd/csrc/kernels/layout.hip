@@ -620,10 +620,10 @@ static int32_t launch_fused_layout(const ExpertIds &idx, int64_t tokens, int64_t
 {
     const LayoutPlan p = plan_layout(tokens, topk, 64);
     if (o.tokens_per_rank || o.token_in_rank)
-        layout_fused_kernel<true><<<p.nblk + 2, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,
+        zb_launch(layout_fused_kernel<true>, p.nblk + 2, ZB_FUSED_THREADS, 0, st, idx, (int)tokens, (int)topk, (int)experts,
                                                                      p.tokens_per_block, ceil_log2(experts), active_mask, o);
     else
-        layout_fused_kernel<false><<<p.nblk + 1, ZB_FUSED_THREADS, 0, st>>>(idx, (int)tokens, (int)topk, (int)experts,
+        zb_launch(layout_fused_kernel<false>, p.nblk + 1, ZB_FUSED_THREADS, 0, st, idx, (int)tokens, (int)topk, (int)experts,
                                                                       p.tokens_per_block, ceil_log2(experts), active_mask, o);
     return zbalhip_check_launch();
 }
@@ -659,10 +659,10 @@ int32_t zbalhip_layout_ranges_internal(const ExpertIds &idx, int64_t tokens, int
     subs = subs < 1 ? 1 : (subs > 8 ? 8 : subs);
     if (subs > tokens_per_block) subs = tokens_per_block;
     if (subs == 1)
-        layout_ranges_kernel<false><<<(unsigned)nblk, ZB_FUSED_THREADS, 0, st>>>(
+        zb_launch(layout_ranges_kernel<false>, (unsigned)nblk, ZB_FUSED_THREADS, 0, st,
             idx, (int)tokens, (int)topk, (int)experts, tokens_per_block, 1, ceil_log2(experts), active_mask, send_token_idx, hist);
     else
-        layout_ranges_kernel<true><<<(unsigned)(nblk * subs), ZB_FUSED_THREADS, 0, st>>>(
+        zb_launch(layout_ranges_kernel<true>, (unsigned)(nblk * subs), ZB_FUSED_THREADS, 0, st,
             idx, (int)tokens, (int)topk, (int)experts, tokens_per_block, (int)subs, ceil_log2(experts), active_mask,
             send_token_idx, hist);
     return zbalhip_check_launch();
@@ -707,10 +707,10 @@ extern "C" int32_t zbalhip_topk_route(const float *logits, int64_t tokens, int64
     const int64_t blocks = (tokens + wpb - 1) / wpb;
     const dim3 grid((unsigned)blocks), block(wpb * 64);
     hipStream_t st = (hipStream_t)stream;
-    if (experts <= 64) topk_route_small_kernel<<<grid, block, 0, st>>>(logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
-    else if (experts <= 128) topk_route_kernel<2><<<grid, block, 0, st>>>(logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
-    else if (experts <= 256) topk_route_kernel<4><<<grid, block, 0, st>>>(logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
-    else topk_route_kernel<ZB_MAX_EXPERTS / 64><<<grid, block, 0, st>>>(logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
+    if (experts <= 64) zb_launch(topk_route_small_kernel, grid, block, 0, st, logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
+    else if (experts <= 128) zb_launch(topk_route_kernel<2>, grid, block, 0, st, logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
+    else if (experts <= 256) zb_launch(topk_route_kernel<4>, grid, block, 0, st, logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
+    else zb_launch(topk_route_kernel<ZB_MAX_EXPERTS / 64>, grid, block, 0, st, logits, (int)tokens, (int)experts, (int)topk, topk_idx, idx_is_i64, topk_w);
     return zbalhip_check_launch();
 }
 
@@ -769,7 +769,7 @@ static int32_t launch_notify(const int32_t *const *tokens_per_expert, int32_t ra
         if (!tokens_per_expert[r]) return ZBALHIP_INVALID;
     const int threads = (int)((experts + 63) / 64 * 64);
     if (ranks == 1) {
-        notify_one_kernel<<<1, threads, 0, st>>>(tokens_per_expert[0], (int)experts, (int)topk, recv_data, put_offset,
+        zb_launch(notify_one_kernel, 1, threads, 0, st, tokens_per_expert[0], (int)experts, (int)topk, recv_data, put_offset,
                                                  recv_tokens_per_expert, total_recv, balance_matrix, host, launch);
         return zbalhip_check_launch();
     }

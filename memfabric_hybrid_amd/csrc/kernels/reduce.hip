@@ -249,7 +249,7 @@ int32_t launch_reduce(const ReducePtrs &ptrs, int n_in, int64_t count, void *out
         sp.chunk = 32;
         blocks = (blocks + 255) / 256 * 256;
     }
-#define ZB_REDUCE(N, ANY) reduce_kernel<DT, OP, N, ANY><<<(unsigned)blocks, threads, 0, st>>>(ptrs, n_in, sp, out)
+#define ZB_REDUCE(N, ANY) zb_launch(reduce_kernel<DT, OP, N, ANY>, (unsigned)blocks, threads, 0, st, ptrs, n_in, sp, out)
     if (!same_offset) ZB_REDUCE(ZBALHIP_MAX_REDUCE_PEERS, true);
     else if (n_in == 1) ZB_REDUCE(1, false);
     else if (n_in == 2) ZB_REDUCE(2, false);
