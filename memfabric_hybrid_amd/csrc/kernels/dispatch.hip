@@ -79,7 +79,18 @@ struct InlineLayout {
     int32_t *row_off;             /* [E + 1] exclusive offsets */
     int64_t *counts_i64;          /* [E] */
     int64_t *nums_typed;          /* [E] counts (type 1) or running sums (type 0) */
+    int part_shift;               /* log2 of how many workgroups share a token's picks, see inline_part_shift */
 };
+
+/* the token of an inline-mode workgroup and which of its picks are this workgroup's: [begin, end) */
+struct PickRange {
+    int token, begin, end, part;
+};
+__device__ __forceinline__ PickRange picks_of_block(const InlineLayout &il, int topk)
+{
+    const int b = (int)blockIdx.x - 1, part = b & ((1 << il.part_shift) - 1);
+    return {b >> il.part_shift, (topk * part) >> il.part_shift, (topk * (part + 1)) >> il.part_shift, part};
+}
 
 /* how many tokens the mask routes (all of them without one); `s` is one word of LDS; holds barriers if there is a mask */
 __device__ __forceinline__ int active_tokens(const uint8_t *mask, int tokens, int32_t *s)
@@ -155,21 +166,22 @@ struct LanePicks {
 };
 
 /*
- * This wave's part of the counts: lane k returns, for pick k of token t, (picks of lower experts) << 16 | (picks that
- * sort before it), over the wave's share of the picks [0, n). my_e: lane k's pick.
+ * This wave's part of the counts: lane k returns, for pick k of token r.token, (picks of lower experts) << 16 | (picks that
+ * sort before it), over the wave's share of the picks [0, n), for the picks of the range. my_e: lane k's pick. KG: picks per pass
+ * over the array.
  */
-__device__ __forceinline__ int32_t count_before(const ExpertIds &idx, int t, int topk, int experts, int n, int my_e)
+template <int KG>
+__device__ __forceinline__ int32_t count_before(const ExpertIds &idx, const PickRange &r, int topk, int experts, int n, int my_e)
 {
     const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63;
-    constexpr int KG = 8;                              /* picks per pass over the array */
     int32_t result = 0;
-    for (int k0 = 0; k0 < topk; k0 += KG) {
+    for (int k0 = r.begin; k0 < r.end; k0 += KG) {
         int32_t first[KG], self[KG], below[KG], before[KG];
 #pragma unroll
         for (int k = 0; k < KG; ++k) {
             const int e = __builtin_amdgcn_readlane(my_e, (k0 + k) & 63);
             first[k] = e << 13;                        /* keys: expert << 13 | pick, kInlineMaxPicks < 2^13 */
-            self[k] = first[k] | (t * topk + k0 + k);
+            self[k] = first[k] | (r.token * topk + k0 + k);
             below[k] = before[k] = 0;
         }
         auto count = [&](int e, int i) __attribute__((always_inline)) {
@@ -414,28 +426,29 @@ __device__ __forceinline__ LanePicks resolve_counts(const GivenPicks &g, const i
 __device__ __forceinline__ int window_of(const PeerRows &pr, int e) { return pr.ranks == 1 ? 0 : e / pr.e_loc; }
 
 /*
- * The workgroup's token in inline mode, in two halves with one barrier of the caller's between them: the wave's counts
+ * The workgroup's token (or its share of one) in inline mode, in two halves with one barrier of the caller's between them: the wave's counts
  * go to LDS, their sums come back as destination rows. Writes the token's expand_idx.
  */
-__device__ __forceinline__ void inline_counts(const ExpertIds &idx, int t, int topk, int experts, int active, int my_e,
-                                              int32_t (*s_cnt)[kInlineMaxTopk])
+__device__ __forceinline__ void inline_counts(const ExpertIds &idx, const PickRange &r, int topk, int experts, int active, int my_e,
+                                              const InlineLayout &il, int32_t (*s_cnt)[kInlineMaxTopk])
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int32_t c = count_before(idx, t, topk, experts, active * topk, my_e);
+    const int32_t c = il.part_shift > 0 ? count_before<2>(idx, r, topk, experts, active * topk, my_e)
+                                        : count_before<8>(idx, r, topk, experts, active * topk, my_e);
     if (lane < topk) s_cnt[wave][lane] = c;
 }
-__device__ __forceinline__ LanePicks inline_rows(int t, int topk, int experts, int active, int my_e, const InlineLayout &il,
+__device__ __forceinline__ LanePicks inline_rows(const PickRange &r, int topk, int experts, int active, int my_e, const InlineLayout &il,
                                                  const PeerRows &pr, int32_t (*s_cnt)[kInlineMaxTopk])
 {
     const int lane = threadIdx.x & 63, nwaves = (blockDim.x + 63) >> 6;
     LanePicks p = {my_e, -1};
-    if (lane < topk) {
+    if (lane >= r.begin && lane < r.end) {
         int32_t c = 0;
         for (int w = 0; w < nwaves; ++w) c += s_cnt[w][lane];
-        const bool valid = my_e >= 0 && my_e < experts, routed = valid && t < active;
-        const int32_t row = c & 0xffff, rank = t >= active ? -2 : (valid ? row - (c >> 16) : -1);
+        const bool valid = my_e >= 0 && my_e < experts, routed = valid && r.token < active;
+        const int32_t row = c & 0xffff, rank = r.token >= active ? -2 : (valid ? row - (c >> 16) : -1);
         if (routed && row < pr.rows_cap) p.row = row;
-        if (threadIdx.x < 64) il.expand_idx[(int64_t)t * topk + lane] = rank;
+        if (threadIdx.x < 64) il.expand_idx[(int64_t)r.token * topk + lane] = rank;
     }
     return p;
 }
@@ -461,7 +474,8 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
         write_inline_layout(topk_idx, topk, experts, il, sh, s_off, s_tmp);
         return;
     }
-    const int t = INLINE ? blockIdx.x - 1 : blockIdx.x;
+    const PickRange mine = INLINE ? picks_of_block(il, topk) : PickRange{(int)blockIdx.x, 0, topk, 0};
+    const int t = mine.token;
     if (!INLINE && sh.end && t == 0) {
         const int n = active_tokens(il.active_mask, il.tokens, s_tmp);
         if (threadIdx.x == 0) *sh.end = (int32_t)(sh.first_row + n);
@@ -493,7 +507,7 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
     int active = 0;
     if constexpr (INLINE) {
         active = active_tokens(il.active_mask, il.tokens, s_tmp);
-        inline_counts(topk_idx, t, topk, experts, active, given.e, s_cnt);
+        inline_counts(topk_idx, mine, topk, experts, active, given.e, il, s_cnt);
     } else if constexpr (TABLE) {
         table_layout(rt, tabv, t / rt.tokens_per_range, experts, t == 0, s_tab, s_off, s_before, s_tmp);
         picks.e = given.e;
@@ -522,9 +536,9 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
         if (lane == 0) red[threadIdx.x >> 6] = amax;
     }
     if constexpr (ROW_MAX || INLINE) __syncthreads();
-    if constexpr (INLINE) picks = inline_rows(t, topk, experts, active, given.e, il, pr, s_cnt);
+    if constexpr (INLINE) picks = inline_rows(mine, topk, experts, active, given.e, il, pr, s_cnt);
     /* rank -2: the layout masked the token out */
-    const bool shares = sh.end && (INLINE ? t < active : __builtin_amdgcn_readlane(given.rank, 0) != -2);
+    const bool shares = sh.end && (INLINE ? mine.part == 0 && t < active : __builtin_amdgcn_readlane(given.rank, 0) != -2);
     /* f(pick's expert, window, row) for every routed pick of the token, and for the shared expert (-1); wave-uniform */
     auto for_each_pick = [&](auto f) __attribute__((always_inline)) {
         for (int k0 = 0; k0 < topk; k0 += 64) {
@@ -532,8 +546,8 @@ permute_quant_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                 picks = resolve_counts(request_given(topk_idx, rank_in_expert, t, topk, k0 + lane), s_off, experts, pr);
             else if (!INLINE && !TABLE && k0 > 0)
                 picks = resolve_given(request_given(topk_idx, rank_in_expert, t, topk, k0 + lane), base, base_inclusive, experts, pr);
-            const int n = topk - k0 < 64 ? topk - k0 : 64;
-            for (int k = 0; k < n; ++k) {
+            const int n = INLINE ? mine.end : (topk - k0 < 64 ? topk - k0 : 64);
+            for (int k = INLINE ? mine.begin : 0; k < n; ++k) {
                 const int32_t row = __builtin_amdgcn_readlane(picks.row, k);
                 if (row < 0) continue;
                 const int e = __builtin_amdgcn_readlane(picks.e, k);
@@ -639,7 +653,8 @@ permute_copy_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
         write_inline_layout(topk_idx, topk, experts, il, SharedRows{}, s_off, s_tmp);
         return;
     }
-    const int t = INLINE ? blockIdx.x - 1 : blockIdx.x, lane = threadIdx.x & 63;
+    const PickRange mine = INLINE ? picks_of_block(il, topk) : PickRange{(int)blockIdx.x, 0, topk, 0};
+    const int t = mine.token, lane = threadIdx.x & 63;
     const int nchunk = hidden / 8;
     const u32x4 *src = reinterpret_cast<const u32x4 *>(x + (int64_t)t * hidden);
     GivenPicks given = {-1, -1};
@@ -659,9 +674,9 @@ permute_copy_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
     LanePicks first;
     if constexpr (INLINE) {
         const int active = active_tokens(il.active_mask, il.tokens, s_tmp);
-        inline_counts(topk_idx, t, topk, experts, active, given.e, s_cnt);
+        inline_counts(topk_idx, mine, topk, experts, active, given.e, il, s_cnt);
         __syncthreads();
-        first = inline_rows(t, topk, experts, active, given.e, il, pr, s_cnt);
+        first = inline_rows(mine, topk, experts, active, given.e, il, pr, s_cnt);
     } else if constexpr (COUNTS) {
         counts_to_offsets(no, experts, topk, t == 0 && threadIdx.x < 64, cnt, s_off);
         first = resolve_counts(given, s_off, experts, pr);
@@ -676,8 +691,8 @@ permute_copy_kernel(const uint16_t *__restrict__ x, ExpertIds topk_idx,
                 picks = resolve_counts(request_given(topk_idx, rank_in_expert, t, topk, k0 + lane), s_off, experts, pr);
             else if (!INLINE && k0 > 0)
                 picks = resolve_given(request_given(topk_idx, rank_in_expert, t, topk, k0 + lane), base, base_inclusive, experts, pr);
-            const int n = topk - k0 < 64 ? topk - k0 : 64;
-            for (int k = 0; k < n; ++k) {
+            const int n = INLINE ? mine.end : (topk - k0 < 64 ? topk - k0 : 64);
+            for (int k = INLINE ? mine.begin : 0; k < n; ++k) {
                 const int32_t row = __builtin_amdgcn_readlane(picks.row, k);
                 if (row < 0) continue;
                 u32x4 *dest = reinterpret_cast<u32x4 *>(pr.dest[window_of(pr, __builtin_amdgcn_readlane(picks.e, k))] + (int64_t)row * hidden * 2);
@@ -702,6 +717,20 @@ struct PermuteExtras {
     const NotifyOut *notify = nullptr;     /* offsets from counts, and what a notify launch writes */
 };
 
+/*
+ * Fewer tokens than half of the CUs: up to eight workgroups, as many as make one per CU, share a token's picks. Each reads the row
+ * and its scale for itself, but counts for its own picks and stores their rows only, and that is what a lone workgroup spends its
+ * time on (one token of 8 picks, 7168 wide, int8: 1.5 us of 4.5 each, a CU storing 50 GB/s). The kernel alone: 1 token 5.31 -> 3.68 us,
+ * 7 tokens 5.53 -> 3.83 (rows as they are 5.05 -> 3.31), 32 of 4096, 128 experts 5.29 -> 3.75, 64 of 7168 5.94 -> 4.80, of 2048 4.64 -> 3.40,
+ * 128 6.58 -> 6.33; two per CU: 64 tokens 6.37, 128 6.96, 512 12.6 -> 15.5.
+ */
+inline int inline_part_shift(int64_t tokens)
+{
+    int shift = 0;
+    while (shift < 3 && tokens << (shift + 1) <= 256) ++shift;
+    return shift;
+}
+
 template <int XDT, int QM, bool SMOOTH>
 int32_t launch_quant(const void *x, const ExpertIds &topk_idx, const int32_t *rank_in_expert, const int32_t *base,
                      int base_inclusive, const float *smooth, int64_t tokens, int64_t hidden, int64_t topk,
@@ -714,7 +743,8 @@ int32_t launch_quant(const void *x, const ExpertIds &topk_idx, const int32_t *ra
     if (ex.inline_layout && tokens * topk > kCountByAll) threads = kThreads;
     const int slots = (nseg + threads - 1) / threads;
     InlineLayout il = ex.inline_layout ? *ex.inline_layout : InlineLayout{};
-    if (!ex.inline_layout) {
+    if (ex.inline_layout) il.part_shift = inline_part_shift(tokens);
+    else {
         il.active_mask = ex.active_mask;
         il.tokens = (int)tokens;
     }
@@ -722,7 +752,7 @@ int32_t launch_quant(const void *x, const ExpertIds &topk_idx, const int32_t *ra
     const NotifyOut no = ex.notify ? *ex.notify : NotifyOut{};
     constexpr bool NOTIFIES = !SMOOTH && QM != QM_INT8_NOEPS;      /* the quantisations of the normal-mode dispatch */
 #define ZB_LAUNCH_I(S, LMV)                                                                                       \
-    zb_launch(permute_quant_kernel<XDT, QM, S, SMOOTH, LMV>, (unsigned)(tokens + (LMV == LM_INLINE ? 1 : 0)), threads, 0, st,  \
+    zb_launch(permute_quant_kernel<XDT, QM, S, SMOOTH, LMV>, (unsigned)(LMV == LM_INLINE ? (tokens << il.part_shift) + 1 : tokens), threads, 0, st, \
         (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, smooth, (int)hidden, (int)topk,       \
         (int)experts, pr, il, rt, ex.shared, no, ex.clear_words, ex.clear_count)
 #define ZB_LAUNCH(S)                                                                                              \
@@ -762,10 +792,13 @@ static int32_t permute_launch(const void *x, int32_t x_dtype, const ExpertIds &t
         int threads = (nchunk + 63) / 64 * 64;
         if (threads > kThreads) threads = kThreads;
         if (ex.inline_layout && tokens * topk > kCountByAll) threads = kThreads;
-        if (ex.inline_layout)
-            zb_launch(permute_copy_kernel<LM_INLINE, 4>, (unsigned)tokens + 1, threads, 0, st,
+        if (ex.inline_layout) {
+            InlineLayout il = *ex.inline_layout;
+            il.part_shift = inline_part_shift(tokens);
+            zb_launch(permute_copy_kernel<LM_INLINE, 4>, (unsigned)(tokens << il.part_shift) + 1, threads, 0, st,
                 (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, (int)hidden, (int)topk, (int)experts, pr,
-                *ex.inline_layout, NotifyOut{});
+                il, NotifyOut{});
+        }
         else if (ex.notify)
             zb_launch(permute_copy_kernel<LM_COUNTS, 4>, (unsigned)tokens, threads, 0, st,
                 (const uint16_t *)x, topk_idx, rank_in_expert, base, base_inclusive, (int)hidden, (int)topk, (int)experts, pr,
