@@ -157,7 +157,8 @@ __global__ void __launch_bounds__(ZB_FUSED_THREADS)
 layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, int nbits,
                     const uint8_t *__restrict__ active_mask, LayoutOutputs o)
 {
-    __shared__ int32_t run[ZB_MAX_EXPERTS], copies[ZB_MAX_EXPERTS];
+    __shared__ int32_t run[ZB_MAX_EXPERTS];
+    __shared__ __align__(16) int32_t copies[ZB_MAX_EXPERTS];
     __shared__ int32_t wsum[ZB_FUSED_THREADS / 64];
     __shared__ int32_t s_active;
     __shared__ __align__(16) uint8_t cnt[ZB_FUSED_THREADS / 64 * ZB_MAX_EXPERTS];
@@ -231,12 +232,20 @@ layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, i
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += blockDim.x) {
         int32_t sum = 0;
-        for (int c = 0; c < 1 << log_copies; ++c) sum += copies[(e << log_copies) + c];
+        if (log_copies >= 2) {
+            i32x4 c[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                c[j] = j < 1 << (log_copies - 2) ? *reinterpret_cast<const i32x4 *>(copies + (e << log_copies) + 4 * j) : i32x4{0, 0, 0, 0};
+            c[0] += c[1] + c[2] + c[3];
+            sum = c[0][0] + c[0][1] + c[0][2] + c[0][3];
+        } else
+            for (int c = 0; c < 1 << log_copies; ++c) sum += copies[(e << log_copies) + c];
         run[e] = sum;
     }
     __syncthreads();
     if (!totals) {
-        rank_picks<false>(idx, p0, p1, own, experts, nbits, run, cnt, o.send_token_idx);
+        rank_picks<ZB_FUSED_THREADS / 64, false>(idx, p0, p1, own, experts, nbits, run, cnt, o.send_token_idx);
         return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -247,12 +256,13 @@ layout_fused_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, i
         int32_t s = zb_wave_scan_dpp(c);
         if (lane == 63) wsum[wave] = s;
         __syncthreads();
-        int32_t add = carry;
-        for (int w = 0; w < wave; ++w) add += wsum[w];
-        s += add;
-        int32_t chunk_total = 0;
-        for (int w = 0; w < ZB_FUSED_THREADS / 64; ++w) chunk_total += wsum[w];
-        carry += chunk_total;
+        s += carry;
+#pragma unroll
+        for (int w = 0; w < ZB_FUSED_THREADS / 64; ++w) {
+            const int32_t of_wave = wsum[w];
+            s += w < wave ? of_wave : 0;
+            carry += of_wave;
+        }
         __syncthreads();
         if (e < experts) {
             if (o.incl_i32) o.incl_i32[e] = s;
@@ -321,7 +331,7 @@ layout_ranges_kernel(ExpertIds idx, int tokens, int topk, int experts, int tpb, 
         __syncthreads();
     }
     const int64_t p0 = (int64_t)sl0 * topk, p1 = (int64_t)sl1 * topk;
-    rank_picks(idx, p0, p1, first_pick(idx, p0, p1), experts, nbits, run, cnt, send_token_idx);
+    rank_picks<ZB_FUSED_THREADS / 64>(idx, p0, p1, first_pick(idx, p0, p1), experts, nbits, run, cnt, send_token_idx);
     /* rank_picks ends on a barrier: run[] counts the range up to this slice's end; the last slice's block has it all */
     if (!SLICED || sub == subs - 1)
         for (int e = threadIdx.x; e < experts; e += blockDim.x) hist[(int64_t)range * experts + e] = run[e];
