@@ -378,7 +378,7 @@ ZBALHIP_API int32_t zbalhip_gmm1_swiglu_quant_shared(const void *a, const float 
                                   int32_t mode, void *q2, float *scale2, float *sgl_ws,
                                   const zbalhip_shared_expert_t *shared, void *stream);
 /*
- * The same with memory for tiles that several workgroups share along K (8-bit modes with few rows per expert): `parts_bytes`
+ * The same with memory for tiles that several workgroups share along K (W8A8 with few rows per expert): `parts_bytes`
  * at `parts`, 16-byte aligned, of which the first ZBALHIP_PART_WORDS 32-bit words are zero; null: no tile is shared. The more bytes,
  * the more rows a shared tile may have. shared may be null.
  */

@@ -817,13 +817,13 @@ public:
         /* int modes: the permute launch clears the row maxima the first GEMM accumulates into (no fill launch) */
         const int32_t clearedFlag = sgl ? ZBALHIP_ROWMAX_CLEARED : 0;
         /*
-         * What the second GEMM's y takes up beyond the row maxima is nobody's during the first: there its workgroups exchange the
+         * What the second GEMM's y takes up beyond the row maxima is nobody's during the first: there W8A8's workgroups exchange the
          * sums of tiles that they share, behind words that the permute launch clears along with the row maxima.
          */
-        uint32_t *clearFrom = sgl ? (uint32_t *)(sgl + allRows * I) : (uint32_t *)y;
+        uint32_t *clearFrom = sgl ? (uint32_t *)(sgl + allRows * I) : nullptr;
         uint32_t *parts = std::max((uint32_t *)y, (uint32_t *)(base + Align256(sgl ? ws.sgl + (uint64_t)allRows * (I + 1) * 4 : 0)));
         int64_t clearCount = sgl ? allRows : 0, partsBytes = (uint8_t *)y + rows * H * 2 - (uint8_t *)parts;
-        if (mode == 3 || partsBytes <= ZBALHIP_PART_WORDS * 4 || parts - clearFrom > clearCount + 1024) parts = nullptr;
+        if (mode != 1 || partsBytes <= ZBALHIP_PART_WORDS * 4 || parts - clearFrom > clearCount + 1024) parts = nullptr;
         else clearCount = parts + ZBALHIP_PART_WORDS - clearFrom;
         /* few rows: the second GEMM takes the first one's values, if y is not where they lie */
         const int32_t valuesFlag = sgl && (uint8_t *)y >= (uint8_t *)(sgl + allRows * (I + 1)) &&
@@ -861,15 +861,14 @@ public:
                                       SI, H, mode, x->dataType, shareOutput->data, stream);
             if (rc != 0) return Launched(op, rc);
         }
-        uint32_t *clearWords = clearCount ? clearFrom : nullptr;
         const int32_t *ids = (const int32_t *)expertIds->data;
         const int32_t permuteMode = qmode | IdsFlag(expertIds);
         int64_t *counts = (int64_t *)expertTokenNums->data;
         rc = ride ? zbalhip_fused_permute_quant_shared(x->data, x->dataType, ids, smooth, activeMask, T, H, K, E, permuteMode, q1, xs,
-                                                       expandIdx, counts, rowOff, clearWords, clearCount, layoutScratch,
+                                                       expandIdx, counts, rowOff, clearFrom, clearCount, layoutScratch,
                                                        ZBALHIP_LAYOUT_MAX_BLOCKS, shareSmooth, stream)
                   : zbalhip_fused_permute_quant(x->data, x->dataType, ids, smooth, activeMask, T, H, K, E, permuteMode, q1, xs,
-                                                expandIdx, counts, rowOff, clearWords, clearCount, layoutScratch,
+                                                expandIdx, counts, rowOff, clearFrom, clearCount, layoutScratch,
                                                 ZBALHIP_LAYOUT_MAX_BLOCKS, stream);
         if (rc != 0) return Launched(op, rc);
         rc = zbalhip_gmm1_swiglu_quant_parts(q1, xs, gmm1Weight->data, gmm1Scale->data, rowOff, E, rows, H, N1,

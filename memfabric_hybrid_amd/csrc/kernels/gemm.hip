@@ -1178,7 +1178,7 @@ static void with_shared(GemmParams &p, const zbalhip_shared_expert_t *shared, in
 }
 
 /*
- * Memory for tiles shared along K (null: none). A shorter K has less to share than the exchange of its sums takes: 64 experts of
+ * Memory for tiles shared along K (W8A8; null: none). A shorter K has less to share than the exchange of its sums takes: 64 experts of
  * 2048 x 2048, 100 tokens Zipf(1.2), layer 79 -> 81 us, 128 of 4096 x 3072, 64 tokens 314 -> 317.
  */
 static void with_parts(GemmParams &p, void *parts, int64_t bytes)
@@ -1222,7 +1222,7 @@ extern "C" int32_t zbalhip_gmm1_swiglu_quant_parts(const void *a, const float *a
     p.out = q2; p.out_scale = scale2; p.sgl_ws = sgl_ws; p.w_is_list = w_is_list;
     with_shared(p, shared, 0);
     if (misaligned16(parts) || (parts && parts_bytes < 0)) return ZBALHIP_INVALID;
-    with_parts(p, parts, parts_bytes);
+    if (mode == MODE_W8A8) with_parts(p, parts, parts_bytes);
     const int n_tiles = (int)(n1 / 2 / 128);
     if (mode == MODE_FP8) return launch_dma<MODE_FP8, true, ZDT_BF16>(p, n_tiles, st);
     if (!sgl_ws) return ZBALHIP_INVALID;

@@ -92,7 +92,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     using S = StreamShape<MODE, TM, SPLIT, VALUES>;
     constexpr int PF = S::PF, NT = S::NT, MTM = S::MTM, LOADS = S::LOADS, NW = S::NW, WRB = S::WRB;
     constexpr int MAX_PARTS = 4;
-    constexpr bool SHARES_K = GMM1 && MODE != MODE_W4A8 && SPLIT == 1;
+    constexpr bool SHARES_K = GMM1 && MODE == MODE_W8A8 && SPLIT == 1;
     constexpr int W_BLOCK_BYTES = 128 * WRB;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     float *lds_sa = reinterpret_cast<float *>(smem + S::A_ALL);
@@ -138,11 +138,12 @@ grouped_gemm_stream_kernel(GemmParams p)
     };
     /*
      * The memory gives every CU the same, so what is over when all CUs have the same number of tiles (`rest`, at the end) runs on
-     * a few CUs, long after the others: fp8, 528 tiles of 7168 x 4096 on 256 CUs, 16 tiles alone for the last 30 of 168 us. Such
-     * tiles are shared along K by up to four workgroups each, which leave their sums in memory; the last of them to get there
-     * adds the parts up, in their order, whichever it is, and has the epilogue. Nobody waits for anybody. Layers with a shared
-     * expert, 32 experts of 7168 x 4096 / 2048 x 7168: fp8, 37 tokens 270 -> 254 us, 12 tokens 245 -> 239, W8A8, 20 tokens 274 -> 257,
-     * 60 tokens 287 -> 273 (up to eight: 254, 238, 261, 275). The words and sums go past the L2s, which are the XCDs' own.
+     * a few CUs, long after the others: 528 tiles of 7168 x 4096 on 256 CUs, 16 tiles alone for the last 30 of 168 us. W8A8: such
+     * tiles are shared along K by up to four workgroups each, which leave their int32 sums in memory; the last of them to get there
+     * adds the parts up and has the epilogue. Nobody waits for anybody. Layers with a shared expert, 32 experts of 7168 x 4096 / 2048 x
+     * 7168: 20 tokens 274 -> 257 us, 60 tokens 287 -> 273 (up to eight: 261, 275). The words and sums go past the L2s, which are the
+     * XCDs' own. Integers add up to the same bits in any parts. fp8's scaled sums do not, and which tiles are over depends on the
+     * whole batch's routing: there a token's bits would depend on the tokens beside it (37 tokens 264 -> 247 us, taken back).
      */
     int part_k = 0, parts = 1, piece = 0;
     int64_t part_rows = 0;
@@ -601,7 +602,7 @@ grouped_gemm_stream_kernel(GemmParams p)
                     }
             };
             each([&](int mt, int nt) __attribute__((always_inline)) {
-                const u32x4 v = MODE == MODE_FP8 ? __builtin_bit_cast(u32x4, accf[mt][nt]) : __builtin_bit_cast(u32x4, acci[mt][nt]);
+                const u32x4 v = __builtin_bit_cast(u32x4, acci[mt][nt]);
                 uint64_t *at = sums_at(part_k, mt, nt);
                 __hip_atomic_store(at, (uint64_t)v[1] << 32 | v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(at + 1, (uint64_t)v[3] << 32 | v[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -612,18 +613,14 @@ grouped_gemm_stream_kernel(GemmParams p)
                 *reinterpret_cast<uint32_t *>(lds_rowmax) = __hip_atomic_fetch_add(p.part_done + xcd * p.part_cus + piece, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __syncthreads();
             if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<uint32_t *>(lds_rowmax)) != (uint32_t)parts - 1) return;
-            each([&](int mt, int nt) __attribute__((always_inline)) {
-                accf[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                acci[mt][nt] = i32x4{0, 0, 0, 0};
-            });
+            each([&](int mt, int nt) __attribute__((always_inline)) { acci[mt][nt] = i32x4{0, 0, 0, 0}; });
             for (int part = 0; part < parts; ++part) {
                 each([&](int mt, int nt) __attribute__((always_inline)) {
                     uint64_t *at = sums_at(part, mt, nt);
                     const uint64_t v0 = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     const uint64_t v1 = __hip_atomic_load(at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     const u32x4 v = {(uint32_t)v0, (uint32_t)(v0 >> 32), (uint32_t)v1, (uint32_t)(v1 >> 32)};
-                    if (MODE == MODE_FP8) accf[mt][nt] += __builtin_bit_cast(f32x4, v);
-                    else acci[mt][nt] += __builtin_bit_cast(i32x4, v);
+                    acci[mt][nt] += __builtin_bit_cast(i32x4, v);
                 });
             }
             __syncthreads();               /* lds_rowmax goes to the epilogue */

@@ -41,7 +41,7 @@ struct GemmParams {
     const void *shared_wscale;
     void *shared_out;        /* GMM2: where row 0 would be if row shared_row is the first */
     /*
-     * For the streaming kernel's tiles that several workgroups share along K (8-bit modes' first GEMM; null: none do): 8 * part_cus
+     * For the streaming kernel's tiles that several workgroups share along K (W8A8's first GEMM; null: none do): 8 * part_cus
      * words that are zero when the launch starts, and room for part_floats sums of every XCD's tiles.
      */
     uint32_t *part_done;

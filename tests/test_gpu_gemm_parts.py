@@ -1,16 +1,13 @@
 """Tiles of the first GEMM that several workgroups share along K: one or two tiles more per XCD than a whole number per CU, with
-room for their sums, with exactly enough and with a row too little, against the launch that shares none. W8A8: the same
-bits. fp8: the sums of up to four parts instead of one chain, so a value next to a rounding boundary of e4m3 may land on the
-neighbouring code, and nothing else."""
-import numpy as np
+room for their sums, with exactly enough and with a row too little. The bits are those of the launch that shares none. fp8
+shares none whatever memory it is given: its sums depend on their order."""
 import pytest
 import torch
 
 from memfabric_hybrid_amd import capi
 from memfabric_hybrid_amd.operators import OperatorBuffer
-from oracle import oracle as zo
-from test_gpu_gemm import assert_requant_close, row_off_dev
-from zbal_testlib import host, rng
+from test_gpu_gemm import row_off_dev
+from zbal_testlib import rng
 
 pytestmark = pytest.mark.gpu
 
@@ -61,15 +58,5 @@ def test_tiles_shared_along_k(buf, mode, K, rest, rows, room):
     want_q2, want_s2, _ = run(False)
     for _ in range(2):
         got_q2, got_s2, shared = run(True)
-        assert shared == (8 * rest if rows <= room else 0)
-        if mode == 1 or not shared:
-            assert torch.equal(got_q2, want_q2) and torch.equal(got_s2, want_s2)
-            continue
-        # the tiles that are not shared have the bits that they had
-        first = int(counts[:cus].sum())
-        assert torch.equal(got_q2[:first], want_q2[:first]) and torch.equal(got_s2[:first], want_s2[:first])
-        blocks = (R, N // 256, 128)
-        q2s, s2s = [host(q) for q in (want_q2, got_q2)], [host(s) for s in (want_s2, got_s2)]
-        assert np.allclose(s2s[1], s2s[0], rtol=1e-4)
-        value = [zo.e4m3_to_f32(q).reshape(blocks) * s[:, :, None] for q, s in zip(q2s, s2s)]
-        assert_requant_close(value[1], value[0], q2s[1], q2s[0])
+        assert shared == (8 * rest if mode == 1 and rows <= room else 0)
+        assert torch.equal(got_q2, want_q2) and torch.equal(got_s2, want_s2)
