@@ -890,7 +890,6 @@ int32_t launch_dma_shape(const GemmParams &p, int n_tiles, hipStream_t st)
     return zbalhip_check_launch();
 }
 
-/* the streaming kernel: every XCD gets a workgroup for each tile it can have (a partial row tile per expert with rows at most) */
 template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1, bool VALUES = false>
 int32_t launch_stream(const GemmParams &p, int n_tiles, hipStream_t st)
 {
@@ -898,9 +897,8 @@ int32_t launch_stream(const GemmParams &p, int n_tiles, hipStream_t st)
     int n_cus = 0;
     const int32_t rc = prepare_stream<MODE, GMM1, OUT_DT, TM, SPLIT, VALUES>(st, &n_cus);
     if (rc != ZBALHIP_OK) return rc;
-    const int64_t partial = p.max_rows < p.experts ? p.max_rows : p.experts;
-    const int64_t per_xcd = (p.max_rows / TM + partial) * ((n_tiles * SPLIT + 7) / 8) + (p.part_sums ? p.part_cus : 0);
-    grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT, VALUES><<<(unsigned)(8 * per_xcd), S::THREADS, S::LDS_BYTES, st>>>(p);
+    const unsigned blocks = (unsigned)stream_workgroups<MODE, GMM1, TM, SPLIT>(p, n_tiles);
+    grouped_gemm_stream_kernel<MODE, GMM1, OUT_DT, TM, SPLIT, VALUES><<<blocks, S::THREADS, S::LDS_BYTES, st>>>(p);
     return zbalhip_check_launch();
 }
 

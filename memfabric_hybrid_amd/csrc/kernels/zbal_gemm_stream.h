@@ -83,6 +83,21 @@ template <int N> __device__ __forceinline__ void wait_w(u32x4 (&w)[2][2])
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]) : "n"(N));
 }
 
+/* which of them share left-over tiles along K, see the kernel */
+template <int MODE, bool GMM1, int SPLIT> constexpr bool stream_shares_k() { return GMM1 && MODE == MODE_W8A8 && SPLIT == 1; }
+
+/*
+ * Workgroups of a launch: every XCD gets one for each tile that it can have (a partial row tile per expert with rows at most),
+ * and where tiles are shared one per CU for the parts. (Given to every launch, those for the parts doubled the grid of one token's first
+ * GEMM: 256 workgroups more that look their tile up and leave, though no time could be measured for them, 70.0 us a layer.)
+ */
+template <int MODE, bool GMM1, int TM, int SPLIT>
+inline int64_t stream_workgroups(const GemmParams &p, int n_tiles)
+{
+    const int64_t partial = p.max_rows < p.experts ? p.max_rows : p.experts;
+    return 8 * ((p.max_rows / TM + partial) * ((n_tiles * SPLIT + 7) / 8) + (stream_shares_k<MODE, GMM1, SPLIT>() && p.part_sums ? p.part_cus : 0));
+}
+
 template <int MODE, bool GMM1, int OUT_DT, int TM, int SPLIT = 1, bool VALUES = false>
 __global__ void __launch_bounds__(512 / SPLIT, 4)
 grouped_gemm_stream_kernel(GemmParams p)
@@ -92,7 +107,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     using S = StreamShape<MODE, TM, SPLIT, VALUES>;
     constexpr int PF = S::PF, NT = S::NT, MTM = S::MTM, LOADS = S::LOADS, NW = S::NW, WRB = S::WRB;
     constexpr int MAX_PARTS = 4;
-    constexpr bool SHARES_K = GMM1 && MODE == MODE_W8A8 && SPLIT == 1;
+    constexpr bool SHARES_K = stream_shares_k<MODE, GMM1, SPLIT>();
     constexpr int W_BLOCK_BYTES = 128 * WRB;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     float *lds_sa = reinterpret_cast<float *>(smem + S::A_ALL);

@@ -16,10 +16,43 @@ PROGRAM = r"""
 #include "zbal_gemm_stream.h"
 #include "zbal_gemm_tall.h"
 
+template <int MODE, bool GMM1, int SPLIT> long workgroups(GemmParams p, int n_tiles, bool parts)
+{
+    static float sums;
+    p.part_sums = parts ? &sums : nullptr;
+    p.part_cus = 32;
+    return stream_workgroups<MODE, GMM1, SPLIT == 2 ? 16 : 64, SPLIT>(p, n_tiles);
+}
+template <int MODE, bool GMM1, int SPLIT> long beyond(const GemmParams &p, int n_tiles)
+{
+    return workgroups<MODE, GMM1, SPLIT>(p, n_tiles, true) - workgroups<MODE, GMM1, SPLIT>(p, n_tiles, false);
+}
+template <int MODE> long beyond(int gmm1, int split, const GemmParams &p, int n_tiles)
+{
+    if (gmm1) return split == 1 ? beyond<MODE, true, 1>(p, n_tiles) : beyond<MODE, true, 2>(p, n_tiles);
+    return split == 1 ? beyond<MODE, false, 1>(p, n_tiles) : beyond<MODE, false, 2>(p, n_tiles);
+}
+long beyond(int mode, int gmm1, int split, int experts, int rows, int n_tiles)
+{
+    GemmParams p = {};
+    p.experts = experts;
+    p.max_rows = rows;
+    const long n = mode == MODE_W8A8 ? beyond<MODE_W8A8>(gmm1, split, p, n_tiles)
+                 : mode == MODE_FP8 ? beyond<MODE_FP8>(gmm1, split, p, n_tiles) : beyond<MODE_W4A8>(gmm1, split, p, n_tiles);
+    if (n != 0 && n != 256) exit(1);
+    return n;
+}
+
 int main()
 {
     int mode, slabs, experts, rows;
     while (scanf("%d %d %d %d", &mode, &slabs, &experts, &rows) == 4) {
+        if (mode >= 10) {                      /* mode - 10: whether memory for shared tiles adds workgroups to a launch of the weight stream */
+            int gmm1, split, n_tiles;
+            if (scanf("%d %d %d", &gmm1, &split, &n_tiles) != 3) return 1;
+            printf("%d\n", beyond(mode - 10, gmm1, split, experts, rows, n_tiles) == 256);
+            continue;
+        }
         if (mode == MODE_W4A8) {
             int n_tiles, cus;
             if (scanf("%d %d", &n_tiles, &cus) != 2) return 1;
@@ -79,3 +112,14 @@ def test_the_taller_w4a8_tile_wants_a_full_chip(accepts, cus):
     assert accepts(low + tall) == [False] * len(low) + [True] * len(tall)
     if cus == 256:
         assert accepts([c[:5] + (0,) for c in low + tall]) == [False] * len(low) + [True] * len(tall)
+
+
+@pytest.mark.parametrize("mode", [1, 2, 3])
+def test_workgroups_for_shared_tiles_only_where_tiles_are_shared(accepts, mode):
+    """Memory for shared tiles adds a workgroup per CU to W8A8's first GEMM with whole tiles, and none to any other launch: a token or two's
+    (two workgroups per tile), the second GEMM's, the other modes'."""
+    shapes = [(33, 8), (33, 264), (1, 1), (300, 5000)]
+    for gmm1 in (1, 0):
+        for split in (1, 2):
+            got = accepts([(10 + mode, 56, e, r, gmm1, split, n) for e, r in shapes for n in (1, 8, 16)])
+            assert got == [mode == 1 and gmm1 == 1 and split == 1] * len(got), (gmm1, split)
