@@ -540,7 +540,7 @@ topk_route_small_kernel(const float *__restrict__ logits, int tokens, int expert
         for (int k = 0; k < topk; ++k) {
             const float best = zb_wave_reduce_dpp<true>(left);
             const uint64_t owners = __ballot(v == best) & avail;
-            if (owners == 0) break;              /* NaN only */
+            if (owners == 0) break;              /* only NaNs are left */
             const int owner = __ffsll((long long)owners) - 1;
             avail &= ~(1ull << owner);
             if (lane == owner) { rank = k; left = -__builtin_inff(); }
@@ -551,14 +551,18 @@ topk_route_small_kernel(const float *__restrict__ logits, int tokens, int expert
             rank += (s > v || (s == v && m < lane)) ? 1 : 0;
         }
     }
-    const bool picked = mine && rank < topk;
+    /* a NaN is no pick; slots for which there is no logit get what the general kernel leaves there, an id that no expert has */
+    const bool number = mine && v == v, picked = number && rank < topk;
+    const int numbers = __popcll(__ballot(number));
     const float p = ex / sum;
     const float wsum = zb_wave_reduce_dpp<false>(picked ? p : 0.0f);
-    if (picked) {
-        if (idx_is_i64) static_cast<int64_t *>(topk_idx)[(int64_t)t * topk + rank] = lane;
-        else static_cast<int32_t *>(topk_idx)[(int64_t)t * topk + rank] = lane;
-        topk_w[(int64_t)t * topk + rank] = p / wsum;
-    }
+    auto put = [&](int slot, int expert, float w) __attribute__((always_inline)) {
+        if (idx_is_i64) static_cast<int64_t *>(topk_idx)[(int64_t)t * topk + slot] = expert;
+        else static_cast<int32_t *>(topk_idx)[(int64_t)t * topk + slot] = expert;
+        topk_w[(int64_t)t * topk + slot] = w;
+    };
+    if (picked) put(rank, lane, p / wsum);
+    if (numbers < topk && lane >= numbers && lane < topk) put(lane, 0x7fffffff, __builtin_nanf(""));
 }
 
 template <int PER_LANE>

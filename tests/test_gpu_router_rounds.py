@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from memfabric_hybrid_amd import capi
 from memfabric_hybrid_amd.operators import OperatorBuffer
 from oracle import oracle as zo
 from zbal_testlib import dev, host, rng
@@ -34,3 +35,28 @@ def test_picks_and_weights(buf, E, K, style):
     ridx, rw = zo.topk_route(logits, K)
     assert np.array_equal(host(idx), ridx)
     assert np.allclose(host(w), rw, rtol=1e-6, atol=0)       # the router's bound: weights within 1e-6 relative
+
+
+# ranks, rounds of one logit per lane, and rounds of two and of sixteen
+@pytest.mark.parametrize("E,K", [(8, 8), (32, 8), (33, 8), (64, 8), (65, 8), (128, 8), (1000, 16)])
+@pytest.mark.parametrize("dt", [torch.int64, torch.int32])
+def test_nan_logits_are_no_picks(buf, E, K, dt):
+    """A NaN is never picked: a row's picks are its other logits in their order, and where there are fewer of them than picks the rest of
+    the row is an id that no expert has. No slot keeps what the memory held. One NaN makes the row's softmax, and so every weight, NaN."""
+    g = rng(E + K)
+    T = 4 * K + 6
+    logits = g.standard_normal((T, E)).astype(np.float32)
+    left = [min(E, max(0, n)) for n in range(-1, K + 3)] + [E - 1, E - 2]
+    for t in range(T):
+        if t % 4:                                # every fourth row as it is
+            logits[t, g.permutation(E)[left[t % len(left)]:]] = np.nan
+    lg = dev(logits)
+    idx, w = torch.full((T, K), 5, dtype=dt, device="cuda"), torch.full((T, K), 0.25, device="cuda")
+    capi.check("route", buf.lib.zbalhip_topk_route(lg.data_ptr(), T, E, K, idx.data_ptr(), int(dt == torch.int64), w.data_ptr(), capi.stream_ptr()))
+    idx, w = host(idx), host(w)
+    for t in range(T):
+        numbers = np.flatnonzero(~np.isnan(logits[t]))
+        want = numbers[np.argsort(-logits[t, numbers], kind="stable")][:K]
+        assert np.array_equal(idx[t, :len(want)], want), (t, idx[t])
+        assert ((idx[t, len(want):] < 0) | (idx[t, len(want):] >= E)).all(), (t, idx[t])
+        assert np.isnan(w[t]).all() if len(numbers) < E else abs(w[t].sum() - 1) < 1e-5, (t, w[t])
