@@ -6,6 +6,7 @@ import torch
 
 from memfabric_hybrid_amd import capi
 from memfabric_hybrid_amd.operators import OperatorBuffer
+from oracle import oracle as zo
 from zbal_testlib import dev, distinct_topk, host
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +76,56 @@ def test_fp8_row_depends_on_its_token_alone(buf):
     for size in (whole, turns):
         out, out_shared, _ = run(T, workspace=torch.empty((size,), dtype=torch.uint8, device="cuda"), **share)
         assert torch.equal(out, alone) and torch.equal(out_shared, shared), size
+
+
+def regions(T, n_experts):
+    """W8A8 workspace in which a shared expert rides along: where the fp32 values and y (apart) begin, y's bytes and those of the values."""
+    rows, all_rows = T * K, T * K + T
+    align = lambda n: (n + 255) // 256 * 256
+    values = sum(align(n) for n in (rows * 4, n_experts * 8, (n_experts + 2) * 4, 50 * n_experts * 4, all_rows * I, all_rows * 4, all_rows * H,
+                                    all_rows * 4))
+    return values, values + align(all_rows * (I + 1) * 4), align(rows * H * 2), align(all_rows * (I + 1) * 4)
+
+
+@pytest.mark.parametrize("together", [False, True])
+def test_w8a8_layer_with_a_tile_shared_along_k(buf, together):
+    """A routed expert's tile on every XCD is left over behind the shared expert's and is shared along K, in the part of y that the second GEMM
+    does not write for the tokens that the mask leaves out: the sums are still there afterwards. Every call on a workspace that the call
+    before has left as it is, and replays of a graph with new inputs, against the oracle; y beside the fp32 values and in their place."""
+    E, T, n = experts(), 96, 56
+    routed, share = weights(1, E, 5), weights(1, 1, 6)
+    args, share_kw = packed(buf, routed), share_args(buf, share)
+    mask = torch.arange(T, device="cuda") < n
+    values, apart, y_bytes, value_bytes = regions(T, E)
+    size, y = (values + max(y_bytes, value_bytes), values) if together else (apart + y_bytes, apart)
+    unwritten = slice(max(y + n * K * H * 2, values + value_bytes if together else 0), y + y_bytes)      # of y, behind the values and the routed rows
+
+    def layer(x, ids, es, out, share_out, ws):
+        return buf.fused_deep_moe(x, ids, *args, es, E, quant_mode=1, x_active_mask=mask, out=out, share_out=share_out, workspace=ws, **share_kw)
+
+    seven = lambda: torch.full((T, H), 7.0, dtype=torch.bfloat16, device="cuda")
+    ws, g_ws = (torch.full((size,), 0x5a, dtype=torch.uint8, device="cuda") for _ in range(2))
+    x, ids, es = inputs(T, E, 30)
+    s_out, s_share = seven(), seven()
+    layer(x, ids, es, s_out, s_share, g_ws)              # first call outside the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layer(x, ids, es, s_out, s_share, g_ws)
+    hosted = [host(t) for t in routed], [host(t) for t in share]
+    for seed in (31, 32, 33):
+        nx, nids, nes = inputs(T, E, seed)
+        assert len(np.unique(host(nids)[:n])) == E
+        ws[unwritten].fill_(0x5a)
+        out, shared, nums = layer(nx, nids, nes, seven(), seven(), ws)
+        assert bool((ws[unwritten] != 0x5a).any()), "no tile was shared"
+        xh, idh, esh = host(nx)[:n], host(nids)[:n].astype(np.int64), host(nes)[:n]
+        want, counts = zo.fused_moe(xh, zo.DT_BF16, idh, esh, *hosted[0], E, 1)
+        want_share, _ = zo.fused_moe(xh, zo.DT_BF16, np.zeros((n, 1), np.int64), np.ones((n, 1), np.float32), *hosted[1], 1, 1)
+        assert np.array_equal(host(nums), counts)
+        assert np.array_equal(host(out)[:n], want) and np.array_equal(host(shared)[:n], want_share)
+        x.copy_(nx), ids.copy_(nids), es.copy_(nes)
+        s_out.fill_(7.0), s_share.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(s_out, out) and torch.equal(s_share, shared), seed

@@ -1,12 +1,15 @@
 """Tiles of the first GEMM that several workgroups share along K: one or two tiles more per XCD than a whole number per CU, with
 room for their sums, with exactly enough and with a row too little. The bits are those of the launch that shares none. fp8
 shares none whatever memory it is given: its sums depend on their order."""
+import ctypes
+
 import pytest
 import torch
 
 from memfabric_hybrid_amd import capi
 from memfabric_hybrid_amd.operators import OperatorBuffer
 from test_gpu_gemm import row_off_dev
+from test_gpu_shared_expert import SharedExpert
 from zbal_testlib import rng
 
 pytestmark = pytest.mark.gpu
@@ -59,4 +62,58 @@ def test_tiles_shared_along_k(buf, mode, K, rest, rows, room):
     for _ in range(2):
         got_q2, got_s2, shared = run(True)
         assert shared == (8 * rest if mode == 1 and rows <= room else 0)
+        assert torch.equal(got_q2, want_q2) and torch.equal(got_s2, want_s2)
+
+
+def tiles_of(rows, tall):
+    """Heights of an expert's row tiles, as the kernel cuts them."""
+    tm = 96 if tall else 64
+    n = -(-rows // tm)
+    height = (-(-rows // n) + 15) & ~15
+    return [min(height, rows - i * height) for i in range(n)]
+
+
+# W8A8, the last experts' rows and the room for a shared tile's. Workgroups per tile: four up to 8 tiles over, three of 9 and 10, two of
+# 11 to 16, one beyond (nothing is shared). Heights on either side of the room in one launch; an expert of two row tiles; a shared expert
+# (the first tile of all); `tall`: 48 rows per expert and more on average, the tile of 96 rows and two slabs in flight.
+@pytest.mark.parametrize("K,last,parts,room,tall,shared", [
+    (4608, [3] * 8, 4, 64, False, 0), (4608, [17] * 9, 3, 64, False, 0), (5120, list(range(8, 18)), 3, 13, False, 20),
+    (4608, [5, 64] * 5 + [16], 2, 40, False, 0), (5120, list(range(9, 25)), 2, 16, False, 64), (4608, [9] * 17, 1, 64, False, 0),
+    (4608, [100], 4, 40, False, 0), (4608, [1, 33], 4, 33, False, 64),
+    (4608, [96], 4, 96, True, 0), (5120, [81, 80, 96, 1], 4, 80, True, 70), (4608, [48, 96] * 5, 3, 90, True, 0),
+    (7168, [95, 64, 17] * 4, 2, 64, True, 96), (4608, [130, 20], 4, 70, True, 0)])
+def test_numbers_of_parts_and_heights_of_tiles(buf, K, last, parts, room, tall, shared):
+    heights = [h for rows in last for h in tiles_of(rows, tall)]
+    rest, N = len(heights), 2048
+    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8
+    first = cus - (1 if shared else 0)
+    counts = rng(K + rest).integers(60, 97, first) if tall else rng(K + rest).integers(1, 20, first)
+    counts = [int(c) for c in counts] + last
+    E, R, I = len(counts), sum(counts), N // 2
+    assert parts == max(1, min(4, cus // rest)) and (R + shared > 48 * (E + bool(shared))) == tall and R + shared <= 87 * E
+    g = torch.Generator(device="cuda").manual_seed(rest)
+    w = torch.randint(-128, 128, (E + 1, N, K), dtype=torch.int8, device="cuda", generator=g)
+    a = torch.randint(-127, 128, (R + shared, K), dtype=torch.int8, device="cuda", generator=g)
+    xs = torch.rand((R + shared,), device="cuda", generator=g) * 0.05 + 0.005
+    ws = torch.rand((E + 1, N), device="cuda", generator=g) * 0.003 + 0.0015
+    off = row_off_dev(counts + [shared])
+    along = SharedExpert(w[E].data_ptr(), ws[E].data_ptr(), shared, None)
+    scratch = torch.full((WORDS + 8 * rest * parts * room * 256,), float("nan"), device="cuda")
+
+    def run(share):
+        q2, s2 = torch.zeros((R + shared, I), dtype=torch.int8, device="cuda"), torch.zeros((R + shared,), device="cuda")
+        sgl = torch.empty(((R + shared) * (I + 1),), device="cuda")
+        scratch[:WORDS].view(torch.int32).zero_()
+        capi.check("gmm1", buf.lib.zbalhip_gmm1_swiglu_quant_parts(
+            a.data_ptr(), xs.data_ptr(), w.data_ptr(), ws.data_ptr(), off.data_ptr(), E, R, K, N, 1, q2.data_ptr(), s2.data_ptr(), sgl.data_ptr(),
+            ctypes.byref(along) if shared else None, scratch.data_ptr() if share else None, scratch.numel() * 4 if share else 0,
+            capi.stream_ptr()))
+        return q2, s2, scratch[:WORDS].view(torch.int32).clone()
+
+    want_q2, want_s2, _ = run(False)
+    assert int((want_q2 != 0).any(dim=1).sum()) == R + shared
+    for _ in range(2):
+        got_q2, got_s2, arrived = run(True)
+        of_xcd = [parts if parts > 1 and h <= room else 0 for h in heights] + [0] * (cus - rest)
+        assert arrived.tolist() == of_xcd * 8 + [0] * (WORDS - 8 * cus)
         assert torch.equal(got_q2, want_q2) and torch.equal(got_s2, want_s2)
