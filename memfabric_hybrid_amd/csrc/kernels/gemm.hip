@@ -1176,8 +1176,9 @@ static void with_shared(GemmParams &p, const zbalhip_shared_expert_t *shared, in
 }
 
 /*
- * Memory for tiles shared along K (W8A8; null: none). A shorter K has less to share than the exchange of its sums takes: 64 experts of
- * 2048 x 2048, 100 tokens Zipf(1.2), layer 79 -> 81 us, 128 of 4096 x 3072, 64 tokens 314 -> 317.
+ * Memory for tiles shared along K (W8A8; null: none). Which of them are is the kernel's business (shared_rows), but not with a K up to
+ * 4096: there the exchange took more than it saved where tiles of any height were shared (64 experts of 2048 x 2048, 100 tokens
+ * Zipf(1.2), layer 79 -> 81 us, 128 of 4096 x 3072, 64 tokens 314 -> 317), and what lower ones would give has not been measured.
  */
 static void with_parts(GemmParams &p, void *parts, int64_t bytes)
 {

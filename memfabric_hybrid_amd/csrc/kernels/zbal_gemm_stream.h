@@ -87,6 +87,19 @@ template <int N> __device__ __forceinline__ void wait_w(u32x4 (&w)[2][2])
 template <int MODE, bool GMM1, int SPLIT> constexpr bool stream_shares_k() { return GMM1 && MODE == MODE_W8A8 && SPLIT == 1; }
 
 /*
+ * Rows up to which an XCD's tiles that are over, `rest` of them, are shared, all of them or none: the longer the K loop, the more a part
+ * saves, and the exchange costs by rows and parts. First W8A8 GEMM, N 2048, an expert per CU and XCD times 1 to 4 and `rest` more, all
+ * with the same rows, per cent of the unshared launch, at 2 / 16 / 32 / 64 / 84 rows:
+ *   - K 4608: rest 1 -13 ... -4 / -10 ... -3 / -6 ... -2 / +1 ... +2 / +3 ... +5; 4 -13 ... -3 / -9 ... -2 / -4 ... 0 / +2 ... +5 / +4 ... +9; 8 -7 ... -1 /
+ *     -3 ... +1 / +2 / +5 ... +11 / +8 ... +16; 10 -7 ... -1 / -4 ... 0 / 0 ... +1 / +4 ... +9 / +6 ... +15;
+ *   - K 7168: rest 1 -18 ... -5 / -15 ... -4 / -11 ... -3 / -6 ... -2 / -2 ... +1; 4 -16 ... -4 / -13 ... -3 / -10 ... -2 / -4 ... -1 / 0 ... +1; 8 -12 ... -3 /
+ *     -9 ... -2 / -5 ... 0 / +1 ... +3 / +3 ... +7; 10 -9 ... -2 / -7 ... -1 / -4 ... 0 / +1 ... +2 / +2 ... +6;
+ *   - K 14336: rest 1 -20 ... -6 / ... / -12 ... -4; 10 -10 ... -2 / ... / -4 ... -1.
+ * Beyond ten tiles (two parts each) 0 ... +10. Where only some of the tiles were shared the others were still the last to end: +2 ... +8.
+ */
+__host__ __device__ inline int shared_rows(int slabs, int rest) { return rest > 10 ? 0 : (slabs - 24) * (11 - rest) / 4; }
+
+/*
  * Workgroups of a launch: every XCD gets one for each tile that it can have (a partial row tile per expert with rows at most),
  * and where tiles are shared one per CU for the parts. (Given to every launch, those for the parts doubled the grid of one token's first
  * GEMM: 256 workgroups more that look their tile up and leave, though no time could be measured for them, 70.0 us a layer.)
@@ -136,7 +149,7 @@ grouped_gemm_stream_kernel(GemmParams p)
     rows_of(0, lo[0], hi[0]);
     rows_of(64, lo[1], hi[1]);
     const int xcd = blockIdx.x & 7;
-    int slot = blockIdx.x >> 3;
+    const int slot = blockIdx.x >> 3;
     auto columns_before = [&](int y) { return (y - xcd + 7) >> 3; };      /* of this XCD, among columns 0 .. y - 1 */
     /* f for 64 experts at a time, one per lane: first of them, and the lane's first row, end row, row tiles, first column and tiles on this XCD; until it is true */
     auto walk = [&](auto f) __attribute__((always_inline)) {
@@ -151,54 +164,67 @@ grouped_gemm_stream_kernel(GemmParams p)
             used += __popcll(busy);
         }
     };
+    int expert = -1, n_tile = 0, m_tile = 0, mt_e = 1, first_row = 0, end_row = 0, tiles = 0;
+    auto find_tile = [&](int wanted, bool count_all) __attribute__((always_inline)) {
+        expert = -1;
+        tiles = 0;
+        walk([&](int base, int l, int h, int m, int c0, int mine) {
+            const int incl = zb_wave_scan_dpp(mine);
+            const uint64_t past = __ballot(tiles + incl > wanted);
+            if (past && expert < 0) {
+                const int src = __ffsll((long long)past) - 1;
+                expert = nth_expert(base + src);
+                mt_e = __builtin_amdgcn_readlane(m, src);
+                first_row = __builtin_amdgcn_readlane(l, src);
+                end_row = __builtin_amdgcn_readlane(h, src);
+                const int at = wanted - tiles - __builtin_amdgcn_readlane(incl - mine, src), col = at / mt_e;
+                m_tile = at - col * mt_e;
+                const int first_col = __builtin_amdgcn_readlane(c0, src);
+                n_tile = (columns_before(first_col) + col) * 8 + xcd - first_col;
+                if (!count_all) return true;
+            }
+            tiles += __builtin_amdgcn_readlane(incl, 63);
+            return false;
+        });
+    };
+    const bool shares = SHARES_K && p.part_sums != nullptr;
+    find_tile(slot, shares);
     /*
      * The memory gives every CU the same, so what is over when all CUs have the same number of tiles (`rest`, at the end) runs on
      * a few CUs, long after the others: 528 tiles of 7168 x 4096 on 256 CUs, 16 tiles alone for the last 30 of 168 us. W8A8: such
-     * tiles are shared along K by up to four workgroups each, which leave their int32 sums in memory; the last of them to get there
-     * adds the parts up and has the epilogue. Nobody waits for anybody. Layers with a shared expert, 32 experts of 7168 x 4096 / 2048 x
-     * 7168: 20 tokens 274 -> 257 us, 60 tokens 287 -> 273 (up to eight: 261, 275). The words and sums go past the L2s, which are the
+     * tiles are shared along K by three or four workgroups each, which leave their int32 sums in memory; the last of them to get there
+     * adds the parts up and has the epilogue. Nobody waits for anybody. The words and sums go past the L2s, which are the
      * XCDs' own. Integers add up to the same bits in any parts. fp8's scaled sums do not, and which tiles are over depends on the
      * whole batch's routing: there a token's bits would depend on the tokens beside it (37 tokens 264 -> 247 us, taken back).
      */
     int part_k = 0, parts = 1, piece = 0;
     int64_t part_rows = 0;
     if constexpr (SHARES_K) {
-        if (p.part_sums != nullptr) {
-            int tiles = 0;
-            walk([&](int, int, int, int, int, int mine) { tiles += __builtin_amdgcn_readlane(zb_wave_scan_dpp(mine), 63); return false; });
-            const int rest = tiles % p.part_cus, whole = tiles - rest;
-            if (rest > 0 && whole > 0 && slot >= whole) {
-                parts = p.part_cus / rest;
-                if (parts > KB / PF) parts = KB / PF;
-                if (parts > MAX_PARTS) parts = MAX_PARTS;
-                const int u = slot - whole;
-                part_k = u / rest;
+        const int rest = shares ? tiles % p.part_cus : 0, whole = tiles - rest;
+        if (rest > 0 && whole > 0 && slot >= whole) {
+            int n = p.part_cus / rest, rows = 0;
+            if (n > KB / PF) n = KB / PF;
+            if (n > MAX_PARTS) n = MAX_PARTS;
+            int before = 0;
+            walk([&](int, int l, int h, int m, int, int mine) {
+                const int incl = zb_wave_scan_dpp(mine), r = h - l;
+                int height = r;
+                if (m > 1) height = ((r + m - 1) / m + 15) & ~15;
+                const int top = __builtin_amdgcn_readfirstlane((int)zb_wave_reduce_dpp<true>(mine > 0 && before + incl > whole ? (float)height : 0.0f));
+                if (top > rows) rows = top;
+                before += __builtin_amdgcn_readlane(incl, 63);
+                return false;
+            });
+            part_rows = p.part_floats / (256 * rest * n);
+            if (rows <= part_rows && rows <= shared_rows(KB, rest)) {
+                parts = n;
+                part_k = (slot - whole) / rest;
                 if (part_k >= parts) return;
-                piece = u - part_k * rest;
-                slot = whole + piece;
-                part_rows = p.part_floats / (256 * rest * parts);
+                piece = slot - whole - part_k * rest;
+                if (part_k > 0) find_tile(whole + piece, false);
             }
         }
     }
-    int expert = -1, n_tile = 0, m_tile = 0, mt_e = 1, first_row = 0, end_row = 0, tiles = 0;
-    walk([&](int base, int l, int h, int m, int c0, int mine) {
-        const int incl = zb_wave_scan_dpp(mine);
-        const uint64_t past = __ballot(tiles + incl > slot);
-        if (past) {
-            const int src = __ffsll((long long)past) - 1;
-            expert = nth_expert(base + src);
-            mt_e = __builtin_amdgcn_readlane(m, src);
-            first_row = __builtin_amdgcn_readlane(l, src);
-            end_row = __builtin_amdgcn_readlane(h, src);
-            const int at = slot - tiles - __builtin_amdgcn_readlane(incl - mine, src), col = at / mt_e;
-            m_tile = at - col * mt_e;
-            const int first_col = __builtin_amdgcn_readlane(c0, src);
-            n_tile = (columns_before(first_col) + col) * 8 + xcd - first_col;
-            return true;
-        }
-        tiles += __builtin_amdgcn_readlane(incl, 63);
-        return false;
-    });
     if (expert < 0) return;
     const int part = SPLIT == 1 ? 0 : n_tile % SPLIT, chan = part * NW + wave;      /* which 32 of the tile's 256 channels are this wave's */
     n_tile /= SPLIT;
@@ -206,12 +232,6 @@ grouped_gemm_stream_kernel(GemmParams p)
     const int row_begin = first_row + m_tile * height;
     const int row_end = row_begin + height < end_row ? row_begin + height : end_row;
     const int last_rel = row_end - 1 - row_begin;
-    if constexpr (SHARES_K) {
-        if (parts > 1 && last_rel >= part_rows) {              /* no room for its sums */
-            if (part_k > 0) return;
-            parts = 1;
-        }
-    }
     /* slabs of this workgroup: whole chunks */
     const int kb_from = SHARES_K ? KB / PF * part_k / parts * PF : 0, kb_to = SHARES_K ? KB / PF * (part_k + 1) / parts * PF : KB;
 

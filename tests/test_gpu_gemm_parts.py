@@ -69,20 +69,26 @@ def tiles_of(rows, tall):
     """Heights of an expert's row tiles, as the kernel cuts them."""
     tm = 96 if tall else 64
     n = -(-rows // tm)
-    height = (-(-rows // n) + 15) & ~15
+    height = (-(-rows // max(n, 1)) + 15) & ~15
     return [min(height, rows - i * height) for i in range(n)]
 
 
-# W8A8, the last experts' rows and the room for a shared tile's. Workgroups per tile: four up to 8 tiles over, three of 9 and 10, two of
-# 11 to 16, one beyond (nothing is shared). Heights on either side of the room in one launch; an expert of two row tiles; a shared expert
-# (the first tile of all); `tall`: 48 rows per expert and more on average, the tile of 96 rows and two slabs in flight.
-@pytest.mark.parametrize("K,last,parts,room,tall,shared", [
-    (4608, [3] * 8, 4, 64, False, 0), (4608, [17] * 9, 3, 64, False, 0), (5120, list(range(8, 18)), 3, 13, False, 20),
-    (4608, [5, 64] * 5 + [16], 2, 40, False, 0), (5120, list(range(9, 25)), 2, 16, False, 64), (4608, [9] * 17, 1, 64, False, 0),
-    (4608, [100], 4, 40, False, 0), (4608, [1, 33], 4, 33, False, 64),
-    (4608, [96], 4, 96, True, 0), (5120, [81, 80, 96, 1], 4, 80, True, 70), (4608, [48, 96] * 5, 3, 90, True, 0),
-    (7168, [95, 64, 17] * 4, 2, 64, True, 96), (4608, [130, 20], 4, 70, True, 0)])
-def test_numbers_of_parts_and_heights_of_tiles(buf, K, last, parts, room, tall, shared):
+def rows_shared(K, rest):
+    """Rows up to which `rest` tiles are shared (shared_rows beside the kernel)."""
+    return 0 if rest > 10 else (K // 128 - 24) * (11 - rest) // 4
+
+
+# The last experts' rows and the room for a shared tile's. Workgroups per tile: four up to 8 tiles over, three of 9 and 10, none beyond.
+# All tiles are shared or none: heights on either side of the line, of the room, and one of them too tall; an expert of two row tiles; a
+# shared expert (the first tile of all); `tall`: 48 rows per expert and more on average, the tile of 96 rows and two slabs in flight.
+@pytest.mark.parametrize("K,last,room,tall,shared", [
+    (4608, [3] * 8, 64, False, 0), (4608, [9] * 8, 64, False, 0), (4608, [9] * 7 + [10], 64, False, 0), (5120, list(range(8)) + [8, 8], 8, False, 20),
+    (7168, [8] * 9 + [1], 24, False, 0), (7168, [9] * 10, 64, False, 0), (14336, [1] * 11, 64, False, 0), (4608, [1, 2], 1, False, 0),
+    (4608, [30], 30, False, 64), (4608, [31], 64, False, 64), (7168, [1, 64], 64, False, 64), (7168, [1, 64, 33], 48, False, 0),
+    (7168, [100], 64, False, 0), (14336, [5, 64] * 4, 64, False, 17),
+    (7168, [80], 80, True, 0), (7168, [81], 96, True, 0), (7168, [40, 96, 1], 96, True, 70), (14336, [96, 3, 95] * 2, 96, True, 96),
+    (14336, [20] * 9, 20, True, 0), (14336, [130, 20], 80, True, 0), (14336, [130, 20], 79, True, 0)])
+def test_numbers_of_parts_and_heights_of_tiles(buf, K, last, room, tall, shared):
     heights = [h for rows in last for h in tiles_of(rows, tall)]
     rest, N = len(heights), 2048
     cus = torch.cuda.get_device_properties(0).multi_processor_count // 8
@@ -90,7 +96,8 @@ def test_numbers_of_parts_and_heights_of_tiles(buf, K, last, parts, room, tall, 
     counts = rng(K + rest).integers(60, 97, first) if tall else rng(K + rest).integers(1, 20, first)
     counts = [int(c) for c in counts] + last
     E, R, I = len(counts), sum(counts), N // 2
-    assert parts == max(1, min(4, cus // rest)) and (R + shared > 48 * (E + bool(shared))) == tall and R + shared <= 87 * E
+    parts = min(4, cus // rest) if max(heights) <= min(room, rows_shared(K, rest)) else 0
+    assert (R + shared > 48 * (E + bool(shared))) == tall and R + shared <= 87 * E
     g = torch.Generator(device="cuda").manual_seed(rest)
     w = torch.randint(-128, 128, (E + 1, N, K), dtype=torch.int8, device="cuda", generator=g)
     a = torch.randint(-127, 128, (R + shared, K), dtype=torch.int8, device="cuda", generator=g)
@@ -98,7 +105,7 @@ def test_numbers_of_parts_and_heights_of_tiles(buf, K, last, parts, room, tall, 
     ws = torch.rand((E + 1, N), device="cuda", generator=g) * 0.003 + 0.0015
     off = row_off_dev(counts + [shared])
     along = SharedExpert(w[E].data_ptr(), ws[E].data_ptr(), shared, None)
-    scratch = torch.full((WORDS + 8 * rest * parts * room * 256,), float("nan"), device="cuda")
+    scratch = torch.full((WORDS + 8 * rest * min(4, cus // rest) * room * 256,), float("nan"), device="cuda")
 
     def run(share):
         q2, s2 = torch.zeros((R + shared, I), dtype=torch.int8, device="cuda"), torch.zeros((R + shared,), device="cuda")
@@ -114,6 +121,5 @@ def test_numbers_of_parts_and_heights_of_tiles(buf, K, last, parts, room, tall, 
     assert int((want_q2 != 0).any(dim=1).sum()) == R + shared
     for _ in range(2):
         got_q2, got_s2, arrived = run(True)
-        of_xcd = [parts if parts > 1 and h <= room else 0 for h in heights] + [0] * (cus - rest)
-        assert arrived.tolist() == of_xcd * 8 + [0] * (WORDS - 8 * cus)
+        assert arrived.tolist() == ([parts] * rest + [0] * (cus - rest)) * 8 + [0] * (WORDS - 8 * cus)
         assert torch.equal(got_q2, want_q2) and torch.equal(got_s2, want_s2)
