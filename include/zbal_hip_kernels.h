@@ -380,7 +380,7 @@ ZBALHIP_API int32_t zbalhip_gmm1_swiglu_quant_shared(const void *a, const float 
 /*
  * The same with memory for tiles that several workgroups share along K (W8A8 with few rows per expert): `parts_bytes`
  * at `parts`, 16-byte aligned, of which the first ZBALHIP_PART_WORDS 32-bit words are zero; null: no tile is shared. The more bytes,
- * the more rows a shared tile may have. shared may be null.
+ * the more rows shared tiles may have, up to what pays. The outputs are the same bits with and without. shared may be null.
  */
 #define ZBALHIP_PART_WORDS 512
 ZBALHIP_API int32_t zbalhip_gmm1_swiglu_quant_parts(const void *a, const float *a_scale, const void *w1, const void *w1scale,

@@ -176,7 +176,7 @@ extern "C" int32_t zbalhip_combine(const void *const *y, int32_t ranks, int32_t 
     src.rows_cap = y_rows;
     if (tokens == 0) return ZBALHIP_OK;
     /*
-     * Fewer tokens than four per CU: the rows are cut into pieces of at least half a chunk per lane of a full workgroup, so that a row is
+     * Fewer tokens than four for each of the 256 CUs: the rows are cut into pieces of at least half a chunk per lane of a full workgroup, so that a row is
      * not read in two or more passes by the few workgroups that there are. Where the line lay at two per CU -> four, the kernel alone: 300
      * tokens x 7168 9.55 -> 9.12 us, 512 14.7 -> 13.9, 900 24.4 -> 23.7, 400 x 4096 7.77 -> 7.54, 1021 15.4 -> 15.05; 512 and 1500 x 2048, 2000 x
      * 4096 the same. At eight per CU 1021 x 4096 16.0, 1500 x 2048 9.8 -> 10.6.

@@ -718,8 +718,8 @@ struct PermuteExtras {
 };
 
 /*
- * Fewer tokens than half of the CUs: up to eight workgroups, as many as make one per CU, share a token's picks. Each reads the row
- * and its scale for itself, but counts for its own picks and stores their rows only, and that is what a lone workgroup spends its
+ * Fewer tokens than half of the CUs: up to eight workgroups, as many as make one for each of the 256 CUs, share a token's picks. Each reads
+ * the row and its scale for itself, but counts for its own picks and stores their rows only, and that is what a lone workgroup spends its
  * time on (one token of 8 picks, 7168 wide, int8: 1.5 us of 4.5 each, a CU storing 50 GB/s). The kernel alone: 1 token 5.31 -> 3.68 us,
  * 7 tokens 5.53 -> 3.83 (rows as they are 5.05 -> 3.31), 32 of 4096, 128 experts 5.29 -> 3.75, 64 of 7168 5.94 -> 4.80, of 2048 4.64 -> 3.40,
  * 128 6.58 -> 6.33; two per CU: 64 tokens 6.37, 128 6.96, 512 12.6 -> 15.5.

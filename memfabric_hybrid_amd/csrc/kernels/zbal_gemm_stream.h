@@ -94,7 +94,7 @@ template <int MODE, bool GMM1, int SPLIT> constexpr bool stream_shares_k() { ret
  *     -3 ... +1 / +2 / +5 ... +11 / +8 ... +16; 10 -7 ... -1 / -4 ... 0 / 0 ... +1 / +4 ... +9 / +6 ... +15;
  *   - K 7168: rest 1 -18 ... -5 / -15 ... -4 / -11 ... -3 / -6 ... -2 / -2 ... +1; 4 -16 ... -4 / -13 ... -3 / -10 ... -2 / -4 ... -1 / 0 ... +1; 8 -12 ... -3 /
  *     -9 ... -2 / -5 ... 0 / +1 ... +3 / +3 ... +7; 10 -9 ... -2 / -7 ... -1 / -4 ... 0 / +1 ... +2 / +2 ... +6;
- *   - K 14336: rest 1 -20 ... -6 / ... / -12 ... -4; 10 -10 ... -2 / ... / -4 ... -1.
+ *   - K 14336: rest 1 -20 ... -6 / ... / -12 ... -4; 10 -10 ... -2 / ... / -4 ... 0.
  * Beyond ten tiles (two parts each) 0 ... +10. Where only some of the tiles were shared the others were still the last to end: +2 ... +8.
  */
 __host__ __device__ inline int shared_rows(int slabs, int rest) { return rest > 10 ? 0 : (slabs - 24) * (11 - rest) / 4; }
